@@ -64,7 +64,7 @@ SHAPES = {0: (4, 64, 5), 1: (4, 64, 9), 2: (16, 16, 5), 3: (8, 32, 9), 4: (8, 32
           5: (8, 64, 5), 6: (4, 32, 9), 7: (2, 64, 5),
           8: (1, 64, 5), 9: (2, 32, 9), 10: (16, 16, 9), 11: (8, 64, 9), 12: (1, 64, 9)}
 PROF_SLOTS = 39
-# pass programs 0..9; filter_gc_first is gc_first preceded by the previous
+# pass programs 0..9 (7 and 8 are never launched); filter_gc_first is gc_first preceded by the previous
 # stage's x filter sweep (rk3 steps with filter fusion, the default)
 PASS_NAMES = ["gc_first", "gc_mid", "gc_last", "visc_mid", "visc_last_rhs",
               "visc_last_rk3_filter", "filter", "gc_last_grad", "gc_last_conv",
@@ -368,7 +368,7 @@ class Flow:
         """{(pass_name, dir): (shape, minb, tuned_ms)} of the passes this case launches."""
         nd = 3 if self.cfg.km > 0 else 2
         used = {0: [0], 1: list(range(1, nd - 1)), 2: [nd - 1], 3: list(range(nd - 1)),
-                4: [nd - 1], 5: [nd - 1], 6: list(range(nd)), 7: [nd - 1], 8: [nd - 1]}
+                4: [nd - 1], 5: [nd - 1], 6: list(range(nd))}
         if self.cfg.semantics != SEM_MAIN:
             used[9] = [0]
         out = {}

@@ -380,7 +380,7 @@ size_t pass_lds_bytes(int shape, int prog) {
   const ShapeInfo& s = kShapes[shape];
   const long long tl = (long long)s.TL * line_stride(s.P, s.R, s.TL);
   const long long one = (2 * tl > 2 * s.NT ? 2 * tl : 2 * s.NT) + kLineOff + 8 + kHaloSlot +
-                        coef_regions(prog) * 2 * s.P * s.R;
+                        coef_regions(prog) * 2 * s.P * s.R + halo_prims(prog, s.TL, true);
   return (size_t)one * sizeof(double);
 }
 
@@ -437,8 +437,8 @@ hipError_t launch_pass(int shape, int prog, int minb, const FlowArgs& a, int dir
 }
 
 // register budget a pass uses until tuned: two workgroups per CU for the
-// gradient/convective passes, one for the others
-int default_minb(int prog) { return prog <= GC_LAST || prog >= GL_GRAD ? 2 : 1; }
+// gradient passes, one for the others
+int default_minb(int prog) { return prog <= GC_LAST || prog == FGC_FIRST ? 2 : 1; }
 
 }  // namespace
 
@@ -453,8 +453,8 @@ struct astr_hip_ctx {
   int shape[kNumProgs][3];
   int minb[kNumProgs][3];
   float tuned_ms[kNumProgs][3];
-  // the last direction's gradient/convective work in two kernels
-  // (GL_GRAD + GL_CONV) instead of GC_LAST; chosen by the autotuner
+  // set and read back by astr_hip_set/get_last_split; the last gradient pass
+  // has one form
   int split_last = 0;
   // rk3_run: each stage's x filter sweep runs in the next stage's first pass
   // (FGC_FIRST) inside one call (fuse_fx, off unless the autotuner finds the
@@ -707,22 +707,15 @@ int pass(astr_hip_ctx* c, int prog, int d, int shape = -1) {
   return 0;
 }
 
-// stats: 0 none, 1 KE/enstrophy, 2 also the dissipation rate
+// stats: the KE/enstrophy partial sums of the current state
 // diss_out (device, nullable): the dissipation rate of the current state,
-// evaluated after the gradient passes (which then store every gradient) and
-// before the viscous passes update q
-int run_rhs(astr_hip_ctx* c, bool rk, bool stats, bool store_last_grad, double* diss_out = nullptr) {
+// evaluated after the gradient passes and before the last pass updates q
+int run_rhs(astr_hip_ctx* c, bool rk, bool stats, double* diss_out = nullptr) {
   FlowArgs& a = c->a;
   const int nd = a.ndir;
-  a.dostats = stats ? 1 : 0;
-  // the shock sensor reads the whole velocity gradient
+  // the shock sensor reads the velocity gradient
   const bool sensor = a.uwd && c->uw.sensor;
-  a.store_last_grad = store_last_grad || diss_out || sensor ? 1 : 0;
   for (int d = 0; d < nd; d++) {
-    if (d == nd - 1 && c->split_last) {
-      if (pass(c, GL_GRAD, d) || (!a.uwd && pass(c, GL_CONV, d))) return -1;
-      continue;
-    }
     const int prog = d == nd - 1 ? GC_LAST : (d == 0 ? (c->fx_pending ? FGC_FIRST : GC_FIRST) : GC_MID);
     if (pass(c, prog, d)) return -1;
     if (d == 0) c->fx_pending = false;
@@ -746,10 +739,12 @@ int run_rhs(astr_hip_ctx* c, bool rk, bool stats, bool store_last_grad, double* 
     hipLaunchKernelGGL(k_diss_sum, dim3(1), dim3(256), 0, c->stream, c->diss_part, nb, diss_out, c->ke_scale);
     HIP_OK(hipGetLastError());
   }
-  a.dostats = 0;
   for (int d = 0; d < nd; d++) {
     const int prog = d == nd - 1 ? (rk ? V_LAST_RK : V_LAST_RHS) : V_MID;
-    if (pass(c, prog, d)) return -1;
+    a.dostats = stats && d == 0 ? 1 : 0;  // the stress pass, along x, sums them
+    const int rc = pass(c, prog, d);
+    a.dostats = 0;
+    if (rc) return -1;
   }
   return 0;
 }
@@ -1147,8 +1142,7 @@ int rk3_run(astr_hip_ctx* c, int nsteps, const StatsBufs& sb, double* ke, double
   double* const diss_keep = c->diss_part;
   a.stats = sb.part;
   c->diss_part = sb.diss;
-  const int stats_prog = c->split_last ? GL_GRAD : GC_LAST;
-  const int ntl = tiles_of(a.n, a.ndir - 1, kShapes[c->shape[stats_prog][a.ndir - 1]].TL);
+  const int ntl = tiles_of(a.n, 0, kShapes[c->shape[V_MID][0]].TL);
   int rc = 0;
   // main path: the last direction's filter sweep of this stage was applied by
   // the previous stage's RK pass (a.rk_filter)
@@ -1170,7 +1164,7 @@ int rk3_run(astr_hip_ctx* c, int nsteps, const StatsBufs& sb, double* ke, double
         if (rc) break;
       }
       a.rk_filter = a.main_sem && c->fuse_main_filter && !(it == nsteps - 1 && s == 2) ? 1 : 0;
-      const int rhs_rc = run_rhs(c, true, want && s == 0, false,
+      const int rhs_rc = run_rhs(c, true, want && s == 0,
                                  diss && s == 0 ? sb.out + kStepStats * it + 2 : nullptr);
       last_filtered = a.rk_filter != 0;
       a.rk_filter = 0;
@@ -1253,6 +1247,7 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   a.const2 = g * ma * ma;
   a.const5 = (g - 1.0) * ma * ma;
   a.const6 = 1.0 / (g - 1.0);
+  a.p0 = 1.0 / a.const2;
   a.reynolds = cfg->reynolds;
   a.prandtl = cfg->prandtl;
   a.suth = cfg->sutherland / cfg->ref_tem;
@@ -1282,8 +1277,9 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
       c->tuned_ms[pr][d] = 0.f;
     }
   }
-  // fields: q 5, qsave 5, qrhs 5, dv 12, sg 9; main path: primitives 6
-  const long long nfield = a.main_sem ? 42 : 36;
+  // fields: q 5, qsave 5, qrhs 5, dv 12, sg 9; then the miniapp's pressure or
+  // the main path's primitives 6
+  const long long nfield = a.main_sem ? 42 : 37;
   size_t bytes = (size_t)(nfield * a.fs) * sizeof(double);
   if (hipMalloc(&c->base, bytes) != hipSuccess) { delete c; return fail("hipMalloc of fields failed"); }
   (void)hipMemset(c->base, 0, bytes);
@@ -1293,6 +1289,7 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   a.dv = a.qrhs + 5 * a.fs;
   a.sg = a.dv + 12 * a.fs;
   a.pr = a.main_sem ? a.sg + 9 * a.fs : nullptr;
+  a.p = a.main_sem ? nullptr : a.sg + 9 * a.fs;
   if (a.main_sem) {
     // halo sources kept by qswap: hx then hy, 5 fields each
     a.hxs = hx_lines(a.n, a.ndir) * kHaloSrcRows;
@@ -1315,7 +1312,7 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   // (then the dissipation rate's block partials)
   int tl_min = 32;
   for (const ShapeInfo& s : kShapes) tl_min = std::min(tl_min, s.TL);
-  const int ntl = tiles_of(a.n, a.ndir - 1, tl_min);
+  const int ntl = tiles_of(a.n, 0, tl_min);
   if (hipMalloc(&c->stats_part, (kTileStats * (size_t)ntl + kDissBlocks) * sizeof(double)) != hipSuccess) {
     (void)hipFree(c->base); (void)hipFree(c->coef); if (c->halo) (void)hipFree(c->halo); delete c;
     return fail("hipMalloc of stats failed");
@@ -1573,7 +1570,7 @@ int astr_hip_filterq(astr_hip_ctx* c) {
 
 int astr_hip_gradcal(astr_hip_ctx* c, double* dvel, double* dtmp) {
   if (check_ctx(c)) return -1;
-  if (ensure_halo(c) || run_rhs(c, false, false, true)) return -1;
+  if (ensure_halo(c) || run_rhs(c, false, false)) return -1;
   if (dvel && xfer(c, dvel, 9, c->a.dv, 0, 0)) return -1;
   if (dtmp && xfer(c, dtmp, 3, c->a.dv + 9 * c->a.fs, 0, 0)) return -1;
   return 0;
@@ -1581,7 +1578,7 @@ int astr_hip_gradcal(astr_hip_ctx* c, double* dvel, double* dtmp) {
 
 int astr_hip_rhscal(astr_hip_ctx* c, double* qrhs) {
   if (check_ctx(c)) return -1;
-  if (ensure_halo(c) || run_rhs(c, false, false, true)) return -1;
+  if (ensure_halo(c) || run_rhs(c, false, false)) return -1;
   if (qrhs && xfer(c, qrhs, 5, c->a.qrhs, 0, 0)) return -1;
   return 0;
 }
@@ -1614,8 +1611,7 @@ int astr_hip_rk3_steps_stats_noalloc(astr_hip_ctx* c, int nsteps, double* ke, do
   if (nsteps < 0) return fail("negative step count");
   if (!c->scratch) return fail("no scratch buffer on this device: " + c->scratch_err);
   const FlowArgs& a = c->a;
-  const int stats_prog = c->split_last ? GL_GRAD : GC_LAST;
-  const long long ntl = tiles_of(a.n, a.ndir - 1, kShapes[c->shape[stats_prog][a.ndir - 1]].TL);
+  const long long ntl = tiles_of(a.n, 0, kShapes[c->shape[V_MID][0]].TL);
   const long long need = kTileStats * ntl + kDissBlocks + kStepStats * (long long)std::max(nsteps, 1);
   if (need > kScratchDoubles)
     return fail("astr_hip_rk3_steps_stats_noalloc: " + std::to_string(need) +
@@ -1682,9 +1678,9 @@ static bool pass_used(int prog, int d, int nd) {
     case GC_FIRST:
     case FGC_FIRST: return d == 0;
     case GC_MID: return d > 0 && d < nd - 1;
-    case GC_LAST:
-    case GL_GRAD:
-    case GL_CONV: return d == nd - 1;
+    case GC_LAST: return d == nd - 1;
+    case RESERVED_7:
+    case RESERVED_8: return false;
     case V_MID: return d < nd - 1;
     case V_LAST_RHS:
     case V_LAST_RK: return d == nd - 1;
@@ -1715,7 +1711,6 @@ int astr_hip_autotune(astr_hip_ctx* c, int reps) {
   a.stage = 0;
   a.rk_a = 1.0; a.rk_b = 0.0; a.rk_c = 1.0;
   a.dostats = 0;
-  a.store_last_grad = 0;
   // the main path's RK pass is timed with the filter sweep it carries in
   // rk3 steps
   a.rk_filter = a.main_sem && c->fuse_main_filter ? 1 : 0;
@@ -1750,26 +1745,6 @@ int astr_hip_autotune(astr_hip_ctx* c, int reps) {
     }
   }
   if (!rc) {
-    // the fused and the split last gradient pass, each timed inside whole
-    // right-hand sides with the selections above (in a step the split form's
-    // second kernel finds the first one's data in cache, which the per-pass
-    // timings do not see)
-    float form_ms[2] = {0.f, 0.f};
-    for (int sp = 0; sp < 2 && !rc; sp++) {
-      c->split_last = sp;
-      if (run_rhs(c, false, false, false)) {
-        rc = -1;
-        break;
-      }
-      hipError_t e = hipEventRecord(e0, c->stream);
-      for (int r = 0; r < reps && e == hipSuccess; r++)
-        if (run_rhs(c, false, false, false)) e = hipErrorUnknown;
-      if (e == hipSuccess) e = hipEventRecord(e1, c->stream);
-      if (e == hipSuccess) e = hipEventSynchronize(e1);
-      if (e == hipSuccess) e = hipEventElapsedTime(&form_ms[sp], e0, e1);
-      if (e != hipSuccess) rc = fail(std::string("autotune rhs: ") + hipGetErrorString(e));
-    }
-    if (!rc) c->split_last = form_ms[1] < form_ms[0];
     // the filtering first pass against the first pass plus the x filter pass
     if (!rc && !a.main_sem)
       c->fuse_fx = c->tuned_ms[FGC_FIRST][0] < c->tuned_ms[GC_FIRST][0] + c->tuned_ms[F_ONLY][0];
@@ -2189,6 +2164,7 @@ int slot_prog(int kind, int d, int nd) {
 }
 const int kSlotKind[8] = {0, 0, 0, 1, 1, 1, 2, 2};
 const int kSlotDir[8] = {0, 1, 2, 0, 1, 2, 1, 0};
+constexpr int kSlotStats = 3;  // V x, which sums the statistics
 
 struct BatchGroup {
   int slot, prog, dir, shape, minb, nblocks;
@@ -2315,9 +2291,8 @@ int upload_jobs(astr_hip_batch* b) {
   std::vector<StatsJob> jobs(nc);
   for (int i = 0; i < nc; i++) {
     astr_hip_ctx* c = b->cases[i];
-    const int nd = c->a.ndir;
     jobs[i].part = c->stats_part;
-    jobs[i].ntiles = tiles_of(c->a.n, nd - 1, kShapes[c->shape[GC_LAST][nd - 1]].TL);
+    jobs[i].ntiles = tiles_of(c->a.n, 0, kShapes[c->shape[V_MID][0]].TL);
     jobs[i].scale = c->ke_scale;
     jobs[i].out = b->d_stats + kBatchStats * (size_t)i * b->stats_cap;
   }
@@ -2329,16 +2304,16 @@ int upload_jobs(astr_hip_batch* b) {
 int enqueue_step(astr_hip_batch* b) {
   static const double rk[3][3] = {{1.0, 0.0, 1.0}, {0.75, 0.25, 0.25}, {1.0 / 3.0, 2.0 / 3.0, 2.0 / 3.0}};
   for (int s = 0; s < 3; s++) {
-    StageArgs sa{s, s == 0 ? 1 : 0, 0, rk[s][0], rk[s][1], rk[s][2]};
+    StageArgs sa{s, s == 0 ? 1 : 0, rk[s][0], rk[s][1], rk[s][2]};
     StageArgs sv = sa;
     sv.dostats = 0;
     for (int sl = 0; sl < 8; sl++) {
       for (auto& g : b->groups) {
         if (g.slot != sl) continue;
-        HIP_OK(launch_batch(g.shape, g.prog, g.minb, g.bl, g.dir, g.prog == GC_LAST ? sa : sv,
-                            g.nblocks, b->stream));
+        HIP_OK(launch_batch(g.shape, g.prog, g.minb, g.bl, g.dir, sl == kSlotStats ? sa : sv, g.nblocks,
+                            b->stream));
       }
-      if (sl == 2 && s == 0) {
+      if (sl == kSlotStats && s == 0) {
         hipLaunchKernelGGL(k_stats_batch, dim3((unsigned)b->cases.size()), dim3(256), 0, b->stream,
                            b->d_jobs, b->d_step);
         HIP_OK(hipGetLastError());
@@ -2499,7 +2474,7 @@ int astr_hip_batch_autotune(astr_hip_batch* b, int reps) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (!rc && (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess))
     rc = fail("hipEventCreate failed");
-  const StageArgs sa{0, 0, 0, 1.0, 0.0, 1.0};
+  const StageArgs sa{0, 0, 1.0, 0.0, 1.0};
   for (int sl = 0; sl < 8 && !rc; sl++) {
     const int kind = kSlotKind[sl], d = kSlotDir[sl];
     // classes: cases of this slot with the same program and the same set of

@@ -23,18 +23,20 @@ struct FlowArgs {
   long long fs;         // doubles between fields
   double inv_d[3];      // 1/dx, 1/dy, 1/dz
   double const2, const5, const6;
+  double p0;            // the reference state's pressure, 1/const2
   double reynolds, prandtl, suth, suth1;
   double rk_a, rk_b, rk_c, dt;
   int trash;            // a point index inside every field's padding
   double alfa, bhalo;   // filter alpha and halo-row beta (LHS of the filter rows)
   int stage;            // 0,1,2
   int dostats;          // stage-1 KE/enstrophy partial sums (1) or none (0)
-  int store_last_grad;  // last GC pass also stores its gradients
   double* q;            // 5 fields
   double* qsave;        // 5 fields
   double* qrhs;         // 5 fields
   double* dv;           // 12 fields: dvel(m,d) at m+3d, dtmp(d) at 9+d
   double* sg;           // 9 fields: sigma 11,12,13,22,23,33, qflux 1,2,3
+  double* p;            // the pressure of q (miniapp; written by the first
+                        // gradient pass, read by the passes that follow)
   double* stats;        // 2 doubles per tile
   const double* dac[3]; // derivative LU tables [ac1|ac2|ac3] per direction
   const double* fac[3]; // filter LU tables
@@ -91,15 +93,23 @@ __host__ __device__ inline int halo_src_index(const int n[3], int ndir, int dir,
   return -1;
 }
 
-// Pass programs.  GL_GRAD + GL_CONV are GC_LAST split in two kernels (the
-// gradient/stress half and the convective half), each with fewer registers.
-// FGC_FIRST is GC_FIRST preceded by the previous stage's filter sweep along
-// the same lines (x): it filters the q it loads, writes it back and goes on
-// with the filtered values (the sweeps along different indices commute, so
-// the x sweep may come last).
-enum Prog { GC_FIRST = 0, GC_MID, GC_LAST, V_MID, V_LAST_RHS, V_LAST_RK, F_ONLY, GL_GRAD, GL_CONV,
-            FGC_FIRST };
-constexpr int kNumProgs = 10;
+// Pass programs.  Per stage: the gradients of u, v, w and T along x, y, z
+// (GC_FIRST, GC_MID, GC_LAST), then per direction the derivative of the whole
+// flux, viscous minus convective (V_MID along x and y, V_LAST_RHS or
+// V_LAST_RK along the last direction).  Taking the two fluxes' difference
+// before the line solve leaves 5 solves per direction where separate
+// derivatives take 9, and qrhs is accumulated once per direction.
+//   V_MID along x (kernel V_FIRST) also forms the stress and heat flux, and
+//   the statistics, from the stored gradients;
+//   FGC_FIRST is GC_FIRST preceded by the previous stage's filter sweep along
+//   the same lines (x): it filters the q it loads, writes it back and goes on
+//   with the filtered values (the sweeps along different indices commute, so
+//   the x sweep may come last).
+// Ids 7 and 8 were the halves of a split last gradient pass; they stay
+// reserved so that the ids of the launch selection keep their meaning.
+enum Prog { GC_FIRST = 0, GC_MID, GC_LAST, V_MID, V_LAST_RHS, V_LAST_RK, F_ONLY, RESERVED_7, RESERVED_8,
+            FGC_FIRST, V_FIRST };
+constexpr int kNumProgs = 10;  // V_FIRST is V_MID's kernel along x, no id of its own
 
 // ntiles of direction dir for lines-per-tile TL
 __host__ __device__ inline int tiles_of(const int n[3], int dir, int TL) {
@@ -177,17 +187,18 @@ template <class C>
 constexpr int lds_coef_offset() {
   return lds_line_doubles<C>() + kHaloSlot;
 }
-// Regions of 2 P R doubles a pass stages: one (the derivative's) in the last
-// gradient pass and the viscous passes, one (the filter's) in the filter
-// pass and in the filtering first gradient pass, two in the RK pass, none in the first two gradient passes, which
-// keep the factors in registers (there the freed registers would not reach
-// another wave per SIMD, and the reloads only cost time).
-constexpr int coef_regions(int prog) {
-  return prog == V_LAST_RK ? 2 : (prog == GC_FIRST || prog == GC_MID ? 0 : 1);
+// Regions of 2 P R doubles a pass stages: two (the derivative's and the
+// filter's) in the RK pass and the filtering first gradient pass, one in the
+// others.
+constexpr int coef_regions(int prog) { return prog == V_LAST_RK || prog == FGC_FIRST ? 2 : 1; }
+// Main path, gradient passes: the primitives u, v, w, T of the halo copies
+// (kHaloSrcRows per line), evaluated once by the slots that own them.
+constexpr int halo_prims(int prog, int TL, bool main_sem) {
+  return main_sem && prog <= GC_LAST ? 4 * kHaloSrcRows * TL : 0;
 }
 template <class C>
-constexpr int lds_doubles(int prog) {
-  return lds_coef_offset<C>() + coef_regions(prog) * 2 * C::P * C::R;
+constexpr int lds_doubles(int prog, bool main_sem = false) {
+  return lds_coef_offset<C>() + coef_regions(prog) * 2 * C::P * C::R + halo_prims(prog, C::TL, main_sem);
 }
 
 // Stage the chunk factors of a line of M rows into coefficient region `region`
@@ -360,10 +371,9 @@ __device__ __forceinline__ Prim prim_of(const FlowArgs& a, double q1, double q2,
 
 // convective flux component m along dir (tgvsolver.F90:559-564, 586-591,
 // 613-618) from q_m, the velocity along dir and p
-__device__ __forceinline__ double conv_flux(int m, int dir, double qm, double q5, double uu,
-                                            double p) {
+__device__ __forceinline__ double conv_flux(int m, int dir, double qm, double uu, double p) {
 #pragma clang fp contract(off)
-  if (m == 4) return (q5 + p) * uu;
+  if (m == 4) return (qm + p) * uu;
   double f = qm * uu;
   if (m == dir + 1) f = f + p;
   return f;
@@ -378,12 +388,11 @@ __device__ __forceinline__ double miucal(const FlowArgs& a, double t) {
 struct StageArgs {
   int stage;            // 0,1,2
   int dostats;          // stage-1 KE/enstrophy partial sums (1) or none (0)
-  int store_last_grad;  // last GC pass also stores its gradients
   double rk_a, rk_b, rk_c;
 };
 
 __device__ __forceinline__ StageArgs stage_of(const FlowArgs& a) {
-  return StageArgs{a.stage, a.dostats, a.store_last_grad, a.rk_a, a.rk_b, a.rk_c};
+  return StageArgs{a.stage, a.dostats, a.rk_a, a.rk_b, a.rk_c};
 }
 
 // q <- a*qsave + b*q + c*qrhs*dt in the reference's order (tgvsolver.F90:1055-1057)
@@ -423,11 +432,11 @@ __device__ __forceinline__ void visc_flux(const FlowArgs& a, const double g[3][3
 // U = sum_n dxi(dir,n) u_n, for the metrics of a uniform Cartesian grid
 // (dxi(dir,n) = 0 for n != dir, so those products add exact zeros)
 __device__ __forceinline__ double conv_flux_main(double jac, double dx, int m, int dir, double qm,
-                                                 double q5, double ud, double p) {
+                                                 double ud, double p) {
 #pragma clang fp contract(off)
   const double uu = dx * ud;
   if (m == 0) return jac * qm * uu;
-  if (m == 4) return jac * (q5 + p) * uu;
+  if (m == 4) return jac * (qm + p) * uu;
   if (m == dir + 1) return jac * (qm * uu + dx * p);
   return jac * (qm * uu);
 }
@@ -458,53 +467,39 @@ __device__ __forceinline__ double jac_of(const FlowArgs& a, unsigned g) {
 
 // convrsdcal6 (src/solver.F90:2196-2207) with the full metric row:
 // U = dxi(d,1) u + dxi(d,2) v + dxi(d,3) w, F_m = J (q_m U + dxi(d,m) p)
-__device__ __forceinline__ double conv_flux_full(const MetRow& M, int m, double qm, double q5,
-                                                 double u, double v, double w, double p) {
+__device__ __forceinline__ double conv_flux_full(const MetRow& M, int m, double qm, double u,
+                                                 double v, double w, double p) {
 #pragma clang fp contract(off)
   const double uu = M.r[0] * u + M.r[1] * v + M.r[2] * w;
   if (m == 0) return M.j * qm * uu;
-  if (m == 4) return M.j * (q5 + p) * uu;
+  if (m == 4) return M.j * (qm + p) * uu;
   return M.j * (qm * uu + M.r[m - 1] * p);
 }
 
 // diffrsdcal6 (src/solver.F90:2623-2635) with the full metric row: column
 // c of direction dir, (s_c1 dxi(d,1) + s_c2 dxi(d,2) + s_c3 dxi(d,3)) J with
 // s_c = the stress row c (c < 3) or the heat flux (c = 3)
-__device__ __forceinline__ double visc_col_full(const FlowArgs& a, int dir, int c, unsigned g) {
+__device__ __forceinline__ double visc_col_row(const MetRow& M, double s0, double s1, double s2) {
 #pragma clang fp contract(off)
-  const MetRow M = met_row(a, dir, g);
-  const int k0 = c == 0 ? 0 : (c == 1 ? 1 : (c == 2 ? 2 : 6));
-  const int k1 = c == 0 ? 1 : (c == 1 ? 3 : (c == 2 ? 4 : 7));
-  const int k2 = c == 0 ? 2 : (c == 1 ? 4 : (c == 2 ? 5 : 8));
-  const double s0 = ldg(a.sg + k0 * a.fs, g), s1 = ldg(a.sg + k1 * a.fs, g), s2 = ldg(a.sg + k2 * a.fs, g);
   return (s0 * M.r[0] + s1 * M.r[1] + s2 * M.r[2]) * M.j;
 }
-
-// element m of a 5-vector by selects: in a loop over m that the compiler
-// keeps rolled, indexing a register array by m would move the array to
-// scratch memory
-__device__ __forceinline__ double pick5(double a0, double a1, double a2, double a3, double a4, int m) {
-  return m == 0 ? a0 : (m == 1 ? a1 : (m == 2 ? a2 : (m == 3 ? a3 : a4)));
+__device__ __forceinline__ int visc_term(int c, int i) {
+  const int k[4][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}, {6, 7, 8}};
+  return k[c][i];
 }
-#define ASTR_QV(m, t) pick5(qv[0][t], qv[1][t], qv[2][t], qv[3][t], qv[4][t], (m))
-#define ASTR_QH(m) pick5(qh[0], qh[1], qh[2], qh[3], qh[4], (m))
+__device__ __forceinline__ double visc_col_full(const FlowArgs& a, int dir, int c, unsigned g) {
+  return visc_col_row(met_row(a, dir, g), ldg(a.sg + visc_term(c, 0) * a.fs, g),
+                      ldg(a.sg + visc_term(c, 1) * a.fs, g), ldg(a.sg + visc_term(c, 2) * a.fs, g));
+}
 
-// Main path: q of the halo copy of slot t.  qswap fills the halo of a line
-// from the filtered q; the lines on boundary planes that a later qswap step
-// averages take the values kept before that step (hx / hy), the others the
-// current q of the source point, which the slot holds.
+// Main path: component m of q of the halo copy of slot t.  qswap fills the
+// halo of a line from the filtered q; the lines on boundary planes that a
+// later qswap step averages take the values kept before that step (hx / hy),
+// the others the current q of the source point, which the slot owns.
 template <class C>
-__device__ __forceinline__ void halo_q(const FlowArgs& a, const Slots<C>& S, int t, int dir,
-                                       const double (&qv)[5][C::NPT], double (&qh)[5]) {
-  if (S.ex[t] >= 0) {
-    const double* src = dir == 0 ? a.hx : a.hy;
-    const long long st = dir == 0 ? a.hxs : a.hys;
-#pragma unroll
-    for (int m = 0; m < 5; m++) qh[m] = src[m * st + S.ex[t]];
-  } else {
-#pragma unroll
-    for (int m = 0; m < 5; m++) qh[m] = qv[m][t];
-  }
+__device__ __forceinline__ double halo_q(const FlowArgs& a, const Slots<C>& S, int t, int dir, int m) {
+  if (S.ex[t] >= 0) return (dir == 0 ? a.hx + m * a.hxs : a.hy + m * a.hys)[S.ex[t]];
+  return ldg(a.q + m * a.fs, S.g[t]);
 }
 
 // main path RK3 update (src/mainloop.F90:441-449):
@@ -518,6 +513,27 @@ __device__ __forceinline__ double rk_update_main(const StageArgs& sa, double dt,
 // ---------------------------------------------------------------------------
 // the pass kernel
 // ---------------------------------------------------------------------------
+// stress and heat flux of a point from its stored gradients (diffusion,
+// tgvsolver.F90:659-694) and its terms of the statistics (stacal, :893-942)
+__device__ __forceinline__ void stress_point(const FlowArgs& a, unsigned o, const Prim& P, double f[9],
+                                             bool stats, double& sk, double& se) {
+  double g[3][3], gt[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+#pragma unroll
+    for (int m = 0; m < 3; m++) g[m][d] = d < a.ndir ? ldg(a.dv + (m + 3 * d) * a.fs, o) : 0.0;
+    gt[d] = d < a.ndir ? ldg(a.dv + (9 + d) * a.fs, o) : 0.0;
+  }
+  visc_flux(a, g, gt, P, f);
+  if (stats) {
+    sk += P.r * (P.u * P.u + P.v * P.v + P.w * P.w);
+    const double o1 = g[2][1] - g[1][2];
+    const double o2 = g[0][2] - g[2][0];
+    const double o3 = g[1][0] - g[0][1];
+    se += P.r * (o1 * o1 + o2 * o2 + o3 * o3);
+  }
+}
+
 // MINB: workgroups per CU the register allocation is held to (each
 // workgroup puts one wave on each SIMD, so MINB waves per SIMD)
 // One tile of one pass.  `a` describes the case, `sa` the stage.
@@ -526,6 +542,9 @@ __device__ __forceinline__ double rk_update_main(const StageArgs& sa, double dt,
 // and their halo copies from the filtered q (qswap), the fluxes carry the
 // metrics J and dxi (convrsdcal6, diffrsdcal6), and the RK pass ends with
 // updatefvar instead of the filter.
+// Each pass reads its chunk factors back from LDS before each solve instead
+// of holding them in registers, and issues a solve's accumulation loads and
+// the next solve's inputs before it, so that their latency overlaps it.
 template <class C, int PROG, bool MAIN = false, bool GEN = false>
 __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa, int dir, int tile,
                                           double* smem) {
@@ -543,131 +562,81 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
   const double idn = a.inv_d[dir];
   const long long fs = a.fs;
 
-  if constexpr (PROG == GC_FIRST || PROG == FGC_FIRST || PROG == GC_MID || PROG == GC_LAST ||
-                PROG == GL_GRAD || PROG == GL_CONV) {
-    constexpr bool FIRST = PROG == GC_FIRST || PROG == FGC_FIRST;
-    constexpr bool LAST = PROG == GC_LAST || PROG == GL_GRAD || PROG == GL_CONV;
-    constexpr bool DO_GRAD = PROG != GL_CONV;
-    constexpr bool DO_CONV = PROG != GL_GRAD;
-    // the last pass, which holds the most registers, reads the chunk factors
-    // back from LDS before each solve; the others keep them in registers
-    ChunkCoef<C::R, false> CDr;
-    const double* cs = nullptr;
-    if constexpr (LAST) cs = stage_chunk_coefs<C>(a.dac[dir], n + 3, smem, 0);
-    else load_chunk_coef<C::R, false>(CDr, a.dac[dir], n + 3, p * C::R);
-    double qv[5][NPT];
-#pragma unroll
-    for (int t = 0; t < NPT; t++)
-#pragma unroll
-      for (int m = 0; m < 5; m++) qv[m][t] = ldg(a.q + m * fs, S.g[t]);
-    if constexpr (PROG == FGC_FIRST) {
-      // the previous stage's filter sweep along these lines (filterq,
-      // tgvsolver.F90:805-825), as the filter pass does it, on the loaded q;
-      // the filtered q is stored and the gradients and fluxes below take it
-      const double* csf = stage_chunk_coefs<C>(a.fac[dir], n + 7, smem, 0);
-      const double c3l = a.fac[dir][2 * (n + 7) + (n + 7) - 1];
-      const FilterCoef fl = stage_halo_coefs<C>(a.fc, smem);
-#pragma unroll
-      for (int m = 0; m < 5; m++) {
-#pragma unroll
-        for (int t = 0; t < NPT; t++) put<C>(T, S, t, qv[m][t]);
-        __syncthreads();
-        {
-          ChunkCoef<C::R, true> CF;
-          lds_chunk_coef_f<C>(CF, csf, p * C::R, n + 7, c3l);
-          solve_line<C::P, C::R, true>(Tl, Xl, n, p, CF, fl);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int t = 0; t < NPT; t++) {
-          qv[m][t] = X[S.s[t]];
-          stg(a.q + m * fs, S.g[t], qv[m][t]);
-        }
-      }
+  // derivative of the staged lines, between the barriers that publish the
+  // staging and the results
+  const double* cs = nullptr;
+  auto derive = [&]() __attribute__((always_inline)) {
+    __syncthreads();
+    {
+      ChunkCoef<C::R, false> CD;
+      lds_chunk_coef<C>(CD, cs, p * C::R);
+      solve_pass_line<C, false, GEN>(Tl, Xl, n, p, CD, a.fc, a.bnd[dir]);
     }
+    __syncthreads();
+  };
+  const double* csf = nullptr;
+  double c3l = 0.0;
+  FilterCoef fl;
+  auto filter_setup = [&](int region) __attribute__((always_inline)) {
+    csf = stage_chunk_coefs<C>(a.fac[dir], n + 7, smem, region);
+    c3l = a.fac[dir][2 * (n + 7) + (n + 7) - 1];
+    fl = stage_halo_coefs<C>(a.fc, smem);
+  };
+  auto filter = [&]() __attribute__((always_inline)) {
+    __syncthreads();
+    {
+      ChunkCoef<C::R, true> CF;
+      lds_chunk_coef_f<C>(CF, csf, p * C::R, n + 7, c3l);
+      solve_pass_line<C, true, GEN>(Tl, Xl, n, p, CF, fl, a.bnd[dir]);
+    }
+    __syncthreads();
+  };
 
-    // main path: the stored primitives the gradient solves take (pv) and
-    // the convective part's u_dir and p are loaded with q, at the start, so
-    // that every load of the pass is in flight at once (these passes run at
-    // two waves per SIMD, whose register budget holds them).  The split last
-    // pass's gradient half loads each just before its solve: the registers
-    // would cost it its third wave per SIMD.
-    constexpr bool PF = MAIN && DO_GRAD && PROG != GL_GRAD;
-    double pv[4][NPT], ud[NPT], pp[NPT];
-    if constexpr (PF) {
+  if constexpr (PROG == GC_FIRST || PROG == FGC_FIRST || PROG == GC_MID) {
+    // gradients of u, v, w, T along dir (gradcal, tgvsolver.F90:450-537;
+    // src/comsolver.F90:280-321)
+    constexpr bool FIRST = PROG != GC_MID;
+    cs = stage_chunk_coefs<C>(a.dac[dir], n + 3, smem, 0);
+    if constexpr (MAIN) {
+      // the stored u, v, w, T; the halo copies from the primitives of the
+      // halo's q (qswap's q2fvar)
+      double pv[4][NPT];
 #pragma unroll
       for (int t = 0; t < NPT; t++)
 #pragma unroll
         for (int c = 0; c < 4; c++) pv[c][t] = ldg(a.pr + (c < 3 ? 1 + c : 5) * fs, S.g[t]);
-      if (DO_CONV && !a.uwd) {
+      double* hal = smem + lds_doubles<C>(PROG);
+      auto hslot = [&](int t) {  // the slot's halo primitives, written and read by its own thread
+        const int l = S.s[t] / C::LT, r = S.s[t] - l * C::LT;
+        return hal + 4 * (l * kHaloSrcRows + (r <= 5 ? r - 1 : r - (n - 5) + 5));
+      };
+#pragma unroll
+      for (int t = 0; t < NPT; t++) {
+        if (S.h[t] != kDummy) {
+          double qh[5];
+#pragma unroll
+          for (int m = 0; m < 5; m++) qh[m] = halo_q<C>(a, S, t, dir, m);
+          const Prim P = prim_of(a, qh[0], qh[1], qh[2], qh[3], qh[4]);
+          double* h = hslot(t);
+          h[0] = P.u; h[1] = P.v; h[2] = P.w; h[3] = P.t;
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
 #pragma unroll
         for (int t = 0; t < NPT; t++) {
-          pp[t] = ldg(a.pr + 4 * fs, S.g[t]);
-          ud[t] = ldg(a.pr + (1 + dir) * fs, S.g[t]);
+          T[kLineOff + S.s[t]] = pv[c][t];
+          if (S.h[t] != kDummy) T[kLineOff + S.h[t]] = hslot(t)[c];
         }
-      }
-    }
-    // main path, halo slots: the halo's pressure (hp) and u_dir (hu), kept
-    // from the gradient part for the convective part (set on halo lanes only)
-    double hp[NPT], hu[NPT];
-    if constexpr (DO_GRAD) {
-    // gradients of u, v, w, T along dir (gradcal, tgvsolver.F90:450-537)
-    double gz[4][NPT];
+        derive();
+        const int fld = c < 3 ? c + 3 * dir : 9 + dir;
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-#pragma unroll
-      for (int t = 0; t < NPT; t++) {
-        if constexpr (MAIN) {
-          // the stored u, v, w or T (gradcal, src/comsolver.F90:280-300);
-          // the halo copy from the primitives of the halo's q (qswap's q2fvar)
-          T[kLineOff + S.s[t]] = PF ? pv[c][t] : ldg(a.pr + (c < 3 ? 1 + c : 5) * fs, S.g[t]);
-          if (S.h[t] != kDummy) {
-            double qh[5];
-            halo_q<C>(a, S, t, dir, qv, qh);
-            double f;
-            if (c < 3) {
-              f = qh[c + 1] / qh[0];
-              if (c == dir) hu[t] = f;
-            } else {
-              const double pr = pressure_of(a, qh[0], qh[1], qh[2], qh[3], qh[4]);
-              hp[t] = pr;
-              f = pr / qh[0] * a.const2;
-            }
-            T[kLineOff + S.h[t]] = f;
-          }
-        } else {
-          double f = 0.0;
-          {
-            if (c < 3) {
-              f = qv[c + 1][t] / qv[0][t];
-            } else {
-              const double pr = pressure_of(a, qv[0][t], qv[1][t], qv[2][t], qv[3][t], qv[4][t]);
-              f = pr / qv[0][t] * a.const2;
-            }
-          }
-          put<C>(T, S, t, f);
-        }
-      }
-      __syncthreads();
-      if constexpr (LAST) {
-        ChunkCoef<C::R, false> CD;
-        lds_chunk_coef<C>(CD, cs, p * C::R);
-        solve_pass_line<C, false, GEN>(Tl, Xl, n, p, CD, a.fc, a.bnd[dir]);
-      } else {
-        solve_pass_line<C, false, GEN>(Tl, Xl, n, p, CDr, a.fc, a.bnd[dir]);
-      }
-      __syncthreads();
-      const int fld = c < 3 ? c + 3 * dir : 9 + dir;
-#pragma unroll
-      for (int t = 0; t < NPT; t++) {
-        if (GEN && a.met) {
-          // gradcal's accumulation dvel(m,n) += D_d(u_m) dxi(d,n) over every
-          // n (src/comsolver.F90:300-321); the last pass adds its terms with
-          // the stress below
+        for (int t = 0; t < NPT; t++) {
+          const unsigned o = S.g[t];
           const double x = X[S.s[t]];
-          gz[c][t] = x;
-          if constexpr (!LAST) {
-            const unsigned o = S.g[t];
+          if (GEN && a.met) {
+            // gradcal's accumulation dvel(m,n) += D_d(u_m) dxi(d,n) over
+            // every n (src/comsolver.F90:300-321)
 #pragma unroll
             for (int nn = 0; nn < 3; nn++) {
 #pragma clang fp contract(off)
@@ -677,53 +646,80 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
               if (FIRST) stg(a.dv + f2 * fs, o, v);
               else stg(a.dv + f2 * fs, o, ldg(a.dv + f2 * fs, o) + v);
             }
+          } else {
+            // dvel(m,n) = D_d(u_m) dxi(d,n): dxi(d,d) of the uniform grid
+            stg(a.dv + fld * fs, o, x * met_of(a, dir).d);
           }
-        } else {
-          // dvel(m,n) = D_d(u_m) dxi(d,n): dxi(d,d) of the uniform grid
-          const double v = X[S.s[t]] * (MAIN ? met_of(a, dir).d : idn);
-          if (!LAST || sa.store_last_grad) stg(a.dv + fld * fs, S.g[t], v);
-          gz[c][t] = v;
         }
       }
+    } else {
+      // the first pass takes q and leaves the pressure for the others
+      double qv[5][NPT];
+#pragma unroll
+      for (int t = 0; t < NPT; t++)
+#pragma unroll
+        for (int m = 0; m < 5; m++) qv[m][t] = ldg(!FIRST && m == 4 ? a.p : a.q + m * fs, S.g[t]);
+      if constexpr (PROG == FGC_FIRST) {
+        // the previous stage's filter sweep along these lines (filterq,
+        // tgvsolver.F90:805-825), as the filter pass does it, on the loaded
+        // q; the filtered q is stored and the gradients below take it
+        filter_setup(1);
+#pragma unroll
+        for (int m = 0; m < 5; m++) {
+#pragma unroll
+          for (int t = 0; t < NPT; t++) put<C>(T, S, t, qv[m][t]);
+          filter();
+#pragma unroll
+          for (int t = 0; t < NPT; t++) {
+            qv[m][t] = X[S.s[t]];
+            stg(a.q + m * fs, S.g[t], qv[m][t]);
+          }
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+#pragma unroll
+        for (int t = 0; t < NPT; t++) {
+          double f;
+          if (c < 3) {
+            f = qv[c + 1][t] / qv[0][t];
+          } else {
+            double pr = qv[4][t];
+            if constexpr (FIRST) {
+              pr = pressure_of(a, qv[0][t], qv[1][t], qv[2][t], qv[3][t], qv[4][t]);
+              stg(a.p, S.g[t], pr);
+            }
+            f = pr / qv[0][t] * a.const2;
+          }
+          put<C>(T, S, t, f);
+        }
+        derive();
+        const int fld = c < 3 ? c + 3 * dir : 9 + dir;
+#pragma unroll
+        for (int t = 0; t < NPT; t++) stg(a.dv + fld * fs, S.g[t], X[S.s[t]] * idn);
+      }
     }
-
-    if constexpr (LAST) {
-      // stress and heat flux (diffusion, tgvsolver.F90:659-694) and the
-      // stage-1 KE / enstrophy partial sums (stacal, :893-942)
+  } else if constexpr (PROG == V_FIRST || PROG == V_MID || PROG == V_LAST_RK) {
+    // The derivative along dir of the viscous (diffusion, tgvsolver.F90:
+    // 700-787) minus the convective flux (convection, :539-633), the sign
+    // qrhs has after rhscal, accumulated over the directions.  Viscous columns
+    // per direction: x (s11,s12,s13,q1), y (s12,s22,s23,q2), z (s13,s23,s33,q3);
+    // density has none.
+    constexpr bool FIRST = PROG == V_FIRST;
+    constexpr bool RK = PROG == V_LAST_RK;
+    // the main path's upwind-biased convection left its part in qrhs
+    const bool uwd = MAIN && a.uwd;
+    cs = stage_chunk_coefs<C>(a.dac[dir], n + 3, smem, 0);
+    double sx[4][FIRST ? NPT : 1];
+    if constexpr (FIRST) {
+      // Stress and heat flux of every point from the stored gradients, here
+      // because x-lines leave a lane only NPT points to hold; columns s11 and
+      // q1, which no other direction reads, stay in registers.  And the
+      // stage-1 KE / enstrophy partial sums.
       double sk = 0.0, se = 0.0;
 #pragma unroll
       for (int t = 0; t < NPT; t++) {
         const unsigned o = S.g[t];
-        double g[3][3], gt[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-          if (GEN && a.met) {
-#pragma clang fp contract(off)
-            // the earlier passes' terms plus this direction's, D_dir(u_m) dxi(dir,d)
-            if (d < a.ndir) {
-              const double md = ldg(a.met + (1 + dir + 3 * d) * fs, o);
-#pragma unroll
-              for (int m = 0; m < 3; m++) g[m][d] = ldg(a.dv + (m + 3 * d) * fs, o) + gz[m][t] * md;
-              gt[d] = ldg(a.dv + (9 + d) * fs, o) + gz[3][t] * md;
-              if (sa.store_last_grad) {
-#pragma unroll
-                for (int m = 0; m < 3; m++) stg(a.dv + (m + 3 * d) * fs, o, g[m][d]);
-                stg(a.dv + (9 + d) * fs, o, gt[d]);
-              }
-            } else {
-              g[0][d] = 0.0; g[1][d] = 0.0; g[2][d] = 0.0; gt[d] = 0.0;
-            }
-          } else if (d == dir) {
-            g[0][d] = gz[0][t]; g[1][d] = gz[1][t]; g[2][d] = gz[2][t]; gt[d] = gz[3][t];
-          } else if (d < a.ndir) {
-            g[0][d] = ldg(a.dv + (0 + 3 * d) * fs, o);
-            g[1][d] = ldg(a.dv + (1 + 3 * d) * fs, o);
-            g[2][d] = ldg(a.dv + (2 + 3 * d) * fs, o);
-            gt[d] = ldg(a.dv + (9 + d) * fs, o);
-          } else {
-            g[0][d] = 0.0; g[1][d] = 0.0; g[2][d] = 0.0; gt[d] = 0.0;
-          }
-        }
         Prim P;
         if constexpr (MAIN) {
           // diffrsdcal6 (src/solver.F90:2433-2545) and the statistics
@@ -735,18 +731,28 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
           P.p = 0.0;
           P.t = ldg(a.pr + 5 * fs, o);
         } else {
-          P = prim_of(a, qv[0][t], qv[1][t], qv[2][t], qv[3][t], qv[4][t]);
+          P.r = ldg(a.q, o);
+          P.u = ldg(a.q + fs, o) / P.r;
+          P.v = ldg(a.q + 2 * fs, o) / P.r;
+          P.w = ldg(a.q + 3 * fs, o) / P.r;
+          P.p = ldg(a.p, o);
+          P.t = P.p / P.r * a.const2;
         }
         double f[9];
-        visc_flux(a, g, gt, P, f);
+        stress_point(a, o, P, f, sa.dostats && ((S.interior >> t) & 1), sk, se);
+        const bool all = GEN && a.met;
 #pragma unroll
-        for (int m = 0; m < 9; m++) stg(a.sg + m * fs, o, f[m]);
-        if (sa.dostats && ((S.interior >> t) & 1)) {
-          sk += P.r * (P.u * P.u + P.v * P.v + P.w * P.w);
-          const double o1 = g[2][1] - g[1][2];
-          const double o2 = g[0][2] - g[2][0];
-          const double o3 = g[1][0] - g[0][1];
-          se += P.r * (o1 * o1 + o2 * o2 + o3 * o3);
+        for (int m = 0; m < 9; m++)
+          if (all || (m != 0 && m != 6)) stg(a.sg + m * fs, o, f[m]);
+        if (all) {
+          const MetRow M = met_row(a, dir, o);
+#pragma unroll
+          for (int c = 0; c < 4; c++)
+            sx[c][t] = visc_col_row(M, f[c == 3 ? 6 : c], f[c == 0 ? 1 : (c == 1 ? 3 : (c == 2 ? 4 : 7))],
+                                    f[c == 0 ? 2 : (c == 1 ? 4 : (c == 2 ? 5 : 8))]);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; c++) sx[c][t] = f[c == 3 ? 6 : c];
         }
       }
       if (sa.dostats) {
@@ -769,210 +775,215 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
         __syncthreads();
       }
     }
-    }
-
-    // the main path's upwind-biased convection replaces this part (uniform
-    // over the workgroup, after the last barrier of the gradient part)
-    if (MAIN && a.uwd) return;
-    if constexpr (DO_CONV) {
-    // convective flux derivatives along dir (convection, tgvsolver.F90:539-633)
-#pragma unroll
-    for (int t = 0; t < NPT; t++) {
-      if constexpr (MAIN) {
-        // convrsdcal6 takes the stored vel and prs (src/solver.F90:2196-2207),
-        // loaded at the start where the pass has gradient solves
-        if constexpr (!PF) {
-          pp[t] = ldg(a.pr + 4 * fs, S.g[t]);
-          ud[t] = ldg(a.pr + (1 + dir) * fs, S.g[t]);
-        }
-      } else {
-        pp[t] = pressure_of(a, qv[0][t], qv[1][t], qv[2][t], qv[3][t], qv[4][t]);
-        ud[t] = (dir == 0 ? qv[1][t] : (dir == 1 ? qv[2][t] : qv[3][t])) / qv[0][t];
-      }
-    }
-    // the main path's flux inputs of component MM: one copy per component
-    // behind a wave-uniform switch, so that q is indexed by constants while
-    // the loop over components (and its solve) stays rolled
-    auto stage_main = [&](auto mc) __attribute__((always_inline)) {
-      constexpr int MM = decltype(mc)::value;
+    // velocity along dir and pressure of the points; hu, hp those of the halo
+    // copies where they differ (main path)
+    double ud[NPT], pp[NPT], hu[NPT], hp[NPT];
+    if (!uwd) {
 #pragma unroll
       for (int t = 0; t < NPT; t++) {
-        // a periodic halo copy carries the source point's metrics, which are this point's
-        if (GEN && a.met) {
-          const unsigned o = S.g[t];
-          const MetRow M = met_row(a, dir, o);
-          const double u = ldg(a.pr + fs, o), v = ldg(a.pr + 2 * fs, o), w = ldg(a.pr + 3 * fs, o);
-          T[kLineOff + S.s[t]] = conv_flux_full(M, MM, qv[MM][t], qv[4][t], u, v, w, pp[t]);
-          if (S.h[t] != kDummy) {
-            double qh[5];
-            halo_q<C>(a, S, t, dir, qv, qh);
-            const double ph = pressure_of(a, qh[0], qh[1], qh[2], qh[3], qh[4]);
-            T[kLineOff + S.h[t]] =
-                conv_flux_full(M, MM, qh[MM], qh[4], qh[1] / qh[0], qh[2] / qh[0], qh[3] / qh[0], ph);
-          }
+        const unsigned o = S.g[t];
+        if constexpr (MAIN) {
+          // convrsdcal6 takes the stored vel and prs (src/solver.F90:2196-2207)
+          pp[t] = ldg(a.pr + 4 * fs, o);
+          ud[t] = ldg(a.pr + (1 + dir) * fs, o);
         } else {
-          const Met M = met_of(a, dir);
-          T[kLineOff + S.s[t]] = conv_flux_main(M.j, M.d, MM, dir, qv[MM][t], qv[4][t], ud[t], pp[t]);
+          pp[t] = ldg(a.p, o);
+          ud[t] = ldg(a.q + (1 + dir) * fs, o) / ldg(a.q, o);
+        }
+      }
+      if constexpr (MAIN) {
+#pragma unroll
+        for (int t = 0; t < NPT; t++) {
           if (S.h[t] != kDummy) {
             double qh[5];
-            halo_q<C>(a, S, t, dir, qv, qh);
-            double ph, uh;
-            if constexpr (DO_GRAD) {
-              ph = hp[t];
-              uh = hu[t];
-            } else {
-              ph = pressure_of(a, qh[0], qh[1], qh[2], qh[3], qh[4]);
-              uh = pick5(0.0, qh[1], qh[2], qh[3], 0.0, 1 + dir) / qh[0];
+#pragma unroll
+            for (int m = 0; m < 5; m++) qh[m] = halo_q<C>(a, S, t, dir, m);
+            hp[t] = pressure_of(a, qh[0], qh[1], qh[2], qh[3], qh[4]);
+            hu[t] = (dir == 0 ? qh[1] : (dir == 1 ? qh[2] : qh[3])) / qh[0];
+          }
+        }
+      }
+    }
+    // inputs of the next solve: q_m and the viscous column (general grids
+    // form their column when it is staged)
+    const bool metg = GEN && a.met;
+    double qn[NPT], vn[NPT];
+    auto load_inputs = [&](int m) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < NPT; t++) {
+        if (!uwd || RK) qn[t] = ldg(a.q + m * fs, S.g[t]);
+        if (!FIRST && m > 0 && !metg) {
+          const int col = m == 4 ? 6 + dir : (dir == 1 ? (m == 1 ? 1 : (m == 2 ? 3 : 4)) : (m == 1 ? 2 : (m == 2 ? 4 : 5)));
+          vn[t] = ldg(a.sg + col * fs, S.g[t]);
+        }
+      }
+    };
+    // Stage component m's flux difference with its halo copies (part 1: the
+    // convective flux alone, 2: the viscous one).  The momentum flux along dir
+    // carries p ~ p0 = 1/(gamma Ma^2), large against everything the
+    // derivative keeps of it; p0 goes off it first, which is exact within a
+    // factor of two of p0 and drops out of the derivative, so the difference
+    // rounds relative to p - p0 and the solve sees the flux's own roundings
+    // only.  Per-point metrics have no such constant: there the two parts are
+    // solved one after the other.
+    auto stage_flux = [&](int m, int part) __attribute__((always_inline)) {
+      const double f0 = m == dir + 1 ? (MAIN ? a.jac * (a.inv_d[dir] * a.p0) : a.p0) : 0.0;
+#pragma unroll
+      for (int t = 0; t < NPT; t++) {
+        const unsigned o = S.g[t];
+        double v = 0.0;
+        if (m > 0 && part != 1) {
+          if constexpr (FIRST) v = sx[m - 1][t];
+          else v = metg ? visc_col_full(a, dir, m - 1, o) : vn[t];
+          if (MAIN && !metg) {
+            // (sigma . dxi(dir,:)) J (diffrsdcal6, src/solver.F90:2623-2635)
+            const Met M = met_of(a, dir);
+            v = v * M.d * M.j;
+          }
+        }
+        if constexpr (!MAIN) {
+          put<C>(T, S, t, v - (conv_flux(m, dir, qn[t], ud[t], pp[t]) - f0));
+        } else {
+          if (uwd || part == 2) {
+            put<C>(T, S, t, v);
+            continue;
+          }
+          if (metg) {
+            // a periodic halo copy carries the source point's metrics, which are this point's
+            const MetRow M = met_row(a, dir, o);
+            T[kLineOff + S.s[t]] = v - conv_flux_full(M, m, qn[t], ldg(a.pr + fs, o), ldg(a.pr + 2 * fs, o),
+                                                      ldg(a.pr + 3 * fs, o), pp[t]);
+            if (S.h[t] != kDummy) {
+              const double r = halo_q<C>(a, S, t, dir, 0);
+              T[kLineOff + S.h[t]] = v - conv_flux_full(M, m, halo_q<C>(a, S, t, dir, m),
+                                                        halo_q<C>(a, S, t, dir, 1) / r, halo_q<C>(a, S, t, dir, 2) / r,
+                                                        halo_q<C>(a, S, t, dir, 3) / r, hp[t]);
             }
-            T[kLineOff + S.h[t]] = conv_flux_main(M.j, M.d, MM, dir, qh[MM], qh[4], uh, ph);
+          } else {
+            const Met M = met_of(a, dir);
+            T[kLineOff + S.s[t]] = v - (conv_flux_main(M.j, M.d, m, dir, qn[t], ud[t], pp[t]) - f0);
+            if (S.h[t] != kDummy) {
+              const double qh = S.ex[t] >= 0 ? halo_q<C>(a, S, t, dir, m) : qn[t];
+              T[kLineOff + S.h[t]] = v - (conv_flux_main(M.j, M.d, m, dir, qh, hu[t], hp[t]) - f0);
+            }
           }
         }
       }
     };
+    // derivative of the staged component; cx: the convective part's, where it
+    // is solved on its own
+    double cx[GEN ? NPT : 1];
+    auto derive_flux = [&](int m) __attribute__((always_inline)) {
+      derive();
+      if constexpr (GEN) {
+        const bool two = metg && m > 0 && !uwd;
 #pragma unroll
-    for (int m = 0; m < 5; m++) {
-      if constexpr (MAIN) {
-        switch (m) {
-          case 0: stage_main(std::integral_constant<int, 0>{}); break;
-          case 1: stage_main(std::integral_constant<int, 1>{}); break;
-          case 2: stage_main(std::integral_constant<int, 2>{}); break;
-          case 3: stage_main(std::integral_constant<int, 3>{}); break;
-          default: stage_main(std::integral_constant<int, 4>{}); break;
-        }
-      } else {
-#pragma unroll
-        for (int t = 0; t < NPT; t++) put<C>(T, S, t, conv_flux(m, dir, ASTR_QV(m, t), qv[4][t], ud[t], pp[t]));
-      }
-      double* dst = a.qrhs + m * fs;
-      double qr[NPT];
-      if (!FIRST) {
-        // issued before the solve so the load latency overlaps it
-#pragma unroll
-        for (int t = 0; t < NPT; t++) qr[t] = ldg(dst, S.g[t]);
-      }
-      __syncthreads();
-      if constexpr (LAST) {
-        ChunkCoef<C::R, false> CD;
-        lds_chunk_coef<C>(CD, cs, p * C::R);
-        solve_pass_line<C, false, GEN>(Tl, Xl, n, p, CD, a.fc, a.bnd[dir]);
-      } else {
-        solve_pass_line<C, false, GEN>(Tl, Xl, n, p, CDr, a.fc, a.bnd[dir]);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int t = 0; t < NPT; t++) {
-        {
-          // the main path's fluxes carry the metrics: no 1/dx after the solve
-          const double v = MAIN ? X[S.s[t]] : X[S.s[t]] * idn;
-          if (FIRST) stg(dst, S.g[t], v);
-          else if (PROG == GC_MID) stg(dst, S.g[t], qr[t] + v);
-          else stg(dst, S.g[t], -(qr[t] + v));
+        for (int t = 0; t < NPT; t++) cx[t] = two ? X[S.s[t]] : 0.0;
+        if (two) {
+          stage_flux(m, 2);
+          derive();
         }
       }
-    }
-    }
-  } else if constexpr (PROG == V_MID || PROG == V_LAST_RHS || PROG == V_LAST_RK) {
-    // viscous-flux derivatives (diffusion, tgvsolver.F90:700-787); columns
-    // per direction: x (s11,s12,s13,q1), y (s12,s22,s23,q2), z (s13,s23,s33,q3).
-    // V_LAST_RK: each variable's RK3 stage update (tgvsolver.F90:1043-1059)
-    // and its filter along dir follow its viscous sum at once, so one sum is
-    // live at a time; density, which has no viscous term, goes first.
-    constexpr bool RK = PROG == V_LAST_RK;
-    // the chunk factors are read back from LDS before each solve, so they do
-    // not hold registers across the pass
-    const double* cs = stage_chunk_coefs<C>(a.dac[dir], n + 3, smem, 0);
-    const int c0 = dir == 0 ? 0 : (dir == 1 ? 1 : 2);
-    const int c1 = dir == 0 ? 1 : (dir == 1 ? 3 : 4);
-    const int c2 = dir == 0 ? 2 : (dir == 1 ? 4 : 5);
-    double nx[NPT];
+    };
+    auto first_part = [&](int m) { return metg && m > 0 && !uwd ? 1 : 0; };
+    // its value at slot t (the main path's fluxes carry the metrics: no 1/dx
+    // after the solve)
+    auto dflux = [&](int t) __attribute__((always_inline)) {
+      const double x = X[S.s[t]];
+      return (MAIN ? x : x * idn) + (GEN ? cx[GEN ? t : 0] : 0.0);
+    };
+    if constexpr (!RK) {
+      const int m0 = uwd ? 1 : 0;
+      load_inputs(m0);
 #pragma unroll
-    for (int t = 0; t < NPT; t++) nx[t] = ldg(a.sg + c0 * fs, S.g[t]);
-    if constexpr (!RK || MAIN) {
-      // MAIN && RK (time_integration_rk, src/mainloop.F90:430-482): each
-      // variable's RK3 update follows its viscous sum, density (no viscous
-      // term) first; updatefvar of the new q ends the pass
-      constexpr bool RKM = RK && MAIN;
-      double qn[5][NPT];
-      if constexpr (RKM) {
+      for (int m = 0; m < 5; m++) {
+        if (m < m0) continue;
+        stage_flux(m, first_part(m));
+        double* dst = a.qrhs + m * fs;
+        double qr[NPT];
+        if (!FIRST || uwd) {
+#pragma unroll
+          for (int t = 0; t < NPT; t++) qr[t] = ldg(dst, S.g[t]);
+        }
+        if (m < 4) load_inputs(m + 1);
+        derive_flux(m);
+#pragma unroll
+        for (int t = 0; t < NPT; t++) stg(dst, S.g[t], FIRST && !uwd ? dflux(t) : qr[t] + dflux(t));
+      }
+    } else {
+      // each variable's RK3 stage update (tgvsolver.F90:1043-1059;
+      // src/mainloop.F90:430-482) and, in the miniapp, its filter along dir
+      // follow its flux derivative at once
+      double qr[NPT], qs[NPT];
+      auto load_rk = [&](int m) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < NPT; t++) {
-          const unsigned o = S.g[t];
-          const double jb = jac_of<GEN>(a, o);
-          const double q0 = ldg(a.q, o);
-          double s0;
-          if (sa.stage == 0) {
-            s0 = q0 * jb;  // qsave = q J (:423-427)
-            stg(a.qsave, o, s0);
-          } else {
-            s0 = ldg(a.qsave, o);
-          }
-          qn[0][t] = rk_update_main(sa, a.dt, jb, s0, q0, ldg(a.qrhs, o));
-          stg(a.q, o, qn[0][t]);
+          qr[t] = ldg(a.qrhs + m * fs, S.g[t]);
+          qs[t] = sa.stage == 0 ? 0.0 : ldg(a.qsave + m * fs, S.g[t]);
         }
-      }
+      };
+      load_inputs(0);
+      load_rk(0);
+      if constexpr (!MAIN) {
+        filter_setup(1);
 #pragma unroll
-      for (int c = 0; c < 4; c++) {
-        // the main path's viscous fluxes carry the metrics:
-        // (sigma . dxi(dir,:)) J (diffrsdcal6, src/solver.F90:2623-2635)
+        for (int m = 0; m < 5; m++) {
+          stage_flux(m, 0);
+          double qo[NPT];
 #pragma unroll
-        for (int t = 0; t < NPT; t++) {
-          if constexpr (MAIN) {
-            if (GEN && a.met) {
-              put<C>(T, S, t, visc_col_full(a, dir, c, S.g[t]));
-            } else {
-              const Met M = met_of(a, dir);
-              put<C>(T, S, t, nx[t] * M.d * M.j);
-            }
-          } else {
-            put<C>(T, S, t, nx[t]);
-          }
-        }
-        // loads for this column's accumulation and the next column's input are
-        // issued before the solve so their latency overlaps it
-        double qr[NPT], qo[NPT], qs[NPT];
-        double* dst = a.qrhs + (1 + c) * fs;
+          for (int t = 0; t < NPT; t++) qo[t] = qn[t];
+          if (m < 4) load_inputs(m + 1);
+          derive_flux(m);
 #pragma unroll
-        for (int t = 0; t < NPT; t++) {
-          qr[t] = ldg(dst, S.g[t]);
-          if constexpr (RKM) {
-            qo[t] = ldg(a.q + (1 + c) * fs, S.g[t]);
-            qs[t] = sa.stage == 0 ? 0.0 : ldg(a.qsave + (1 + c) * fs, S.g[t]);
-          }
-        }
-        if (c < 3) {
-          const int col = c == 0 ? c1 : (c == 1 ? c2 : 6 + dir);
-#pragma unroll
-          for (int t = 0; t < NPT; t++) nx[t] = ldg(a.sg + col * fs, S.g[t]);
-        }
-        __syncthreads();
-        {
-          ChunkCoef<C::R, false> CD;
-          lds_chunk_coef<C>(CD, cs, p * C::R);
-          solve_pass_line<C, false, GEN>(Tl, Xl, n, p, CD, a.fc, a.bnd[dir]);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int t = 0; t < NPT; t++) {
-          const double v = qr[t] + (MAIN ? X[S.s[t]] : X[S.s[t]] * idn);
-          if constexpr (RKM) {
-            const double jb = jac_of<GEN>(a, S.g[t]);
+          for (int t = 0; t < NPT; t++) {
+            const double v = qr[t] + dflux(t);
             double s0 = qs[t];
             if (sa.stage == 0) {
-              s0 = qo[t] * jb;
-              stg(a.qsave + (1 + c) * fs, S.g[t], s0);
+              stg(a.qsave + m * fs, S.g[t], qo[t]);
+              s0 = qo[t];
             }
-            qn[1 + c][t] = rk_update_main(sa, a.dt, jb, s0, qo[t], v);
-            stg(a.q + (1 + c) * fs, S.g[t], qn[1 + c][t]);
-          } else {
-            stg(dst, S.g[t], v);
+            put<C>(T, S, t, rk_update(sa, a.dt, s0, qo[t], v));
+          }
+          if (m < 4) load_rk(m + 1);
+          filter();
+#pragma unroll
+          for (int t = 0; t < NPT; t++) stg(a.q + m * fs, S.g[t], X[S.s[t]]);
+        }
+      } else {
+        // the new q, whose updatefvar ends the pass
+        double qw[5][NPT];
+#pragma unroll
+        for (int m = 0; m < 5; m++) {
+          const bool solve = m > 0 || !uwd;  // without convection density has no flux
+          if (solve) stage_flux(m, first_part(m));
+          double qo[NPT], ro[NPT], so[NPT];
+#pragma unroll
+          for (int t = 0; t < NPT; t++) {
+            qo[t] = qn[t];
+            ro[t] = qr[t];
+            so[t] = qs[t];
+          }
+          if (m < 4) {
+            load_inputs(m + 1);
+            load_rk(m + 1);
+          }
+          if (solve) derive_flux(m);
+#pragma unroll
+          for (int t = 0; t < NPT; t++) {
+            const double v = solve ? ro[t] + dflux(t) : ro[t];
+            const double jb = jac_of<GEN>(a, S.g[t]);
+            double s0 = so[t];
+            if (sa.stage == 0) {
+              s0 = qo[t] * jb;  // qsave = q J (src/mainloop.F90:423-427)
+              stg(a.qsave + m * fs, S.g[t], s0);
+            }
+            qw[m][t] = rk_update_main(sa, a.dt, jb, s0, qo[t], v);
           }
         }
-      }
-      if constexpr (RKM) {
         // updatefvar (fludyna.F90:191-242): rho, u, v, w, p, T of the new q
 #pragma unroll
         for (int t = 0; t < NPT; t++) {
-          const Prim P = prim_of(a, qn[0][t], qn[1][t], qn[2][t], qn[3][t], qn[4][t]);
+          const Prim P = prim_of(a, qw[0][t], qw[1][t], qw[2][t], qw[3][t], qw[4][t]);
           const unsigned o = S.g[t];
           stg(a.pr, o, P.r);
           stg(a.pr + fs, o, P.u);
@@ -986,121 +997,33 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
           // as the filter pass does it, on the new q held in registers; the
           // primitives above stay those of the unfiltered q, as after the
           // reference's filterq.  The barrier before the solve orders the
-          // staging below after every read of the viscous part's LDS.
-          const double* csf = stage_chunk_coefs<C>(a.fac[dir], n + 7, smem, 1);
-          const double c3l = a.fac[dir][2 * (n + 7) + (n + 7) - 1];
-          const FilterCoef fl = stage_halo_coefs<C>(a.fc, smem);
+          // staging below after every read of the flux part's LDS.
+          filter_setup(1);
 #pragma unroll
           for (int m = 0; m < 5; m++) {
 #pragma unroll
-            for (int t = 0; t < NPT; t++) put<C>(T, S, t, qn[m][t]);
-            __syncthreads();
-            {
-              ChunkCoef<C::R, true> CF;
-              lds_chunk_coef_f<C>(CF, csf, p * C::R, n + 7, c3l);
-              solve_pass_line<C, true, GEN>(Tl, Xl, n, p, CF, fl, a.bnd[dir]);
-            }
-            __syncthreads();
+            for (int t = 0; t < NPT; t++) put<C>(T, S, t, qw[m][t]);
+            filter();
 #pragma unroll
             for (int t = 0; t < NPT; t++) stg(a.q + m * fs, S.g[t], X[S.s[t]]);
           }
+        } else {
+          // q last: the halo copies of general grids are read from it above
+#pragma unroll
+          for (int t = 0; t < NPT; t++)
+#pragma unroll
+            for (int m = 0; m < 5; m++) stg(a.q + m * fs, S.g[t], qw[m][t]);
         }
-      }
-    } else {
-      const double* csf = stage_chunk_coefs<C>(a.fac[dir], n + 7, smem, 1);
-      const double c3l = a.fac[dir][2 * (n + 7) + (n + 7) - 1];
-      const FilterCoef fl = stage_halo_coefs<C>(a.fc, smem);
-      // Loads run two solves ahead: variable c+1's qrhs, q, qsave are issued
-      // before variable c's filter solve, the next stress column before
-      // variable c's derivative solve.
-      double qr[NPT], qo[NPT], qs[NPT];
-#pragma unroll
-      for (int t = 0; t < NPT; t++) {
-        const unsigned o = S.g[t];
-        const double q0 = ldg(a.q, o);
-        double s0 = q0;
-        if (sa.stage == 0) stg(a.qsave, o, q0);
-        else s0 = ldg(a.qsave, o);
-        put<C>(T, S, t, rk_update(sa, a.dt, s0, q0, ldg(a.qrhs, o)));
-      }
-#pragma unroll
-      for (int t = 0; t < NPT; t++) {
-        qr[t] = ldg(a.qrhs + fs, S.g[t]);
-        qo[t] = ldg(a.q + fs, S.g[t]);
-        qs[t] = sa.stage == 0 ? 0.0 : ldg(a.qsave + fs, S.g[t]);
-      }
-      __syncthreads();
-      {
-          ChunkCoef<C::R, true> CF;
-          lds_chunk_coef_f<C>(CF, csf, p * C::R, n + 7, c3l);
-          solve_line<C::P, C::R, true>(Tl, Xl, n, p, CF, fl);
-        }
-      __syncthreads();
-#pragma unroll
-      for (int t = 0; t < NPT; t++) stg(a.q, S.g[t], X[S.s[t]]);
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-#pragma unroll
-        for (int t = 0; t < NPT; t++)
-          put<C>(T, S, t, nx[t]);
-        if (c < 3) {
-          const int col = c == 0 ? c1 : (c == 1 ? c2 : 6 + dir);
-#pragma unroll
-          for (int t = 0; t < NPT; t++) nx[t] = ldg(a.sg + col * fs, S.g[t]);
-        }
-        __syncthreads();
-        {
-          ChunkCoef<C::R, false> CD;
-          lds_chunk_coef<C>(CD, cs, p * C::R);
-          solve_line<C::P, C::R, false>(Tl, Xl, n, p, CD, a.fc);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int t = 0; t < NPT; t++) {
-          const double v = qr[t] + X[S.s[t]] * idn;
-          double s0 = qs[t];
-          if (sa.stage == 0) {
-            stg(a.qsave + (1 + c) * fs, S.g[t], qo[t]);
-            s0 = qo[t];
-          }
-          put<C>(T, S, t, rk_update(sa, a.dt, s0, qo[t], v));
-        }
-        if (c < 3) {
-#pragma unroll
-          for (int t = 0; t < NPT; t++) {
-            qr[t] = ldg(a.qrhs + (2 + c) * fs, S.g[t]);
-            qo[t] = ldg(a.q + (2 + c) * fs, S.g[t]);
-            qs[t] = sa.stage == 0 ? 0.0 : ldg(a.qsave + (2 + c) * fs, S.g[t]);
-          }
-        }
-        __syncthreads();
-        {
-          ChunkCoef<C::R, true> CF;
-          lds_chunk_coef_f<C>(CF, csf, p * C::R, n + 7, c3l);
-          solve_line<C::P, C::R, true>(Tl, Xl, n, p, CF, fl);
-        }
-        __syncthreads();
-        double* dq = a.q + (1 + c) * fs;
-#pragma unroll
-        for (int t = 0; t < NPT; t++) stg(dq, S.g[t], X[S.s[t]]);
       }
     }
   } else {  // F_ONLY: filter of q along dir, in place (filterq, tgvsolver.F90:791-883)
-    const double* csf = stage_chunk_coefs<C>(a.fac[dir], n + 7, smem, 0);
-    const double c3l = a.fac[dir][2 * (n + 7) + (n + 7) - 1];
-    const FilterCoef fl = stage_halo_coefs<C>(a.fc, smem);
+    filter_setup(0);
 #pragma unroll
     for (int m = 0; m < 5; m++) {
 #pragma unroll
       for (int t = 0; t < NPT; t++)
         put<C>(T, S, t, ldg(a.q + m * fs, S.g[t]));
-      __syncthreads();
-      {
-        ChunkCoef<C::R, true> CF;
-        lds_chunk_coef_f<C>(CF, csf, p * C::R, n + 7, c3l);
-        solve_pass_line<C, true, GEN>(Tl, Xl, n, p, CF, fl, a.bnd[dir]);
-      }
-      __syncthreads();
+      filter();
       double* dst = a.q + m * fs;
 #pragma unroll
       for (int t = 0; t < NPT; t++)
@@ -1156,14 +1079,18 @@ hipError_t launch_batch_c(int prog, const BatchLaunch& bl, int dir, const StageA
   dim3 g(nblocks), b(C::NT);
   switch (prog) {
     case GC_FIRST: hipLaunchKernelGGL((k_pass_batch<C, GC_FIRST, MINB>), g, b, lds, st, bl, dir, sa); break;
-    case GC_MID: hipLaunchKernelGGL((k_pass_batch<C, GC_MID, MINB>), g, b, lds, st, bl, dir, sa); break;
-    case GC_LAST: hipLaunchKernelGGL((k_pass_batch<C, GC_LAST, MINB>), g, b, lds, st, bl, dir, sa); break;
-    case V_MID: hipLaunchKernelGGL((k_pass_batch<C, V_MID, MINB>), g, b, lds, st, bl, dir, sa); break;
-    case V_LAST_RHS: hipLaunchKernelGGL((k_pass_batch<C, V_LAST_RHS, MINB>), g, b, lds, st, bl, dir, sa); break;
+    case GC_MID:
+    case GC_LAST: hipLaunchKernelGGL((k_pass_batch<C, GC_MID, MINB>), g, b, lds, st, bl, dir, sa); break;
+    case V_MID:
+      if (dir == 0) hipLaunchKernelGGL((k_pass_batch<C, V_FIRST, MINB>), g, b, lds, st, bl, dir, sa);
+      else hipLaunchKernelGGL((k_pass_batch<C, V_MID, MINB>), g, b, lds, st, bl, dir, sa);
+      break;
     case V_LAST_RK: hipLaunchKernelGGL((k_pass_batch<C, V_LAST_RK, MINB>), g, b, lds, st, bl, dir, sa); break;
-    case GL_GRAD: hipLaunchKernelGGL((k_pass_batch<C, GL_GRAD, MINB>), g, b, lds, st, bl, dir, sa); break;
-    case GL_CONV: hipLaunchKernelGGL((k_pass_batch<C, GL_CONV, MINB>), g, b, lds, st, bl, dir, sa); break;
-    case FGC_FIRST: return hipErrorInvalidValue;  // single-case passes only
+    // single-case passes only
+    case V_LAST_RHS:
+    case FGC_FIRST:
+    case RESERVED_7:
+    case RESERVED_8: return hipErrorInvalidValue;
     default: hipLaunchKernelGGL((k_pass_batch<C, F_ONLY, MINB>), g, b, lds, st, bl, dir, sa); break;
   }
   return hipGetLastError();
@@ -1172,17 +1099,20 @@ hipError_t launch_batch_c(int prog, const BatchLaunch& bl, int dir, const StageA
 template <class C, int MINB, bool MAIN, bool GEN>
 void launch_pass_m(int prog, const FlowArgs& a, int dir, hipStream_t st) {
   const int nt = tiles_of(a.n, dir, C::TL);
-  const size_t lds = (size_t)lds_doubles<C>(prog) * sizeof(double);
+  const size_t lds = (size_t)lds_doubles<C>(prog, MAIN) * sizeof(double);
   dim3 g(nt), b(C::NT);
   switch (prog) {
     case GC_FIRST: hipLaunchKernelGGL((k_pass<C, GC_FIRST, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
-    case GC_MID: hipLaunchKernelGGL((k_pass<C, GC_MID, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
-    case GC_LAST: hipLaunchKernelGGL((k_pass<C, GC_LAST, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
-    case V_MID: hipLaunchKernelGGL((k_pass<C, V_MID, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
-    case V_LAST_RHS: hipLaunchKernelGGL((k_pass<C, V_LAST_RHS, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
+    case GC_MID:
+    case GC_LAST: hipLaunchKernelGGL((k_pass<C, GC_MID, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
+    case V_MID:
+      if (dir == 0) {
+        hipLaunchKernelGGL((k_pass<C, V_FIRST, MINB, MAIN, GEN>), g, b, lds, st, a, dir);
+        break;
+      }
+      [[fallthrough]];
+    case V_LAST_RHS: hipLaunchKernelGGL((k_pass<C, V_MID, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
     case V_LAST_RK: hipLaunchKernelGGL((k_pass<C, V_LAST_RK, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
-    case GL_GRAD: hipLaunchKernelGGL((k_pass<C, GL_GRAD, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
-    case GL_CONV: hipLaunchKernelGGL((k_pass<C, GL_CONV, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
     // the filtering first pass exists for the miniapp's stage only (the main
     // path filters at the start of its stage); launch_pass_c refuses it there
     case FGC_FIRST:
@@ -1196,6 +1126,7 @@ void launch_pass_m(int prog, const FlowArgs& a, int dir, hipStream_t st) {
 template <class C, int MINB>
 hipError_t launch_pass_c(int prog, const FlowArgs& a, int dir, hipStream_t st) {
   if (prog == FGC_FIRST && (a.main_sem || dir != 0)) return hipErrorInvalidValue;
+  if (prog == RESERVED_7 || prog == RESERVED_8) return hipErrorInvalidValue;
   if (a.main_sem && (a.met || a.bnd[dir])) launch_pass_m<C, MINB, true, true>(prog, a, dir, st);
   else if (a.main_sem) launch_pass_m<C, MINB, true, false>(prog, a, dir, st);
   else launch_pass_m<C, MINB, false, false>(prog, a, dir, st);

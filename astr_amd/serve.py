@@ -68,11 +68,11 @@ class Result:
 
 
 def case_bytes(cfg: A.Config) -> int:
-    """Device memory of one context: 36 padded FP64 fields plus tables."""
+    """Device memory of one context: 37 padded FP64 fields plus tables."""
     pitch = (cfg.im + 1 + 15) // 16 * 16
     plane = pitch * (cfg.jm + 1)
     fs = (plane * (cfg.km + 1) + 1 + 63) // 64 * 64
-    return 36 * fs * 8 + 64 * 1024
+    return 37 * fs * 8 + 64 * 1024
 
 
 def h2_air(names, W, phi):

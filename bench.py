@@ -31,24 +31,19 @@ FP64_PEAK_TFS = 78.6
 
 # Algorithmic FP64 words per lattice point moved by the reference operators
 # each pass fuses (one streaming sweep per operator, reads + writes):
-#   gc_first  : gradients x (4+4) + convective x (7+5)                 = 20
-#   gc_mid    : gradients y (4+4) + convective y (12+5)                = 25
-#   gc_last   : gradients z (4+4) + convective z (12+5)
-#               + pointwise stress/heat flux (16+9)                    = 50
-#   visc_mid  : viscous derivative (4+4 read, 4 write)                 = 12
-#   visc_last_rk3_filter: viscous z (12) + RK3 update (15+5)
-#               + filter z (5+5)                                       = 42
+#   gc_first, gc_mid, gc_last: gradients of one direction (4+4)        =  8
+#   visc_mid x: pointwise stress/heat flux (16+9), convective x (7+5),
+#               viscous x (4+4 read, 4 write)                          = 49
+#   visc_mid y: convective y (12+5) + viscous y (12)                   = 29
+#   visc_last_rhs: convective z (17) + viscous z (12)                  = 29
+#   visc_last_rk3_filter: those + RK3 update (15+5) + filter z (5+5)   = 59
 #   filter    : one filter sweep (5+5)                                 = 10
-#   filter_gc_first: gc_first with the previous stage's x filter sweep = 30
-# Summed over a 3-D stage: 20+25+50+12+12+42+10+10 = 181, plus the
+#   filter_gc_first: gc_first with the previous stage's x filter sweep = 18
+# Summed over a 3-D stage: 3*8 + 49 + 29 + 59 + 2*10 = 181, plus the
 # reference's updatefvar (5+6 = 11) that the passes make unnecessary:
 # 192 words = 1536 B per point per stage.
-# When the last gradient/convective pass runs split, its halves carry the
-# gradients + stress/heat flux (4+4 + 16+9 = 33) and the convective
-# derivatives (12+5 = 17) of the same 50 words.
-PASS_WORDS = {"gc_first": 20, "gc_mid": 25, "gc_last": 50, "visc_mid": 12,
-              "visc_last_rhs": 12, "visc_last_rk3_filter": 42, "filter": 10,
-              "gc_last_grad": 33, "gc_last_conv": 17, "filter_gc_first": 30}
+PASS_WORDS = {"gc_first": 8, "gc_mid": 8, "gc_last": 8, "visc_mid_x": 49, "visc_mid_y": 29,
+              "visc_last_rhs": 29, "visc_last_rk3_filter": 59, "filter": 10, "filter_gc_first": 18}
 STAGE_BYTES = 1536
 
 
@@ -560,7 +555,7 @@ def main():
     # dominant kernel by total time
     (pname, pdir), (ms_tot, cnt) = max(prof.items(), key=lambda kv: kv[1][0])
     avg_s = ms_tot / cnt / 1e3
-    alg_bytes = PASS_WORDS[pname] * 8 * pts
+    alg_bytes = PASS_WORDS.get(f"{pname}_{pdir}", PASS_WORDS.get(pname)) * 8 * pts
     achieved = alg_bytes / avg_s / 1e9
     tr = load_traffic(n)
     traffic = None

@@ -147,7 +147,7 @@ int astr_hip_rk3_steps_stats(astr_hip_ctx *ctx, int nsteps, double *ke, double *
  * statistics buffers (per-tile partial sums, dissipation block partials, the
  * per-step values) live in a fixed 8 MiB device array, one copy per GPU, held
  * until the process ends.  It calls no hipMalloc/hipFree.  Limit:
- * 2 x (tiles of the last gradient pass) + 1024 + 3 x nsteps doubles must fit
+ * 2 x (x-line tiles of the stress pass) + 1024 + 3 x nsteps doubles must fit
  * in 2^20 (e.g. nsteps <= 170000 at 512^3); larger requests return an error
  * before any work is queued.  Every call on one GPU shares that GPU's array,
  * so calls that overlap on one GPU (other threads, other contexts on other
@@ -222,13 +222,13 @@ int astr_hip_set_convection(astr_hip_ctx *ctx, int upwind, int recon_schem, int 
 
 /* Per-pass timing with HIP events on the context's stream (no reference
  * counterpart; the reference's timerept accumulators, src/utility.F90:27-297,
- * are no-ops).  Slot = pass*3 + direction, pass 0..8 = convective+gradient
- * first/middle/last, viscous middle/last(rhs)/last(RK3+filter), filter, and
- * the two halves of the split last convective+gradient pass (gradients and
- * stress, convective); 9..11 = the upwind-biased convection's split,
- * interface-flux and shock-sensor kernels (the sensor in slot 33); 12 = the
- * first convective+gradient pass with the previous stage's x filter sweep
- * (program 9, slot 36). */
+ * are no-ops).  Slot = pass*3 + direction, pass 0..6 = gradients
+ * first/middle/last, flux derivative (viscous minus convective; along x with
+ * the stress, the heat flux and the statistics) middle/last(rhs)/last(RK3 +
+ * filter), filter; 7 and 8 stay empty; 9..11 = the upwind-biased
+ * convection's split, interface-flux and shock-sensor kernels (the sensor in
+ * slot 33); 12 = the first gradient pass with the previous stage's x filter
+ * sweep (program 9, slot 36). */
 #define ASTR_PROF_SLOTS 39
 int astr_hip_profile_begin(astr_hip_ctx *ctx, int max_launches);
 int astr_hip_profile_end(astr_hip_ctx *ctx, double *ms, int *count);
@@ -244,15 +244,16 @@ int astr_hip_profile_end(astr_hip_ctx *ctx, double *ms, int *count);
  * each, on the context's stream, state restored afterwards) and keeps the
  * fastest; get/set read and override single selections. */
 int astr_hip_autotune(astr_hip_ctx *ctx, int reps);
-/* The last direction's gradient/convective work as one pass (split = 0) or as
- * two lighter passes (split = 1, programs 7 and 8); astr_hip_autotune sets
- * it from the timings. */
+/* Selected between two forms of the last gradient/convective pass when that
+ * pass carried both; the gradient passes have one form now, and the setting
+ * is only kept and read back.  Programs 7 and 8, its halves, are never
+ * launched. */
 int astr_hip_set_last_split(astr_hip_ctx *ctx, int split);
 /* Filter-sweep fusion of astr_hip_rk3_steps* (no reference counterpart).
  * filterq's sweeps act on different indices and are linear, so they commute.
  * - Compact-scheme solver's stage: it ends with z (in the RK pass), then y,
  *   then x.  With on != 0 the x sweep of every stage but a call's last runs
- *   inside the next stage's first convective+gradient pass (program 9),
+ *   inside the next stage's first gradient pass (program 9),
  *   which loads the same x-lines.  Off by default; astr_hip_autotune turns
  *   it on when its timing of program 9 is below those of programs 0 and 6
  *   along x together.

@@ -380,7 +380,8 @@ size_t pass_lds_bytes(int shape, int prog) {
   const ShapeInfo& s = kShapes[shape];
   const long long tl = (long long)s.TL * line_stride(s.P, s.R, s.TL);
   const long long one = (2 * tl > 2 * s.NT ? 2 * tl : 2 * s.NT) + kLineOff + 8 + kHaloSlot +
-                        coef_regions(prog) * 2 * s.P * s.R + halo_prims(prog, s.TL, true);
+                        coef_regions(prog) * 2 * s.P * s.R +
+                        halo_prims(prog == V_MID ? V_FIRST_G : prog, s.TL, true);
   return (size_t)one * sizeof(double);
 }
 
@@ -436,9 +437,36 @@ hipError_t launch_pass(int shape, int prog, int minb, const FlowArgs& a, int dir
   }
 }
 
-// register budget a pass uses until tuned: two workgroups per CU for the
-// gradient passes, one for the others
-int default_minb(int prog) { return prog <= GC_LAST || prog == FGC_FIRST ? 2 : 1; }
+// The launch shape a pass uses until tuned, from sweeps of every shape over
+// boxes of side 32..256 and 64^2..512^2 (microseconds per launch in brackets).
+// The shortest chunks that hold the line win wherever the kernels wait on
+// their own chains, which is everywhere below about 150 points a side: the 16 x 5
+// shape to n = 73, the 32 x 5 shape to n = 153 (stress pass at 96 x 80 x 63,
+// main path: 56 against 150 on 16 x 9).  Longer lines: one line per wavefront
+// along x; along y and z 8-line tiles, whose 64-byte row segments the memory
+// system needs once a pass is bound by it (256^3 y gradients 380 on 8 lines,
+// 436 on 4, 593 on 2), in the register footprint the pass has room for.  With
+// fewer lines than fill the chip with such tiles, two lines per workgroup
+// (2-D 300 x 181: RK pass 23 against 32).
+int default_shape(int prog, int dir, const int n3[3], int ndir) {
+  const int n = n3[dir];
+  const long long lines = (long long)(n3[0] + 1) * (n3[1] + 1) * (n3[2] + 1) / (n + 1);
+  const bool few = lines < 1024;
+  if (n <= 73 && !few) return 2;
+  if (n <= 153 && !few) return 4;
+  if (n <= 313) {
+    if (few) return dir == 0 ? 8 : 7;
+    if (dir == 0) return prog == F_ONLY && n <= 281 ? 6 : 8;
+    if (prog == V_LAST_RK) return 0;
+    if (n <= 281 && (prog == F_ONLY || prog == V_MID || prog == V_LAST_RHS)) return 3;
+    return 5;
+  }
+  if (dir == 0) return 12;
+  return few || ndir == 2 ? 1 : 11;
+}
+// and its register budget: the larger one only for the 64 x 9 shapes, which
+// spill at two waves per SIMD (512 x 512 RK pass 44 against 55)
+int default_minb(int shape) { return shape == 1 || shape == 12 ? 1 : 2; }
 
 }  // namespace
 
@@ -707,15 +735,30 @@ int pass(astr_hip_ctx* c, int prog, int d, int shape = -1) {
   return 0;
 }
 
+// Whether the stress pass may compute the x gradients: not where they
+// accumulate per-point metrics or take the closed form, and only on the x
+// gradient pass's launch shape, so that the gradients have the bits that pass
+// would give them (a shape's chunks fix how its solves round).
+bool own_gradx(const astr_hip_ctx* c) {
+  const FlowArgs& a = c->a;
+  return !(a.met || a.bnd[0] || a.bnd[1] || a.bnd[2]) && c->shape[GC_FIRST][0] == c->shape[V_MID][0];
+}
+
 // stats: the KE/enstrophy partial sums of the current state
 // diss_out (device, nullable): the dissipation rate of the current state,
-// evaluated after the gradient passes and before the last pass updates q
-int run_rhs(astr_hip_ctx* c, bool rk, bool stats, double* diss_out = nullptr) {
+// evaluated after the stress pass, which is the last to form gradients, and
+// before the last pass updates q
+// store_gx: every gradient is stored (gradcal)
+int run_rhs(astr_hip_ctx* c, bool rk, bool stats, double* diss_out = nullptr, bool store_gx = false) {
   FlowArgs& a = c->a;
   const int nd = a.ndir;
   // the shock sensor reads the velocity gradient
   const bool sensor = a.uwd && c->uw.sensor;
-  for (int d = 0; d < nd; d++) {
+  // the stress pass computes the x gradients itself unless they are needed
+  // before it or come with the x filter sweep
+  a.gradx = !sensor && !c->fx_pending && own_gradx(c) ? 1 : 0;
+  a.store_gx = a.gradx && (store_gx || diss_out) ? 1 : 0;
+  for (int d = a.gradx ? 1 : 0; d < nd; d++) {
     const int prog = d == nd - 1 ? GC_LAST : (d == 0 ? (c->fx_pending ? FGC_FIRST : GC_FIRST) : GC_MID);
     if (pass(c, prog, d)) return -1;
     if (d == 0) c->fx_pending = false;
@@ -731,20 +774,20 @@ int run_rhs(astr_hip_ctx* c, bool rk, bool stats, double* diss_out = nullptr) {
         return -1;
     }
   }
-  if (diss_out) {
-    const long long npts = (long long)a.n[0] * a.n[1] * (a.n[2] > 0 ? a.n[2] : 1);
-    const int nb = (int)std::min<long long>(kDissBlocks, (npts + 255) / 256);
-    hipLaunchKernelGGL(k_diss_part, dim3(nb), dim3(256), 0, c->stream, a, c->diss_part);
-    HIP_OK(hipGetLastError());
-    hipLaunchKernelGGL(k_diss_sum, dim3(1), dim3(256), 0, c->stream, c->diss_part, nb, diss_out, c->ke_scale);
-    HIP_OK(hipGetLastError());
-  }
   for (int d = 0; d < nd; d++) {
     const int prog = d == nd - 1 ? (rk ? V_LAST_RK : V_LAST_RHS) : V_MID;
     a.dostats = stats && d == 0 ? 1 : 0;  // the stress pass, along x, sums them
     const int rc = pass(c, prog, d);
     a.dostats = 0;
     if (rc) return -1;
+    if (d == 0 && diss_out) {
+        const long long npts = (long long)a.n[0] * a.n[1] * (a.n[2] > 0 ? a.n[2] : 1);
+        const int nb = (int)std::min<long long>(kDissBlocks, (npts + 255) / 256);
+        hipLaunchKernelGGL(k_diss_part, dim3(nb), dim3(256), 0, c->stream, a, c->diss_part);
+        HIP_OK(hipGetLastError());
+        hipLaunchKernelGGL(k_diss_sum, dim3(1), dim3(256), 0, c->stream, c->diss_part, nb, diss_out, c->ke_scale);
+        HIP_OK(hipGetLastError());
+    }
   }
   return 0;
 }
@@ -1138,6 +1181,9 @@ int rk3_run(astr_hip_ctx* c, int nsteps, const StatsBufs& sb, double* ke, double
   static const double rk[3][3] = {{1.0, 0.0, 1.0}, {0.75, 0.25, 0.25}, {1.0 / 3.0, 2.0 / 3.0, 2.0 / 3.0}};
   const bool want = ke || ens || diss;
   FlowArgs& a = c->a;
+  double* const q_home = a.q;
+  double* const qsave_home = a.qsave;
+  double* const qrhs_home = a.qrhs;
   double* const stats_keep = a.stats;
   double* const diss_keep = c->diss_part;
   a.stats = sb.part;
@@ -1172,6 +1218,14 @@ int rk3_run(astr_hip_ctx* c, int nsteps, const StatsBufs& sb, double* ke, double
         rc = -1;
         break;
       }
+      // the arrays change roles (FlowArgs::q)
+      if (s == 0) std::swap(a.q, a.qsave);
+      if (s == 1) std::swap(a.q, a.qrhs);
+      if (s == 2) {
+        a.q = q_home;
+        a.qsave = qsave_home;
+        a.qrhs = qrhs_home;
+      }
       if (want && s == 0) {
         hipLaunchKernelGGL(k_stats_reduce, dim3(1), dim3(256), 0, c->stream, sb.part, ntl,
                            sb.out + kStepStats * it, c->ke_scale);
@@ -1194,6 +1248,9 @@ int rk3_run(astr_hip_ctx* c, int nsteps, const StatsBufs& sb, double* ke, double
     }
   }
   c->fx_pending = false;
+  a.q = q_home;
+  a.qsave = qsave_home;
+  a.qrhs = qrhs_home;
   // the RK passes changed q after the last qswap
   c->halo_valid = false;
   a.stats = stats_keep;
@@ -1265,15 +1322,14 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   filter_coefs(cfg->alfa_filter, cfg->beta_halo, a.fc, h33);
   c->ke_scale = 1.0 / ((double)cfg->im * cfg->jm * (cfg->km > 0 ? cfg->km : 1));
   for (int d = 0; d < a.ndir; d++) {
-    const int sh = pick_shape(a.n[d]);
-    if (sh < 0) { delete c; return fail("no launch shape fits this line length"); }
+    if (pick_shape(a.n[d]) < 0) { delete c; return fail("no launch shape fits this line length"); }
     for (int pr = 0; pr < kNumProgs; pr++) {
-      int use = sh;
+      int use = default_shape(pr, d, a.n, a.ndir);
       for (int k = 0; k < kNumShapes && !selection_ok(use, pr, a.n[d], c->device); k++)
         use = k;
       if (!selection_ok(use, pr, a.n[d], c->device)) { delete c; return fail("no launch shape fits the LDS"); }
       c->shape[pr][d] = use;
-      c->minb[pr][d] = default_minb(pr);
+      c->minb[pr][d] = default_minb(use);
       c->tuned_ms[pr][d] = 0.f;
     }
   }
@@ -1570,7 +1626,7 @@ int astr_hip_filterq(astr_hip_ctx* c) {
 
 int astr_hip_gradcal(astr_hip_ctx* c, double* dvel, double* dtmp) {
   if (check_ctx(c)) return -1;
-  if (ensure_halo(c) || run_rhs(c, false, false)) return -1;
+  if (ensure_halo(c) || run_rhs(c, false, false, nullptr, true)) return -1;
   if (dvel && xfer(c, dvel, 9, c->a.dv, 0, 0)) return -1;
   if (dtmp && xfer(c, dtmp, 3, c->a.dv + 9 * c->a.fs, 0, 0)) return -1;
   return 0;
@@ -1711,16 +1767,23 @@ int astr_hip_autotune(astr_hip_ctx* c, int reps) {
   a.stage = 0;
   a.rk_a = 1.0; a.rk_b = 0.0; a.rk_c = 1.0;
   a.dostats = 0;
+  const bool gradx = !(a.met || a.bnd[0] || a.bnd[1] || a.bnd[2]);
+  a.gradx = gradx ? 1 : 0;
+  a.store_gx = 0;
   // the main path's RK pass is timed with the filter sweep it carries in
   // rk3 steps
   a.rk_filter = a.main_sem && c->fuse_main_filter ? 1 : 0;
   int rc = 0;
-  for (int pr = 0; pr < kNumProgs && !rc; pr++) {
+  for (int k = 0; k < kNumProgs && !rc; k++) {
+    const int pr = (k + 1) % kNumProgs;  // GC_FIRST last
     for (int d = 0; d < a.ndir && !rc; d++) {
       if (!pass_used(pr, d, a.ndir) || (pr == FGC_FIRST && a.main_sem)) continue;
       float best = 1e30f;
       for (int sh = 0; sh < kNumShapes && !rc; sh++) {
         if (!selection_ok(sh, pr, a.n[d], c->device)) continue;
+        // the x gradient pass takes the stress pass's shape (own_gradx),
+        // which is tuned before it
+        if (pr == GC_FIRST && gradx && sh != c->shape[V_MID][0]) continue;
         for (int mb = 1; mb <= kMinbVariants && !rc; mb++) {
           hipError_t e = launch_pass(sh, pr, mb, a, d, c->stream);
           if (e == hipSuccess) e = hipEventRecord(e0, c->stream);
@@ -1745,9 +1808,28 @@ int astr_hip_autotune(astr_hip_ctx* c, int reps) {
     }
   }
   if (!rc) {
-    // the filtering first pass against the first pass plus the x filter pass
-    if (!rc && !a.main_sem)
-      c->fuse_fx = c->tuned_ms[FGC_FIRST][0] < c->tuned_ms[GC_FIRST][0] + c->tuned_ms[F_ONLY][0];
+    // the x sweep inside the first gradient pass, which then stores the x
+    // gradients, against the x filter pass and the stress pass that computes
+    // them: each form's launches up to the stress pass, timed together
+    if (!rc && !a.main_sem && gradx) {
+      float form_ms[2] = {0.f, 0.f};
+      for (int f = 0; f < 2 && !rc; f++) {
+        a.gradx = f ? 0 : 1;
+        auto form = [&]() -> int {
+          if (pass(c, f ? FGC_FIRST : F_ONLY, 0)) return -1;
+          return pass(c, a.ndir == 2 ? GC_LAST : GC_MID, 1) || pass(c, V_MID, 0) ? -1 : 0;
+        };
+        if (form()) rc = -1;
+        hipError_t e = rc ? hipErrorUnknown : hipEventRecord(e0, c->stream);
+        for (int r = 0; r < reps && e == hipSuccess; r++)
+          if (form()) e = hipErrorUnknown;
+        if (e == hipSuccess) e = hipEventRecord(e1, c->stream);
+        if (e == hipSuccess) e = hipEventSynchronize(e1);
+        if (e == hipSuccess) e = hipEventElapsedTime(&form_ms[f], e0, e1);
+        if (e != hipSuccess && !rc) rc = fail(std::string("autotune forms: ") + hipGetErrorString(e));
+      }
+      if (!rc) c->fuse_fx = form_ms[1] < form_ms[0];
+    }
   }
   a = keep;
   hipError_t e = hipMemcpyAsync(a.q, snap, qbytes, hipMemcpyDeviceToDevice, c->stream);
@@ -2157,14 +2239,21 @@ hipError_t launch_batch(int shape, int prog, int minb, const BatchLaunch& bl, in
 // the eight pass slots of a stage: GC x,y,z; V x,y,z; F y,x (the filter
 // sweeps in the single-case stage's order).  The program a case of nd
 // directions runs in slot (kind, d), or -1.
+// The x gradients come with the stress pass (V x).
 int slot_prog(int kind, int d, int nd) {
-  if (kind == 0) return d < nd ? (d == nd - 1 ? GC_LAST : (d == 0 ? GC_FIRST : GC_MID)) : -1;
+  if (kind == 0) return d > 0 && d < nd ? (d == nd - 1 ? GC_LAST : GC_MID) : -1;
   if (kind == 1) return d < nd ? (d == nd - 1 ? V_LAST_RK : V_MID) : -1;
   return d < nd - 1 ? F_ONLY : -1;
 }
 const int kSlotKind[8] = {0, 0, 0, 1, 1, 1, 2, 2};
 const int kSlotDir[8] = {0, 1, 2, 0, 1, 2, 1, 0};
 constexpr int kSlotStats = 3;  // V x, which sums the statistics
+
+// work items of a batched pass of nt tiles
+int batch_items(int prog, int dir, int nt) {
+  if ((prog == V_MID && dir == 0) || !pass_one(prog, false, dir == 1, nt)) return nt;
+  return nt * pass_fields(prog, false);
+}
 
 struct BatchGroup {
   int slot, prog, dir, shape, minb, nblocks;
@@ -2253,7 +2342,8 @@ int build_groups(astr_hip_batch* b) {
     // budget keeps resident (minb per CU), never more than the tiles
     // (a 128-thread workgroup is half a 256-thread one: twice as many fit)
     const int cap = b->ncu * g.minb * (kShapes[g.shape].NT < 256 ? 256 / kShapes[g.shape].NT : 1);
-    int nb = g.bl.total < cap ? g.bl.total : cap;
+    const int items = batch_items(g.prog, g.dir, g.bl.total);
+    int nb = items < cap ? items : cap;
     g.nblocks = (nb + 7) / 8 * 8;
   }
   return 0;
@@ -2304,14 +2394,16 @@ int upload_jobs(astr_hip_batch* b) {
 int enqueue_step(astr_hip_batch* b) {
   static const double rk[3][3] = {{1.0, 0.0, 1.0}, {0.75, 0.25, 0.25}, {1.0 / 3.0, 2.0 / 3.0, 2.0 / 3.0}};
   for (int s = 0; s < 3; s++) {
-    StageArgs sa{s, s == 0 ? 1 : 0, rk[s][0], rk[s][1], rk[s][2]};
+    StageArgs sa{s, s == 0 ? 1 : 0, rk[s][0], rk[s][1], rk[s][2], s};
     StageArgs sv = sa;
     sv.dostats = 0;
+    StageArgs sf = sv;  // the filter passes after the update
+    sf.alt = (s + 1) % 3;
     for (int sl = 0; sl < 8; sl++) {
       for (auto& g : b->groups) {
         if (g.slot != sl) continue;
-        HIP_OK(launch_batch(g.shape, g.prog, g.minb, g.bl, g.dir, sl == kSlotStats ? sa : sv, g.nblocks,
-                            b->stream));
+        HIP_OK(launch_batch(g.shape, g.prog, g.minb, g.bl, g.dir,
+                            sl == kSlotStats ? sa : (kSlotKind[sl] == 2 ? sf : sv), g.nblocks, b->stream));
       }
       if (sl == kSlotStats && s == 0) {
         hipLaunchKernelGGL(k_stats_batch, dim3((unsigned)b->cases.size()), dim3(256), 0, b->stream,
@@ -2474,7 +2566,7 @@ int astr_hip_batch_autotune(astr_hip_batch* b, int reps) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (!rc && (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess))
     rc = fail("hipEventCreate failed");
-  const StageArgs sa{0, 0, 1.0, 0.0, 1.0};
+  const StageArgs sa{0, 0, 1.0, 0.0, 1.0, 0};
   for (int sl = 0; sl < 8 && !rc; sl++) {
     const int kind = kSlotKind[sl], d = kSlotDir[sl];
     // classes: cases of this slot with the same program and the same set of
@@ -2518,7 +2610,8 @@ int astr_hip_batch_autotune(astr_hip_batch* b, int reps) {
         BatchLaunch bl{dargs, dts, nm, ts[nm]};
         for (int mb = 1; mb <= kMinbVariants && !rc; mb++) {
           const int cap = b->ncu * mb * (kShapes[sh].NT < 256 ? 256 / kShapes[sh].NT : 1);
-          const int nb = ((bl.total < cap ? bl.total : cap) + 7) / 8 * 8;
+          const int items = batch_items(prog, d, bl.total);
+          const int nb = ((items < cap ? items : cap) + 7) / 8 * 8;
           hipError_t e = launch_batch(sh, prog, mb, bl, d, sa, nb, b->stream);
           if (e == hipSuccess) e = hipEventRecord(e0, b->stream);
           for (int r = 0; r < reps && e == hipSuccess; r++) e = launch_batch(sh, prog, mb, bl, d, sa, nb, b->stream);
@@ -2540,6 +2633,9 @@ int astr_hip_batch_autotune(astr_hip_batch* b, int reps) {
           b->cases[i]->shape[prog][d] = bsh;
           b->cases[i]->minb[prog][d] = bmb;
           b->cases[i]->tuned_ms[prog][d] = best / reps;
+          // the batch's stress pass computes the x gradients; so does the
+          // case's own with both on one shape (own_gradx)
+          if (prog == V_MID && d == 0) b->cases[i]->shape[GC_FIRST][0] = bsh;
         }
     }
   }

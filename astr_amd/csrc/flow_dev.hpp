@@ -30,13 +30,19 @@ struct FlowArgs {
   double alfa, bhalo;   // filter alpha and halo-row beta (LHS of the filter rows)
   int stage;            // 0,1,2
   int dostats;          // stage-1 KE/enstrophy partial sums (1) or none (0)
+  // q holds the current state.  No RK stage updates it in place or copies it:
+  // the arrays change roles (rk3_run).  The first stage leaves q as the saved
+  // state and writes the new one to qsave; the second writes it over qrhs,
+  // whose values it is the last to read; the third, with the second's q as
+  // its qrhs, writes it over the saved state, so a step starts and ends in
+  // one array.
   double* q;            // 5 fields
   double* qsave;        // 5 fields
   double* qrhs;         // 5 fields
   double* dv;           // 12 fields: dvel(m,d) at m+3d, dtmp(d) at 9+d
   double* sg;           // 9 fields: sigma 11,12,13,22,23,33, qflux 1,2,3
-  double* p;            // the pressure of q (miniapp; written by the first
-                        // gradient pass, read by the passes that follow)
+  double* p;            // the pressure of q (miniapp; written by the stage's
+                        // first gradient pass, read by the passes that follow)
   double* stats;        // 2 doubles per tile
   const double* dac[3]; // derivative LU tables [ac1|ac2|ac3] per direction
   const double* fac[3]; // filter LU tables
@@ -64,6 +70,9 @@ struct FlowArgs {
   // main path: the RK pass also applies the next stage's filterq sweep along
   // its direction to the new q, after updatefvar took the primitives
   int rk_filter;
+  // the stress pass computes the x gradients itself (its lines are x-lines),
+  // no x gradient pass before it; store_gx: it also stores them
+  int gradx, store_gx;
 };
 
 // Halo sources kept by qswap for the lines whose halo the reference fills
@@ -93,14 +102,19 @@ __host__ __device__ inline int halo_src_index(const int n[3], int ndir, int dir,
   return -1;
 }
 
-// Pass programs.  Per stage: the gradients of u, v, w and T along x, y, z
-// (GC_FIRST, GC_MID, GC_LAST), then per direction the derivative of the whole
-// flux, viscous minus convective (V_MID along x and y, V_LAST_RHS or
-// V_LAST_RK along the last direction).  Taking the two fluxes' difference
-// before the line solve leaves 5 solves per direction where separate
-// derivatives take 9, and qrhs is accumulated once per direction.
-//   V_MID along x (kernel V_FIRST) also forms the stress and heat flux, and
-//   the statistics, from the stored gradients;
+// Pass programs.  Per stage: the gradients of u, v, w and T along y and z
+// (GC_MID, GC_LAST), then per direction the derivative of the whole flux,
+// viscous minus convective (V_MID along x and y, V_LAST_RHS or V_LAST_RK along
+// the last direction).  Taking the two fluxes' difference before the line
+// solve leaves 5 solves per direction where separate derivatives take 9, and
+// qrhs is accumulated once per direction.
+//   V_MID along x (kernels V_FIRST and V_FIRST_G) also forms the stress and
+//   heat flux, and the statistics, from the gradients; V_FIRST_G computes the
+//   x gradients itself, on the lines it holds anyway, which saves a pass that
+//   would read q and store four fields for this one to read back;
+//   GC_FIRST is the x gradients on their own, stored, where something else
+//   reads them: the shock sensor, per-point metrics (whose gradients
+//   accumulate over the directions), physical ends;
 //   FGC_FIRST is GC_FIRST preceded by the previous stage's filter sweep along
 //   the same lines (x): it filters the q it loads, writes it back and goes on
 //   with the filtered values (the sweeps along different indices commute, so
@@ -108,8 +122,8 @@ __host__ __device__ inline int halo_src_index(const int n[3], int ndir, int dir,
 // Ids 7 and 8 were the halves of a split last gradient pass; they stay
 // reserved so that the ids of the launch selection keep their meaning.
 enum Prog { GC_FIRST = 0, GC_MID, GC_LAST, V_MID, V_LAST_RHS, V_LAST_RK, F_ONLY, RESERVED_7, RESERVED_8,
-            FGC_FIRST, V_FIRST };
-constexpr int kNumProgs = 10;  // V_FIRST is V_MID's kernel along x, no id of its own
+            FGC_FIRST, V_FIRST, V_FIRST_G };
+constexpr int kNumProgs = 10;  // V_FIRST, V_FIRST_G: V_MID's kernels along x, no ids of their own
 
 // ntiles of direction dir for lines-per-tile TL
 __host__ __device__ inline int tiles_of(const int n[3], int dir, int TL) {
@@ -194,7 +208,7 @@ constexpr int coef_regions(int prog) { return prog == V_LAST_RK || prog == FGC_F
 // Main path, gradient passes: the primitives u, v, w, T of the halo copies
 // (kHaloSrcRows per line), evaluated once by the slots that own them.
 constexpr int halo_prims(int prog, int TL, bool main_sem) {
-  return main_sem && prog <= GC_LAST ? 4 * kHaloSrcRows * TL : 0;
+  return main_sem && (prog <= GC_LAST || prog == V_FIRST_G) ? 4 * kHaloSrcRows * TL : 0;
 }
 template <class C>
 constexpr int lds_doubles(int prog, bool main_sem = false) {
@@ -381,6 +395,7 @@ __device__ __forceinline__ double conv_flux(int m, int dir, double qm, double uu
 
 // Sutherland (tgvsolver.F90:123-140)
 __device__ __forceinline__ double miucal(const FlowArgs& a, double t) {
+#pragma clang fp contract(off)
   return t * sqrt(t) * a.suth1 / (t + a.suth);
 }
 
@@ -389,10 +404,21 @@ struct StageArgs {
   int stage;            // 0,1,2
   int dostats;          // stage-1 KE/enstrophy partial sums (1) or none (0)
   double rk_a, rk_b, rk_c;
+  int alt;              // batches: stages whose change of array roles applies (0, 1, 2)
 };
 
+// the arrays in their roles after `alt` stages of a step
+struct Arrays {
+  double *q, *qsave, *qrhs;
+};
+__device__ __forceinline__ Arrays arrays_of(const FlowArgs& a, int alt) {
+  if (alt == 0) return Arrays{a.q, a.qsave, a.qrhs};
+  if (alt == 1) return Arrays{a.qsave, a.q, a.qrhs};
+  return Arrays{a.qrhs, a.q, a.qsave};
+}
+
 __device__ __forceinline__ StageArgs stage_of(const FlowArgs& a) {
-  return StageArgs{a.stage, a.dostats, a.rk_a, a.rk_b, a.rk_c};
+  return StageArgs{a.stage, a.dostats, a.rk_a, a.rk_b, a.rk_c, 0};
 }
 
 // q <- a*qsave + b*q + c*qrhs*dt in the reference's order (tgvsolver.F90:1055-1057)
@@ -497,9 +523,10 @@ __device__ __forceinline__ double visc_col_full(const FlowArgs& a, int dir, int 
 // later qswap step averages take the values kept before that step (hx / hy),
 // the others the current q of the source point, which the slot owns.
 template <class C>
-__device__ __forceinline__ double halo_q(const FlowArgs& a, const Slots<C>& S, int t, int dir, int m) {
+__device__ __forceinline__ double halo_q(const FlowArgs& a, const double* q, const Slots<C>& S, int t, int dir,
+                                         int m) {
   if (S.ex[t] >= 0) return (dir == 0 ? a.hx + m * a.hxs : a.hy + m * a.hys)[S.ex[t]];
-  return ldg(a.q + m * a.fs, S.g[t]);
+  return ldg(q + m * a.fs, S.g[t]);
 }
 
 // main path RK3 update (src/mainloop.F90:441-449):
@@ -513,16 +540,20 @@ __device__ __forceinline__ double rk_update_main(const StageArgs& sa, double dt,
 // ---------------------------------------------------------------------------
 // the pass kernel
 // ---------------------------------------------------------------------------
-// stress and heat flux of a point from its stored gradients (diffusion,
-// tgvsolver.F90:659-694) and its terms of the statistics (stacal, :893-942)
-__device__ __forceinline__ void stress_point(const FlowArgs& a, unsigned o, const Prim& P, double f[9],
-                                             bool stats, double& sk, double& se) {
+// stress and heat flux of a point from its gradients (diffusion,
+// tgvsolver.F90:659-694) and its terms of the statistics (stacal, :893-942);
+// gx: the x gradients of u, v, w, T where the pass has them, nullptr: stored
+__device__ __forceinline__ void stress_point(const FlowArgs& a, unsigned o, const Prim& P, const double* gx,
+                                             double f[9], bool stats, double& sk, double& se) {
+#pragma clang fp contract(off)
   double g[3][3], gt[3];
 #pragma unroll
   for (int d = 0; d < 3; d++) {
+    const bool own = d == 0 && gx;
 #pragma unroll
-    for (int m = 0; m < 3; m++) g[m][d] = d < a.ndir ? ldg(a.dv + (m + 3 * d) * a.fs, o) : 0.0;
-    gt[d] = d < a.ndir ? ldg(a.dv + (9 + d) * a.fs, o) : 0.0;
+    for (int m = 0; m < 3; m++)
+      g[m][d] = own ? gx[m] : (d < a.ndir ? ldg(a.dv + (m + 3 * d) * a.fs, o) : 0.0);
+    gt[d] = own ? gx[3] : (d < a.ndir ? ldg(a.dv + (9 + d) * a.fs, o) : 0.0);
   }
   visc_flux(a, g, gt, P, f);
   if (stats) {
@@ -545,9 +576,16 @@ __device__ __forceinline__ void stress_point(const FlowArgs& a, unsigned o, cons
 // Each pass reads its chunk factors back from LDS before each solve instead
 // of holding them in registers, and issues a solve's accumulation loads and
 // the next solve's inputs before it, so that their latency overlaps it.
-template <class C, int PROG, bool MAIN = false, bool GEN = false>
-__device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa, int dir, int tile,
-                                          double* smem) {
+// A: the arrays of the current state, the saved one and qrhs (FlowArgs::q).
+// ONE: the workgroup takes one component (`field`) of the pass, five or four
+// workgroups share a tile.  The components' solves are independent, and
+// where a pass has few tiles their serial chain in one workgroup is its time.
+template <class C, int PROG, bool MAIN = false, bool GEN = false, bool ONE = false>
+__device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa, const Arrays& A, int dir, int tile,
+                                          double* smem, int field = 0) {
+  double* const qc = A.q;
+  double* const qo = A.qsave;
+  double* const qrhs = A.qrhs;
   constexpr int NPT = C::NPT;
   constexpr int kDummy = C::TL * C::LT;
   const int n = a.n[dir];
@@ -592,77 +630,46 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
     __syncthreads();
   };
 
-  if constexpr (PROG == GC_FIRST || PROG == FGC_FIRST || PROG == GC_MID) {
-    // gradients of u, v, w, T along dir (gradcal, tgvsolver.F90:450-537;
-    // src/comsolver.F90:280-321)
-    constexpr bool FIRST = PROG != GC_MID;
-    cs = stage_chunk_coefs<C>(a.dac[dir], n + 3, smem, 0);
+  // Gradients of u, v, w, T along dir (gradcal, tgvsolver.F90:450-537;
+  // src/comsolver.F90:280-321).  Miniapp: of q; the stage's first gradient
+  // pass forms the pressure and leaves it for the others.  Main path: of the
+  // stored primitives, with the halo copies from the primitives of the halo's
+  // q (qswap's q2fvar).
+  constexpr bool GRAD = PROG == GC_FIRST || PROG == FGC_FIRST || PROG == GC_MID || PROG == V_FIRST_G;
+  double pv[4][GRAD ? NPT : 1];
+  double* hal = smem + lds_doubles<C>(PROG);
+  auto hslot = [&](int t) {  // the slot's halo primitives, written and read by its own thread
+    const int l = S.s[t] / C::LT, r = S.s[t] - l * C::LT;
+    return hal + 4 * (l * kHaloSrcRows + (r <= 5 ? r - 1 : r - (n - 5) + 5));
+  };
+  auto load_prims = [&]() __attribute__((always_inline)) {
     if constexpr (MAIN) {
-      // the stored u, v, w, T; the halo copies from the primitives of the
-      // halo's q (qswap's q2fvar)
-      double pv[4][NPT];
 #pragma unroll
       for (int t = 0; t < NPT; t++)
 #pragma unroll
         for (int c = 0; c < 4; c++) pv[c][t] = ldg(a.pr + (c < 3 ? 1 + c : 5) * fs, S.g[t]);
-      double* hal = smem + lds_doubles<C>(PROG);
-      auto hslot = [&](int t) {  // the slot's halo primitives, written and read by its own thread
-        const int l = S.s[t] / C::LT, r = S.s[t] - l * C::LT;
-        return hal + 4 * (l * kHaloSrcRows + (r <= 5 ? r - 1 : r - (n - 5) + 5));
-      };
 #pragma unroll
       for (int t = 0; t < NPT; t++) {
         if (S.h[t] != kDummy) {
           double qh[5];
 #pragma unroll
-          for (int m = 0; m < 5; m++) qh[m] = halo_q<C>(a, S, t, dir, m);
+          for (int m = 0; m < 5; m++) qh[m] = halo_q<C>(a, qc, S, t, dir, m);
           const Prim P = prim_of(a, qh[0], qh[1], qh[2], qh[3], qh[4]);
           double* h = hslot(t);
           h[0] = P.u; h[1] = P.v; h[2] = P.w; h[3] = P.t;
         }
       }
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-#pragma unroll
-        for (int t = 0; t < NPT; t++) {
-          T[kLineOff + S.s[t]] = pv[c][t];
-          if (S.h[t] != kDummy) T[kLineOff + S.h[t]] = hslot(t)[c];
-        }
-        derive();
-        const int fld = c < 3 ? c + 3 * dir : 9 + dir;
-#pragma unroll
-        for (int t = 0; t < NPT; t++) {
-          const unsigned o = S.g[t];
-          const double x = X[S.s[t]];
-          if (GEN && a.met) {
-            // gradcal's accumulation dvel(m,n) += D_d(u_m) dxi(d,n) over
-            // every n (src/comsolver.F90:300-321)
-#pragma unroll
-            for (int nn = 0; nn < 3; nn++) {
-#pragma clang fp contract(off)
-              if (nn >= a.ndir) continue;
-              const int f2 = c < 3 ? c + 3 * nn : 9 + nn;
-              const double v = x * ldg(a.met + (1 + dir + 3 * nn) * fs, o);
-              if (FIRST) stg(a.dv + f2 * fs, o, v);
-              else stg(a.dv + f2 * fs, o, ldg(a.dv + f2 * fs, o) + v);
-            }
-          } else {
-            // dvel(m,n) = D_d(u_m) dxi(d,n): dxi(d,d) of the uniform grid
-            stg(a.dv + fld * fs, o, x * met_of(a, dir).d);
-          }
-        }
-      }
     } else {
-      // the first pass takes q and leaves the pressure for the others
+      constexpr bool PRES = PROG == GC_FIRST || PROG == FGC_FIRST;
       double qv[5][NPT];
 #pragma unroll
       for (int t = 0; t < NPT; t++)
 #pragma unroll
-        for (int m = 0; m < 5; m++) qv[m][t] = ldg(!FIRST && m == 4 ? a.p : a.q + m * fs, S.g[t]);
+        for (int m = 0; m < 5; m++) qv[m][t] = ldg(!PRES && m == 4 ? a.p : qc + m * fs, S.g[t]);
       if constexpr (PROG == FGC_FIRST) {
         // the previous stage's filter sweep along these lines (filterq,
         // tgvsolver.F90:805-825), as the filter pass does it, on the loaded
-        // q; the filtered q is stored and the gradients below take it
+        // q; the filtered q is stored and the gradients take it
         filter_setup(1);
 #pragma unroll
         for (int m = 0; m < 5; m++) {
@@ -672,74 +679,170 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
 #pragma unroll
           for (int t = 0; t < NPT; t++) {
             qv[m][t] = X[S.s[t]];
-            stg(a.q + m * fs, S.g[t], qv[m][t]);
+            stg(qc + m * fs, S.g[t], qv[m][t]);
           }
         }
       }
 #pragma unroll
-      for (int c = 0; c < 4; c++) {
-#pragma unroll
-        for (int t = 0; t < NPT; t++) {
-          double f;
-          if (c < 3) {
-            f = qv[c + 1][t] / qv[0][t];
-          } else {
-            double pr = qv[4][t];
-            if constexpr (FIRST) {
-              pr = pressure_of(a, qv[0][t], qv[1][t], qv[2][t], qv[3][t], qv[4][t]);
-              stg(a.p, S.g[t], pr);
-            }
-            f = pr / qv[0][t] * a.const2;
-          }
-          put<C>(T, S, t, f);
+      for (int t = 0; t < NPT; t++) {
+        double pr = qv[4][t];
+        if constexpr (PRES) {
+          pr = pressure_of(a, qv[0][t], qv[1][t], qv[2][t], qv[3][t], qv[4][t]);
+          stg(a.p, S.g[t], pr);
         }
-        derive();
-        const int fld = c < 3 ? c + 3 * dir : 9 + dir;
 #pragma unroll
-        for (int t = 0; t < NPT; t++) stg(a.dv + fld * fs, S.g[t], X[S.s[t]] * idn);
+        for (int c = 0; c < 3; c++) pv[c][t] = qv[c + 1][t] / qv[0][t];
+        pv[3][t] = pr / qv[0][t] * a.const2;
       }
     }
-  } else if constexpr (PROG == V_FIRST || PROG == V_MID || PROG == V_LAST_RK) {
+  };
+  // derivative of component c (u, v, w, T), left in X
+  auto gradient = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < NPT; t++) {
+      if constexpr (MAIN) {
+        T[kLineOff + S.s[t]] = pv[c][t];
+        if (S.h[t] != kDummy) T[kLineOff + S.h[t]] = hslot(t)[c];
+      } else {
+        put<C>(T, S, t, pv[c][t]);
+      }
+    }
+    derive();
+  };
+
+  // one component's primitive alone, in pv[0]
+  auto load_one = [&](int c) __attribute__((always_inline)) {
+    if constexpr (MAIN) {
+#pragma unroll
+      for (int t = 0; t < NPT; t++) pv[0][t] = ldg(a.pr + (c < 3 ? 1 + c : 5) * fs, S.g[t]);
+#pragma unroll
+      for (int t = 0; t < NPT; t++) {
+        if (S.h[t] != kDummy) {
+          const double r = halo_q<C>(a, qc, S, t, dir, 0);
+          if (c < 3) {
+            hslot(t)[0] = halo_q<C>(a, qc, S, t, dir, c + 1) / r;
+          } else {
+            double qh[5];
+#pragma unroll
+            for (int m = 1; m < 5; m++) qh[m] = halo_q<C>(a, qc, S, t, dir, m);
+            hslot(t)[0] = prim_of(a, r, qh[1], qh[2], qh[3], qh[4]).t;
+          }
+        }
+      }
+    } else {
+      constexpr bool PRES = PROG == GC_FIRST;
+      double r[NPT];
+#pragma unroll
+      for (int t = 0; t < NPT; t++) {
+        r[t] = ldg(qc, S.g[t]);
+        pv[0][t] = ldg(c < 3 ? qc + (c + 1) * fs : (PRES ? qc + 4 * fs : a.p), S.g[t]);
+      }
+      if (c < 3) {
+#pragma unroll
+        for (int t = 0; t < NPT; t++) pv[0][t] = pv[0][t] / r[t];
+      } else {
+#pragma unroll
+        for (int t = 0; t < NPT; t++) {
+          if constexpr (PRES) {
+            pv[0][t] = pressure_of(a, r[t], ldg(qc + fs, S.g[t]), ldg(qc + 2 * fs, S.g[t]), ldg(qc + 3 * fs, S.g[t]),
+                                   pv[0][t]);
+            stg(a.p, S.g[t], pv[0][t]);
+          }
+          pv[0][t] = pv[0][t] / r[t] * a.const2;
+        }
+      }
+    }
+  };
+
+  if constexpr (GRAD && PROG != V_FIRST_G) {
+    cs = stage_chunk_coefs<C>(a.dac[dir], n + 3, smem, 0);
+    if constexpr (ONE) load_one(field);
+    else load_prims();
+#pragma unroll
+    for (int cc = 0; cc < (ONE ? 1 : 4); cc++) {
+      const int c = ONE ? field : cc;
+      gradient(cc);
+      const int fld = c < 3 ? c + 3 * dir : 9 + dir;
+#pragma unroll
+      for (int t = 0; t < NPT; t++) {
+        const unsigned o = S.g[t];
+        const double x = X[S.s[t]];
+        if (GEN && a.met) {
+          // gradcal's accumulation dvel(m,n) += D_d(u_m) dxi(d,n) over
+          // every n (src/comsolver.F90:300-321)
+#pragma unroll
+          for (int nn = 0; nn < 3; nn++) {
+#pragma clang fp contract(off)
+            if (nn >= a.ndir) continue;
+            const int f2 = c < 3 ? c + 3 * nn : 9 + nn;
+            const double v = x * ldg(a.met + (1 + dir + 3 * nn) * fs, o);
+            if (PROG == GC_FIRST) stg(a.dv + f2 * fs, o, v);
+            else stg(a.dv + f2 * fs, o, ldg(a.dv + f2 * fs, o) + v);
+          }
+        } else {
+          // dvel(m,n) = D_d(u_m) dxi(d,n): dxi(d,d) of the uniform grid
+          stg(a.dv + fld * fs, o, x * (MAIN ? met_of(a, dir).d : idn));
+        }
+      }
+    }
+  } else if constexpr (PROG == V_FIRST || PROG == V_FIRST_G || PROG == V_MID || PROG == V_LAST_RK) {
     // The derivative along dir of the viscous (diffusion, tgvsolver.F90:
     // 700-787) minus the convective flux (convection, :539-633), the sign
     // qrhs has after rhscal, accumulated over the directions.  Viscous columns
     // per direction: x (s11,s12,s13,q1), y (s12,s22,s23,q2), z (s13,s23,s33,q3);
     // density has none.
-    constexpr bool FIRST = PROG == V_FIRST;
+    constexpr bool FIRST = PROG == V_FIRST || PROG == V_FIRST_G;
     constexpr bool RK = PROG == V_LAST_RK;
     // the main path's upwind-biased convection left its part in qrhs
     const bool uwd = MAIN && a.uwd;
     cs = stage_chunk_coefs<C>(a.dac[dir], n + 3, smem, 0);
     double sx[4][FIRST ? NPT : 1];
     if constexpr (FIRST) {
-      // Stress and heat flux of every point from the stored gradients, here
+      // Stress and heat flux of every point from the gradients, here
       // because x-lines leave a lane only NPT points to hold; columns s11 and
       // q1, which no other direction reads, stay in registers.  And the
       // stage-1 KE / enstrophy partial sums.
+      double gx[4][PROG == V_FIRST_G ? NPT : 1];
+      if constexpr (PROG == V_FIRST_G) {
+        load_prims();
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          gradient(c);
+#pragma unroll
+          for (int t = 0; t < NPT; t++) {
+            gx[c][t] = X[S.s[t]] * (MAIN ? met_of(a, dir).d : idn);
+            if (a.store_gx) stg(a.dv + (c < 3 ? c : 9) * fs, S.g[t], gx[c][t]);
+          }
+        }
+      }
       double sk = 0.0, se = 0.0;
 #pragma unroll
       for (int t = 0; t < NPT; t++) {
         const unsigned o = S.g[t];
         Prim P;
-        if constexpr (MAIN) {
+        P.p = 0.0;
+        if constexpr (PROG == V_FIRST_G) {
+          P.r = sa.dostats ? ldg(MAIN ? a.pr : qc, o) : 0.0;
+          P.u = pv[0][t]; P.v = pv[1][t]; P.w = pv[2][t]; P.t = pv[3][t];
+        } else if constexpr (MAIN) {
           // diffrsdcal6 (src/solver.F90:2433-2545) and the statistics
           // (statistic.F90:871-992) take the stored rho, vel, tmp
           P.r = sa.dostats ? ldg(a.pr, o) : 0.0;
           P.u = ldg(a.pr + fs, o);
           P.v = ldg(a.pr + 2 * fs, o);
           P.w = ldg(a.pr + 3 * fs, o);
-          P.p = 0.0;
           P.t = ldg(a.pr + 5 * fs, o);
         } else {
-          P.r = ldg(a.q, o);
-          P.u = ldg(a.q + fs, o) / P.r;
-          P.v = ldg(a.q + 2 * fs, o) / P.r;
-          P.w = ldg(a.q + 3 * fs, o) / P.r;
-          P.p = ldg(a.p, o);
-          P.t = P.p / P.r * a.const2;
+          P.r = ldg(qc, o);
+          P.u = ldg(qc + fs, o) / P.r;
+          P.v = ldg(qc + 2 * fs, o) / P.r;
+          P.w = ldg(qc + 3 * fs, o) / P.r;
+          P.t = ldg(a.p, o) / P.r * a.const2;
         }
-        double f[9];
-        stress_point(a, o, P, f, sa.dostats && ((S.interior >> t) & 1), sk, se);
+        double f[9], gp[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) gp[c] = PROG == V_FIRST_G ? gx[c][PROG == V_FIRST_G ? t : 0] : 0.0;
+        stress_point(a, o, P, PROG == V_FIRST_G ? gp : nullptr, f, sa.dostats && ((S.interior >> t) & 1), sk, se);
         const bool all = GEN && a.met;
 #pragma unroll
         for (int m = 0; m < 9; m++)
@@ -784,11 +887,11 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
         const unsigned o = S.g[t];
         if constexpr (MAIN) {
           // convrsdcal6 takes the stored vel and prs (src/solver.F90:2196-2207)
-          pp[t] = ldg(a.pr + 4 * fs, o);
-          ud[t] = ldg(a.pr + (1 + dir) * fs, o);
+          if (!ONE || field == 4 || field == dir + 1) pp[t] = ldg(a.pr + 4 * fs, o);
+          ud[t] = PROG == V_FIRST_G ? pv[0][t] : ldg(a.pr + (1 + dir) * fs, o);
         } else {
-          pp[t] = ldg(a.p, o);
-          ud[t] = ldg(a.q + (1 + dir) * fs, o) / ldg(a.q, o);
+          if (!ONE || field == 4 || field == dir + 1) pp[t] = ldg(a.p, o);
+          ud[t] = PROG == V_FIRST_G ? pv[0][t] : ldg(qc + (1 + dir) * fs, o) / ldg(qc, o);
         }
       }
       if constexpr (MAIN) {
@@ -797,7 +900,7 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
           if (S.h[t] != kDummy) {
             double qh[5];
 #pragma unroll
-            for (int m = 0; m < 5; m++) qh[m] = halo_q<C>(a, S, t, dir, m);
+            for (int m = 0; m < 5; m++) qh[m] = halo_q<C>(a, qc, S, t, dir, m);
             hp[t] = pressure_of(a, qh[0], qh[1], qh[2], qh[3], qh[4]);
             hu[t] = (dir == 0 ? qh[1] : (dir == 1 ? qh[2] : qh[3])) / qh[0];
           }
@@ -811,7 +914,7 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
     auto load_inputs = [&](int m) __attribute__((always_inline)) {
 #pragma unroll
       for (int t = 0; t < NPT; t++) {
-        if (!uwd || RK) qn[t] = ldg(a.q + m * fs, S.g[t]);
+        if (!uwd || RK) qn[t] = ldg(qc + m * fs, S.g[t]);
         if (!FIRST && m > 0 && !metg) {
           const int col = m == 4 ? 6 + dir : (dir == 1 ? (m == 1 ? 1 : (m == 2 ? 3 : 4)) : (m == 1 ? 2 : (m == 2 ? 4 : 5)));
           vn[t] = ldg(a.sg + col * fs, S.g[t]);
@@ -854,16 +957,16 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
             T[kLineOff + S.s[t]] = v - conv_flux_full(M, m, qn[t], ldg(a.pr + fs, o), ldg(a.pr + 2 * fs, o),
                                                       ldg(a.pr + 3 * fs, o), pp[t]);
             if (S.h[t] != kDummy) {
-              const double r = halo_q<C>(a, S, t, dir, 0);
-              T[kLineOff + S.h[t]] = v - conv_flux_full(M, m, halo_q<C>(a, S, t, dir, m),
-                                                        halo_q<C>(a, S, t, dir, 1) / r, halo_q<C>(a, S, t, dir, 2) / r,
-                                                        halo_q<C>(a, S, t, dir, 3) / r, hp[t]);
+              const double r = halo_q<C>(a, qc, S, t, dir, 0);
+              T[kLineOff + S.h[t]] = v - conv_flux_full(M, m, halo_q<C>(a, qc, S, t, dir, m),
+                                                        halo_q<C>(a, qc, S, t, dir, 1) / r, halo_q<C>(a, qc, S, t, dir, 2) / r,
+                                                        halo_q<C>(a, qc, S, t, dir, 3) / r, hp[t]);
             }
           } else {
             const Met M = met_of(a, dir);
             T[kLineOff + S.s[t]] = v - (conv_flux_main(M.j, M.d, m, dir, qn[t], ud[t], pp[t]) - f0);
             if (S.h[t] != kDummy) {
-              const double qh = S.ex[t] >= 0 ? halo_q<C>(a, S, t, dir, m) : qn[t];
+              const double qh = S.ex[t] >= 0 ? halo_q<C>(a, qc, S, t, dir, m) : qn[t];
               T[kLineOff + S.h[t]] = v - (conv_flux_main(M.j, M.d, m, dir, qh, hu[t], hp[t]) - f0);
             }
           }
@@ -894,18 +997,20 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
     };
     if constexpr (!RK) {
       const int m0 = uwd ? 1 : 0;
-      load_inputs(m0);
+      if (ONE && field < m0) return;  // without convection density has no flux
+      load_inputs(ONE ? field : m0);
 #pragma unroll
-      for (int m = 0; m < 5; m++) {
+      for (int mm = 0; mm < (ONE ? 1 : 5); mm++) {
+        const int m = ONE ? field : mm;
         if (m < m0) continue;
         stage_flux(m, first_part(m));
-        double* dst = a.qrhs + m * fs;
+        double* dst = qrhs + m * fs;
         double qr[NPT];
         if (!FIRST || uwd) {
 #pragma unroll
           for (int t = 0; t < NPT; t++) qr[t] = ldg(dst, S.g[t]);
         }
-        if (m < 4) load_inputs(m + 1);
+        if (!ONE && m < 4) load_inputs(m + 1);
         derive_flux(m);
 #pragma unroll
         for (int t = 0; t < NPT; t++) stg(dst, S.g[t], FIRST && !uwd ? dflux(t) : qr[t] + dflux(t));
@@ -914,52 +1019,44 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
       // each variable's RK3 stage update (tgvsolver.F90:1043-1059;
       // src/mainloop.F90:430-482) and, in the miniapp, its filter along dir
       // follow its flux derivative at once
+      // the state the step began with (qsave of the reference) is q itself
+      // in the first stage
+      double* const qnew = sa.stage == 1 ? qrhs : qo;
       double qr[NPT], qs[NPT];
       auto load_rk = [&](int m) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < NPT; t++) {
-          qr[t] = ldg(a.qrhs + m * fs, S.g[t]);
-          qs[t] = sa.stage == 0 ? 0.0 : ldg(a.qsave + m * fs, S.g[t]);
+          qr[t] = ldg(qrhs + m * fs, S.g[t]);
+          qs[t] = sa.stage == 0 ? 0.0 : ldg(qo + m * fs, S.g[t]);
         }
       };
-      load_inputs(0);
-      load_rk(0);
       if constexpr (!MAIN) {
+        // one component per workgroup (pass_one)
+        const int m = field;
+        load_inputs(m);
+        load_rk(m);
         filter_setup(1);
+        stage_flux(m, 0);
+        derive_flux(m);
 #pragma unroll
-        for (int m = 0; m < 5; m++) {
-          stage_flux(m, 0);
-          double qo[NPT];
+        for (int t = 0; t < NPT; t++)
+          put<C>(T, S, t, rk_update(sa, a.dt, sa.stage == 0 ? qn[t] : qs[t], qn[t], qr[t] + dflux(t)));
+        filter();
 #pragma unroll
-          for (int t = 0; t < NPT; t++) qo[t] = qn[t];
-          if (m < 4) load_inputs(m + 1);
-          derive_flux(m);
-#pragma unroll
-          for (int t = 0; t < NPT; t++) {
-            const double v = qr[t] + dflux(t);
-            double s0 = qs[t];
-            if (sa.stage == 0) {
-              stg(a.qsave + m * fs, S.g[t], qo[t]);
-              s0 = qo[t];
-            }
-            put<C>(T, S, t, rk_update(sa, a.dt, s0, qo[t], v));
-          }
-          if (m < 4) load_rk(m + 1);
-          filter();
-#pragma unroll
-          for (int t = 0; t < NPT; t++) stg(a.q + m * fs, S.g[t], X[S.s[t]]);
-        }
+        for (int t = 0; t < NPT; t++) stg(qnew + m * fs, S.g[t], X[S.s[t]]);
       } else {
+        load_inputs(0);
+        load_rk(0);
         // the new q, whose updatefvar ends the pass
         double qw[5][NPT];
 #pragma unroll
         for (int m = 0; m < 5; m++) {
           const bool solve = m > 0 || !uwd;  // without convection density has no flux
           if (solve) stage_flux(m, first_part(m));
-          double qo[NPT], ro[NPT], so[NPT];
+          double qm[NPT], ro[NPT], so[NPT];
 #pragma unroll
           for (int t = 0; t < NPT; t++) {
-            qo[t] = qn[t];
+            qm[t] = qn[t];
             ro[t] = qr[t];
             so[t] = qs[t];
           }
@@ -972,12 +1069,9 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
           for (int t = 0; t < NPT; t++) {
             const double v = solve ? ro[t] + dflux(t) : ro[t];
             const double jb = jac_of<GEN>(a, S.g[t]);
-            double s0 = so[t];
-            if (sa.stage == 0) {
-              s0 = qo[t] * jb;  // qsave = q J (src/mainloop.F90:423-427)
-              stg(a.qsave + m * fs, S.g[t], s0);
-            }
-            qw[m][t] = rk_update_main(sa, a.dt, jb, s0, qo[t], v);
+            // qsave = q J (src/mainloop.F90:423-427)
+            const double s0 = (sa.stage == 0 ? qm[t] : so[t]) * jb;
+            qw[m][t] = rk_update_main(sa, a.dt, jb, s0, qm[t], v);
           }
         }
         // updatefvar (fludyna.F90:191-242): rho, u, v, w, p, T of the new q
@@ -1005,26 +1099,27 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
             for (int t = 0; t < NPT; t++) put<C>(T, S, t, qw[m][t]);
             filter();
 #pragma unroll
-            for (int t = 0; t < NPT; t++) stg(a.q + m * fs, S.g[t], X[S.s[t]]);
+            for (int t = 0; t < NPT; t++) stg(qnew + m * fs, S.g[t], X[S.s[t]]);
           }
         } else {
           // q last: the halo copies of general grids are read from it above
 #pragma unroll
           for (int t = 0; t < NPT; t++)
 #pragma unroll
-            for (int m = 0; m < 5; m++) stg(a.q + m * fs, S.g[t], qw[m][t]);
+            for (int m = 0; m < 5; m++) stg(qnew + m * fs, S.g[t], qw[m][t]);
         }
       }
     }
   } else {  // F_ONLY: filter of q along dir, in place (filterq, tgvsolver.F90:791-883)
     filter_setup(0);
 #pragma unroll
-    for (int m = 0; m < 5; m++) {
+    for (int mm = 0; mm < (ONE ? 1 : 5); mm++) {
+      const int m = ONE ? field : mm;
 #pragma unroll
       for (int t = 0; t < NPT; t++)
-        put<C>(T, S, t, ldg(a.q + m * fs, S.g[t]));
+        put<C>(T, S, t, ldg(qc + m * fs, S.g[t]));
       filter();
-      double* dst = a.q + m * fs;
+      double* dst = qc + m * fs;
 #pragma unroll
       for (int t = 0; t < NPT; t++)
         stg(dst, S.g[t], X[S.s[t]]);
@@ -1040,7 +1135,43 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
 template <class C, int PROG, int MINB, bool MAIN = false, bool GEN = false>
 __global__ __launch_bounds__(C::NT, MINB) void k_pass(FlowArgs a, int dir) {
   extern __shared__ double smem[];
-  pass_body<C, PROG, MAIN, GEN>(a, stage_of(a), dir, xcd_tile(blockIdx.x, gridDim.x), smem);
+  pass_body<C, PROG, MAIN, GEN>(a, stage_of(a), arrays_of(a, 0), dir, xcd_tile(blockIdx.x, gridDim.x), smem);
+}
+
+// Components a pass runs as separate workgroups, 0: it cannot (the stress
+// pass's fluxes share the stress, the main path's RK pass ends with
+// updatefvar of all five).
+constexpr int pass_fields(int prog, bool main_sem) {
+  if (prog == GC_FIRST || prog == GC_MID || prog == GC_LAST) return 4;
+  if (prog == V_MID || prog == V_LAST_RHS || prog == F_ONLY || (prog == V_LAST_RK && !main_sem)) return 5;
+  return 0;
+}
+// Whether a pass of nt tiles runs one component per workgroup.  With few
+// tiles its time is one workgroup's chain of solves, which this divides by
+// the components; with many it only repeats each tile's set-up (the slots'
+// index arithmetic, the coefficients) and the loads components share.
+// Measured, us per launch, whole tile -> components: filter sweep 33^3 (69
+// tiles) 17 -> 9, 65^3 (265) 20 -> 15.6, 97^3 (1177) 34 -> 38; flux derivative
+// 11.7 -> 8.4, 16.1 -> 15.5, 33 -> 39; gradients 10.3 -> 7.6, 13.5 -> 12.2,
+// 23.8 -> 25.7, and where they form the pressure too 10.3 -> 9.2, 13.8 -> 16.5.
+// The RK pass solves twice per component and gains at every size (33^3 23.5
+// -> 12, 129^3 132 -> 129, 257^3 1080 -> 1034), so it has that form only.
+constexpr bool pass_one(int prog, bool main_sem, bool pres, int nt) {
+  if (pass_fields(prog, main_sem) == 0) return false;
+  if (prog == V_LAST_RK) return true;
+  if (prog == F_ONLY) return nt <= 512;
+  if (prog <= GC_LAST) return nt <= (pres ? 128 : 384);
+  return nt <= 320;
+}
+
+// one component of one pass per workgroup: the tile's components are
+// neighbouring blocks of one XCD, so what they share is read once into its L2
+template <class C, int PROG, int MINB, bool MAIN = false, bool GEN = false>
+__global__ __launch_bounds__(C::NT, MINB) void k_pass_one(FlowArgs a, int dir) {
+  extern __shared__ double smem[];
+  constexpr int NF = pass_fields(PROG, MAIN);
+  const int b = xcd_tile(blockIdx.x, gridDim.x);
+  pass_body<C, PROG, MAIN, GEN, true>(a, stage_of(a), arrays_of(a, 0), dir, b / NF, smem, b % NF);
 }
 
 // The tiles of one pass over several cases: case k owns global tiles
@@ -1055,19 +1186,23 @@ struct BatchLaunch {
 // one pass over a batch of cases: persistent blocks (grid a multiple of 8);
 // the blocks of XCD x walk the contiguous range [x*total/8, (x+1)*total/8) so
 // neighbouring tiles share that XCD's L2
-template <class C, int PROG, int MINB>
+template <class C, int PROG, int MINB, bool ONE = false>
 __global__ __launch_bounds__(C::NT, MINB) void k_pass_batch(BatchLaunch bl, int dir, StageArgs sa) {
   extern __shared__ double smem[];
   const int x = blockIdx.x & 7, per = gridDim.x >> 3;
-  const int lo = (int)((long long)bl.total * x / 8), hi = (int)((long long)bl.total * (x + 1) / 8);
-  for (int g = lo + (int)(blockIdx.x >> 3); g < hi; g += per) {
+  constexpr int NF = ONE ? pass_fields(PROG, false) : 1;
+  const long long total = (long long)bl.total * NF;
+  const int lo = (int)(total * x / 8), hi = (int)(total * (x + 1) / 8);
+  for (int e = lo + (int)(blockIdx.x >> 3); e < hi; e += per) {
+    const int g = e / NF;
     int kl = 0, kh = bl.ncases;  // tstart[kl] <= g < tstart[kh]
     while (kh - kl > 1) {
       const int mid = (kl + kh) >> 1;
       if (bl.tstart[mid] <= g) kl = mid;
       else kh = mid;
     }
-    pass_body<C, PROG>(bl.cases[kl], sa, dir, g - bl.tstart[kl], smem);
+    const FlowArgs& a = bl.cases[kl];
+    pass_body<C, PROG, false, false, ONE>(a, sa, arrays_of(a, sa.alt), dir, g - bl.tstart[kl], smem, e % NF);
     __syncthreads();
   }
 }
@@ -1077,22 +1212,38 @@ hipError_t launch_batch_c(int prog, const BatchLaunch& bl, int dir, const StageA
                           hipStream_t st) {
   const size_t lds = (size_t)lds_doubles<C>(prog) * sizeof(double);
   dim3 g(nblocks), b(C::NT);
+#define ASTR_BATCH_PASS(P, O) hipLaunchKernelGGL((k_pass_batch<C, P, MINB, O>), g, b, lds, st, bl, dir, sa)
+  const bool one = pass_one(prog, false, dir == 1, bl.total);
   switch (prog) {
-    case GC_FIRST: hipLaunchKernelGGL((k_pass_batch<C, GC_FIRST, MINB>), g, b, lds, st, bl, dir, sa); break;
+    // the y gradient pass is a stage's first: it forms the pressure
     case GC_MID:
-    case GC_LAST: hipLaunchKernelGGL((k_pass_batch<C, GC_MID, MINB>), g, b, lds, st, bl, dir, sa); break;
-    case V_MID:
-      if (dir == 0) hipLaunchKernelGGL((k_pass_batch<C, V_FIRST, MINB>), g, b, lds, st, bl, dir, sa);
-      else hipLaunchKernelGGL((k_pass_batch<C, V_MID, MINB>), g, b, lds, st, bl, dir, sa);
+    case GC_LAST:
+      if (dir == 1) {
+        if (one) ASTR_BATCH_PASS(GC_FIRST, true);
+        else ASTR_BATCH_PASS(GC_FIRST, false);
+      } else {
+        if (one) ASTR_BATCH_PASS(GC_MID, true);
+        else ASTR_BATCH_PASS(GC_MID, false);
+      }
       break;
-    case V_LAST_RK: hipLaunchKernelGGL((k_pass_batch<C, V_LAST_RK, MINB>), g, b, lds, st, bl, dir, sa); break;
+    case V_MID:
+      if (dir == 0) ASTR_BATCH_PASS(V_FIRST_G, false);
+      else if (one) ASTR_BATCH_PASS(V_MID, true);
+      else ASTR_BATCH_PASS(V_MID, false);
+      break;
+    case V_LAST_RK: ASTR_BATCH_PASS(V_LAST_RK, true); break;
     // single-case passes only
+    case GC_FIRST:
     case V_LAST_RHS:
     case FGC_FIRST:
     case RESERVED_7:
     case RESERVED_8: return hipErrorInvalidValue;
-    default: hipLaunchKernelGGL((k_pass_batch<C, F_ONLY, MINB>), g, b, lds, st, bl, dir, sa); break;
+    default:
+      if (one) ASTR_BATCH_PASS(F_ONLY, true);
+      else ASTR_BATCH_PASS(F_ONLY, false);
+      break;
   }
+#undef ASTR_BATCH_PASS
   return hipGetLastError();
 }
 
@@ -1101,18 +1252,64 @@ void launch_pass_m(int prog, const FlowArgs& a, int dir, hipStream_t st) {
   const int nt = tiles_of(a.n, dir, C::TL);
   const size_t lds = (size_t)lds_doubles<C>(prog, MAIN) * sizeof(double);
   dim3 g(nt), b(C::NT);
+  if constexpr (!GEN) {
+    const bool pres = !MAIN && (prog == GC_FIRST || (a.gradx && dir == 1));
+    if (!(prog == V_MID && dir == 0) && pass_one(prog, MAIN, pres, nt)) {
+      switch (prog) {
+        case GC_FIRST:
+        case GC_MID:
+        case GC_LAST:
+          if (pres || prog == GC_FIRST)
+            hipLaunchKernelGGL((k_pass_one<C, GC_FIRST, MINB, MAIN>), dim3(4 * nt), b, lds, st, a, dir);
+          else
+            hipLaunchKernelGGL((k_pass_one<C, GC_MID, MINB, MAIN>), dim3(4 * nt), b, lds, st, a, dir);
+          return;
+        case V_MID:
+        case V_LAST_RHS:
+          hipLaunchKernelGGL((k_pass_one<C, V_MID, MINB, MAIN>), dim3(5 * nt), b, lds, st, a, dir);
+          return;
+        case V_LAST_RK:
+          if constexpr (!MAIN) {
+            hipLaunchKernelGGL((k_pass_one<C, V_LAST_RK, MINB, false>), dim3(5 * nt), b, lds, st, a, dir);
+            return;
+          }
+          break;
+        case F_ONLY: hipLaunchKernelGGL((k_pass_one<C, F_ONLY, MINB, false>), dim3(5 * nt), b, lds, st, a, dir); return;
+        default: break;
+      }
+    }
+  }
   switch (prog) {
     case GC_FIRST: hipLaunchKernelGGL((k_pass<C, GC_FIRST, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
     case GC_MID:
-    case GC_LAST: hipLaunchKernelGGL((k_pass<C, GC_MID, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
+    case GC_LAST:
+      // miniapp, without an x gradient pass: the stage's first, which forms
+      // the pressure
+      if constexpr (!MAIN) {
+        if (a.gradx && dir == 1) {
+          hipLaunchKernelGGL((k_pass<C, GC_FIRST, MINB, false, false>), g, b, lds, st, a, dir);
+          break;
+        }
+      }
+      hipLaunchKernelGGL((k_pass<C, GC_MID, MINB, MAIN, GEN>), g, b, lds, st, a, dir);
+      break;
     case V_MID:
       if (dir == 0) {
+        if constexpr (!GEN) {
+          if (a.gradx) {
+            const size_t ldsg = (size_t)lds_doubles<C>(V_FIRST_G, MAIN) * sizeof(double);
+            hipLaunchKernelGGL((k_pass<C, V_FIRST_G, MINB, MAIN, false>), g, b, ldsg, st, a, dir);
+            break;
+          }
+        }
         hipLaunchKernelGGL((k_pass<C, V_FIRST, MINB, MAIN, GEN>), g, b, lds, st, a, dir);
         break;
       }
       [[fallthrough]];
     case V_LAST_RHS: hipLaunchKernelGGL((k_pass<C, V_MID, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
-    case V_LAST_RK: hipLaunchKernelGGL((k_pass<C, V_LAST_RK, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
+    case V_LAST_RK:
+      if constexpr (MAIN) hipLaunchKernelGGL((k_pass<C, V_LAST_RK, MINB, MAIN, GEN>), g, b, lds, st, a, dir);
+      break;
     // the filtering first pass exists for the miniapp's stage only (the main
     // path filters at the start of its stage); launch_pass_c refuses it there
     case FGC_FIRST:

@@ -223,9 +223,10 @@ int astr_hip_set_convection(astr_hip_ctx *ctx, int upwind, int recon_schem, int 
 /* Per-pass timing with HIP events on the context's stream (no reference
  * counterpart; the reference's timerept accumulators, src/utility.F90:27-297,
  * are no-ops).  Slot = pass*3 + direction, pass 0..6 = gradients
- * first/middle/last, flux derivative (viscous minus convective; along x with
- * the stress, the heat flux and the statistics) middle/last(rhs)/last(RK3 +
- * filter), filter; 7 and 8 stay empty; 9..11 = the upwind-biased
+ * first/middle/last (first: along x, only where the stress pass does not
+ * compute the x gradients itself), flux derivative (viscous minus
+ * convective; along x with the x gradients, the stress, the heat flux and the
+ * statistics) middle/last(rhs)/last(RK3 + filter), filter; 7 and 8 stay empty; 9..11 = the upwind-biased
  * convection's split, interface-flux and shock-sensor kernels (the sensor in
  * slot 33); 12 = the first gradient pass with the previous stage's x filter
  * sweep (program 9, slot 36). */
@@ -237,6 +238,8 @@ int astr_hip_profile_end(astr_hip_ctx *ctx, double *ms, int *count);
  * reference's loops have no launch parameters).  A pass is identified by its
  * program (0..6 as in the profile slots) and direction; its selection is a
  * launch shape and a register budget minb (1 or 2 workgroups per CU).  The
+ * stress pass (3 along x) computes the x gradients itself when it and program
+ * 0 have one shape, whose chunks fix how the solves round.  The
  * shapes (256 threads each) are 0: 4 lines x 64 chunks of 5 unknowns,
  * 1: 4 x 64 x 9, 2: 16 x 16 x 5, 3: 8 x 32 x 9, 4: 8 x 32 x 5; a shape fits a
  * line of n intervals when its chunks hold n+7 unknowns.  astr_hip_autotune times
@@ -254,9 +257,10 @@ int astr_hip_set_last_split(astr_hip_ctx *ctx, int split);
  * - Compact-scheme solver's stage: it ends with z (in the RK pass), then y,
  *   then x.  With on != 0 the x sweep of every stage but a call's last runs
  *   inside the next stage's first gradient pass (program 9),
- *   which loads the same x-lines.  Off by default; astr_hip_autotune turns
- *   it on when its timing of program 9 is below those of programs 0 and 6
- *   along x together.
+ *   which loads the same x-lines; that stage's stress pass then reads the x
+ *   gradients it stored.  Off by default; astr_hip_autotune turns it on when
+ *   it times that form's passes below the x filter pass and a stress pass
+ *   that computes them.
  * - Main path (ASTR_SEM_MAIN), whose stage starts with filterq: with
  *   on != 0 (the default) every RK pass but a call's last also applies the
  *   next stage's sweep along the last direction to the new q, after

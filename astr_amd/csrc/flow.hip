@@ -872,6 +872,93 @@ __global__ void k_bprims(FlowArgs a, int dir) {
   a.pr[5 * fs + o] = P.t;
 }
 
+// The main path's whole qswap where every direction is periodic, one thread
+// per set of duplicates of a boundary point: their mean along i, then j, then
+// k, as the steps in turn give it, and (3-D) the primitives of the result;
+// and the halo sources (k_halo_src) of the lines through them, which the same
+// thread holds from before the averages.  It touches the boundary planes
+// only, so the eight launches of the separate steps were its cost: 113 of
+// 2500 us a step at 129^3.
+__global__ __launch_bounds__(256) void k_qswap_box(FlowArgs a) {
+  const int n0 = a.n[0], n1 = a.n[1], n2 = a.n[2];
+  const bool d3 = a.ndir == 3;
+  const int m2 = d3 ? n2 : 1;
+  const long long A = (long long)n1 * m2, B = (long long)(n0 - 1) * m2, D = d3 ? (long long)(n0 - 1) * (n1 - 1) : 0;
+  long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+  int i, j, k;
+  if (e < A) {
+    i = 0; j = (int)(e % n1); k = (int)(e / n1);
+  } else if ((e -= A) < B) {
+    i = 1 + (int)(e % (n0 - 1)); j = 0; k = (int)(e / (n0 - 1));
+  } else if ((e -= B) < D) {
+    i = 1 + (int)(e % (n0 - 1)); j = 1 + (int)(e / (n0 - 1)); k = 0;
+  } else {
+    return;
+  }
+  const int ci = i == 0 ? 2 : 1, cj = j == 0 ? 2 : 1, ck = d3 && k == 0 ? 2 : 1;
+  auto off = [&](int x, int y, int z) {
+    return (long long)(z ? n2 : k) * a.plane + (long long)(y ? n1 : j) * a.pitch + (x ? n0 : i);
+  };
+  // source rows of the halos: 1..5 and n-5..n-1
+  auto hrow = [](int r, int n) { return r >= 1 && r <= 5 ? r - 1 : (r >= n - 5 && r <= n - 1 ? r - (n - 5) + 5 : -1); };
+  const int hi = hrow(i, n0), hj = hrow(j, n1);
+  const bool src_x = hi >= 0 && (cj == 2 || ck == 2), src_y = d3 && hj >= 0 && ck == 2;
+  double v[5];
+#pragma unroll
+  for (int m = 0; m < 5; m++) {
+    double* q = a.q + m * a.fs;
+    double s[2][2][2];  // z, y, x
+#pragma unroll
+    for (int z = 0; z < 2; z++)
+#pragma unroll
+      for (int y = 0; y < 2; y++)
+#pragma unroll
+        for (int x = 0; x < 2; x++)
+          if (x < ci && y < cj && z < ck) s[z][y][x] = q[off(x, y, z)];
+#pragma unroll
+    for (int z = 0; z < 2; z++)
+#pragma unroll
+      for (int y = 0; y < 2; y++) {
+        if (y >= cj || z >= ck) continue;
+        if (src_x)
+          const_cast<double*>(a.hx)[m * a.hxs + halo_src_index(a.n, a.ndir, 0, i, y ? n1 : j, z ? n2 : k, hi)] =
+              s[z][y][0];
+        if (ci == 2) s[z][y][0] = 0.5 * (s[z][y][0] + s[z][y][1]);
+        if (src_y)
+#pragma unroll
+          for (int x = 0; x < 2; x++)
+            if (x < ci)
+              const_cast<double*>(a.hy)[m * a.hys + halo_src_index(a.n, a.ndir, 1, x ? n0 : i, j, z ? n2 : k, hj)] =
+                  s[z][y][0];
+      }
+#pragma unroll
+    for (int z = 0; z < 2; z++)
+      if (z < ck && cj == 2) s[z][0][0] = 0.5 * (s[z][0][0] + s[z][1][0]);
+    v[m] = ck == 2 ? 0.5 * (s[0][0][0] + s[1][0][0]) : s[0][0][0];
+#pragma unroll
+    for (int z = 0; z < 2; z++)
+#pragma unroll
+      for (int y = 0; y < 2; y++)
+#pragma unroll
+        for (int x = 0; x < 2; x++)
+          if (x < ci && y < cj && z < ck) q[off(x, y, z)] = v[m];
+  }
+  if (!d3) return;  // 2-D: every point's primitives are refreshed after it
+  const Prim P = prim_of(a, v[0], v[1], v[2], v[3], v[4]);
+  const double pv[6] = {P.r, P.u, P.v, P.w, P.p, P.t};
+#pragma unroll
+  for (int z = 0; z < 2; z++)
+#pragma unroll
+    for (int y = 0; y < 2; y++)
+#pragma unroll
+      for (int x = 0; x < 2; x++)
+        if (x < ci && y < cj && z < ck) {
+          const long long o = off(x, y, z);
+#pragma unroll
+          for (int m = 0; m < 6; m++) a.pr[m * a.fs + o] = pv[m];
+        }
+}
+
 // updatefvar (fludyna.F90:191-242): rho, u, v, w, p, T of q at every computed
 // point into the stored primitives
 __global__ void k_updatefvar(FlowArgs a) {
@@ -1125,6 +1212,19 @@ int updatefvar_dev(astr_hip_ctx* c) {
 // reference's dataswap of q gives).
 int qswap_main(astr_hip_ctx* c, bool average) {
   const FlowArgs& a = c->a;
+  if (average && !a.bnd[0] && !a.bnd[1] && !a.bnd[2]) {
+    const long long m2 = a.ndir == 3 ? a.n[2] : 1;
+    const long long cnt = a.n[1] * m2 + (a.n[0] - 1) * m2 + (a.ndir == 3 ? (long long)(a.n[0] - 1) * (a.n[1] - 1) : 0);
+    hipLaunchKernelGGL(k_qswap_box, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, c->stream, a);
+    HIP_OK(hipGetLastError());
+    // a 2-D case still takes the k step, see below
+    if (a.ndir == 2) {
+      hipLaunchKernelGGL(k_updatefvar, pt_grid(a), dim3(64), 0, c->stream, a);
+      HIP_OK(hipGetLastError());
+    }
+    c->halo_valid = true;
+    return 0;
+  }
   auto avg = [&](int d) -> int {
     const int d1 = d == 0 ? 1 : 0, d2 = d == 2 ? 1 : 2;
     const long long cnt = 5LL * (a.n[d1] + 1) * (a.n[d2] + 1);
@@ -2251,8 +2351,8 @@ constexpr int kSlotStats = 3;  // V x, which sums the statistics
 
 // work items of a batched pass of nt tiles
 int batch_items(int prog, int dir, int nt) {
-  if ((prog == V_MID && dir == 0) || !pass_one(prog, false, dir == 1, nt)) return nt;
-  return nt * pass_fields(prog, false);
+  if ((prog == V_MID && dir == 0) || !pass_one(prog, dir == 1, nt)) return nt;
+  return nt * pass_fields(prog);
 }
 
 struct BatchGroup {

@@ -1030,17 +1030,40 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
           qs[t] = sa.stage == 0 ? 0.0 : ldg(qo + m * fs, S.g[t]);
         }
       };
-      if constexpr (!MAIN) {
-        // one component per workgroup (pass_one)
+      if constexpr (ONE) {
         const int m = field;
+        const bool solve = m > 0 || !uwd;  // without convection density has no flux
         load_inputs(m);
         load_rk(m);
-        filter_setup(1);
-        stage_flux(m, 0);
-        derive_flux(m);
+        if (solve) {
+          stage_flux(m, 0);
+          derive_flux(m);
+        }
+        double qw[NPT];
 #pragma unroll
-        for (int t = 0; t < NPT; t++)
-          put<C>(T, S, t, rk_update(sa, a.dt, sa.stage == 0 ? qn[t] : qs[t], qn[t], qr[t] + dflux(t)));
+        for (int t = 0; t < NPT; t++) {
+          const double v = solve ? qr[t] + dflux(t) : qr[t];
+          const double s0 = sa.stage == 0 ? qn[t] : qs[t];
+          qw[t] = MAIN ? rk_update_main(sa, a.dt, a.jac, s0 * a.jac, qn[t], v)  // qsave = q J (mainloop.F90:423-427)
+                       : rk_update(sa, a.dt, s0, qn[t], v);
+        }
+        if (MAIN && !a.rk_filter) {
+#pragma unroll
+          for (int t = 0; t < NPT; t++) stg(qnew + m * fs, S.g[t], qw[t]);
+          return;
+        }
+        if constexpr (MAIN) {
+          // updatefvar needs all five components of the unfiltered state:
+          // they go to the first fields of the gradients, which the flux
+          // passes no longer read, for k_fvar
+#pragma unroll
+          for (int t = 0; t < NPT; t++) stg(a.dv + m * fs, S.g[t], qw[t]);
+        }
+        // the filter sweep along dir: the miniapp's of this stage, the main
+        // path's of the next (comsolver.F90:514-632)
+        filter_setup(1);
+#pragma unroll
+        for (int t = 0; t < NPT; t++) put<C>(T, S, t, qw[t]);
         filter();
 #pragma unroll
         for (int t = 0; t < NPT; t++) stg(qnew + m * fs, S.g[t], X[S.s[t]]);
@@ -1139,11 +1162,10 @@ __global__ __launch_bounds__(C::NT, MINB) void k_pass(FlowArgs a, int dir) {
 }
 
 // Components a pass runs as separate workgroups, 0: it cannot (the stress
-// pass's fluxes share the stress, the main path's RK pass ends with
-// updatefvar of all five).
-constexpr int pass_fields(int prog, bool main_sem) {
+// pass's fluxes share the stress).
+constexpr int pass_fields(int prog) {
   if (prog == GC_FIRST || prog == GC_MID || prog == GC_LAST) return 4;
-  if (prog == V_MID || prog == V_LAST_RHS || prog == F_ONLY || (prog == V_LAST_RK && !main_sem)) return 5;
+  if (prog == V_MID || prog == V_LAST_RHS || prog == F_ONLY || prog == V_LAST_RK) return 5;
   return 0;
 }
 // Whether a pass of nt tiles runs one component per workgroup.  With few
@@ -1154,10 +1176,11 @@ constexpr int pass_fields(int prog, bool main_sem) {
 // tiles) 17 -> 9, 65^3 (265) 20 -> 15.6, 97^3 (1177) 34 -> 38; flux derivative
 // 11.7 -> 8.4, 16.1 -> 15.5, 33 -> 39; gradients 10.3 -> 7.6, 13.5 -> 12.2,
 // 23.8 -> 25.7, and where they form the pressure too 10.3 -> 9.2, 13.8 -> 16.5.
-// The RK pass solves twice per component and gains at every size (33^3 23.5
-// -> 12, 129^3 132 -> 129, 257^3 1080 -> 1034), so it has that form only.
-constexpr bool pass_one(int prog, bool main_sem, bool pres, int nt) {
-  if (pass_fields(prog, main_sem) == 0) return false;
+// The RK pass solves twice per component and gains at every size (miniapp
+// 33^3 23.5 -> 12, 129^3 132 -> 129, 257^3 1080 -> 1034), so it has that
+// form only, but for directions of the general-grid kernels.
+constexpr bool pass_one(int prog, bool pres, int nt) {
+  if (pass_fields(prog) == 0) return false;
   if (prog == V_LAST_RK) return true;
   if (prog == F_ONLY) return nt <= 512;
   if (prog <= GC_LAST) return nt <= (pres ? 128 : 384);
@@ -1169,9 +1192,27 @@ constexpr bool pass_one(int prog, bool main_sem, bool pres, int nt) {
 template <class C, int PROG, int MINB, bool MAIN = false, bool GEN = false>
 __global__ __launch_bounds__(C::NT, MINB) void k_pass_one(FlowArgs a, int dir) {
   extern __shared__ double smem[];
-  constexpr int NF = pass_fields(PROG, MAIN);
+  constexpr int NF = pass_fields(PROG);
   const int b = xcd_tile(blockIdx.x, gridDim.x);
   pass_body<C, PROG, MAIN, GEN, true>(a, stage_of(a), arrays_of(a, 0), dir, b / NF, smem, b % NF);
+}
+
+// updatefvar (fludyna.F90:191-242) after the main path's RK pass: rho, u, v,
+// w, p, T at every computed point of the state q
+__global__ __launch_bounds__(256) inline void k_fvar(FlowArgs a, const double* q) {
+  const unsigned rows = (a.n[1] + 1) * (a.n[2] + 1);
+  const unsigned e = blockIdx.x * 256 + threadIdx.x;
+  const unsigned row = e / a.pitch, i = e - row * a.pitch;
+  if (row >= rows || i > (unsigned)a.n[0]) return;
+  const unsigned o = e * 8u;  // rows are contiguous
+  const long long fs = a.fs;
+  const Prim P = prim_of(a, ldg(q, o), ldg(q + fs, o), ldg(q + 2 * fs, o), ldg(q + 3 * fs, o), ldg(q + 4 * fs, o));
+  stg(a.pr, o, P.r);
+  stg(a.pr + fs, o, P.u);
+  stg(a.pr + 2 * fs, o, P.v);
+  stg(a.pr + 3 * fs, o, P.w);
+  stg(a.pr + 4 * fs, o, P.p);
+  stg(a.pr + 5 * fs, o, P.t);
 }
 
 // The tiles of one pass over several cases: case k owns global tiles
@@ -1190,7 +1231,7 @@ template <class C, int PROG, int MINB, bool ONE = false>
 __global__ __launch_bounds__(C::NT, MINB) void k_pass_batch(BatchLaunch bl, int dir, StageArgs sa) {
   extern __shared__ double smem[];
   const int x = blockIdx.x & 7, per = gridDim.x >> 3;
-  constexpr int NF = ONE ? pass_fields(PROG, false) : 1;
+  constexpr int NF = ONE ? pass_fields(PROG) : 1;
   const long long total = (long long)bl.total * NF;
   const int lo = (int)(total * x / 8), hi = (int)(total * (x + 1) / 8);
   for (int e = lo + (int)(blockIdx.x >> 3); e < hi; e += per) {
@@ -1213,7 +1254,7 @@ hipError_t launch_batch_c(int prog, const BatchLaunch& bl, int dir, const StageA
   const size_t lds = (size_t)lds_doubles<C>(prog) * sizeof(double);
   dim3 g(nblocks), b(C::NT);
 #define ASTR_BATCH_PASS(P, O) hipLaunchKernelGGL((k_pass_batch<C, P, MINB, O>), g, b, lds, st, bl, dir, sa)
-  const bool one = pass_one(prog, false, dir == 1, bl.total);
+  const bool one = pass_one(prog, dir == 1, bl.total);
   switch (prog) {
     // the y gradient pass is a stage's first: it forms the pressure
     case GC_MID:
@@ -1254,7 +1295,7 @@ void launch_pass_m(int prog, const FlowArgs& a, int dir, hipStream_t st) {
   dim3 g(nt), b(C::NT);
   if constexpr (!GEN) {
     const bool pres = !MAIN && (prog == GC_FIRST || (a.gradx && dir == 1));
-    if (!(prog == V_MID && dir == 0) && pass_one(prog, MAIN, pres, nt)) {
+    if (!(prog == V_MID && dir == 0) && pass_one(prog, pres, nt)) {
       switch (prog) {
         case GC_FIRST:
         case GC_MID:
@@ -1269,11 +1310,13 @@ void launch_pass_m(int prog, const FlowArgs& a, int dir, hipStream_t st) {
           hipLaunchKernelGGL((k_pass_one<C, V_MID, MINB, MAIN>), dim3(5 * nt), b, lds, st, a, dir);
           return;
         case V_LAST_RK:
-          if constexpr (!MAIN) {
-            hipLaunchKernelGGL((k_pass_one<C, V_LAST_RK, MINB, false>), dim3(5 * nt), b, lds, st, a, dir);
-            return;
+          hipLaunchKernelGGL((k_pass_one<C, V_LAST_RK, MINB, MAIN>), dim3(5 * nt), b, lds, st, a, dir);
+          if constexpr (MAIN) {
+            const unsigned pts = (unsigned)a.pitch * (a.n[1] + 1) * (a.n[2] + 1);
+            const double* q = a.rk_filter ? a.dv : (a.stage == 1 ? a.qrhs : a.qsave);
+            hipLaunchKernelGGL(k_fvar, dim3((pts + 255) / 256), dim3(256), 0, st, a, q);
           }
-          break;
+          return;
         case F_ONLY: hipLaunchKernelGGL((k_pass_one<C, F_ONLY, MINB, false>), dim3(5 * nt), b, lds, st, a, dir); return;
         default: break;
       }
@@ -1308,7 +1351,7 @@ void launch_pass_m(int prog, const FlowArgs& a, int dir, hipStream_t st) {
       [[fallthrough]];
     case V_LAST_RHS: hipLaunchKernelGGL((k_pass<C, V_MID, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
     case V_LAST_RK:
-      if constexpr (MAIN) hipLaunchKernelGGL((k_pass<C, V_LAST_RK, MINB, MAIN, GEN>), g, b, lds, st, a, dir);
+      if constexpr (GEN) hipLaunchKernelGGL((k_pass<C, V_LAST_RK, MINB, MAIN, GEN>), g, b, lds, st, a, dir);
       break;
     // the filtering first pass exists for the miniapp's stage only (the main
     // path filters at the start of its stage); launch_pass_c refuses it there

@@ -62,6 +62,26 @@ struct Mech {
   double pnu[NRMAX][NTERM];
   double dnu[NRMAX];       // sum of product minus reactant coefficients
   double p0;               // standard-state pressure of the thermo data, Pa
+  // the same data in the form the cell kernels read it, laid out once by
+  // prepare_cells: every access is uniform over a wavefront, so a record comes
+  // in with a few scalar loads, and no division is left to the cells
+  double iW[NSMAX], rW[NSMAX];  // 1/W, kRref/W
+  struct Range {           // one NASA range: cp/R, h/RT and g/RT as polynomials
+    double a0, a1, a2, a3, a4;
+    double h1, h2, h3, h4;  // a1/2, a2/3, a3/4, a4/5
+    double g1, g2, g3, g4;  // -a1/2, -a2/6, -a3/12, -a4/20
+    double a5, a6;
+  } th[NSMAX][2];
+  struct Rx {
+    double lnA, b, EaR;
+    unsigned sp;           // unit terms: 3 reactants, 3 products, 4 bits each
+    unsigned fl;           // bits 0-1 / 2-3: unit terms per side, 4: reversible, 5: three-body,
+                           // 6: a product of unit terms on both sides
+    double nu[NSMAX];      // product minus reactant coefficients
+    double eff[NSMAX];
+  } rx[NRMAX];
+  double lnp0R;            // ln(p0 / kRgas)
+  int unit;                // every order is a whole number and a side has at most NTERM of them
 };
 
 // ---------------------------------------------------------------------------
@@ -130,74 +150,189 @@ __device__ __forceinline__ void kinetics(const Mech* __restrict__ M, double T, d
   }
 }
 
-// The net molar production rates w (kmol/m^3/s) of one cell at (T, rho, y):
-// k_chem's arithmetic, in the same order, without the mixture cp and h.
-// k_chem keeps its own copy: with this function inlined in it, its register
-// peak rose from 164 VGPRs to 256 and its occupancy fell from three waves per
-// SIMD to one.  NSA as in k_chem.
-template <int NSA>
-__device__ __forceinline__ void cell_rates(const Mech* __restrict__ M, double T, double rho,
-                                           const double* y, double* w) {
-  const int ns = NSA == NSMAX ? M->ns : NSA, nr = M->nr;
-  double c[NSA], g[NSA];
-  const double logT = log(T), invT = 1.0 / T;
-  const double T2 = T * T, T3 = T2 * T, T4 = T3 * T;
-  for (int k = 0; k < ns; k++) {
-    c[k] = rho * y[k] / M->W[k];
-    double hrt, sr;
-    {
-      double hr[2], srr[2];
-#pragma unroll
-      for (int q = 0; q < 2; q++) {
-        const double* a = q == 0 ? M->lo[k] : M->hi[k];
-        hr[q] = a[0] + a[1] * T / 2.0 + a[2] * T2 / 3.0 + a[3] * T3 / 4.0 + a[4] * T4 / 5.0 +
-                a[5] * invT;
-        srr[q] = a[0] * logT + a[1] * T + a[2] * T2 / 2.0 + a[3] * T3 / 3.0 + a[4] * T4 / 4.0 + a[6];
-      }
-      const int q = T <= M->tmid[k] ? 0 : 1;
-      hrt = q == 0 ? hr[0] : hr[1];
-      sr = q == 0 ? srr[0] : srr[1];
-    }
-    g[k] = hrt - sr;
-    w[k] = 0.0;
+// An array in registers read at an index that is uniform over the wavefront.
+// Kept as two vectors of 32-bit halves: a register tuple exists for every
+// count of 9..12 32-bit elements, while an array of 9 doubles is rounded up to
+// a tuple of 16 (32 registers for 18).
+// N < NSMAX: one more element, 1, where unit()'s unused indices point.
+template <int N>
+struct RegArray {
+  static constexpr bool PAD = N < NSMAX;
+  typedef unsigned V __attribute__((ext_vector_type(N + PAD)));
+  V lo, hi;
+  __device__ __forceinline__ RegArray() {
+    if constexpr (PAD) set(N, 1.0);
   }
-  const double lc0 = log(M->p0 / (kRgas * T));  // ln of the standard concentration
-  for (int r = 0; r < nr; r++) {
-    const double kf = exp(M->lnA[r] + M->b[r] * logT - M->EaR[r] * invT);
-    double fwd = kf;
-    double dg = 0.0;
-    for (int j = 0; j < M->nre[r]; j++) {
-      fwd *= conc_pow(c[M->rsp[r][j]], M->rnu[r][j]);
-      dg -= M->rnu[r][j] * g[M->rsp[r][j]];
-    }
-    double rv = 0.0;
-    if (M->rev[r]) {
-      double pp = 1.0;
-      for (int j = 0; j < M->npr[r]; j++) {
-        pp *= conc_pow(c[M->psp[r][j]], M->pnu[r][j]);
-        dg += M->pnu[r][j] * g[M->psp[r][j]];
-      }
-      // kr = kf / Kc, Kc = exp(-dG/RT) * (p0/RT)^dnu
-      const double kr = exp(M->lnA[r] + M->b[r] * logT - M->EaR[r] * invT + dg - M->dnu[r] * lc0);
-      rv = kr * pp;
-    }
-    double q = fwd - rv;
-    if (M->tb[r]) {
-      double cm = 0.0;
-      for (int k = 0; k < ns; k++) cm += M->eff[r][k] * c[k];
-      q *= cm;
-    }
-    for (int j = 0; j < M->nre[r]; j++) w[M->rsp[r][j]] -= M->rnu[r][j] * q;
-    for (int j = 0; j < M->npr[r]; j++) w[M->psp[r][j]] += M->pnu[r][j] * q;
+  __device__ __forceinline__ void set(int k, double x) {
+    lo[k] = (unsigned)__double2loint(x);
+    hi[k] = (unsigned)__double2hiint(x);
+  }
+  __device__ __forceinline__ double get(int k) const { return __hiloint2double((int)hi[k], (int)lo[k]); }
+  // the product of up to three elements: 4-bit indices in sp, their count in
+  // the low bits of fl; with the pad, three without a branch
+  __device__ __forceinline__ double unit(unsigned sp, unsigned fl) const {
+    double p = get(sp & 15);
+    if (PAD || (fl & 3) > 1) p *= get(sp >> 4 & 15);
+    if (PAD || (fl & 3) > 2) p *= get(sp >> 8 & 15);
+    return p;
+  }
+};
+
+// e^x for the rate constants: x = n ln 2 + r with the nearest n (Cody and
+// Waite's two-part ln 2), e^r = 1 + r + r^2 P(r) with P of degree 9 through
+// the Chebyshev nodes of |r| <= ln 2 / 2 (its error 2e-17), scaled by 2^n.
+// About 20 instructions where exp takes 33: exp's constants sit in vector
+// registers that its multiply-adds overwrite, so each is copied first; here
+// they are scalar operands (ExpK, made once per thread in scalar registers),
+// and the checks for overflow and underflow are one comparison, with exp's
+// own result for the lanes outside +-700.
+struct ExpK {
+  double l2e = 0x1.71547652b82fep+0, rnd = 0x1.8p52, hi = 0x1.62e42fefa39efp-1, lo = 0x1.abc9e3b39803fp-56;
+  double c3 = 0x1.5555555555556p-3, c4 = 0x1.5555555553d4fp-5, c5 = 0x1.11111111109adp-7,
+         c6 = 0x1.6c16c17893833p-10, c7 = 0x1.a01a01a7c8d47p-13, c8 = 0x1.a019b8ef67c6cp-16,
+         c9 = 0x1.71de0d9c145d0p-19, c10 = 0x1.2891a8c1d838dp-22, c11 = 0x1.af38d53857513p-26;
+  __device__ __forceinline__ ExpK() {
+    asm volatile("" : "+s"(l2e), "+s"(rnd), "+s"(hi), "+s"(lo), "+s"(c3), "+s"(c4), "+s"(c5), "+s"(c6));
+    asm volatile("" : "+s"(c7), "+s"(c8), "+s"(c9), "+s"(c10), "+s"(c11));
+  }
+};
+__device__ __forceinline__ double rate_exp_in(double x, const ExpK& K) {  // |x| < 700
+  const double t = fma(x, K.l2e, K.rnd);  // n in the low bits
+  const double n = t - K.rnd;
+  const double r = fma(-n, K.lo, fma(-n, K.hi, x));
+  double p = fma(K.c11, r, K.c10);
+  p = fma(p, r, K.c9);
+  p = fma(p, r, K.c8);
+  p = fma(p, r, K.c7);
+  p = fma(p, r, K.c6);
+  p = fma(p, r, K.c5);
+  p = fma(p, r, K.c4);
+  p = fma(p, r, K.c3);
+  p = fma(p, r, 0.5);
+  return ldexp(1.0 + fma(r * r, p, r), __double2loint(t));
+}
+__device__ __forceinline__ double rate_exp(double x, const ExpK& K) {
+  double e = rate_exp_in(x, K);
+  const bool in = fabs(x) < 700.0;
+  if (__any(!in)) e = in ? e : exp(x);
+  return e;
+}
+// both at once, with one branch after the two chains of multiply-adds
+__device__ __forceinline__ void rate_exp2(double x, double y, const ExpK& K, double& ex, double& ey) {
+  ex = rate_exp_in(x, K);
+  ey = rate_exp_in(y, K);
+  const bool in = fabs(x) < 700.0 && fabs(y) < 700.0;
+  if (__any(!in)) {
+    ex = fabs(x) < 700.0 ? ex : exp(x);
+    ey = fabs(y) < 700.0 ? ey : exp(y);
   }
 }
 
-// NSA: the per-cell arrays' size.  NSA = NSMAX serves any mechanism (loops
-// to M->ns); an instance with NSA = the mechanism's species count keeps four
-// arrays of that size in registers instead of NSMAX, with the same arithmetic
-// in the same order.
-template <int NSA>
-__global__ __launch_bounds__(256) void k_chem(const Mech* __restrict__ M, long long n,
+// cp/R, h/RT and g/RT - ln(p0/RT) of species k, from both NASA ranges
+// (uniform coefficients, one scalar operand per multiply-add) and the cell's
+// range picked.  With ln(p0/RT) in g, ln kr = ln kf + sum nu_k g_k: the
+// equilibrium constant's (p0/RT)^dnu needs no term of its own.
+struct Thermo {
+  double cp, h, g;
+};
+__device__ __forceinline__ Thermo species(const Mech* __restrict__ M, int k, double T, double invT,
+                                          double omlogT, double lc0) {
+  Thermo t[2];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    const Mech::Range& R = M->th[k][q];
+    const double b = R.a5 * invT;
+    t[q].cp = R.a0 + T * (R.a1 + T * (R.a2 + T * (R.a3 + T * R.a4)));
+    t[q].h = R.a0 + T * (R.h1 + T * (R.h2 + T * (R.h3 + T * R.h4))) + b;
+    t[q].g = R.a0 * omlogT + T * (R.g1 + T * (R.g2 + T * (R.g3 + T * R.g4))) + b - R.a6 - lc0;
+  }
+  const bool low = T <= M->tmid[k];
+  return {low ? t[0].cp : t[1].cp, low ? t[0].h : t[1].h, low ? t[0].g : t[1].g};
+}
+
+// The net molar production rates w (kmol/m^3/s) of one cell from its
+// concentrations c and its g (as species() returns it).  What a reaction adds
+// to dg and takes from q goes over all species with its row of coefficients:
+// nine multiply-adds with a scalar operand each, against three to six indexed
+// register accesses of about eight instructions.  A reaction whose rate is
+// not finite must leave the species alone that take no part in it: it makes
+// every w of that sum NaN, w[0] too, and the sums are then formed again with
+// the zeros of the rows skipped (CAREFUL).  c, g and the coefficients past ns
+// are zero.  UNIT: every mass-action product is one of at most NTERM
+// concentrations; otherwise the reactions that have other orders go through
+// conc_pow, whose call to pow sets the register peak of the whole kernel
+// (2^20 cells of 9 species 114 us with it, 88 us without).
+template <int NSA, bool UNIT, bool CAREFUL>
+__device__ __forceinline__ void reaction_sums(const Mech* __restrict__ M, int ns, double logT, double invT,
+                                              const RegArray<NSA>& c, const double (&g)[NSA], double (&w)[NSA]) {
+  const int nr = M->nr;
+  const ExpK K;
+#pragma unroll
+  for (int k = 0; k < NSA; k++) w[k] = 0.0;
+#pragma unroll 1
+  for (int r = 0; r < nr; r++) {
+    const Mech::Rx& R = M->rx[r];
+    double nu[NSA];  // read with the record's head, ahead of the exponentials
+#pragma unroll
+    for (int k = 0; k < NSA; k++) nu[k] = R.nu[k];
+    const unsigned fl = R.fl;
+    const double lkf = R.lnA + R.b * logT - R.EaR * invT;
+    double fw = 1.0, q;
+    if (UNIT || (fl & 64)) {
+      fw = c.unit(R.sp, fl);
+    } else {
+      for (int j = 0; j < M->nre[r]; j++) fw *= conc_pow(c.get(M->rsp[r][j]), M->rnu[r][j]);
+    }
+    if (fl & 16) {
+      double dg = 0.0, bw = 1.0, kf, kr;
+#pragma unroll
+      for (int k = 0; k < NSA; k++) dg += nu[k] * g[k];
+      if (UNIT || (fl & 64)) {
+        bw = c.unit(R.sp >> 12, fl >> 2);
+      } else {
+        for (int j = 0; j < M->npr[r]; j++) bw *= conc_pow(c.get(M->psp[r][j]), M->pnu[r][j]);
+      }
+      rate_exp2(lkf, lkf + dg, K, kf, kr);  // kr = kf / Kc
+      q = kf * fw - kr * bw;
+    } else {
+      q = rate_exp(lkf, K) * fw;
+    }
+    if (fl & 32) {
+      double cm = 0.0;
+#pragma unroll
+      for (int k = 0; k < NSA; k++) cm += R.eff[k] * c.get(k);
+      q *= cm;
+    }
+#pragma unroll
+    for (int k = 0; k < NSA; k++)
+      if (!CAREFUL || nu[k] != 0.0) w[k] += nu[k] * q;
+  }
+}
+
+template <int NSA, bool UNIT>
+__device__ __forceinline__ void cell_rates(const Mech* __restrict__ M, int ns, double logT, double invT,
+                                           const RegArray<NSA>& c, const double (&g)[NSA], double (&w)[NSA]) {
+  reaction_sums<NSA, UNIT, false>(M, ns, logT, invT, c, g, w);
+  if (__any(!(fabs(w[0]) <= 1.7976931348623157e308)))
+    reaction_sums<NSA, UNIT, true>(M, ns, logT, invT, c, g, w);
+}
+
+// cells per workgroup: one wavefront, so that few cells spread over many
+// compute units (1000 cells 14 us, 16 with four wavefronts; 2^20 alike)
+constexpr int kCellBlock = 64;
+
+// NSA: the per-cell arrays' size.  NSA = NSMAX serves any mechanism (up to
+// M->ns); an instance with NSA = the mechanism's species count has every loop
+// over the species unrolled.  Bound by FP64 arithmetic: about 2400 vector
+// instructions a cell with 9 species and 19 reactions (two exponentials per
+// reaction are 760 of them), 64 us of issue for 2^20 cells against 38 us for
+// the cells' 176 bytes.  124 registers leave four wavefronts per SIMD to cover
+// the scalar loads of the reaction records (96 spill: 220 us; three: 93 us).
+// 2^20 cells 178 -> 88 us, 1000 cells 29 -> 13 us against divisions in the
+// thermodynamics, indexed sums and the library's exponential; 8 species in
+// the NSMAX instance 253 -> 129 us, with general orders 264 -> 168 us.
+template <int NSA, bool UNIT>
+__global__ __launch_bounds__(kCellBlock, NSA == NSMAX ? 2 : UNIT ? 4 : 3) void k_chem(const Mech* __restrict__ M, long long n,
                                               const double* __restrict__ Tin,
                                               const double* __restrict__ RPin, int input_is_p,
                                               const double* __restrict__ Y, double* __restrict__ wdot,
@@ -205,76 +340,39 @@ __global__ __launch_bounds__(256) void k_chem(const Mech* __restrict__ M, long l
                                               double* __restrict__ hk) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int ns = NSA == NSMAX ? M->ns : NSA, nr = M->nr;
+  const int ns = NSA == NSMAX ? M->ns : NSA;
   const double T = Tin[i];
-  double y[NSA], c[NSA], g[NSA], w[NSA];
+  double y[NSA], g[NSA], w[NSA];
+  RegArray<NSA> c;
   double winv = 0.0;
-  for (int k = 0; k < ns; k++) {
-    y[k] = Y[k * n + i];
-    winv += y[k] / M->W[k];
+#pragma unroll
+  for (int k = 0; k < NSA; k++) {
+    y[k] = NSA != NSMAX || k < ns ? Y[k * n + i] * M->iW[k] : 0.0;
+    winv += y[k];
   }
   const double rho = input_is_p ? RPin[i] / (kRgas * T * winv) : RPin[i];
   const double logT = log(T), invT = 1.0 / T;
-  const double T2 = T * T, T3 = T2 * T, T4 = T3 * T;
+  const double lc0 = M->lnp0R - logT;  // ln of the standard concentration
   double cp = 0.0, h = 0.0;
-  for (int k = 0; k < ns; k++) {
-    c[k] = rho * y[k] / M->W[k];
-    // NASA 7-coefficient polynomials, evaluated with both ranges' coefficients
-    // (uniform, so they stay in scalar registers) and the cell's range picked
-    double cpr, hrt, sr;
-    {
-      double cr[2], hr[2], srr[2];
 #pragma unroll
-      for (int q = 0; q < 2; q++) {
-        const double* a = q == 0 ? M->lo[k] : M->hi[k];
-        cr[q] = a[0] + a[1] * T + a[2] * T2 + a[3] * T3 + a[4] * T4;
-        hr[q] = a[0] + a[1] * T / 2.0 + a[2] * T2 / 3.0 + a[3] * T3 / 4.0 + a[4] * T4 / 5.0 +
-                a[5] * invT;
-        srr[q] = a[0] * logT + a[1] * T + a[2] * T2 / 2.0 + a[3] * T3 / 3.0 + a[4] * T4 / 4.0 + a[6];
-      }
-      const int q = T <= M->tmid[k] ? 0 : 1;
-      cpr = q == 0 ? cr[0] : cr[1];
-      hrt = q == 0 ? hr[0] : hr[1];
-      sr = q == 0 ? srr[0] : srr[1];
-    }
-    g[k] = hrt - sr;
-    cp += y[k] * cpr / M->W[k];
-    const double hks = hrt * (kRref / M->W[k]) * T;
-    h += y[k] * hks;
-    if (hk) hk[k * n + i] = hks;
-    w[k] = 0.0;
+  for (int k = 0; k < NSA; k++) {
+    c.set(k, NSA != NSMAX || k < ns ? rho * y[k] : 0.0);
+    g[k] = 0.0;
+    if (NSA == NSMAX && k >= ns) continue;
+    const Thermo t = species(M, k, T, invT, 1.0 - logT, lc0);
+    g[k] = t.g;
+    cp += y[k] * t.cp;
+    h += y[k] * t.h;
+    // evaluated here: sunk to their uses, all species' polynomials would wait
+    // there with all their coefficients in (spilled) scalar registers
+    asm volatile("" : "+v"(g[k]), "+v"(cp), "+v"(h));
+    if (hk) hk[k * n + i] = t.h * M->rW[k] * T;
   }
-  const double lc0 = log(M->p0 / (kRgas * T));  // ln of the standard concentration
-  for (int r = 0; r < nr; r++) {
-    const double kf = exp(M->lnA[r] + M->b[r] * logT - M->EaR[r] * invT);
-    double fwd = kf;
-    double dg = 0.0;
-    for (int j = 0; j < M->nre[r]; j++) {
-      fwd *= conc_pow(c[M->rsp[r][j]], M->rnu[r][j]);
-      dg -= M->rnu[r][j] * g[M->rsp[r][j]];
-    }
-    double rv = 0.0;
-    if (M->rev[r]) {
-      double pp = 1.0;
-      for (int j = 0; j < M->npr[r]; j++) {
-        pp *= conc_pow(c[M->psp[r][j]], M->pnu[r][j]);
-        dg += M->pnu[r][j] * g[M->psp[r][j]];
-      }
-      // kr = kf / Kc, Kc = exp(-dG/RT) * (p0/RT)^dnu
-      const double kr = exp(M->lnA[r] + M->b[r] * logT - M->EaR[r] * invT + dg - M->dnu[r] * lc0);
-      rv = kr * pp;
-    }
-    double q = fwd - rv;
-    if (M->tb[r]) {
-      double cm = 0.0;
-      for (int k = 0; k < ns; k++) cm += M->eff[r][k] * c[k];
-      q *= cm;
-    }
-    for (int j = 0; j < M->nre[r]; j++) w[M->rsp[r][j]] -= M->rnu[r][j] * q;
-    for (int j = 0; j < M->npr[r]; j++) w[M->psp[r][j]] += M->pnu[r][j] * q;
-  }
-  for (int k = 0; k < ns; k++) wdot[k * n + i] = w[k] * M->W[k];
-  if (hmix) hmix[i] = h;
+  cell_rates<NSA, UNIT>(M, ns, logT, invT, c, g, w);
+#pragma unroll
+  for (int k = 0; k < NSA; k++)
+    if (NSA != NSMAX || k < ns) wdot[k * n + i] = w[k] * M->W[k];
+  if (hmix) hmix[i] = h * kRref * T;
   if (cpmix) cpmix[i] = cp * kRgas;
 }
 
@@ -284,27 +382,40 @@ __global__ __launch_bounds__(256) void k_chem(const Mech* __restrict__ M, long l
 // tmp, jacob: (-hm:im+hm, -hm:jm+hm, -hm:km+hm), spc: the same with a last
 // species index, qrhs: (0:im, 0:jm, 0:km, 1:numq), all column-major as the
 // reference allocates them (commarray.F90).
-template <int NSA>
-__global__ __launch_bounds__(256) void k_srccomb(const Mech* __restrict__ M, int im, int jm, int km,
+template <int NSA, bool UNIT>
+__global__ __launch_bounds__(kCellBlock, NSA == NSMAX ? 2 : UNIT ? 4 : 3) void k_srccomb(const Mech* __restrict__ M, int im, int jm, int km,
                                                  int hm, const double* __restrict__ rho,
                                                  const double* __restrict__ tmp,
                                                  const double* __restrict__ spc,
                                                  const double* __restrict__ jacob,
                                                  double* __restrict__ qrhs) {
   const long long nx = im + 1, ny = jm + 1, ncell = nx * ny * (km + 1);
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
+  const long long cell = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (cell >= ncell) return;
   const int ns = NSA == NSMAX ? M->ns : NSA;
-  const long long i = c % nx, j = (c / nx) % ny, k = c / (nx * ny);
+  const long long i = cell % nx, j = (cell / nx) % ny, k = cell / (nx * ny);
   const long long sx = im + 1 + 2 * hm, sy = jm + 1 + 2 * hm, sz = km + 1 + 2 * hm;
   const long long hp = ((k + hm) * sy + (j + hm)) * sx + (i + hm);
   const long long hs = sx * sy * sz;
-  double y[NSA], w[NSA];
-  for (int s = 0; s < ns; s++) y[s] = spc[s * hs + hp];
-  cell_rates<NSA>(M, tmp[hp], rho[hp], y, w);
+  const double T = tmp[hp], r = rho[hp];
+  const double logT = log(T), invT = 1.0 / T;
+  double g[NSA], w[NSA];
+  RegArray<NSA> c;
+#pragma unroll
+  for (int s = 0; s < NSA; s++) {
+    c.set(s, 0.0);
+    g[s] = 0.0;
+    if (NSA == NSMAX && s >= ns) continue;
+    c.set(s, r * (spc[s * hs + hp] * M->iW[s]));
+    g[s] = species(M, s, T, invT, 1.0 - logT, M->lnp0R - logT).g;
+    asm volatile("" : "+v"(g[s]));  // as in k_chem
+  }
+  cell_rates<NSA, UNIT>(M, ns, logT, invT, c, g, w);
   const double jac = jacob[hp];
-  for (int s = 0; s < ns; s++) {
-    double* q = qrhs + (5 + s) * ncell + c;
+#pragma unroll
+  for (int s = 0; s < NSA; s++) {
+    if (NSA == NSMAX && s >= ns) continue;
+    double* q = qrhs + (5 + s) * ncell + cell;
     *q = *q + (w[s] * M->W[s]) * jac;
   }
 }
@@ -1249,6 +1360,52 @@ bool ea_factor(const std::string& units, double& f) {
   return true;
 }
 
+// the cell kernels' form of the mechanism (Mech::th, rx)
+void prepare_cells(Mech& m) {
+  m.lnp0R = std::log(m.p0 / kRgas);
+  for (int k = 0; k < m.ns; k++) {
+    m.iW[k] = 1.0 / m.W[k];
+    m.rW[k] = kRref / m.W[k];
+    for (int q = 0; q < 2; q++) {
+      const double* a = q == 0 ? m.lo[k] : m.hi[k];
+      m.th[k][q] = {a[0], a[1], a[2], a[3], a[4], a[1] / 2.0, a[2] / 3.0, a[3] / 4.0, a[4] / 5.0,
+                    -a[1] / 2.0, -a[2] / 6.0, -a[3] / 12.0, -a[4] / 20.0, a[5], a[6]};
+    }
+  }
+  m.unit = 1;
+  for (int r = 0; r < m.nr; r++) {
+    Mech::Rx& R = m.rx[r];
+    R.lnA = m.lnA[r];
+    R.b = m.b[r];
+    R.EaR = m.EaR[r];
+    R.sp = 0;
+    R.fl = (m.rev[r] ? 16u : 0u) | (m.tb[r] ? 32u : 0u) | 64u;
+    for (int k = 0; k < m.ns; k++) {
+      R.nu[k] = 0.0;
+      R.eff[k] = m.eff[r][k];
+    }
+    for (int side = 0; side < 2; side++) {
+      const int n = side ? m.npr[r] : m.nre[r];
+      const int* sp = side ? m.psp[r] : m.rsp[r];
+      const double* nu = side ? m.pnu[r] : m.rnu[r];
+      int terms = 0;
+      for (int j = 0; j < n; j++) {
+        R.nu[sp[j]] += side ? nu[j] : -nu[j];
+        const int whole = nu[j] == 1.0 ? 1 : nu[j] == 2.0 ? 2 : nu[j] == 3.0 ? 3 : NTERM + 1;
+        for (int i = 0; i < whole && terms <= NTERM; i++, terms++)
+          if (terms < NTERM) R.sp |= (unsigned)sp[j] << (12 * side + 4 * terms);
+      }
+      if (terms < 1 || terms > NTERM) {
+        R.fl &= ~64u;
+        m.unit = 0;
+      }
+      for (int i = terms; i < NTERM; i++)  // RegArray's pad
+        if (m.ns < NSMAX) R.sp |= (unsigned)m.ns << (12 * side + 4 * i);
+      R.fl |= (unsigned)(terms & 3) << (2 * side);
+    }
+  }
+}
+
 int parse_ctml(const std::string& path, const std::string& phase_id, Mech& m,
                std::vector<std::string>& names) {
   std::ifstream f(path);
@@ -1390,6 +1547,7 @@ int parse_ctml(const std::string& path, const std::string& phase_id, Mech& m,
     r++;
   }
   m.nr = r;
+  prepare_cells(m);
   return 0;
 }
 
@@ -1472,14 +1630,13 @@ int astr_hip_chem_rates_device(astr_chem* c, long long n, const double* T, const
   if (n == 0) return 0;
   if (!T || !rho_or_p || !Y || !wdot) return cfail("null buffer");
   CHIP_OK(hipSetDevice(c->device));
-  const int bs = 256;
+  const int bs = kCellBlock;
   const dim3 grid((unsigned)((n + bs - 1) / bs));
-  if (c->host.ns == 9)
-    hipLaunchKernelGGL(k_chem<9>, grid, dim3(bs), 0, (hipStream_t)stream, c->dev, n, T, rho_or_p,
-                       input_is_p, Y, wdot, h_mix, cp_mix, h_k);
-  else
-    hipLaunchKernelGGL(k_chem<NSMAX>, grid, dim3(bs), 0, (hipStream_t)stream, c->dev, n, T, rho_or_p,
-                       input_is_p, Y, wdot, h_mix, cp_mix, h_k);
+  const bool nine = c->host.ns == 9, unit = c->host.unit != 0;
+  auto kern = nine ? (unit ? k_chem<9, true> : k_chem<9, false>)
+                   : (unit ? k_chem<NSMAX, true> : k_chem<NSMAX, false>);
+  hipLaunchKernelGGL(kern, grid, dim3(bs), 0, (hipStream_t)stream, c->dev, n, T, rho_or_p, input_is_p,
+                     Y, wdot, h_mix, cp_mix, h_k);
   CHIP_OK(hipGetLastError());
   return 0;
 }
@@ -1539,14 +1696,13 @@ int astr_hip_srccomb_device(astr_chem* c, int im, int jm, int km, int hm, int nu
   if (int rc = srccomb_check(c, im, jm, km, hm, numq, rho, tmp, spc, jacob, qrhs)) return rc;
   CHIP_OK(hipSetDevice(c->device));
   const long long ncell = (long long)(im + 1) * (jm + 1) * (km + 1);
-  const int bs = 256;
+  const int bs = kCellBlock;
   const dim3 grid((unsigned)((ncell + bs - 1) / bs));
-  if (c->host.ns == 9)
-    hipLaunchKernelGGL(k_srccomb<9>, grid, dim3(bs), 0, (hipStream_t)stream, c->dev, im, jm, km, hm,
-                       rho, tmp, spc, jacob, qrhs);
-  else
-    hipLaunchKernelGGL(k_srccomb<NSMAX>, grid, dim3(bs), 0, (hipStream_t)stream, c->dev, im, jm, km,
-                       hm, rho, tmp, spc, jacob, qrhs);
+  const bool nine = c->host.ns == 9, unit = c->host.unit != 0;
+  auto kern = nine ? (unit ? k_srccomb<9, true> : k_srccomb<9, false>)
+                   : (unit ? k_srccomb<NSMAX, true> : k_srccomb<NSMAX, false>);
+  hipLaunchKernelGGL(kern, grid, dim3(bs), 0, (hipStream_t)stream, c->dev, im, jm, km, hm, rho, tmp, spc,
+                     jacob, qrhs);
   CHIP_OK(hipGetLastError());
   return 0;
 }

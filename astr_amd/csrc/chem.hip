@@ -20,6 +20,7 @@
 #include <map>
 #include <sstream>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/astr_hip.h"
@@ -700,26 +701,11 @@ __device__ __forceinline__ void add_at(double (&v)[NS], int idx, double x) {
 // Lanes of a reactor team (one DPP row); the team kernel is further down.
 constexpr int kTeam = 16;
 
-// The sum of v over the 16 lanes of a team: a fixed tree into the team's
-// lane 0 (the same association on every team), then lane 0's sum to every
-// lane, so that all lanes of the team hold the same bits.
-__device__ __forceinline__ double team_sum(double v) {
-  v += __shfl_down(v, 8, kTeam);
-  v += __shfl_down(v, 4, kTeam);
-  v += __shfl_down(v, 2, kTeam);
-  v += __shfl_down(v, 1, kTeam);
-  return __shfl(v, 0, kTeam);
-}
-
 // Inlined at every call, so that the caller's state arrays stay in registers
-// (a call would take them by address, in scratch memory).  LANES = kTeam:
-// the team evaluates one right-hand side together, lane l taking reactions
-// l, l + 16, ...; each species rate is then summed over the team (team_sum),
-// and every lane ends with the same f.  LANES = 1: one thread, every
-// reaction in order.
-template <int NS, int LANES = 1>
+// (a call would take them by address, in scratch memory).
+template <int NS>
 __device__ __forceinline__ void reactor_rhs_n(const Mech* __restrict__ M, double p, const double (&yv)[NS + 1],
-                                              double (&f)[NS + 1], int lane = 0) {
+                                              double (&f)[NS + 1]) {
   const double T = yv[0];
   double c[NS], g[NS], w[NS], cpr[NS], hrt[NS];
   double winv = 0.0;
@@ -741,7 +727,7 @@ __device__ __forceinline__ void reactor_rhs_n(const Mech* __restrict__ M, double
     w[k] = 0.0;
   }
   const double lc0 = log(M->p0 / (kRgas * T));
-  for (int r = LANES > 1 ? lane : 0; r < M->nr; r += LANES) {
+  for (int r = 0; r < M->nr; r++) {
     const double kf = exp(M->lnA[r] + M->b[r] * logT - M->EaR[r] * invT);
     double fwd = kf;
     double dg = 0.0;
@@ -770,10 +756,6 @@ __device__ __forceinline__ void reactor_rhs_n(const Mech* __restrict__ M, double
     }
     for (int j = 0; j < M->nre[r]; j++) add_at<NS>(w, M->rsp[r][j], -M->rnu[r][j] * q);
     for (int j = 0; j < M->npr[r]; j++) add_at<NS>(w, M->psp[r][j], M->pnu[r][j] * q);
-  }
-  if constexpr (LANES > 1) {
-#pragma unroll
-    for (int k = 0; k < NS; k++) w[k] = team_sum(w[k]);
   }
   double cp = 0.0, dh = 0.0;
 #pragma unroll
@@ -1098,19 +1080,29 @@ __global__ __launch_bounds__(64) void k_reactor_eval(const Mech* __restrict__ M,
 
 // ---------------------------------------------------------------------------
 // The same reactor integrated by a team of 16 lanes (one DPP row), four
-// reactors per wavefront, for latency: each right-hand side is evaluated by
-// the whole team (the reactions split over the lanes, the species rates
-// summed over the team into identical values on every lane), the step's
-// Jacobian columns, which do not depend on each other, by separate lanes at
-// once (lane j the analytic column j), and the LU elimination runs one row
-// per lane.  The pivot search, both triangular solves, the stage sums and
-// the step control are done by every lane of the team, in the one-thread
-// kernel's order; only the species-rate sums associate differently.
+// reactors per wavefront, for latency.  A few dozen reactors leave almost the
+// whole chip idle, and what an ignition takes is the length of one reactor's
+// chain of operations; so every vector of the method is spread over the lanes
+// and nothing is computed twice:
+//   lane l < N holds component l of the state and of every stage vector (0 the
+//     temperature, 1 + k species k, whose thermodynamics it evaluates);
+//   lane r evaluates reactions r, r + 16, r + 32, its records in registers;
+//   lane j < N forms column j of the analytic Jacobian from the reactions'
+//     derivatives, and after a transposition holds row j of I - gamma h J for
+//     the elimination and the triangular solves.
+// Sums over species and the solves' broadcasts go through DPP row operations;
+// concentrations, reaction rates and the reactions' derivative rows go through
+// the team's LDS, where each lane reads the species of its own reactions.
+// A step attempt (six right-hand sides, a Jacobian, a factorisation, six
+// solves) takes 18 us, against 167 us with the whole right-hand side's species
+// part, the stage sums and the triangular solves repeated by every lane
+// (20 attempts: 40 reactors 4.0 -> 0.94 ms, 4096 3.7 -> 0.41, 16384 14.6 ->
+// 1.6; the one-thread kernel 13 ms at each).
 // A team's lanes hold identical scalars (t, h, err), so its control flow is
 // uniform; teams of one wavefront may diverge, which is why the kernel uses
-// no workgroup barrier.  The team's matrix sits in LDS; a team is part of one
-// wavefront, whose LDS accesses complete in order, so a wave barrier (for
-// the compiler) orders one lane's write before another lane's read.
+// no workgroup barrier.  A team is part of one wavefront, whose LDS accesses
+// complete in order, so a wave barrier (for the compiler) orders one lane's
+// write before another lane's read.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void team_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1118,140 +1110,417 @@ __device__ __forceinline__ void team_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// ro_stages for a team: the same six stages in the same arithmetic, with the
-// stage vectors U_s in the team's LDS (Us, 6 N doubles) instead of in each
-// lane's registers.  Every lane computes each stage (the right-hand side and
-// the triangular solves, as the one-thread kernel does); lane k < N then
-// stores component k of U_s, and the next stage reads them all back.  The
-// stage loop stays rolled, so that the right-hand side is inlined once.
-template <int NS>
-__device__ __forceinline__ double ro_stages_team(const Mech* __restrict__ M, double p, double h, const double* a,
-                                                 const int (&piv)[NS + 1], const double (&y)[NS + 1],
-                                                 const double (&f0)[NS + 1], double (&ynew)[NS + 1],
-                                                 double rtol, double atol, double* Us, int lane) {
-  constexpr int N = NS + 1;
-  double u[N], yt[N], f1[N];
-  const double gh = kRoGamma * h;
-#pragma unroll
-  for (int k = 0; k < N; k++) u[k] = f0[k];
-  lu_solve_n<N, 1>(a, piv, u);
-#pragma unroll
-  for (int k = 0; k < N; k++) u[k] = gh * u[k];
-  if (lane < N) Us[lane] = pick<N>(u, lane);
-  team_sync();
-#pragma unroll 1
-  for (int s = 1; s < 6; s++) {
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-      double v = y[k];
-      // Y_s = y + sum_j a_sj U_j (s < 5); Y_6 = Y_5 + U_5
-      const int nj = s < 5 ? s : 4;
-      const int ra = s < 5 ? s - 1 : 3;
-#pragma unroll 1
-      for (int j = 0; j < nj; j++) v += kRoA[ra][j] * Us[j * N + k];
-      if (s == 5) v = v + Us[4 * N + k];
-      yt[k] = v;
-    }
-    reactor_rhs_n<NS, kTeam>(M, p, yt, f1, lane);
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-      double c = 0.0;
-#pragma unroll 1
-      for (int j = 0; j < s; j++) c += (kRoC[s - 1][j] / h) * Us[j * N + k];
-      u[k] = f1[k] + c;
-    }
-    lu_solve_n<N, 1>(a, piv, u);
-#pragma unroll
-    for (int k = 0; k < N; k++) u[k] = gh * u[k];
-    if (s < 5) {
-      if (lane < N) Us[s * N + lane] = pick<N>(u, lane);
-      team_sync();
-    }
-  }
-  double err = 0.0;
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    const double yn = yt[k] + u[k];
-    const double sc = (k == 0 ? 1e-6 : atol) + rtol * fmax(fabs(y[k]), fabs(yn));
-    const double e = fabs(u[k]) / sc;
-    if (!(e <= err)) err = e;  // a NaN makes err NaN and rejects the step
-    ynew[k] = yn;
-  }
-  return err;
+template <int CTRL>
+__device__ __forceinline__ double row_dpp(double v) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false));
 }
+// lane L's v on every lane of the team
+template <int L>
+__device__ __forceinline__ double row_lane(double v) {
+  return row_dpp<0x150 + L>(v);  // row_newbcast
+}
+// The sum over the team, the same bits on every lane: after each rotation two
+// lanes that differ by it hold the same pair of addends.
+__device__ __forceinline__ double row_sum(double v) {
+  v += row_dpp<0x128>(v);  // row_ror
+  v += row_dpp<0x124>(v);
+  v += row_dpp<0x122>(v);
+  v += row_dpp<0x121>(v);
+  return v;
+}
+// the largest bit pattern over the team
+__device__ __forceinline__ unsigned long long row_max(unsigned long long u) {
+  auto step = [&](double r) {
+    const unsigned long long o = (unsigned long long)__double_as_longlong(r);
+    u = o > u ? o : u;
+  };
+  step(row_dpp<0x128>(__longlong_as_double((long long)u)));
+  step(row_dpp<0x124>(__longlong_as_double((long long)u)));
+  step(row_dpp<0x122>(__longlong_as_double((long long)u)));
+  step(row_dpp<0x121>(__longlong_as_double((long long)u)));
+  return u;
+}
+// F(integral_constant<0>) ... F(integral_constant<N - 1>)
+template <int N, class F, int K = 0>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (K < N) {
+    f(std::integral_constant<int, K>{});
+    static_for<N, F, K + 1>(static_cast<F&&>(f));
+  }
+}
+
+// RODAS4's coefficients by the stage vector that they multiply: stage s > j
+// takes kTeamA[j][s - 1 - j] U_j into its argument and kTeamC[j][s - 1 - j] / h
+// U_j into its right-hand side.  Stage 5's argument is stage 4's plus U_4.
+struct TeamCoef {
+  double a[5][5] = {}, c[5][5] = {};
+  constexpr TeamCoef() {
+    for (int j = 0; j < 5; j++)
+      for (int s = j + 1; s < 6; s++) {
+        a[j][s - 1 - j] = s < 5 ? kRoA[s - 1][j] : j < 4 ? kRoA[3][j] : 1.0;
+        c[j][s - 1 - j] = kRoC[s - 1][j];
+      }
+  }
+};
+__constant__ const TeamCoef kTeamCoef;
+
+template <int NS>
+struct Team {
+  static constexpr int N = NS + 1;
+  static constexpr int RS = N + 2;  // row of the reactions' derivatives: N columns and where pads go
+  struct Lds {
+    double c[NS + 1], g[NS + 1], h[NS + 1];  // with a pad: 1, 0, 0
+    double q[NRMAX];                         // zero past the last reaction
+    double d[NRMAX][RS];
+    double a[N][N];
+  };
+  // one reaction, with one side's terms at a time
+  struct Rx {
+    double lnA, b, EaR, of, ob, eff[NS];
+    unsigned sp, fl;
+  };
+  struct Side {
+    double prod, g, h, td[3];  // td: the product's derivative by each term's concentration
+    int ix[3];
+  };
+
+  const Mech* __restrict__ M;
+  Lds& S;
+  const int lane, nr;
+  const double p, ip;
+  double W, iW, tmid, lo[15], hi[15];  // this lane's species (lanes without one: W = 0, iW = 0)
+  Rx rx0, rx1;                         // reactions lane and lane + 16
+  double nu[32];                       // this species' coefficients in reactions 0..31
+  const ExpK K;
+  // of the last rhs()
+  double T, invT, rho, winv, yw, cpr, hrt, cp;
+
+  __device__ __forceinline__ static Rx record(const Mech* __restrict__ M, int r, int nr) {
+    Rx x;
+    const Mech::Rx& R = M->rx[r < nr ? r : 0];
+    const bool tb = R.fl & 32;
+    x.lnA = R.lnA, x.b = R.b, x.EaR = R.EaR, x.sp = R.sp, x.fl = r < nr ? R.fl : 0;
+    x.of = x.ob = 0.0;
+    for (int j = 0; j < M->nre[r < nr ? r : 0]; j++) x.of += M->rnu[r < nr ? r : 0][j];
+    for (int j = 0; j < M->npr[r < nr ? r : 0]; j++) x.ob += M->pnu[r < nr ? r : 0][j];
+#pragma unroll
+    for (int k = 0; k < NS; k++) x.eff[k] = tb ? R.eff[k] : 0.0;
+    return x;
+  }
+
+  __device__ __forceinline__ Team(const Mech* __restrict__ M_, Lds& S_, int lane_, double p_)
+      : M(M_), S(S_), lane(lane_), nr(M_->nr), p(p_), ip(1.0 / p_) {
+    const bool has = lane >= 1 && lane <= NS;
+    const int k = has ? lane - 1 : 0;
+    W = has ? M->W[k] : 0.0;
+    iW = has ? M->iW[k] : 0.0;
+    tmid = M->tmid[k];
+    const double* c0 = &M->th[k][0].a0;
+    const double* c1 = &M->th[k][1].a0;
+#pragma unroll
+    for (int j = 0; j < 15; j++) lo[j] = c0[j], hi[j] = c1[j];
+    rx0 = record(M, lane, nr);
+    rx1 = record(M, lane + kTeam, nr);
+#pragma unroll
+    for (int r = 0; r < 32; r++) nu[r] = has && r < nr ? M->rx[r].nu[k] : 0.0;
+    if (lane == 0) S.c[NS] = 1.0, S.g[NS] = 0.0, S.h[NS] = 0.0;
+    for (int r = lane; r < NRMAX; r += kTeam) S.q[r] = 0.0;
+    team_sync();
+  }
+
+  // one side of a reaction from the concentrations in LDS
+  template <bool DER>
+  __device__ __forceinline__ Side side(const Rx& x, int r, bool products) const {
+    Side s;
+    if (x.fl & 64) {
+      const unsigned sp = products ? x.sp >> 12 : x.sp;
+#pragma unroll
+      for (int j = 0; j < 3; j++) s.ix[j] = sp >> (4 * j) & 15;
+      const double c0 = S.c[s.ix[0]], c1 = S.c[s.ix[1]], c2 = S.c[s.ix[2]];
+      s.g = S.g[s.ix[0]] + S.g[s.ix[1]] + S.g[s.ix[2]];
+      s.prod = c0 * c1 * c2;
+      if (DER) {
+        s.h = S.h[s.ix[0]] + S.h[s.ix[1]] + S.h[s.ix[2]];
+        s.td[0] = c1 * c2, s.td[1] = c0 * c2, s.td[2] = c0 * c1;
+      }
+      return s;
+    }
+    s.prod = 1.0, s.g = s.h = 0.0;
+    double c[3], v[3], w[3];
+    const int n = products ? M->npr[r] : M->nre[r];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      s.ix[j] = j < n ? (products ? M->psp[r][j] : M->rsp[r][j]) : NS;
+      v[j] = j < n ? (products ? M->pnu[r][j] : M->rnu[r][j]) : 0.0;
+      c[j] = S.c[s.ix[j]];
+      w[j] = j < n ? conc_pow(c[j], v[j]) : 1.0;
+      s.prod *= w[j];
+      s.g += v[j] * S.g[s.ix[j]];
+      s.h += v[j] * S.h[s.ix[j]];
+    }
+    if (DER) {
+#pragma unroll
+      for (int j = 0; j < 3; j++)
+        s.td[j] = j < n ? conc_pow_d(c[j], v[j]) * w[(j + 1) % 3] * w[(j + 2) % 3] : 0.0;
+    }
+    return s;
+  }
+
+  // reaction r: its rate, into S.q; DER: its row of derivatives, into S.d:
+  // column 0 dq/dT at fixed Y, column 1 + m dq/dY_m divided by rho/W_m
+  template <bool DER>
+  __device__ __forceinline__ void reaction(const Rx& x, int r, double logT) const {
+    if (r >= nr) return;
+    const double lkf = x.lnA + x.b * logT - x.EaR * invT;
+    const Side f = side<DER>(x, r, false), b = side<DER>(x, r, true);
+    const bool rev = x.fl & 16, tb = x.fl & 32;
+    double kf, kr;
+    rate_exp2(lkf, rev ? lkf + (b.g - f.g) : 0.0, K, kf, kr);
+    if (!rev) kr = 0.0;
+    double cm = 0.0;
+#pragma unroll
+    for (int k = 0; k < NS; k++) cm += x.eff[k] * S.c[k];
+    if (!tb) cm = 1.0;
+    const double fw = kf * f.prod, bw = rev ? kr * b.prod : 0.0, net = fw - bw;
+    S.q[r] = cm * net;
+    if constexpr (DER) {
+      const double dlf = x.b * invT + x.EaR * invT * invT;
+      const double dlr = dlf - (b.h - f.h) * invT + (x.ob - x.of) * invT;
+      const double one = tb ? 1.0 : 0.0;
+      const double s = cm * ((x.of + one) * fw - (x.ob + one) * bw);
+      const double base = s / (rho * winv);
+      double* d = S.d[r];
+      d[0] = cm * (fw * dlf - bw * dlr) - s * invT;
+#pragma unroll
+      for (int k = 0; k < NS; k++) d[1 + k] = net * x.eff[k] - base;
+      const double cf = cm * kf, cb = rev ? -cm * kr : 0.0;
+#pragma unroll
+      for (int j = 0; j < 3; j++) add(&d[1 + f.ix[j]], cf * f.td[j]);
+      if (rev) {
+#pragma unroll
+        for (int j = 0; j < 3; j++) add(&d[1 + b.ix[j]], cb * b.td[j]);
+      }
+    }
+  }
+  // an addition that nothing waits for; one lane's own row, in its order
+  __device__ __forceinline__ static void add(double* a, double v) {
+    __builtin_amdgcn_ds_atomic_fadd_f64((__attribute__((address_space(3))) double*)a, v);
+  }
+
+  // this lane's component of f(y); y = 0 on the lanes past the last one
+  template <bool DER>
+  __device__ __forceinline__ double rhs(double y) {
+    T = row_lane<0>(y);
+    invT = 1.0 / T;
+    const double logT = log(T), omlogT = 1.0 - logT, lc0 = M->lnp0R - logT;
+    yw = y * iW;
+    winv = row_sum(yw);
+    const double rtw = kRgas * T * winv;
+    rho = p / rtw;
+    const bool low = T <= tmid;
+    const auto poly = [&](const double (&r)[15], double& cpo, double& ho, double& go) {
+      const double b = r[13] * invT;
+      cpo = r[0] + T * (r[1] + T * (r[2] + T * (r[3] + T * r[4])));
+      ho = r[0] + T * (r[5] + T * (r[6] + T * (r[7] + T * r[8]))) + b;
+      go = r[0] * omlogT + T * (r[9] + T * (r[10] + T * (r[11] + T * r[12]))) + b - r[14] - lc0;
+    };
+    double c0, h0, g0, c1, h1, g1;
+    poly(lo, c0, h0, g0);
+    poly(hi, c1, h1, g1);
+    cpr = low ? c0 : c1;
+    hrt = low ? h0 : h1;
+    if (lane >= 1 && lane <= NS) {
+      S.c[lane - 1] = rho * yw;
+      S.g[lane - 1] = low ? g0 : g1;
+      if (DER) S.h[lane - 1] = hrt;
+    }
+    team_sync();
+    reaction<DER>(rx0, lane, logT);
+    if (nr > kTeam) reaction<DER>(rx1, lane + kTeam, logT);
+    if (nr > 2 * kTeam) {
+      const Rx x = record(M, lane + 2 * kTeam, nr);
+      reaction<DER>(x, lane + 2 * kTeam, logT);
+    }
+    team_sync();
+    double w[4] = {0.0, 0.0, 0.0, 0.0};
+    const auto sum8 = [&](auto first) {
+#pragma unroll
+      for (int r = decltype(first)::value; r < decltype(first)::value + 8; r++) w[r & 3] += nu[r] * S.q[r];
+    };
+    sum8(std::integral_constant<int, 0>{});
+    sum8(std::integral_constant<int, 8>{});
+    if (nr > 16) sum8(std::integral_constant<int, 16>{});
+    if (nr > 24) sum8(std::integral_constant<int, 24>{});
+    if (nr > 32 && lane >= 1 && lane <= NS)
+      for (int r = 32; r < nr; r++) w[r & 3] += M->rx[r].nu[lane - 1] * S.q[r];
+    const double dY = ((w[0] + w[1]) + (w[2] + w[3])) * W * (rtw * ip);
+    cp = row_sum(yw * cpr);
+    const double dh = row_sum(hrt * T * iW * dY);
+    return lane == 0 ? -dh / cp : dY;
+  }
+
+  // Row `lane` of A = I - gh J at the last rhs<true>(), f its result there.
+  // Column j by lane j: with dw_k = sum_r nu_rk dq_r/dY_j,
+  //   dY_k' = W_k/rho dw_k + f_k / (W_j sum Y/W)  (dT column: + f_k / T),
+  //   dT'   = -(sum_k h_k dY_k' + f_T dcp) / cp.
+  __device__ __forceinline__ void matrix(double f, double gh, double (&row)[N]) {
+    double dw[NS];
+#pragma unroll
+    for (int k = 0; k < NS; k++) dw[k] = 0.0;
+    const int j = lane < N ? lane : 0;
+#pragma unroll 2
+    for (int r = 0; r < nr; r++) {
+      const double q = S.d[r][j];
+#pragma unroll
+      for (int k = 0; k < NS; k++) dw[k] += M->rx[r].nu[k] * q;
+    }
+    const bool low = T <= tmid;
+    const auto dpoly = [&](const double (&r)[15]) {
+      return r[1] + T * (2.0 * r[2] + T * (3.0 * r[3] + T * (4.0 * r[4])));
+    };
+    const double dcpT = row_sum(yw * (low ? dpoly(lo) : dpoly(hi)));
+    const double dcp = lane == 0 ? dcpT : cpr * iW;
+    const double irho = kRgas * T * winv * ip;
+    const double sc = lane == 0 ? irho : iW;       // rho/W_j of the derivatives' scaling, times 1/rho
+    const double fs = lane == 0 ? invT : iW / winv;
+    const double hk = hrt * T * iW, ck = cpr * iW;
+    double dH = 0.0;
+    static_for<NS>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      const double fk = row_lane<1 + k>(f);
+      const double v = row_lane<1 + k>(W) * sc * dw[k] + fk * fs;
+      dw[k] = v;
+      dH += row_lane<1 + k>(hk) * v;
+      const double cT = row_lane<1 + k>(ck) * fk;
+      dH += lane == 0 ? cT : 0.0;
+    });
+    const double top = -(dH + row_lane<0>(f) * dcp) / cp;
+    if (lane < N) {
+      S.a[0][lane] = (lane == 0 ? 1.0 : 0.0) - gh * top;
+#pragma unroll
+      for (int k = 0; k < NS; k++) S.a[1 + k][lane] = (lane == 1 + k ? 1.0 : 0.0) - gh * dw[k];
+    }
+    team_sync();
+#pragma unroll
+    for (int k = 0; k < N; k++) row[k] = S.a[j][k];
+    team_sync();
+  }
+
+  // LU of the matrix whose row `lane` is a: pivots by the largest element (its
+  // low four bits give way to the lane, so that one maximum finds both), rows
+  // left where they are until the end, when lane i takes row src, position i.
+  // lw: the multipliers left of the diagonal, up: the row right of it divided
+  // by the diagonal element, dinv its reciprocal; zeros elsewhere.
+  __device__ __forceinline__ bool factor(double (&a)[N], double (&lw)[N], double (&up)[N], double& dinv,
+                                         int& src) {
+    bool used = lane >= N, ok = true;
+    double inv_own = 0.0;
+    src = lane;
+    static_for<N>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      const unsigned long long mag = (unsigned long long)__double_as_longlong(fabs(a[k]));
+      const unsigned long long best = row_max(used ? 0ull : (mag & ~15ull) | (unsigned)(15 - lane));
+      const double inv = 1.0 / a[k];
+      const int pk = 15 - (int)(best & 15);
+      if (lane == k) src = pk;
+      double piv[N];
+#pragma unroll
+      for (int c = k; c < N; c++) piv[c] = __shfl(a[c], pk, kTeam);
+      ok = ok && fabs(piv[k]) > 0.0;
+      const double pinv = __shfl(inv, pk, kTeam);
+      if (lane == pk) {
+        used = true;
+        inv_own = inv;
+      }
+      const double l = used ? 0.0 : a[k] * pinv;
+      if (!used) a[k] = l;
+#pragma unroll
+      for (int c = k + 1; c < N; c++) a[c] -= l * piv[c];
+    });
+    dinv = __shfl(inv_own, src, kTeam);
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const double v = __shfl(a[k], src, kTeam);
+      lw[k] = k < lane && lane < N ? v : 0.0;
+      up[k] = k > lane ? v * dinv : 0.0;
+    }
+    return ok;
+  }
+
+  // this lane's component of the solution for the right-hand side b
+  __device__ __forceinline__ double solve(const double (&lw)[N], const double (&up)[N], double dinv, int src,
+                                          double b) const {
+    b = __shfl(b, src, kTeam);
+    static_for<N - 1>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      b -= lw[k] * row_lane<k>(b);
+    });
+    b *= dinv;
+    static_for<N - 1>([&](auto kc) {
+      constexpr int k = N - 1 - decltype(kc)::value;
+      b -= up[k] * row_lane<k>(b);
+    });
+    return b;
+  }
+};
 
 template <int NS>
 __global__ __launch_bounds__(64) void k_reactor_team(const Mech* __restrict__ M, ReactorPool P,
                                                      int max_tries, double rtol, double atol) {
+  using TeamN = Team<NS>;
   constexpr int N = NS + 1;
   constexpr int TPB = 64 / kTeam;
-  static_assert(N < kTeam, "a team needs a lane per column and one for the unperturbed state");
-  __shared__ double sA[TPB][N * N];
-  __shared__ double sU[TPB][6 * N];
+  static_assert(N <= kTeam && NRMAX <= 3 * kTeam, "a lane per component, three reactions per lane");
+  __shared__ typename TeamN::Lds lds[TPB];
   const int team = threadIdx.x / kTeam, lane = threadIdx.x % kTeam;
   const int i = blockIdx.x * TPB + team;
   if (i >= P.cap || P.status[i] != RX_RUN) return;  // the whole team leaves
-  double* a = sA[team];
-#define AT(r, c) a[(r) * N + (c)]
-  const double gam = kRoGamma;
-  double y[N], f0[N], f1[N], yt[N];
-  int piv[N];
-#pragma unroll
-  for (int k = 0; k < N; k++) y[k] = P.y[(size_t)k * P.cap + i];
+  TeamN R(M, lds[team], lane, P.p[i]);
+  double y = lane < N ? P.y[(size_t)lane * P.cap + i] : 0.0;
   double t = P.t[i], h = P.h[i];
-  const double tend = P.tend[i], p = P.p[i];
+  const double tend = P.tend[i];
   int nstep = P.nstep[i], nrej = P.nrej[i], st = RX_RUN;
   for (int it = 0; it < max_tries; it++) {
     if (t >= tend) { st = RX_DONE; break; }
     if (h > tend - t) h = tend - t;
     if (!(h > 1e-18)) { st = RX_FAIL; break; }
-    // f(y) by the whole team, then lane j < N: column j of the analytic Jacobian
-    reactor_rhs_n<NS, kTeam>(M, p, y, f0, lane);
-    if (lane < N) {
-      reactor_jac_col<NS>(M, p, y, f0, lane, f1);
+    const double gh = kRoGamma * h, ih = 1.0 / h;
+    double f = R.template rhs<true>(y);
+    double a[N], lw[N], up[N], dinv;
+    int src;
+    R.matrix(f, gh, a);
+    const bool ok = R.factor(a, lw, up, dinv, src);
+    double err = 2.0, yn = y;
+    if (ok) {
+      // the arguments and the U sums of the stages still to come, [0] the next
+      double ya[5], cs[5];
 #pragma unroll
-      for (int k = 0; k < N; k++) AT(k, lane) = -gam * h * f1[k];
-      AT(lane, lane) += 1.0;
+      for (int s = 0; s < 5; s++) ya[s] = y, cs[s] = 0.0;
+      double u = gh * R.solve(lw, up, dinv, src, f);
+#pragma unroll 1
+      for (int j = 0; j < 5; j++) {
+#pragma unroll
+        for (int s = 0; s < 5; s++) {
+          ya[s] += kTeamCoef.a[j][s] * u;
+          cs[s] += (kTeamCoef.c[j][s] * ih) * u;
+        }
+        yn = ya[0];
+        f = R.template rhs<false>(yn);
+        u = gh * R.solve(lw, up, dinv, src, f + cs[0]);
+#pragma unroll
+        for (int s = 0; s < 4; s++) ya[s] = ya[s + 1], cs[s] = cs[s + 1];
+      }
+      yn += u;
+      const double sc = (lane == 0 ? 1e-6 : atol) + rtol * fmax(fabs(y), fabs(yn));
+      // the largest of the lanes' errors; a NaN's bits are above all others,
+      // it makes err NaN and rejects the step
+      const double e = lane < N ? fabs(fabs(u) / sc) : 0.0;
+      err = __longlong_as_double((long long)row_max((unsigned long long)__double_as_longlong(e)));
     }
-    team_sync();
-    // LU with partial pivoting: rows swapped one column per lane, then
-    // eliminated one row per lane
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-      int pk = k;
-      double m = fabs(AT(k, k));
-#pragma unroll
-      for (int r = k + 1; r < N; r++) {
-        const double v = fabs(AT(r, k));
-        if (v > m) { m = v; pk = r; }
-      }
-      piv[k] = pk;
-      ok = ok && (m > 0.0);
-      team_sync();
-      if (pk != k && lane < N) {
-        const double tmp = AT(k, lane);
-        AT(k, lane) = AT(pk, lane);
-        AT(pk, lane) = tmp;
-      }
-      team_sync();
-      const double inv = 1.0 / AT(k, k);
-      if (lane > k && lane < N) {
-        const double l = AT(lane, k) * inv;
-        AT(lane, k) = l;
-#pragma unroll
-        for (int c = k + 1; c < N; c++) AT(lane, c) -= l * AT(k, c);
-      }
-      team_sync();
-    }
-    double err = 2.0;
-    if (ok) err = ro_stages_team<NS>(M, p, h, a, piv, y, f0, yt, rtol, atol, sU[team], lane);
-    // the next step's matrix writes must follow every lane's solve reads
-    team_sync();
     if (err <= 1.0) {
       t += h;
-#pragma unroll
-      for (int k = 0; k < N; k++) y[k] = yt[k];
+      y = yn;
       nstep++;
       h *= ro_factor(err, true);
     } else {
@@ -1260,10 +1529,8 @@ __global__ __launch_bounds__(64) void k_reactor_team(const Mech* __restrict__ M,
     }
     if (t >= tend) { st = RX_DONE; break; }
   }
-#undef AT
+  if (lane < N) P.y[(size_t)lane * P.cap + i] = y;
   if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < N; k++) P.y[(size_t)k * P.cap + i] = y[k];
     P.t[i] = t;
     P.h[i] = h;
     P.nstep[i] = nstep;

@@ -91,3 +91,48 @@ def test_gpu_a_cell_without_a_finite_rate_leaves_the_others_alone(tmp_path, orde
     assert np.array_equal(wd2[:, keep], wd[:, keep])
     assert np.array_equal(h2[keep], h[keep]) and np.array_equal(cp2[keep], cp[keep])
     assert wd2[ix["N2"], 70] == 0.0 and np.isnan(wd2[ix["H2O2"], 70])
+
+
+def _repeated(tmp_path, times, base):
+    """The mechanism with its reactions repeated (with a pre-exponential
+    factor divided by the count, the same chemistry): 19 * times records."""
+    x = open(base).read()
+    a, b = x.index("<reaction "), x.rindex("</reaction>") + len("</reaction>")
+    import re
+    body = re.sub(r"(<A[^>]*>)([^<]+)(</A>)", lambda m: m[1] + repr(float(m[2]) / times) + m[3], x[a:b])
+    p = tmp_path / "many.xml"
+    p.write_text(x[:a] + "\n".join([body] * times) + x[b:])
+    return str(p)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("times,form", [(2, (False, False, False)), (1, (False, True, True)), (2, (False, True, False)),
+                                        (1, (False, False, True))])
+def test_gpu_reactor_team_on_derived_mechanisms(tmp_path, times, form):
+    """A team's third reaction per lane (38 reactions), general orders and
+    irreversible reactions: ignitions by the team and by the one-thread kernel
+    agree to the integrator's tolerance, in about the same number of steps (a
+    wrong Jacobian costs steps).  Nine reactors: a last wavefront with one."""
+    gm = AC.Mechanism(_repeated(tmp_path, times, variant(tmp_path, *form)))
+    assert gm.nr == 19 * times
+    ix = {s: k for k, s in enumerate(gm.names)}
+    rng = np.random.default_rng(41)
+    reqs = []
+    for _ in range(9):
+        X = np.zeros(gm.ns)
+        X[ix["H2"]], X[ix["O2"]], X[ix["N2"]] = 2.0 * rng.uniform(0.5, 2.0), 1.0, 3.76
+        reqs.append((rng.uniform(1050.0, 1400.0), rng.uniform(1.0, 10.0) * 101325.0, X * gm.W / (X * gm.W).sum()))
+    out = {}
+    for lanes in (1, 16):
+        pool = AC.ReactorPool(gm, 10, rtol=1e-6, atol=1e-12, lanes=lanes)
+        for k, (T0, p, Y) in enumerate(reqs):
+            pool.set(k, T0, p, Y, 2e-4)
+        st = pool.run(max_tries=500)
+        assert np.all(st[:9] == AC.ReactorPool.DONE) and st[9] == AC.ReactorPool.FREE
+        out[lanes] = [pool.get(k) for k in range(9)]
+        pool.close()
+    for a, b in zip(out[1], out[16]):
+        assert a[0] == b[0] and a[3] > 5
+        assert abs(b[1] / a[1] - 1.0) < 1e-5
+        assert np.abs(b[2] - a[2]).max() < 1e-6
+        assert abs(a[3] - b[3]) <= max(2, a[3] // 20)

@@ -18,6 +18,7 @@
 #include <cstring>
 #include <fstream>
 #include <map>
+#include <mutex>
 #include <sstream>
 #include <string>
 #include <type_traits>
@@ -1539,6 +1540,39 @@ __global__ __launch_bounds__(64) void k_reactor_team(const Mech* __restrict__ M,
   }
 }
 
+// A slot's state in and out: one launch each (set: 17 copies of 4 or 8 bytes
+// before, get: 13).  A reactor set, read and released takes 47 us, 290 with
+// the copies.
+struct SlotState {
+  double y[NYMAX], h, tend, p;
+};
+__global__ __launch_bounds__(64) void k_reactor_set(ReactorPool P, int slot, int n, SlotState s) {
+  const int k = threadIdx.x;
+#pragma unroll
+  for (int j = 0; j < NYMAX; j++)
+    if (k == j && j < n) P.y[(size_t)j * P.cap + slot] = s.y[j];
+  if (k == 0) {
+    P.t[slot] = 0.0;
+    P.h[slot] = s.h;
+    P.tend[slot] = s.tend;
+    P.p[slot] = s.p;
+    P.nstep[slot] = 0;
+    P.nrej[slot] = 0;
+    P.status[slot] = RX_RUN;
+  }
+}
+
+// out: y, then at NYMAX t and the two step counts
+__global__ __launch_bounds__(64) void k_reactor_get(ReactorPool P, int slot, int n, double* __restrict__ out) {
+  const int k = threadIdx.x;
+  if (k < n) out[k] = P.y[(size_t)k * P.cap + slot];
+  if (k == NYMAX) out[k] = P.t[slot];
+  if (k == NYMAX + 1) out[k] = (double)P.nstep[slot];
+  if (k == NYMAX + 2) out[k] = (double)P.nrej[slot];
+}
+
+__global__ void k_reactor_mark(ReactorPool P, int slot, int status) { P.status[slot] = status; }
+
 // ---------------------------------------------------------------------------
 // CTML reading (the subset the reference's mechanisms use)
 // ---------------------------------------------------------------------------
@@ -1834,6 +1868,8 @@ struct astr_reactor_pool {
   double rtol = 1e-6, atol = 1e-12;
   hipStream_t stream = nullptr;
   int lanes = 1;  // lanes per reactor: 1, or kTeam for the team kernel
+  double* pin = nullptr;  // pinned host memory that k_reactor_get writes, one call at a time
+  std::mutex pin_mutex;
 };
 
 extern "C" {
@@ -2060,8 +2096,11 @@ int astr_hip_reactor_create(astr_chem* chem, int capacity, double rtol, double a
   r->P.nrej = iv + 2 * cap;
   r->P.cap = capacity;
   r->lanes = chem->host.ns == 9 ? kTeam : 1;
-  if (hipMemset(r->base, 0, bytes) != hipSuccess || hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking) != hipSuccess) {
+  if (hipHostMalloc(&r->pin, (NYMAX + 3) * sizeof(double), hipHostMallocDefault) != hipSuccess ||
+      hipMemset(r->base, 0, bytes) != hipSuccess ||
+      hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking) != hipSuccess) {
     (void)hipFree(r->base);
+    if (r->pin) (void)hipHostFree(r->pin);
     delete r;
     return cfail("reactor pool set-up failed");
   }
@@ -2074,6 +2113,7 @@ int astr_hip_reactor_destroy(astr_reactor_pool* r) {
   (void)hipSetDevice(r->chem->device);
   (void)hipStreamSynchronize(r->stream);
   (void)hipFree(r->base);
+  (void)hipHostFree(r->pin);
   (void)hipStreamDestroy(r->stream);
   delete r;
   return 0;
@@ -2086,20 +2126,14 @@ int astr_hip_reactor_set(astr_reactor_pool* r, int slot, double T0, double p, co
   if (!(T0 > 0.0) || !(p > 0.0) || !(t_end >= 0.0) || !(h0 > 0.0)) return cfail("bad reactor state");
   CHIP_OK(hipSetDevice(r->chem->device));
   const int ns = r->chem->host.ns;
-  const size_t cap = (size_t)r->P.cap;
-  double yv[NYMAX];
-  yv[0] = T0;
-  for (int k = 0; k < ns; k++) yv[1 + k] = Y0[k];
-  for (int k = 0; k <= ns; k++)
-    CHIP_OK(hipMemcpyAsync(r->P.y + k * cap + slot, &yv[k], sizeof(double), hipMemcpyHostToDevice, r->stream));
-  const double sc[4] = {0.0, h0, t_end, p};
-  double* dst[4] = {r->P.t, r->P.h, r->P.tend, r->P.p};
-  for (int q = 0; q < 4; q++)
-    CHIP_OK(hipMemcpyAsync(dst[q] + slot, &sc[q], sizeof(double), hipMemcpyHostToDevice, r->stream));
-  const int iv[3] = {RX_RUN, 0, 0};
-  int* idst[3] = {r->P.status, r->P.nstep, r->P.nrej};
-  for (int q = 0; q < 3; q++)
-    CHIP_OK(hipMemcpyAsync(idst[q] + slot, &iv[q], sizeof(int), hipMemcpyHostToDevice, r->stream));
+  SlotState st{};
+  st.y[0] = T0;
+  for (int k = 0; k < ns; k++) st.y[1 + k] = Y0[k];
+  st.h = h0;
+  st.tend = t_end;
+  st.p = p;
+  hipLaunchKernelGGL(k_reactor_set, dim3(1), dim3(64), 0, r->stream, r->P, slot, ns + 1, st);
+  CHIP_OK(hipGetLastError());
   CHIP_OK(hipStreamSynchronize(r->stream));
   return 0;
 }
@@ -2171,14 +2205,14 @@ int astr_hip_reactor_get(astr_reactor_pool* r, int slot, double* t, double* yv, 
   if (slot < 0 || slot >= r->P.cap) return cfail("reactor slot out of range");
   CHIP_OK(hipSetDevice(r->chem->device));
   const int n = r->chem->host.ns + 1;
-  const size_t cap = (size_t)r->P.cap;
-  if (yv)
-    for (int k = 0; k < n; k++)
-      CHIP_OK(hipMemcpyAsync(&yv[k], r->P.y + k * cap + slot, sizeof(double), hipMemcpyDeviceToHost, r->stream));
-  if (t) CHIP_OK(hipMemcpyAsync(t, r->P.t + slot, sizeof(double), hipMemcpyDeviceToHost, r->stream));
-  if (nstep) CHIP_OK(hipMemcpyAsync(nstep, r->P.nstep + slot, sizeof(int), hipMemcpyDeviceToHost, r->stream));
-  if (nrej) CHIP_OK(hipMemcpyAsync(nrej, r->P.nrej + slot, sizeof(int), hipMemcpyDeviceToHost, r->stream));
+  std::lock_guard<std::mutex> lock(r->pin_mutex);
+  hipLaunchKernelGGL(k_reactor_get, dim3(1), dim3(64), 0, r->stream, r->P, slot, n, r->pin);
+  CHIP_OK(hipGetLastError());
   CHIP_OK(hipStreamSynchronize(r->stream));
+  if (yv) std::memcpy(yv, r->pin, n * sizeof(double));
+  if (t) *t = r->pin[NYMAX];
+  if (nstep) *nstep = (int)r->pin[NYMAX + 1];
+  if (nrej) *nrej = (int)r->pin[NYMAX + 2];
   return 0;
 }
 
@@ -2186,8 +2220,8 @@ int astr_hip_reactor_release(astr_reactor_pool* r, int slot) {
   if (!r) return cfail("null pool");
   if (slot < 0 || slot >= r->P.cap) return cfail("reactor slot out of range");
   CHIP_OK(hipSetDevice(r->chem->device));
-  const int v = RX_FREE;
-  CHIP_OK(hipMemcpyAsync(r->P.status + slot, &v, sizeof(int), hipMemcpyHostToDevice, r->stream));
+  hipLaunchKernelGGL(k_reactor_mark, dim3(1), dim3(1), 0, r->stream, r->P, slot, (int)RX_FREE);
+  CHIP_OK(hipGetLastError());
   CHIP_OK(hipStreamSynchronize(r->stream));
   return 0;
 }

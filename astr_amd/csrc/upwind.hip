@@ -19,7 +19,8 @@
 //                qrhs(i) + Fh(i) - Fh(i-1).  x-lines: one lane per
 //                interface, 63 points per wavefront, Fh(i-1) from the
 //                neighbouring lane; y- and z-lines: one lane per line and
-//                a run of 16 points, Fh(i-1) carried in registers.
+//                a run of up to 16 points (of one component, without
+//                the projection), Fh(i-1) carried in registers.
 // The sensor: k_ssf (the Ducros ratio from the stored velocity gradient and
 // the pressure with its halo values) and k_lshock (its maximum over the
 // cross of offsets -4..5 against shkcrt).
@@ -35,7 +36,14 @@
 namespace astr {
 namespace {
 
-constexpr int kRun = 16;  // points per lane of a y- or z-line
+// Points per lane of a y- or z-line: up to kRun, fewer (a quarter more work
+// at 4) until there are four wavefronts per SIMD.
+constexpr int kRun = 16;
+int run_length(long long lanes_per_point, int points) {
+  int run = kRun;
+  while (run > 4 && lanes_per_point * ((points + run - 1) / run) < 4 * 64 * 1024) run /= 2;
+  return run;
+}
 
 // ---------------------------------------------------------------------------
 // pointwise pieces
@@ -237,9 +245,14 @@ __device__ __forceinline__ double recons(const double* f, double bfac, bool shoc
 
 // chardecomp (solver.F90:1958-2162, no species); l, r = rho, u, v, w, p, E,
 // dxi row; rev, lev row-major 5 x 5.  A zero averaged metric row (where the
-// reference stops) cannot occur on the grids the host accepts.
-__device__ __forceinline__ void chardecomp(double gamma, const double* l, const double* r, double* rev,
-                                           double* lev) {
+// reference stops) cannot occur on the grids the host accepts.  The left
+// eigenvectors are formed before the projection and the right ones after it,
+// both from the Roe state, so that only one set is held at a time.
+struct Roe {
+  double u1, u2, u3, H, Css, b1, b2, rcs, g1, g2, g3, ugp;
+  int axis;  // the first metric component that is not zero
+};
+__device__ __forceinline__ Roe roe_state(double gamma, const double* l, const double* r) {
   const double rero = 1.0e-12;
   const double WRoe = sqrt(l[0]) / (sqrt(l[0]) + sqrt(r[0]));
   const double WRoe1 = 1.0 - WRoe;
@@ -260,6 +273,11 @@ __device__ __forceinline__ void chardecomp(double gamma, const double* l, const 
   const double ugp = u1 * g1 + u2 * g2 + u3 * g3;
   const double b1 = (gamma - 1.0) / (Css * Css);
   const double b2 = 1.0 + 2.0 * b1 * KRoe - b1 * HRoe;
+  return {u1, u2, u3, HRoe, Css, b1, b2, rcs, g1, g2, g3, ugp, fabs(var1) > rero ? 0 : fabs(var2) > rero ? 1 : 2};
+}
+__device__ __forceinline__ void left_vectors(const Roe& q, double* lev) {
+  const double u1 = q.u1, u2 = q.u2, u3 = q.u3, b1 = q.b1, b2 = q.b2, rcs = q.rcs, g1 = q.g1, g2 = q.g2, g3 = q.g3,
+               ugp = q.ugp;
   lev[0] = 0.5 * (b2 + ugp * rcs);
   lev[1] = -0.5 * (b1 * u1 + g1 * rcs);
   lev[2] = -0.5 * (b1 * u2 + g2 * rcs);
@@ -270,39 +288,47 @@ __device__ __forceinline__ void chardecomp(double gamma, const double* l, const 
   lev[7] = b1 * u2;
   lev[8] = b1 * u3;
   lev[9] = -b1;
-  rev[0] = 1.0; rev[5] = u1 - Css * g1; rev[10] = u2 - Css * g2; rev[15] = u3 - Css * g3;
-  rev[20] = HRoe - ugp * Css;
-  rev[1] = 1.0; rev[6] = u1; rev[11] = u2; rev[16] = u3; rev[21] = HRoe - 1.0 / b1;
-  if (fabs(var1) > rero) {
+  if (q.axis == 0) {
     const double rgp = 1.0 / g1;
     lev[10] = (ugp * g2 - u2) * rgp; lev[11] = -g2; lev[12] = (1.0 - g2 * g2) * rgp;
     lev[13] = -(g2 * g3 * rgp); lev[14] = 0.0;
     lev[15] = (ugp * g3 - u3) * rgp; lev[16] = -g3; lev[17] = -(g2 * g3 * rgp);
     lev[18] = (1.0 - g3 * g3) * rgp; lev[19] = 0.0;
-    rev[2] = 0.0; rev[7] = -g2; rev[12] = g1; rev[17] = 0.0; rev[22] = u2 * g1 - u1 * g2;
-    rev[3] = 0.0; rev[8] = -g3; rev[13] = 0.0; rev[18] = g1; rev[23] = u3 * g1 - u1 * g3;
-  } else if (fabs(var2) > rero) {
+  } else if (q.axis == 1) {
     const double rgp = 1.0 / g2;
     lev[10] = (ugp * g1 - u1) * rgp; lev[11] = (1.0 - g1 * g1) * rgp; lev[12] = -g1;
     lev[13] = -(g1 * g3 * rgp); lev[14] = 0.0;
     lev[15] = (ugp * g3 - u3) * rgp; lev[16] = -(g1 * g3 * rgp); lev[17] = -g3;
     lev[18] = (1.0 - g3 * g3) * rgp; lev[19] = 0.0;
-    rev[2] = 0.0; rev[7] = g2; rev[12] = -g1; rev[17] = 0.0; rev[22] = u1 * g2 - u2 * g1;
-    rev[3] = 0.0; rev[8] = 0.0; rev[13] = -g3; rev[18] = g2; rev[23] = u3 * g2 - u2 * g3;
   } else {
     const double rgp = 1.0 / g3;
     lev[10] = (ugp * g1 - u1) * rgp; lev[11] = (1.0 - g1 * g1) * rgp; lev[12] = -(g1 * g2 * rgp);
     lev[13] = -g1; lev[14] = 0.0;
     lev[15] = (ugp * g2 - u2) * rgp; lev[16] = -(g1 * g2 * rgp); lev[17] = (1.0 - g2 * g2) * rgp;
     lev[18] = -g2; lev[19] = 0.0;
-    rev[2] = 0.0; rev[7] = g3; rev[12] = 0.0; rev[17] = -g1; rev[22] = u1 * g3 - u3 * g1;
-    rev[3] = 0.0; rev[8] = 0.0; rev[13] = g3; rev[18] = -g2; rev[23] = u2 * g3 - u3 * g2;
   }
   lev[20] = 0.5 * (b2 - ugp * rcs);
   lev[21] = -0.5 * (b1 * u1 - g1 * rcs);
   lev[22] = -0.5 * (b1 * u2 - g2 * rcs);
   lev[23] = -0.5 * (b1 * u3 - g3 * rcs);
   lev[24] = 0.5 * b1;
+}
+__device__ __forceinline__ void right_vectors(const Roe& q, double* rev) {
+  const double u1 = q.u1, u2 = q.u2, u3 = q.u3, Css = q.Css, HRoe = q.H, b1 = q.b1, g1 = q.g1, g2 = q.g2, g3 = q.g3,
+               ugp = q.ugp;
+  rev[0] = 1.0; rev[5] = u1 - Css * g1; rev[10] = u2 - Css * g2; rev[15] = u3 - Css * g3;
+  rev[20] = HRoe - ugp * Css;
+  rev[1] = 1.0; rev[6] = u1; rev[11] = u2; rev[16] = u3; rev[21] = HRoe - 1.0 / b1;
+  if (q.axis == 0) {
+    rev[2] = 0.0; rev[7] = -g2; rev[12] = g1; rev[17] = 0.0; rev[22] = u2 * g1 - u1 * g2;
+    rev[3] = 0.0; rev[8] = -g3; rev[13] = 0.0; rev[18] = g1; rev[23] = u3 * g1 - u1 * g3;
+  } else if (q.axis == 1) {
+    rev[2] = 0.0; rev[7] = g2; rev[12] = -g1; rev[17] = 0.0; rev[22] = u1 * g2 - u2 * g1;
+    rev[3] = 0.0; rev[8] = 0.0; rev[13] = -g3; rev[18] = g2; rev[23] = u3 * g2 - u2 * g3;
+  } else {
+    rev[2] = 0.0; rev[7] = g3; rev[12] = 0.0; rev[17] = -g1; rev[22] = u1 * g3 - u3 * g1;
+    rev[3] = 0.0; rev[8] = 0.0; rev[13] = g3; rev[18] = -g2; rev[23] = u2 * g3 - u3 * g2;
+  }
   rev[4] = 1.0; rev[9] = u1 + Css * g1; rev[14] = u2 + Css * g2; rev[19] = u3 + Css * g3;
   rev[24] = HRoe + ugp * Css;
 }
@@ -496,32 +522,41 @@ template <int SCH, bool CD>
 __device__ __forceinline__ void face_flux(const UwArgs& u, long long c0, long long rs, bool lsh, double* Fh) {
   const double* sw = u.sw;
   const long long S = u.sws;
-  double Fhc[5];
   if constexpr (CD) {
     if (lsh) {
+      double Fhc[5] = {};
       double sl[9], sr[9], lev[25], rev[25];
 #pragma unroll
       for (int m = 0; m < 9; m++) {
         sl[m] = sw[(kUwFields + m) * S + c0];
         sr[m] = sw[(kUwFields + m) * S + c0 + rs];
       }
-      chardecomp(u.gamma, sl, sr, rev, lev);
+      const Roe R = roe_state(u.gamma, sl, sr);
+      left_vectors(R, lev);
+      // iwind8: '+' element k is row i+k-3, '-' element k is row i+4-k; one
+      // side at a time, in one copy of the code, so that its 8 x 5 window and
+      // the left vectors are all that the registers hold
+#pragma unroll 1
+      for (int side = 0; side < 2; side++) {
+        const double* sf = sw + 5 * side * S + c0 + (side ? 4 : -3) * rs;
+        const long long step = side ? -rs : rs;
+        double x[8][5];
 #pragma unroll
-      for (int m = 0; m < 5; m++) {
-        double wp[8], wm[8];
+        for (int k = 0; k < 8; k++)
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-          // iwind8: '+' element k is row i+k-3, '-' element k is row i+4-k
-          const long long ip = c0 + (long long)(k - 3) * rs, im = c0 + (long long)(4 - k) * rs;
-          wp[k] = lev[5 * m] * sw[ip] + lev[5 * m + 1] * sw[S + ip] + lev[5 * m + 2] * sw[2 * S + ip] +
-                  lev[5 * m + 3] * sw[3 * S + ip] + lev[5 * m + 4] * sw[4 * S + ip];
-          wm[k] = lev[5 * m] * sw[5 * S + im] + lev[5 * m + 1] * sw[6 * S + im] + lev[5 * m + 2] * sw[7 * S + im] +
-                  lev[5 * m + 3] * sw[8 * S + im] + lev[5 * m + 4] * sw[9 * S + im];
+          for (int c = 0; c < 5; c++) x[k][c] = sf[c * S + k * step];
+#pragma unroll
+        for (int m = 0; m < 5; m++) {
+          double w[8];
+#pragma unroll
+          for (int k = 0; k < 8; k++)
+            w[k] = lev[5 * m] * x[k][0] + lev[5 * m + 1] * x[k][1] + lev[5 * m + 2] * x[k][2] +
+                   lev[5 * m + 3] * x[k][3] + lev[5 * m + 4] * x[k][4];
+          const double v = recons<SCH>(w, u.bfac, lsh);
+          Fhc[m] = side ? Fhc[m] + v : v;
         }
-        const double v1 = recons<SCH>(wp, u.bfac, lsh);
-        const double v2 = recons<SCH>(wm, u.bfac, lsh);
-        Fhc[m] = v1 + v2;
       }
+      right_vectors(R, rev);
 #pragma unroll
       for (int m = 0; m < 5; m++)
         Fh[m] = rev[5 * m] * Fhc[0] + rev[5 * m + 1] * Fhc[1] + rev[5 * m + 2] * Fhc[2] + rev[5 * m + 3] * Fhc[3] +
@@ -556,7 +591,7 @@ __device__ __forceinline__ void face_update1(const FlowArgs& a, int m, long long
 // x-lines: lane l of a wavefront takes interface i0 - 1 + l of segment
 // (L, sg); lanes 1..63 update points i0..i0+62
 template <int SCH, bool CD>
-__global__ __launch_bounds__(256) void k_uw_face_x(FlowArgs a, UwArgs u, int first, int last) {
+__global__ __launch_bounds__(256, CD ? 2 : 1) void k_uw_face_x(FlowArgs a, UwArgs u, int first, int last) {
   const int n = a.n[0];
   const int NR = n + 9;
   const long long NL = uw_lines(a.n, 0);
@@ -580,72 +615,73 @@ __global__ __launch_bounds__(256) void k_uw_face_x(FlowArgs a, UwArgs u, int fir
 }
 
 // y- and z-lines without the characteristic projection: one lane per line
-// and a run of kRun points; per component the 8-row windows of F+ and F-
-// slide along the run in registers (one new row of each per point)
+// and a run of kRun points of one component (the grid's y): the 8-row windows
+// of F+ and F- slide along the run in registers (one new row of each per
+// point).  With the components one after the other in each lane, 97^3 left
+// one wavefront per SIMD with its serial windows: MP7 88 us, now 46 (the bytes
+// of the split buffer and qrhs, 150 MB, take 33).
 template <int SCH, int DIR>
-__global__ __launch_bounds__(256) void k_uw_face_yz(FlowArgs a, UwArgs u, int first, int last) {
+__global__ __launch_bounds__(256) void k_uw_face_yz(FlowArgs a, UwArgs u, int len, int first, int last) {
   constexpr int dir = DIR;
   const int n = a.n[dir];
   const long long NL = uw_lines(a.n, dir);
-  const int nruns = (n + 1 + kRun - 1) / kRun;
+  const int nruns = (n + len) / len;
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= NL * nruns) return;
   const int run = (int)(idx / NL);
   const long long L = idx - (long long)run * NL;
-  const int r0 = run * kRun, r1 = min(r0 + kRun - 1, n);
+  const int r0 = run * len, r1 = min(r0 + len - 1, n);
   int c3[3];
   const long long o0 = line_base(a, dir, L, c3);
   const long long st = dir_stride(a, dir);
   const double* sw = u.sw;
   const long long S = u.sws;
   bool shp = face_shock(u, o0, st, r0 - 1, n);
-#pragma unroll 1
-  for (int m = 0; m < 5; m++) {
-    // rows r0-4 .. r0+3: the window of interface r0-1
-    double wp[8], wr[8];
+  const int m = blockIdx.y;
+  // rows r0-4 .. r0+3: the window of interface r0-1
+  double wp[8], wr[8];
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const long long c = (long long)(r0 - 4 + k + 4) * NL + L;
-      wp[k] = sw[m * S + c];
-      wr[k] = sw[(5 + m) * S + c];
+  for (int k = 0; k < 8; k++) {
+    const long long c = (long long)(r0 - 4 + k + 4) * NL + L;
+    wp[k] = sw[m * S + c];
+    wr[k] = sw[(5 + m) * S + c];
+  }
+  double wm[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) wm[k] = wr[7 - k];
+  double prev = recons<SCH>(wp, u.bfac, shp) + recons<SCH>(wm, u.bfac, shp);
+#pragma unroll 1
+  for (int t = r0; t <= r1; t++) {
+#pragma unroll
+    for (int k = 0; k < 7; k++) {
+      wp[k] = wp[k + 1];
+      wr[k] = wr[k + 1];
     }
-    double wm[8];
+    const long long c = (long long)(t + 4 + 4) * NL + L;
+    wp[7] = sw[m * S + c];
+    wr[7] = sw[(5 + m) * S + c];
 #pragma unroll
     for (int k = 0; k < 8; k++) wm[k] = wr[7 - k];
-    double prev = recons<SCH>(wp, u.bfac, shp) + recons<SCH>(wm, u.bfac, shp);
-#pragma unroll 1
-    for (int t = r0; t <= r1; t++) {
-#pragma unroll
-      for (int k = 0; k < 7; k++) {
-        wp[k] = wp[k + 1];
-        wr[k] = wr[k + 1];
-      }
-      const long long c = (long long)(t + 4 + 4) * NL + L;
-      wp[7] = sw[m * S + c];
-      wr[7] = sw[(5 + m) * S + c];
-#pragma unroll
-      for (int k = 0; k < 8; k++) wm[k] = wr[7 - k];
-      const bool sh = face_shock(u, o0, st, t, n);
-      const double cur = recons<SCH>(wp, u.bfac, sh) + recons<SCH>(wm, u.bfac, sh);
-      face_update1(a, m, o0 + (long long)t * st, cur, prev, first, last);
-      prev = cur;
-    }
+    const bool sh = face_shock(u, o0, st, t, n);
+    const double cur = recons<SCH>(wp, u.bfac, sh) + recons<SCH>(wm, u.bfac, sh);
+    face_update1(a, m, o0 + (long long)t * st, cur, prev, first, last);
+    prev = cur;
   }
 }
 
 // y- and z-lines with the characteristic projection: one lane per line
 // and a run of kRun points, the five components of each interface together
 template <int SCH, int DIR>
-__global__ __launch_bounds__(256) void k_uw_face_yz_cd(FlowArgs a, UwArgs u, int first, int last) {
+__global__ __launch_bounds__(256, 2) void k_uw_face_yz_cd(FlowArgs a, UwArgs u, int len, int first, int last) {
   constexpr int dir = DIR;
   const int n = a.n[dir];
   const long long NL = uw_lines(a.n, dir);
-  const int nruns = (n + 1 + kRun - 1) / kRun;
+  const int nruns = (n + len) / len;
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= NL * nruns) return;
   const int run = (int)(idx / NL);
   const long long L = idx - (long long)run * NL;
-  const int r0 = run * kRun, r1 = min(r0 + kRun - 1, n);
+  const int r0 = run * len, r1 = min(r0 + len - 1, n);
   int c3[3];
   const long long o0 = line_base(a, dir, L, c3);
   const long long st = dir_stride(a, dir);
@@ -728,12 +764,10 @@ __global__ __launch_bounds__(64) void k_lshock(FlowArgs a, UwArgs u) {
 // (k_cuw_face) and its difference into qrhs (k_cuw_diff).
 // ---------------------------------------------------------------------------
 
-// split-buffer index of row r (-4..n+4) of line L for the compact scheme's
-// lane-per-line sweeps (with the characteristic projection), which keep
-// every direction's lines fastest, so that one lane per line coalesces
-template <int DIR>
-__device__ __forceinline__ long long cuw_at(long long L, int r, int NR, long long NL) {
-  (void)NR;
+// split-buffer index of row r (-4..n+4) of line L for the compact scheme with
+// the characteristic projection, which keeps every direction's lines fastest:
+// consecutive lanes take consecutive lines
+__device__ __forceinline__ long long cuw_at(long long L, int r, long long NL) {
   return (long long)(r + 4) * NL + L;
 }
 
@@ -749,76 +783,18 @@ __device__ __forceinline__ double mp5(const double* u, double ul, bool shock) {
   return ul;
 }
 
-// flux_compact (flux.F90:125-150, compact_flux_rhs :163-254, the Thomas
-// sweeps of tridiagonal_thomas_solver, commfunc.F90:790-813) of one line and
-// one split component (0..4 F+ with the upwind scheme, 5..9 F- with the
-// downwind one): rows -2..n+1, the end rows the explicit 6th-order interface
-// value, rows -1..n the 5th-order compact one.  The forward sweep leaves d'
-// in the output rows, the backward sweep overwrites them with the solution;
-// rows -1..n are the interface fluxes fh(-1:n).  One lane per (component,
-// line); for y and z the lanes of a wavefront take consecutive lines, so
-// every access coalesces.
+// The interface flux Fh(i), i = -1..n, of convrsdcmp (solver.F90:1366-1490)
+// with the characteristic projection: the windows Flcp(m, n) =
+// fplus(i+n-3), Flcm(m, n) = fminus(i+4-n), n = 1..5 (iwind6) and the compact
+// values, all of them projected on the Roe-state characteristics of rows i,
+// i+1, each limited by MP5 (no crinod: hdiss false), summed, projected back.
+// Fh(i) replaces the compact value of F+ component m at row i (this lane's own
+// row, read before).  Both sides unrolled with both sets of eigenvectors took
+// 310 registers, one wavefront per SIMD and 102 us at 73^3; one side at a time
+// takes 168, three wavefronts and 51 us (its bytes 20).
 template <int DIR>
-__global__ __launch_bounds__(256) void k_cuw_solve(FlowArgs a, UwArgs u) {
+__global__ __launch_bounds__(256, 3) void k_cuw_face(FlowArgs a, UwArgs u) {
   const int n = a.n[DIR];
-  const int NR = n + 9;
-  const long long NL = uw_lines(a.n, DIR);
-  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= 10 * NL) return;
-  const int f = (int)(idx / NL);
-  const long long L = idx - (long long)f * NL;
-  const bool plus = f < 5;
-  const double* __restrict__ ac = u.cuw_ac + cuw_ac_offset(a.n, DIR, plus);
-  const double* __restrict__ src = u.sw + f * u.sws;
-  double* __restrict__ dst = u.fhc + f * u.sws;
-  const double b = u.bfac;
-  const double k118 = 1.0 / 18.0, k136 = 1.0 / 36.0, k1918 = 19.0 / 18.0, k59 = 5.0 / 9.0, k936 = 9.0 / 36.0;
-  const double w0 = k118 - k136 * b, w1 = k1918 - k936 * b, w2 = k59 + k936 * b, w3 = k136 * b;
-  const double c37 = 37.0 / 60.0, c2 = 2.0 / 15.0, c1 = 1.0 / 60.0;
-  auto F = [&](int r) { return src[cuw_at<DIR>(L, r, NR, NL)]; };
-  auto end_row = [&](int j) {
-    const double v1 = F(j) + F(j + 1), v2 = F(j - 1) + F(j + 2), v3 = F(j - 2) + F(j + 3);
-    return c37 * v1 - c2 * v2 + c1 * v3;
-  };
-  const int N = n + 4;
-  double dp = end_row(-2);
-  dst[cuw_at<DIR>(L, -2, NR, NL)] = dp;
-  // interior rows j = -1..n: the window F(j-1..j+2) slides one row a step;
-  // unrolled so that the loads of later rows issue ahead of the recurrence
-  double f0 = F(-2), f1 = F(-1), f2 = F(0);
-#pragma unroll 8
-  for (int r = 1; r < N - 1; r++) {
-    const int j = r - 2;
-    const double f3 = F(j + 2);
-    const double d = plus ? w0 * f0 + w1 * f1 + w2 * f2 + w3 * f3 : w0 * f3 + w1 * f2 + w2 * f1 + w3 * f0;
-    dp = d * ac[3 * r + 1] - dp * ac[3 * r + 2];
-    dst[cuw_at<DIR>(L, j, NR, NL)] = dp;
-    f0 = f1;
-    f1 = f2;
-    f2 = f3;
-  }
-  dp = end_row(n + 1) * ac[3 * (N - 1) + 1] - dp * ac[3 * (N - 1) + 2];
-  dst[cuw_at<DIR>(L, n + 1, NR, NL)] = dp;
-  double x = dp;
-#pragma unroll 8
-  for (int r = N - 2; r >= 0; r--) {
-    const int j = r - 2;
-    const long long c = cuw_at<DIR>(L, j, NR, NL);
-    x = dst[c] - ac[3 * r] * x;
-    dst[c] = x;
-  }
-}
-
-// The interface flux Fh(i), i = -1..n, of convrsdcmp (solver.F90:1366-1490):
-// the windows Flcp(m, n) = fplus(i+n-3), Flcm(m, n) = fminus(i+4-n), n =
-// 1..5 (iwind6) and the compact values, with CD all of them projected on the
-// Roe-state characteristics of rows i, i+1, each limited by MP5 (no crinod:
-// hdiss false), summed, projected back.  Fh(i) replaces the compact value of
-// F+ component m at row i (this lane's own row, read before).
-template <int DIR, bool CD>
-__global__ __launch_bounds__(256) void k_cuw_face(FlowArgs a, UwArgs u) {
-  const int n = a.n[DIR];
-  const int NR = n + 9;
   const long long NL = uw_lines(a.n, DIR);
   const long long NI = n + 2;
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
@@ -828,65 +804,51 @@ __global__ __launch_bounds__(256) void k_cuw_face(FlowArgs a, UwArgs u) {
   const long long L = idx - (long long)(i + 1) * NL;
   int c3[3];
   const long long o0 = line_base(a, DIR, L, c3);
-  const long long st = dir_stride(a, DIR);
-  const bool lsh = face_shock(u, o0, st, i, n);
+  const bool lsh = face_shock(u, o0, dir_stride(a, DIR), i, n);
   const double* sw = u.sw;
   const long long S = u.sws;
-  const long long ci = cuw_at<DIR>(L, i, NR, NL);
-  auto at = [&](int r) { return cuw_at<DIR>(L, r, NR, NL); };
-  double hp[5], hm[5], Fh[5];
+  const long long ci = cuw_at(L, i, NL);
+  double sl[9], sr[9], lev[25], rev[25], Fhc[5] = {};
+  const long long cr = cuw_at(L, i + 1, NL);
 #pragma unroll
-  for (int m = 0; m < 5; m++) {
-    hp[m] = u.fhc[m * S + ci];
-    hm[m] = u.fhc[(5 + m) * S + ci];
+  for (int m = 0; m < 9; m++) {
+    sl[m] = sw[(kUwFields + m) * S + ci];
+    sr[m] = sw[(kUwFields + m) * S + cr];
   }
-  if constexpr (CD) {
-    double sl[9], sr[9], lev[25], rev[25];
-    const long long cr = at(i + 1);
+  const Roe R = roe_state(u.gamma, sl, sr);
+  left_vectors(R, lev);
+  // one side at a time, in one copy of the code, as face_flux does
+#pragma unroll 1
+  for (int side = 0; side < 2; side++) {
+    const double* sf = sw + 5 * side * S + cuw_at(L, side ? i + 3 : i - 2, NL);
+    const double* hf = u.fhc + 5 * side * S + ci;
+    const long long step = side ? -NL : NL;
+    double x[5][5], h[5];
 #pragma unroll
-    for (int m = 0; m < 9; m++) {
-      sl[m] = sw[(kUwFields + m) * S + ci];
-      sr[m] = sw[(kUwFields + m) * S + cr];
-    }
-    chardecomp(u.gamma, sl, sr, rev, lev);
-    double Fhc[5];
+    for (int k = 0; k < 5; k++)
+#pragma unroll
+      for (int c = 0; c < 5; c++) x[k][c] = sf[c * S + k * step];
+#pragma unroll
+    for (int c = 0; c < 5; c++) h[c] = hf[c * S];
 #pragma unroll
     for (int m = 0; m < 5; m++) {
-      double wp[5], wm[5];
+      double w[5];
 #pragma unroll
-      for (int k = 0; k < 5; k++) {
-        const long long ip = at(i + k - 2), im = at(i + 3 - k);
-        wp[k] = lev[5 * m] * sw[ip] + lev[5 * m + 1] * sw[S + ip] + lev[5 * m + 2] * sw[2 * S + ip] +
-                lev[5 * m + 3] * sw[3 * S + ip] + lev[5 * m + 4] * sw[4 * S + ip];
-        wm[k] = lev[5 * m] * sw[5 * S + im] + lev[5 * m + 1] * sw[6 * S + im] + lev[5 * m + 2] * sw[7 * S + im] +
-                lev[5 * m + 3] * sw[8 * S + im] + lev[5 * m + 4] * sw[9 * S + im];
-      }
-      const double lp = lev[5 * m] * hp[0] + lev[5 * m + 1] * hp[1] + lev[5 * m + 2] * hp[2] +
-                        lev[5 * m + 3] * hp[3] + lev[5 * m + 4] * hp[4];
-      const double lm = lev[5 * m] * hm[0] + lev[5 * m + 1] * hm[1] + lev[5 * m + 2] * hm[2] +
-                        lev[5 * m + 3] * hm[3] + lev[5 * m + 4] * hm[4];
-      const double v1 = mp5(wp, lp, lsh);
-      const double v2 = mp5(wm, lm, lsh);
-      Fhc[m] = v1 + v2;
-    }
-#pragma unroll
-    for (int m = 0; m < 5; m++)
-      Fh[m] = rev[5 * m] * Fhc[0] + rev[5 * m + 1] * Fhc[1] + rev[5 * m + 2] * Fhc[2] + rev[5 * m + 3] * Fhc[3] +
-              rev[5 * m + 4] * Fhc[4];
-  } else {
-#pragma unroll
-    for (int m = 0; m < 5; m++) {
-      double wp[5], wm[5];
-#pragma unroll
-      for (int k = 0; k < 5; k++) {
-        wp[k] = sw[m * S + at(i + k - 2)];
-        wm[k] = sw[(5 + m) * S + at(i + 3 - k)];
-      }
-      const double v1 = mp5(wp, hp[m], lsh);
-      const double v2 = mp5(wm, hm[m], lsh);
-      Fh[m] = v1 + v2;
+      for (int k = 0; k < 5; k++)
+        w[k] = lev[5 * m] * x[k][0] + lev[5 * m + 1] * x[k][1] + lev[5 * m + 2] * x[k][2] +
+               lev[5 * m + 3] * x[k][3] + lev[5 * m + 4] * x[k][4];
+      const double l = lev[5 * m] * h[0] + lev[5 * m + 1] * h[1] + lev[5 * m + 2] * h[2] + lev[5 * m + 3] * h[3] +
+                       lev[5 * m + 4] * h[4];
+      const double v = mp5(w, l, lsh);
+      Fhc[m] = side ? Fhc[m] + v : v;
     }
   }
+  right_vectors(R, rev);
+  double Fh[5];
+#pragma unroll
+  for (int m = 0; m < 5; m++)
+    Fh[m] = rev[5 * m] * Fhc[0] + rev[5 * m + 1] * Fhc[1] + rev[5 * m + 2] * Fhc[2] + rev[5 * m + 3] * Fhc[3] +
+            rev[5 * m + 4] * Fhc[4];
 #pragma unroll
   for (int m = 0; m < 5; m++) u.fhc[m * S + ci] = Fh[m];
 }
@@ -914,7 +876,7 @@ __global__ __launch_bounds__(256) void k_cuw_diff(FlowArgs a, UwArgs u, int firs
   int c3[3];
   const long long o0 = line_base(a, DIR, L, c3);
   const long long o = o0 + (long long)t * dir_stride(a, DIR);
-  const long long c = cuw_at<DIR>(L, t, NR, NL), cp = cuw_at<DIR>(L, t - 1, NR, NL);
+  const long long c = cuw_at(L, t, NL), cp = cuw_at(L, t - 1, NL);
 #pragma unroll
   for (int m = 0; m < 5; m++)
     face_update1(a, m, o, u.fhc[m * u.sws + c], u.fhc[m * u.sws + cp], first, last);
@@ -939,7 +901,7 @@ __global__ __launch_bounds__(kDtThreads) void k_cuw_diff_xt(FlowArgs a, UwArgs u
     const int rr = e / kDtLines, l = e % kDtLines;
     const int t = t0 - 1 + rr;  // -1 .. n: the rows fh(-1:n) holds
     if (t <= n && L0 + l < NL) {
-      const long long c = cuw_at<0>(L0 + l, t, NR, NL);
+      const long long c = cuw_at(L0 + l, t, NL);
 #pragma unroll
       for (int m = 0; m < 5; m++) sb[m][rr * kDtPad + l] = u.fhc[m * u.sws + c];
     }
@@ -990,7 +952,11 @@ __device__ __forceinline__ void load_cuw_coef(CuwCoef<R>& C, const double* __res
   }
 }
 
-// flux_compact of one line in LDS: T holds f(-8 .. P*R+2) at offset
+// flux_compact (flux.F90:125-150, compact_flux_rhs :163-254, the Thomas
+// sweeps of tridiagonal_thomas_solver, commfunc.F90:790-813) of one line and
+// one split component (F+ with the upwind scheme, F- with the downwind one):
+// rows -2..n+1, the end rows the explicit 6th-order interface value, rows
+// -1..n the 5th-order compact one.  The line is in LDS: T holds f(-8 .. P*R+2) at offset
 // kLineOff (f(-4..n+4) the split values, zeros elsewhere), X receives
 // fh(-1..n) at X[0..n+1]
 template <int P, int R, bool PLUS>
@@ -1061,6 +1027,15 @@ __device__ __forceinline__ void solve_line_cuw(const double* __restrict__ T, dou
   }
 }
 
+// compact_flux_rhs's weights of f(j-1..j+2) with the bandwidth factor b
+__device__ __forceinline__ void cuw_weights(double b, double (&wt)[4]) {
+  const double k118 = 1.0 / 18.0, k136 = 1.0 / 36.0, k1918 = 19.0 / 18.0, k59 = 5.0 / 9.0, k936 = 9.0 / 36.0;
+  wt[0] = k118 - k136 * b;
+  wt[1] = k1918 - k936 * b;
+  wt[2] = k59 + k936 * b;
+  wt[3] = k136 * b;
+}
+
 template <class C>
 constexpr size_t cuw_line_lds() {
   return 4 * (size_t)C::TL * C::LT * sizeof(double);
@@ -1083,9 +1058,8 @@ __global__ __launch_bounds__(C::NT) void k_cuw_line(FlowArgs a, UwArgs u, int fi
   CuwCoef<R> Cp, Cm;
   load_cuw_coef<R>(Cp, u.cuw_ac + cuw_ac_offset(a.n, DIR, true), n + 4, p * R);
   load_cuw_coef<R>(Cm, u.cuw_ac + cuw_ac_offset(a.n, DIR, false), n + 4, p * R);
-  const double b = u.bfac;
-  const double k118 = 1.0 / 18.0, k136 = 1.0 / 36.0, k1918 = 19.0 / 18.0, k59 = 5.0 / 9.0, k936 = 9.0 / 36.0;
-  const double wt[4] = {k118 - k136 * b, k1918 - k936 * b, k59 + k936 * b, k136 * b};
+  double wt[4];
+  cuw_weights(u.bfac, wt);
   // the rows the split does not fill read as zeros (only the padding of the
   // chunks past the system's last row and the windows' outer edge touch them)
   for (int e = threadIdx.x; e < 2 * TL * LT; e += NT) smem[e] = 0.0;
@@ -1149,20 +1123,67 @@ __global__ __launch_bounds__(C::NT) void k_cuw_line(FlowArgs a, UwArgs u, int fi
   }
 }
 
+// The compact interface fluxes fh(-1..n) of one split component (the grid's
+// y) of TL lines, for the characteristic projection, which needs all ten of
+// an interface at once: read and stored once with the lines side by side, the
+// recurrences by the line engine's chunks in LDS.  One lane per line and
+// component, sweeping through memory, took 65 us at 73^3 with fewer than one
+// wavefront per SIMD; 24 us now (its bytes 15).
+template <class C>
+constexpr size_t cuw_solve_lds() {
+  return 2 * (size_t)C::TL * C::LT * sizeof(double);
+}
+template <class C, int DIR>
+__global__ __launch_bounds__(C::NT) void k_cuw_solve(FlowArgs a, UwArgs u) {
+  extern __shared__ double smem[];
+  constexpr int TL = C::TL, P = C::P, R = C::R, LT = C::LT, NT = C::NT;
+  const int n = a.n[DIR];
+  const long long NL = uw_lines(a.n, DIR);
+  const long long L0 = (long long)blockIdx.x * TL;
+  const int f = blockIdx.y;
+  const bool plus = f < 5;
+  double* T = smem;
+  double* X = smem + TL * LT;
+  const int ln = threadIdx.x / P, p = threadIdx.x % P;
+  CuwCoef<R> K;
+  load_cuw_coef<R>(K, u.cuw_ac + cuw_ac_offset(a.n, DIR, plus), n + 4, p * R);
+  double wt[4];
+  cuw_weights(u.bfac, wt);
+  // the rows the split does not fill read as zeros, as in k_cuw_line
+  for (int e = threadIdx.x; e < TL * LT; e += NT) T[e] = 0.0;
+  __syncthreads();
+  const double* src = u.sw + f * u.sws + L0;
+  const bool full = L0 + TL <= NL;
+  for (int e = threadIdx.x; e < TL * (n + 9); e += NT) {
+    const int l = e % TL, rr = e / TL;
+    if (full || L0 + l < NL) T[l * LT + kLineOff + rr - 4] = src[(long long)rr * NL + l];
+  }
+  __syncthreads();
+  if (plus) solve_line_cuw<P, R, true>(T + ln * LT, X + ln * LT, n, p, K, wt);
+  else solve_line_cuw<P, R, false>(T + ln * LT, X + ln * LT, n, p, K, wt);
+  __syncthreads();
+  double* dst = u.fhc + f * u.sws + L0;
+  for (int e = threadIdx.x; e < TL * (n + 2); e += NT) {
+    const int l = e % TL, i = e / TL;  // row i - 1
+    if (full || L0 + l < NL) dst[(long long)(i + 3) * NL + l] = X[l * LT + i];
+  }
+}
+
 // launch shapes of k_cuw_line: the first whose chunks hold the n+4 rows
 using CuwCfg16 = LineCfg<256, 16, 5, 5>;  // P = 16: n <= 76
 using CuwCfg32 = LineCfg<256, 8, 5, 5>;   // P = 32: n <= 156
 using CuwCfg64 = LineCfg<512, 8, 5, 5>;   // P = 64: n <= 316
 using CuwCfg64b = LineCfg<512, 8, 9, 9>;  // P = 64, 9 rows per chunk: n <= 572
 
-// The compact scheme along dir runs the three-kernel sweeps (one lane per
-// line and component, the split buffer holding the lines fastest) rather
-// than the LDS-resident pass: with the characteristic projection, or for
-// lines longer than the LDS pass holds (the flow passes stop at 569 points,
-// below its 572).  The x split and the face launch both follow it.
-bool cuw_sweeps(const FlowArgs& a, const UwArgs& u, int dir) {
-  return u.compact && (u.chardec || a.n[dir] + 4 > CuwCfg64b::P * CuwCfg64b::R);
-}
+// and of k_cuw_solve: half the LDS per line, so 16 lines (128 bytes of every
+// row) also at P = 32
+using CuwSolve32 = LineCfg<512, 16, 5, 5>;
+
+// With the characteristic projection the compact scheme runs three kernels
+// along dir (solves, faces, difference) with the lines fastest in the split
+// buffer, without it one pass with the lines in LDS.  The x split and the face
+// launch both follow it.
+bool cuw_sweeps(const UwArgs& u) { return u.compact && u.chardec; }
 
 template <class C, int DIR>
 hipError_t cuw_line_launch(const FlowArgs& a, const UwArgs& u, bool first, bool last, hipStream_t st) {
@@ -1171,27 +1192,38 @@ hipError_t cuw_line_launch(const FlowArgs& a, const UwArgs& u, bool first, bool 
   hipLaunchKernelGGL((k_cuw_line<C, DIR>), g, dim3(C::NT), cuw_line_lds<C>(), st, a, u, (int)first, (int)last);
   return hipGetLastError();
 }
+template <class C, int DIR>
+hipError_t cuw_solve_launch(const FlowArgs& a, const UwArgs& u, hipStream_t st) {
+  const long long NL = uw_lines(a.n, DIR);
+  const dim3 g((unsigned)((NL + C::TL - 1) / C::TL), 10);
+  hipLaunchKernelGGL((k_cuw_solve<C, DIR>), g, dim3(C::NT), cuw_solve_lds<C>(), st, a, u);
+  return hipGetLastError();
+}
 
 template <int DIR>
 hipError_t cuw_launch_dir(const FlowArgs& a, const UwArgs& u, bool first, bool last, hipStream_t st) {
-  if (!cuw_sweeps(a, u, DIR)) {
-    const int n = a.n[DIR];
-    if (n + 4 <= CuwCfg16::P * CuwCfg16::R) return cuw_line_launch<CuwCfg16, DIR>(a, u, first, last, st);
-    if (n + 4 <= CuwCfg32::P * CuwCfg32::R) return cuw_line_launch<CuwCfg32, DIR>(a, u, first, last, st);
-    if (n + 4 <= CuwCfg64::P * CuwCfg64::R) return cuw_line_launch<CuwCfg64, DIR>(a, u, first, last, st);
-    if (n + 4 <= CuwCfg64b::P * CuwCfg64b::R) return cuw_line_launch<CuwCfg64b, DIR>(a, u, first, last, st);
+  const int n = a.n[DIR];
+  const auto holds = [n](int rows) { return n + 4 <= rows; };
+  if (!cuw_sweeps(u)) {
+    if (holds(CuwCfg16::P * CuwCfg16::R)) return cuw_line_launch<CuwCfg16, DIR>(a, u, first, last, st);
+    if (holds(CuwCfg32::P * CuwCfg32::R)) return cuw_line_launch<CuwCfg32, DIR>(a, u, first, last, st);
+    if (holds(CuwCfg64::P * CuwCfg64::R)) return cuw_line_launch<CuwCfg64, DIR>(a, u, first, last, st);
+    if (holds(CuwCfg64b::P * CuwCfg64b::R)) return cuw_line_launch<CuwCfg64b, DIR>(a, u, first, last, st);
+    return hipErrorInvalidValue;  // the flow passes stop at 569 points, below CuwCfg64b's 572
   }
   const long long NL = uw_lines(a.n, DIR);
-  hipLaunchKernelGGL(k_cuw_solve<DIR>, dim3((unsigned)((10 * NL + 255) / 256)), dim3(256), 0, st, a, u);
-  hipError_t e = hipGetLastError();
+  hipError_t e = hipErrorInvalidValue;
+  if (holds(CuwCfg16::P * CuwCfg16::R)) e = cuw_solve_launch<CuwCfg16, DIR>(a, u, st);
+  else if (holds(CuwSolve32::P * CuwSolve32::R)) e = cuw_solve_launch<CuwSolve32, DIR>(a, u, st);
+  else if (holds(CuwCfg64::P * CuwCfg64::R)) e = cuw_solve_launch<CuwCfg64, DIR>(a, u, st);
+  else if (holds(CuwCfg64b::P * CuwCfg64b::R)) e = cuw_solve_launch<CuwCfg64b, DIR>(a, u, st);
   if (e != hipSuccess) return e;
-  const dim3 gf((unsigned)(((a.n[DIR] + 2) * NL + 255) / 256));
-  if (u.chardec) hipLaunchKernelGGL((k_cuw_face<DIR, true>), gf, dim3(256), 0, st, a, u);
-  else hipLaunchKernelGGL((k_cuw_face<DIR, false>), gf, dim3(256), 0, st, a, u);
+  const dim3 gf((unsigned)(((n + 2) * NL + 255) / 256));
+  hipLaunchKernelGGL(k_cuw_face<DIR>, gf, dim3(256), 0, st, a, u);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (DIR == 0) {
-    const long long nb = (long long)((a.n[0] + 1 + kDtRows - 1) / kDtRows) * ((NL + kDtLines - 1) / kDtLines);
+    const long long nb = (long long)((n + 1 + kDtRows - 1) / kDtRows) * ((NL + kDtLines - 1) / kDtLines);
     if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_cuw_diff_xt, dim3((unsigned)nb), dim3(kDtThreads), 0, st, a, u, (int)first, (int)last);
     return hipGetLastError();
@@ -1213,7 +1245,7 @@ hipError_t uw_launch_sensor(const FlowArgs& a, const UwArgs& u, hipStream_t st) 
 }
 
 hipError_t uw_launch_split(const FlowArgs& a, const UwArgs& u, int dir, hipStream_t st) {
-  if (dir == 0 && cuw_sweeps(a, u, 0)) {
+  if (dir == 0 && cuw_sweeps(u)) {
     const long long nb = (long long)((a.n[0] + 9 + kXtRows - 1) / kXtRows) *
                          ((uw_lines(a.n, 0) + kXtLines - 1) / kXtLines);
     if (nb > 0x7fffffffLL) return hipErrorInvalidValue;
@@ -1238,13 +1270,13 @@ hipError_t launch_face_s(const FlowArgs& a, const UwArgs& u, int dir, bool first
     else
       hipLaunchKernelGGL((k_uw_face_x<SCH, false>), g, dim3(256), 0, st, a, u, (int)first, (int)last);
   } else {
-    const long long nt = NL * ((a.n[dir] + 1 + kRun - 1) / kRun);
-    const dim3 g((unsigned)((nt + 255) / 256));
-    const int f = first, l = last;
-    if (u.chardec && dir == 1) hipLaunchKernelGGL((k_uw_face_yz_cd<SCH, 1>), g, dim3(256), 0, st, a, u, f, l);
-    else if (u.chardec) hipLaunchKernelGGL((k_uw_face_yz_cd<SCH, 2>), g, dim3(256), 0, st, a, u, f, l);
-    else if (dir == 1) hipLaunchKernelGGL((k_uw_face_yz<SCH, 1>), g, dim3(256), 0, st, a, u, f, l);
-    else hipLaunchKernelGGL((k_uw_face_yz<SCH, 2>), g, dim3(256), 0, st, a, u, f, l);
+    const int f = first, l = last, np = a.n[dir] + 1;
+    const int len = run_length(u.chardec ? NL : 5 * NL, np);
+    const long long nt = NL * ((np + len - 1) / len);
+    const dim3 g((unsigned)((nt + 255) / 256), u.chardec ? 1 : 5);
+    auto kern = u.chardec ? (dir == 1 ? k_uw_face_yz_cd<SCH, 1> : k_uw_face_yz_cd<SCH, 2>)
+                          : (dir == 1 ? k_uw_face_yz<SCH, 1> : k_uw_face_yz<SCH, 2>);
+    hipLaunchKernelGGL(kern, g, dim3(256), 0, st, a, u, len, f, l);
   }
   return hipGetLastError();
 }

@@ -1391,7 +1391,13 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   std::memset(&a, 0, sizeof(a));
   a.n[0] = cfg->im; a.n[1] = cfg->jm; a.n[2] = cfg->km;
   a.ndir = cfg->km > 0 ? 3 : 2;
-  a.pitch = ((cfg->im + 1) + 15) / 16 * 16;
+  // rows start on a cache line of 128 bytes, or, from 400 000 points on, on half
+  // of one: there the passes are bound by bytes and shorter rows are fewer
+  // (129^3 3.7% and 257^3 1% of a step, 97x81x64 1%), below it by latency and
+  // by requests (33^3 1.4% slower with half lines, 98x62x46 0.7%)
+  const long long points = (long long)(cfg->im + 1) * (cfg->jm + 1) * (cfg->km + 1);
+  const int unit = points < 400000 ? 16 : 8;
+  a.pitch = (cfg->im + unit) / unit * unit;
   a.plane = (long long)a.pitch * (cfg->jm + 1);
   a.trash = (int)(a.plane * (cfg->km + 1));
   a.fs = (a.plane * (cfg->km + 1) + 1 + 63) / 64 * 64;

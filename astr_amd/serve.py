@@ -69,7 +69,8 @@ class Result:
 
 def case_bytes(cfg: A.Config) -> int:
     """Device memory of one context: 37 padded FP64 fields plus tables."""
-    pitch = (cfg.im + 1 + 15) // 16 * 16
+    unit = 16 if (cfg.im + 1) * (cfg.jm + 1) * (cfg.km + 1) < 400000 else 8
+    pitch = (cfg.im + unit) // unit * unit
     plane = pitch * (cfg.jm + 1)
     fs = (plane * (cfg.km + 1) + 1 + 63) // 64 * 64
     return 37 * fs * 8 + 64 * 1024

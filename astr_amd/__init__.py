@@ -417,7 +417,7 @@ def vortex_config(im, jm=None, mach=0.5, reynolds=1.0e5, length=10.0, cfl=0.67, 
 
 
 class Batch:
-    """Many independent cases advanced together (persistent batched passes,
+    """Many independent cases advanced together (batched passes,
     optionally one hipGraph per RK3 step).  The Flow objects stay owned by the
     caller and must outlive the batch."""
 

@@ -2301,7 +2301,7 @@ int astr_hip_set_convection(astr_hip_ctx* c, int upwind, int recon_schem, int lc
 // ---------------------------------------------------------------------------
 // batching: many independent cases advanced together.  Every pass of a stage
 // is launched once per group of cases sharing (program, launch shape,
-// register budget) as a persistent kernel over the groups' concatenated
+// register budget) as one launch over the groups' concatenated
 // tiles; a whole RK3 step can be captured in a hipGraph and replayed.
 // ---------------------------------------------------------------------------
 namespace {
@@ -2374,7 +2374,6 @@ struct BatchGroup {
 struct astr_hip_batch {
   std::vector<astr_hip_ctx*> cases;
   int device = 0;
-  int ncu = 256;
   hipStream_t stream = nullptr;
   std::vector<BatchGroup> groups;  // in slot order
   StatsJob* d_jobs = nullptr;
@@ -2444,12 +2443,7 @@ int build_groups(astr_hip_batch* b) {
     g.bl.tstart = g.d_tstart;
     g.bl.ncases = nm;
     g.bl.total = ts[nm];
-    // persistent grid: a multiple of 8 blocks, at most as many blocks as the
-    // budget keeps resident (minb per CU), never more than the tiles
-    // (a 128-thread workgroup is half a 256-thread one: twice as many fit)
-    const int cap = b->ncu * g.minb * (kShapes[g.shape].NT < 256 ? 256 / kShapes[g.shape].NT : 1);
-    const int items = batch_items(g.prog, g.dir, g.bl.total);
-    int nb = items < cap ? items : cap;
+    const int nb = batch_items(g.prog, g.dir, g.bl.total);
     g.nblocks = (nb + 7) / 8 * 8;
   }
   return 0;
@@ -2563,8 +2557,6 @@ int astr_hip_batch_create(astr_hip_ctx* const* cases, int ncases, astr_hip_batch
   b->device = cases[0]->device;
   int rc = 0;
   if (hipSetDevice(b->device) != hipSuccess) rc = fail("hipSetDevice failed");
-  if (!rc && hipDeviceGetAttribute(&b->ncu, hipDeviceAttributeMultiprocessorCount, b->device) != hipSuccess)
-    rc = fail("device attribute query failed");
   if (!rc && hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
     rc = fail("hipStreamCreate failed");
   if (!rc && hipMalloc(&b->d_step, sizeof(int)) != hipSuccess) rc = fail("hipMalloc failed");
@@ -2715,9 +2707,7 @@ int astr_hip_batch_autotune(astr_hip_batch* b, int reps) {
         }
         BatchLaunch bl{dargs, dts, nm, ts[nm]};
         for (int mb = 1; mb <= kMinbVariants && !rc; mb++) {
-          const int cap = b->ncu * mb * (kShapes[sh].NT < 256 ? 256 / kShapes[sh].NT : 1);
-          const int items = batch_items(prog, d, bl.total);
-          const int nb = ((items < cap ? items : cap) + 7) / 8 * 8;
+          const int nb = (batch_items(prog, d, bl.total) + 7) / 8 * 8;
           hipError_t e = launch_batch(sh, prog, mb, bl, d, sa, nb, b->stream);
           if (e == hipSuccess) e = hipEventRecord(e0, b->stream);
           for (int r = 0; r < reps && e == hipSuccess; r++) e = launch_batch(sh, prog, mb, bl, d, sa, nb, b->stream);

@@ -274,7 +274,7 @@ int astr_hip_set_pass_config(astr_hip_ctx *ctx, int prog, int dir, int shape, in
 /* ------------------------------------------------------------------------
  * Batching (no reference counterpart: the reference runs one case per job).
  * A batch advances many independent contexts together:
- *   - each pass of a stage is one persistent launch per group of cases that
+ *   - each pass of a stage is one launch per group of cases that
  *     share program, launch shape and register budget;
  *   - with use_graph != 0, a whole RK3 step is captured once as a hipGraph
  *     and replayed.

@@ -213,20 +213,18 @@ __device__ __forceinline__ double rate_exp_in(double x, const ExpK& K) {  // |x|
   p = fma(p, r, 0.5);
   return ldexp(1.0 + fma(r * r, p, r), __double2loint(t));
 }
-__device__ __forceinline__ double rate_exp(double x, const ExpK& K) {
-  double e = rate_exp_in(x, K);
-  const bool in = fabs(x) < 700.0;
-  if (__any(!in)) e = in ? e : exp(x);
-  return e;
-}
-// both at once, with one branch after the two chains of multiply-adds
-__device__ __forceinline__ void rate_exp2(double x, double y, const ExpK& K, double& ex, double& ey) {
-  ex = rate_exp_in(x, K);
-  ey = rate_exp_in(y, K);
-  const bool in = fabs(x) < 700.0 && fabs(y) < 700.0;
+// several at once, with one branch after their chains of multiply-adds
+template <int N>
+__device__ __forceinline__ void rate_exps(const double (&x)[N], const ExpK& K, double (&e)[N]) {
+  bool in = true;
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    e[j] = rate_exp_in(x[j], K);
+    in = in && fabs(x[j]) < 700.0;
+  }
   if (__any(!in)) {
-    ex = fabs(x) < 700.0 ? ex : exp(x);
-    ey = fabs(y) < 700.0 ? ey : exp(y);
+#pragma unroll
+    for (int j = 0; j < N; j++) e[j] = fabs(x[j]) < 700.0 ? e[j] : exp(x[j]);
   }
 }
 
@@ -286,7 +284,7 @@ __device__ __forceinline__ void reaction_sums(const Mech* __restrict__ M, int ns
       for (int j = 0; j < M->nre[r]; j++) fw *= conc_pow(c.get(M->rsp[r][j]), M->rnu[r][j]);
     }
     if (fl & 16) {
-      double dg = 0.0, bw = 1.0, kf, kr;
+      double dg = 0.0, bw = 1.0, k[2];
 #pragma unroll
       for (int k = 0; k < NSA; k++) dg += nu[k] * g[k];
       if (UNIT || (fl & 64)) {
@@ -294,10 +292,12 @@ __device__ __forceinline__ void reaction_sums(const Mech* __restrict__ M, int ns
       } else {
         for (int j = 0; j < M->npr[r]; j++) bw *= conc_pow(c.get(M->psp[r][j]), M->pnu[r][j]);
       }
-      rate_exp2(lkf, lkf + dg, K, kf, kr);  // kr = kf / Kc
-      q = kf * fw - kr * bw;
+      rate_exps({lkf, lkf + dg}, K, k);  // kr = kf / Kc
+      q = k[0] * fw - k[1] * bw;
     } else {
-      q = rate_exp(lkf, K) * fw;
+      double k[1];
+      rate_exps({lkf}, K, k);
+      q = k[0] * fw;
     }
     if (fl & 32) {
       double cm = 0.0;
@@ -1097,8 +1097,8 @@ __global__ __launch_bounds__(64) void k_reactor_eval(const Mech* __restrict__ M,
 // A step attempt (six right-hand sides, a Jacobian, a factorisation, six
 // solves) takes 18 us, against 167 us with the whole right-hand side's species
 // part, the stage sums and the triangular solves repeated by every lane
-// (20 attempts: 40 reactors 4.0 -> 0.94 ms, 4096 3.7 -> 0.41, 16384 14.6 ->
-// 1.6; the one-thread kernel 13 ms at each).
+// (20 attempts: 40 reactors 4.0 -> 0.36 ms, 1024 3.4 -> 0.32, 16384 14.6 ->
+// 1.4; the one-thread kernel 13 ms at each).
 // A team's lanes hold identical scalars (t, h, err), so its control flow is
 // uniform; teams of one wavefront may diverge, which is why the kernel uses
 // no workgroup barrier.  A team is part of one wavefront, whose LDS accesses
@@ -1166,7 +1166,7 @@ struct TeamCoef {
 };
 __constant__ const TeamCoef kTeamCoef;
 
-template <int NS>
+template <int NS, bool UNIT>
 struct Team {
   static constexpr int N = NS + 1;
   static constexpr int RS = N + 2;  // row of the reactions' derivatives: N columns and where pads go
@@ -1191,7 +1191,7 @@ struct Team {
   const int lane, nr;
   const double p, ip;
   double W, iW, tmid, lo[15], hi[15];  // this lane's species (lanes without one: W = 0, iW = 0)
-  Rx rx0, rx1;                         // reactions lane and lane + 16
+  Rx rx[2];                            // reactions lane and lane + 16
   double nu[32];                       // this species' coefficients in reactions 0..31
   const ExpK K;
   // of the last rhs()
@@ -1221,8 +1221,8 @@ struct Team {
     const double* c1 = &M->th[k][1].a0;
 #pragma unroll
     for (int j = 0; j < 15; j++) lo[j] = c0[j], hi[j] = c1[j];
-    rx0 = record(M, lane, nr);
-    rx1 = record(M, lane + kTeam, nr);
+    rx[0] = record(M, lane, nr);
+    rx[1] = record(M, lane + kTeam, nr);
 #pragma unroll
     for (int r = 0; r < 32; r++) nu[r] = has && r < nr ? M->rx[r].nu[k] : 0.0;
     if (lane == 0) S.c[NS] = 1.0, S.g[NS] = 0.0, S.h[NS] = 0.0;
@@ -1234,7 +1234,7 @@ struct Team {
   template <bool DER>
   __device__ __forceinline__ Side side(const Rx& x, int r, bool products) const {
     Side s;
-    if (x.fl & 64) {
+    if (UNIT || (x.fl & 64)) {
       const unsigned sp = products ? x.sp >> 12 : x.sp;
 #pragma unroll
       for (int j = 0; j < 3; j++) s.ix[j] = sp >> (4 * j) & 15;
@@ -1268,39 +1268,52 @@ struct Team {
     return s;
   }
 
-  // reaction r: its rate, into S.q; DER: its row of derivatives, into S.d:
-  // column 0 dq/dT at fixed Y, column 1 + m dq/dY_m divided by rho/W_m
-  template <bool DER>
-  __device__ __forceinline__ void reaction(const Rx& x, int r, double logT) const {
-    if (r >= nr) return;
-    const double lkf = x.lnA + x.b * logT - x.EaR * invT;
-    const Side f = side<DER>(x, r, false), b = side<DER>(x, r, true);
-    const bool rev = x.fl & 16, tb = x.fl & 32;
-    double kf, kr;
-    rate_exp2(lkf, rev ? lkf + (b.g - f.g) : 0.0, K, kf, kr);
-    if (!rev) kr = 0.0;
-    double cm = 0.0;
+  // The rates of NR reactions a lane, the first being r, into S.q, without a
+  // branch (UNIT) so that their chains overlap; past the last reaction a lane
+  // evaluates reaction 0 and stores zero.  DER: their rows of derivatives, into
+  // S.d: column 0 dq/dT at fixed Y, column 1 + m dq/dY_m divided by rho/W_m.
+  template <bool DER, int NR>
+  __device__ __forceinline__ void reactions(const Rx* x, int r, double logT) const {
+    Side f[NR], b[NR];
+    double ex[2 * NR], k[2 * NR], cm[NR];
 #pragma unroll
-    for (int k = 0; k < NS; k++) cm += x.eff[k] * S.c[k];
-    if (!tb) cm = 1.0;
-    const double fw = kf * f.prod, bw = rev ? kr * b.prod : 0.0, net = fw - bw;
-    S.q[r] = cm * net;
-    if constexpr (DER) {
-      const double dlf = x.b * invT + x.EaR * invT * invT;
-      const double dlr = dlf - (b.h - f.h) * invT + (x.ob - x.of) * invT;
-      const double one = tb ? 1.0 : 0.0;
-      const double s = cm * ((x.of + one) * fw - (x.ob + one) * bw);
-      const double base = s / (rho * winv);
-      double* d = S.d[r];
-      d[0] = cm * (fw * dlf - bw * dlr) - s * invT;
+    for (int i = 0; i < NR; i++) {
+      const int ri = r + kTeam * i < nr ? r + kTeam * i : 0;
+      f[i] = side<DER>(x[i], ri, false);
+      b[i] = side<DER>(x[i], ri, true);
+      ex[2 * i] = x[i].lnA + x[i].b * logT - x[i].EaR * invT;
+      ex[2 * i + 1] = x[i].fl & 16 ? ex[2 * i] + (b[i].g - f[i].g) : 0.0;
+      cm[i] = 0.0;
+    }
 #pragma unroll
-      for (int k = 0; k < NS; k++) d[1 + k] = net * x.eff[k] - base;
-      const double cf = cm * kf, cb = rev ? -cm * kr : 0.0;
+    for (int s = 0; s < NS; s++) {
+      const double c = S.c[s];
 #pragma unroll
-      for (int j = 0; j < 3; j++) add(&d[1 + f.ix[j]], cf * f.td[j]);
-      if (rev) {
+      for (int i = 0; i < NR; i++) cm[i] += x[i].eff[s] * c;
+    }
+    rate_exps(ex, K, k);
 #pragma unroll
-        for (int j = 0; j < 3; j++) add(&d[1 + b.ix[j]], cb * b.td[j]);
+    for (int i = 0; i < NR; i++) {
+      const bool rev = x[i].fl & 16, tb = x[i].fl & 32;
+      const double kf = k[2 * i], kr = rev ? k[2 * i + 1] : 0.0;
+      if (!tb) cm[i] = 1.0;
+      const double fw = kf * f[i].prod, bw = rev ? kr * b[i].prod : 0.0, net = fw - bw;
+      S.q[r + kTeam * i] = r + kTeam * i < nr ? cm[i] * net : 0.0;
+      if constexpr (DER) {
+        const double dlf = x[i].b * invT + x[i].EaR * invT * invT;
+        const double dlr = dlf - (b[i].h - f[i].h) * invT + (x[i].ob - x[i].of) * invT;
+        const double one = tb ? 1.0 : 0.0;
+        const double s = cm[i] * ((x[i].of + one) * fw - (x[i].ob + one) * bw);
+        const double base = s / (rho * winv);
+        double* d = S.d[r + kTeam * i];
+        d[0] = cm[i] * (fw * dlf - bw * dlr) - s * invT;
+#pragma unroll
+        for (int m = 0; m < NS; m++) d[1 + m] = net * x[i].eff[m] - base;
+        const double cf = cm[i] * kf, cb = rev ? -cm[i] * kr : 0.0;
+#pragma unroll
+        for (int j = 0; j < 3; j++) add(&d[1 + f[i].ix[j]], cf * f[i].td[j]);
+#pragma unroll
+        for (int j = 0; j < 3; j++) add(&d[1 + b[i].ix[j]], rev ? cb * b[i].td[j] : 0.0);
       }
     }
   }
@@ -1337,11 +1350,11 @@ struct Team {
       if (DER) S.h[lane - 1] = hrt;
     }
     team_sync();
-    reaction<DER>(rx0, lane, logT);
-    if (nr > kTeam) reaction<DER>(rx1, lane + kTeam, logT);
+    if (nr > kTeam) reactions<DER, 2>(rx, lane, logT);
+    else reactions<DER, 1>(rx, lane, logT);
     if (nr > 2 * kTeam) {
       const Rx x = record(M, lane + 2 * kTeam, nr);
-      reaction<DER>(x, lane + 2 * kTeam, logT);
+      reactions<DER, 1>(&x, lane + 2 * kTeam, logT);
     }
     team_sync();
     double w[4] = {0.0, 0.0, 0.0, 0.0};
@@ -1466,10 +1479,10 @@ struct Team {
   }
 };
 
-template <int NS>
+template <int NS, bool UNIT>
 __global__ __launch_bounds__(64) void k_reactor_team(const Mech* __restrict__ M, ReactorPool P,
                                                      int max_tries, double rtol, double atol) {
-  using TeamN = Team<NS>;
+  using TeamN = Team<NS, UNIT>;
   constexpr int N = NS + 1;
   constexpr int TPB = 64 / kTeam;
   static_assert(N <= kTeam && NRMAX <= 3 * kTeam, "a lane per component, three reactions per lane");
@@ -2145,8 +2158,9 @@ int astr_hip_reactor_advance(astr_reactor_pool* r, int max_tries) {
   const int bs = 64;
   const dim3 grid((r->P.cap + bs - 1) / bs);
   if (r->lanes == kTeam)
-    hipLaunchKernelGGL(k_reactor_team<9>, dim3((r->P.cap + bs / kTeam - 1) / (bs / kTeam)), dim3(bs), 0,
-                       r->stream, r->chem->dev, r->P, max_tries, r->rtol, r->atol);
+    hipLaunchKernelGGL((r->chem->host.unit ? k_reactor_team<9, true> : k_reactor_team<9, false>),
+                       dim3((r->P.cap + bs / kTeam - 1) / (bs / kTeam)), dim3(bs), 0, r->stream, r->chem->dev, r->P,
+                       max_tries, r->rtol, r->atol);
   else if (r->chem->host.ns == 9)
     hipLaunchKernelGGL(k_reactor_n<9>, grid, dim3(bs), 0, r->stream, r->chem->dev, r->P, max_tries,
                        r->rtol, r->atol);

@@ -230,7 +230,7 @@ class ReactorPool:
 
     @property
     def lanes(self):
-        """Lanes per reactor: 1 (throughput) or 16 (a team, for latency)."""
+        """Lanes per reactor: 1, or 16 (a team; the default for 9 species)."""
         v = C.c_int()
         _chk(_bind().astr_hip_reactor_get_lanes(self.h, C.byref(v)))
         return v.value

@@ -77,7 +77,7 @@ bool test_fail_alloc() {
       return fail(std::string(#x) + ": " + hipGetErrorString(e_));                 \
   } while (0)
 
-// Per-tile partial sums left by the last gradient pass: rho|u|^2, rho|w|^2.
+// Per-tile partial sums left by the x flux pass: rho|u|^2, rho|w|^2.
 constexpr int kTileStats = 2;
 // Statistics per step of a single case: KE, enstrophy, dissipation rate.
 constexpr int kStepStats = 3;
@@ -1143,7 +1143,7 @@ double* scratch_address(int device, std::string* err) {
 }
 
 // Device buffers of the per-step statistics: the per-tile partial sums the
-// last gradient pass leaves (2 per tile), the dissipation rate's block
+// x flux pass leaves (2 per tile), the dissipation rate's block
 // partials (kDissBlocks) and the per-step results (kStepStats per step).
 struct StatsBufs {
   double* part;

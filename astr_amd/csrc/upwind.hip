@@ -857,7 +857,6 @@ __global__ __launch_bounds__(256, 3) void k_cuw_face(FlowArgs a, UwArgs u) {
 template <int DIR>
 __global__ __launch_bounds__(256) void k_cuw_diff(FlowArgs a, UwArgs u, int first, int last) {
   const int n = a.n[DIR];
-  const int NR = n + 9;
   const long long NL = uw_lines(a.n, DIR);
   const long long NP = n + 1;
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
@@ -892,7 +891,6 @@ constexpr int kDtRows = 16, kDtLines = 64, kDtPad = kDtLines + 2, kDtThreads = k
 __global__ __launch_bounds__(kDtThreads) void k_cuw_diff_xt(FlowArgs a, UwArgs u, int first, int last) {
   __shared__ double sb[5][(kDtRows + 1) * kDtPad];
   const int n = a.n[0];
-  const int NR = n + 9;
   const long long NL = uw_lines(a.n, 0);
   const int ntt = (n + 1 + kDtRows - 1) / kDtRows;
   const int t0 = (int)(blockIdx.x % ntt) * kDtRows;

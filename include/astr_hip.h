@@ -384,10 +384,9 @@ int astr_hip_chem_temperature_device(astr_chem *chem, long long n, const double 
  * c32, c41..c43, c51..c54, c61..c65 (26 values; n must be at least 26).
  *
  * Lanes per reactor (set_lanes / get_lanes): 1, one thread per reactor and 64
- * reactors per wavefront, for throughput over many thousands of reactors; or
- * 16, a team per reactor that evaluates the Jacobian's columns on separate
- * lanes and eliminates one matrix row per lane, for latency when reactors are
- * few (the default for 9-species mechanisms; other sizes use 1).
+ * reactors per wavefront; or 16, a team per reactor with one component of the
+ * state and one matrix row per lane (the default for 9-species mechanisms, and
+ * the faster one from 1 to at least 16384 reactors; other sizes use 1).
  *
  * A pool holds `capacity` slots:
  *   - set starts a reactor in a slot;

@@ -791,9 +791,10 @@ __device__ __forceinline__ double mp5(const double* u, double ul, bool shock) {
 // Fh(i) replaces the compact value of F+ component m at row i (this lane's own
 // row, read before).  Both sides unrolled with both sets of eigenvectors took
 // 310 registers, one wavefront per SIMD and 102 us at 73^3; one side at a time
-// takes 168, three wavefronts and 51 us (its bytes 20).
+// takes 179, two wavefronts and 44 us (its bytes 20).  Held to three
+// wavefronts it spills 11 registers (51 us), to four many more (78 us).
 template <int DIR>
-__global__ __launch_bounds__(256, 3) void k_cuw_face(FlowArgs a, UwArgs u) {
+__global__ __launch_bounds__(256, 2) void k_cuw_face(FlowArgs a, UwArgs u) {
   const int n = a.n[DIR];
   const long long NL = uw_lines(a.n, DIR);
   const long long NI = n + 2;

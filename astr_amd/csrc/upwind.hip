@@ -792,7 +792,8 @@ __device__ __forceinline__ double mp5(const double* u, double ul, bool shock) {
 // row, read before).  Both sides unrolled with both sets of eigenvectors took
 // 310 registers, one wavefront per SIMD and 102 us at 73^3; one side at a time
 // takes 179, two wavefronts and 44 us (its bytes 20).  Held to three
-// wavefronts it spills 11 registers (51 us), to four many more (78 us).
+// wavefronts it spills 11 registers (51 us), to four far more (a step of the
+// scheme 1985 us, 1560 with two).
 template <int DIR>
 __global__ __launch_bounds__(256, 2) void k_cuw_face(FlowArgs a, UwArgs u) {
   const int n = a.n[DIR];

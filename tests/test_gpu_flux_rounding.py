@@ -1,0 +1,108 @@
+"""The viscous flux must not cost the right-hand side of the convective flux's
+accuracy.  Each flux derivative is taken of the difference of the two; formed
+from a rounded convective flux, the difference rounds a second time at that
+flux's size (the viscous flux is 1e-3 of it), and the right-hand side's error
+grows by a fifth to a quarter, as a double against an extended-precision
+restatement of the line operators shows.  Formed by one fused operation it
+rounds once, as the convective flux alone does.
+
+Measure: the RMS distance from the same right-hand side in extended precision,
+with the viscous flux (Re 1600) over that without (Re 1e30), at Mach 1, where
+pressure, kinetic energy and momentum fluxes are all of order one.  The viscous
+part's own error is 1e-3 of the convective one's.  The RMS over 16 000 points
+or more of errors that are correlated over a few points is good to about 1%;
+the bound, 1.05, leaves five of those."""
+import numpy as np
+import pytest
+
+import astr_amd as A
+from fields import periodic_field
+
+LD = np.longdouble
+
+
+def derivative(f, axis):
+    """df_compact of lines with periodic halo (derivative.F90:63-306), not
+    divided by the spacing: explicit 6th-order rows at -1 and n+1, compact ones
+    between."""
+    f = np.moveaxis(f, axis, 0)
+    n = f.shape[0] - 1
+    ext = np.concatenate([f[n - 5:n], f, f[1:6]])  # rows -5 .. n+5
+    row = lambda s: ext[4 + s:n + 7 + s]  # rows -1 .. n+1, shifted by s  # noqa: E731
+    b = LD(7) / 9 * (row(1) - row(-1)) + LD(1) / 36 * (row(2) - row(-2))
+    for r in (0, n + 2):
+        e = lambda s: ext[r + 4 + s]  # noqa: E731
+        b[r] = LD(3) / 4 * (e(1) - e(-1)) - LD(3) / 20 * (e(2) - e(-2)) + LD(1) / 60 * (e(3) - e(-3))
+    # x(r-1)/3 + x(r) + x(r+1)/3 = b(r) between the end rows, x = b at them
+    a, c = LD(1) / 3, np.zeros(n + 3, LD)
+    for r in range(1, n + 2):
+        m = 1 - a * c[r - 1]
+        c[r] = a / m
+        b[r] = (b[r] - a * b[r - 1]) / m
+    for r in range(n + 1, 0, -1):
+        b[r] -= c[r] * b[r + 1]
+    return np.moveaxis(b[1:n + 2], 0, axis)
+
+
+def rhs_extended(cfg, q, viscous):
+    """rhscal (tgvsolver.F90:450-787) of q in extended precision."""
+    nd = 3 if cfg.km > 0 else 2
+    inv = [LD(cfg.im) / LD(cfg.lx), LD(cfg.jm) / LD(cfg.ly), LD(max(cfg.km, 1)) / LD(cfg.lz)]
+    q = q.astype(LD)
+    g1 = LD(cfg.gamma) - 1
+    u = [q[1 + m] / q[0] for m in range(3)]
+    p = g1 * (q[4] - (q[1] * u[0] + q[2] * u[1] + q[3] * u[2]) / 2)
+    T = p / q[0] * LD(cfg.gamma) * LD(cfg.mach) ** 2
+    D = lambda f, d: derivative(f, 2 - d) * inv[d]  # noqa: E731
+    zero = np.zeros_like(p)
+    out = [zero.copy() for _ in range(5)]
+    if viscous:
+        g = [[D(u[m], d) if d < nd else zero for d in range(3)] for m in range(3)]
+        gt = [D(T, d) if d < nd else zero for d in range(3)]
+        s = LD(cfg.sutherland) / LD(cfg.ref_tem)
+        mu = T * np.sqrt(T) * (1 + s) / (T + s) / LD(cfg.reynolds)
+        k = mu / LD(cfg.prandtl) / (g1 * LD(cfg.mach) ** 2)
+        div = (g[0][0] + g[1][1] + g[2][2]) / 3
+        sg = [[mu * (g[a][b] + g[b][a]) - (2 * mu * div if a == b else 0) for b in range(3)] for a in range(3)]
+    for d in range(nd):
+        for m in range(5):
+            f = -(q[4] + p) * u[d] if m == 4 else -q[m] * u[d] - (p if m == d + 1 else 0)
+            if viscous and 0 < m < 4:
+                f = f + sg[d][m - 1]
+            if viscous and m == 4:
+                f = f + k * gt[d] + sg[d][0] * u[0] + sg[d][1] * u[1] + sg[d][2] * u[2]
+            out[m] += D(f, d)
+    return np.array(out)
+
+
+def test_extended_derivative_is_sixth_order():
+    err = []
+    for n in (32, 64):
+        x = LD(2) * LD(np.pi) * np.arange(n + 1) / n
+        f = np.sin(x)[None, :, None] * np.ones((2, 1, 3), LD)
+        err.append(float(np.abs(derivative(f, 1) * (n / (2 * LD(np.pi))) - np.cos(x)[None, :, None]).max()))
+    assert err[1] < 3e-9 and err[0] / err[1] > 40
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("main", [False, True])
+@pytest.mark.parametrize("dims", [(28, 27, 24), (41, 26, 33), (150, 131, 0)])
+def test_viscous_flux_adds_no_rounding_at_the_convective_size(main, dims):
+    make = A.main_config if main else A.tgv_config
+    err = {}
+    for re in (1600.0, 1e30):
+        f = A.Flow(make(*dims, mach=1.0, reynolds=re))
+        q = periodic_field(f.cfg, 8)
+        f.upload(q)
+        got = f.rhscal()
+        want = rhs_extended(f.cfg, q, re < 1e20)
+        if main:  # the main path's right-hand side carries the Jacobian
+            got = got / (f.cfg.lx / dims[0] * (f.cfg.ly / dims[1]) * (f.cfg.lz / dims[2] if dims[2] else 1.0))
+        assert float(np.abs(got - want).max() / np.abs(want).max()) < 1e-12
+        err[re] = np.sqrt(((got - want).astype(float) ** 2).mean(axis=(1, 2, 3)))
+        f.close()
+    ratio = err[1600.0] / np.maximum(err[1e30], 1e-300)
+    for m in (1, 2, 3, 4):
+        if m == 3 and dims[2] == 0:
+            continue
+        assert ratio[m] < 1.05, (m, ratio)

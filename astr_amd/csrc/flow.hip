@@ -1410,7 +1410,6 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   a.const2 = g * ma * ma;
   a.const5 = (g - 1.0) * ma * ma;
   a.const6 = 1.0 / (g - 1.0);
-  a.p0 = 1.0 / a.const2;
   a.reynolds = cfg->reynolds;
   a.prandtl = cfg->prandtl;
   a.suth = cfg->sutherland / cfg->ref_tem;

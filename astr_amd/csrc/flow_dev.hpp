@@ -23,7 +23,6 @@ struct FlowArgs {
   long long fs;         // doubles between fields
   double inv_d[3];      // 1/dx, 1/dy, 1/dz
   double const2, const5, const6;
-  double p0;            // the reference state's pressure, 1/const2
   double reynolds, prandtl, suth, suth1;
   double rk_a, rk_b, rk_c, dt;
   int trash;            // a point index inside every field's padding
@@ -163,6 +162,11 @@ __device__ __forceinline__ T* uniform_ptr(T* p) {
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
   const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
   return reinterpret_cast<T*>(((unsigned long long)hi << 32) | lo);
+}
+// a value that is the same on every lane, kept in scalar registers
+__device__ __forceinline__ double uniform(double x) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(x)));
 }
 // The accesses are made through global (address space 1) pointers so the
 // compiler emits global, not flat, instructions.
@@ -335,6 +339,17 @@ __device__ __forceinline__ void make_slots(Slots<C>& S, const FlowArgs& a, int d
   }
 }
 
+// byte offset of row 0 of a tile's first line
+template <class C>
+__device__ __forceinline__ unsigned tile_first(const FlowArgs& a, int dir, int tile) {
+  if (dir == 0) {
+    const int L = tile * C::TL, rows = a.n[1] + 1;
+    return (unsigned)((long long)(L / rows) * a.plane + (long long)(L % rows) * a.pitch) * 8u;
+  }
+  const int ni = (a.n[0] + C::TL) / C::TL;
+  return (unsigned)((long long)(tile / ni) * (dir == 1 ? a.plane : a.pitch) + tile % ni * C::TL) * 8u;
+}
+
 // store slot t's value into its input line with the periodic halo copies
 // q(-h)=q(n-h), q(n+h)=q(h) (tgvsolver.F90:371-440)
 template <class C>
@@ -390,11 +405,13 @@ __device__ __forceinline__ Prim prim_of(const FlowArgs& a, double q1, double q2,
 // alone does; formed from the rounded product it rounds twice there (at 28 x 27
 // x 24, Mach 1, the energy right-hand side's error is 1.12 times that of the
 // convective part alone with two roundings, 1.01 with one).  The momentum along
-// dir keeps the reference's q_m u + p, from which f0 goes off exactly first.
-__device__ __forceinline__ double flux_diff(int m, int dir, double qm, double uu, double p, double f0, double v) {
+// dir keeps the reference's q_m u + p, from which f0 goes off first.
+enum FluxKind { FLUX_PLAIN, FLUX_ALONG, FLUX_ENERGY };
+template <int KIND>
+__device__ __forceinline__ double flux_diff(double qm, double uu, double p, double f0, double v) {
 #pragma clang fp contract(off)
-  if (m == dir + 1) return v - (qm * uu + p - f0);
-  return fma(-(m == 4 ? qm + p : qm), uu, v);
+  if (KIND == FLUX_ALONG) return v - (qm * uu + p - f0);
+  return fma(-(KIND == FLUX_ENERGY ? qm + p : qm), uu, v);
 }
 
 // Sutherland (tgvsolver.F90:123-140)
@@ -462,12 +479,13 @@ __device__ __forceinline__ void visc_flux(const FlowArgs& a, const double g[3][3
 // U = sum_n dxi(dir,n) u_n, for the metrics of a uniform Cartesian grid
 // (dxi(dir,n) = 0 for n != dir, so those products add exact zeros); v minus it
 // as in flux_diff
-__device__ __forceinline__ double flux_diff_main(double jac, double dx, int m, int dir, double qm, double ud,
-                                                 double p, double f0, double v) {
+template <int KIND>
+__device__ __forceinline__ double flux_diff_main(double jac, double dx, double qm, double ud, double p, double f0,
+                                                 double v) {
 #pragma clang fp contract(off)
   const double uu = dx * ud;
-  if (m == dir + 1) return v - (jac * (qm * uu + dx * p) - f0);
-  return fma(-(jac * (m == 4 ? qm + p : qm)), uu, v);
+  if (KIND == FLUX_ALONG) return v - (jac * (qm * uu + dx * p) - f0);
+  return fma(-(jac * (KIND == FLUX_ENERGY ? qm + p : qm)), uu, v);
 }
 
 // Main path: the Jacobian J and dxi(dir,dir) of a point on a uniform grid
@@ -584,8 +602,9 @@ __device__ __forceinline__ void stress_point(const FlowArgs& a, unsigned o, cons
 // workgroups share a tile.  The components' solves are independent, and
 // where a pass has few tiles their serial chain in one workgroup is its time.
 template <class C, int PROG, bool MAIN = false, bool GEN = false, bool ONE = false>
-__device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa, const Arrays& A, int dir, int tile,
+__device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa, const Arrays& A, int dir_, int tile,
                                           double* smem, int field = 0) {
+  const int dir = PROG == FGC_FIRST || PROG == V_FIRST || PROG == V_FIRST_G ? 0 : dir_;
   double* const qc = A.q;
   double* const qo = A.qsave;
   double* const qrhs = A.qrhs;
@@ -926,13 +945,21 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
     };
     // Stage component m's flux difference with its halo copies (part 1: the
     // convective flux alone, 2: the viscous one).  The momentum flux along dir
-    // carries p ~ p0 = 1/(gamma Ma^2), large against everything the
-    // derivative keeps of it; p0 goes off it first, which is exact within a
-    // factor of two of p0 and drops out of the derivative.  Per-point metrics
-    // have no such constant: there the two parts are solved one after the
-    // other.
-    auto stage_flux = [&](int m, int part) __attribute__((always_inline)) {
-      const double f0 = m == dir + 1 ? (MAIN ? a.jac * (a.inv_d[dir] * a.p0) : a.p0) : 0.0;
+    // carries p ~ 1/(gamma Ma^2), large against everything the derivative keeps
+    // of it; f0, the pressure of the tile's first point, drops out of the
+    // derivative and goes off it first, exactly where p is within a factor of
+    // two of it.  (The reference pressure in its place would round a state of
+    // another pressure level at its own size.)  Per-point metrics have no such
+    // constant: there the two parts are solved one after the other.
+    double f0 = 0.0;
+    if (!uwd && !metg && (!ONE || field == dir + 1)) {
+#pragma clang fp contract(off)
+      f0 = ldg(MAIN ? a.pr + 4 * fs : a.p, tile_first<C>(a, dir, tile));
+      if (MAIN) f0 = a.jac * (a.inv_d[dir] * f0);
+      f0 = uniform(__builtin_isfinite(f0) ? f0 : 0.0);
+    }
+    auto stage_kind = [&](auto kind, int m, int part) __attribute__((always_inline)) {
+      constexpr int KIND = decltype(kind)::value;
 #pragma unroll
       for (int t = 0; t < NPT; t++) {
         const unsigned o = S.g[t];
@@ -947,7 +974,7 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
           }
         }
         if constexpr (!MAIN) {
-          put<C>(T, S, t, flux_diff(m, dir, qn[t], ud[t], pp[t], f0, v));
+          put<C>(T, S, t, flux_diff<KIND>(qn[t], ud[t], pp[t], f0, v));
         } else {
           if (uwd || part == 2) {
             put<C>(T, S, t, v);
@@ -966,14 +993,19 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
             }
           } else {
             const Met M = met_of(a, dir);
-            T[kLineOff + S.s[t]] = flux_diff_main(M.j, M.d, m, dir, qn[t], ud[t], pp[t], f0, v);
+            T[kLineOff + S.s[t]] = flux_diff_main<KIND>(M.j, M.d, qn[t], ud[t], pp[t], f0, v);
             if (S.h[t] != kDummy) {
               const double qh = S.ex[t] >= 0 ? halo_q<C>(a, qc, S, t, dir, m) : qn[t];
-              T[kLineOff + S.h[t]] = flux_diff_main(M.j, M.d, m, dir, qh, hu[t], hp[t], f0, v);
+              T[kLineOff + S.h[t]] = flux_diff_main<KIND>(M.j, M.d, qh, hu[t], hp[t], f0, v);
             }
           }
         }
       }
+    };
+    auto stage_flux = [&](int m, int part) __attribute__((always_inline)) {
+      if (m == 4) stage_kind(std::integral_constant<int, FLUX_ENERGY>{}, m, part);
+      else if (m == dir + 1) stage_kind(std::integral_constant<int, FLUX_ALONG>{}, m, part);
+      else stage_kind(std::integral_constant<int, FLUX_PLAIN>{}, m, part);
     };
     // derivative of the staged component; cx: the convective part's, where it
     // is solved on its own

@@ -106,3 +106,50 @@ def test_viscous_flux_adds_no_rounding_at_the_convective_size(main, dims):
         if m == 3 and dims[2] == 0:
             continue
         assert ratio[m] < 1.05, (m, ratio)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("main", [False, True])
+@pytest.mark.parametrize("dims", [(28, 27, 24), (150, 131, 0)])
+def test_pressures_far_from_the_reference_state(main, dims):
+    """The convective right-hand side does not depend on the configuration's
+    Mach number, nor may its error: a state whose pressures are a hundredth of
+    the reference pressure 1/(gamma Ma^2) of Mach 0.1, against the same state
+    under Mach 1, whose reference pressure it has."""
+    make = A.main_config if main else A.tgv_config
+    err = []
+    for mach in (1.0, 0.1):
+        f = A.Flow(make(*dims, mach=mach, reynolds=1e30))
+        q = periodic_field(make(*dims, mach=1.0), 8)
+        f.upload(q)
+        got = f.rhscal()
+        if main:
+            got = got / (f.cfg.lx / dims[0] * (f.cfg.ly / dims[1]) * (f.cfg.lz / dims[2] if dims[2] else 1.0))
+        want = rhs_extended(f.cfg, q, False)
+        err.append(np.sqrt(((got - want).astype(float) ** 2).mean(axis=(1, 2, 3))))
+        f.close()
+    for m in (1, 2, 3):
+        if m == 3 and dims[2] == 0:
+            continue
+        assert err[1][m] < 1.05 * err[0][m], (m, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("main", [False, True])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_a_point_that_is_not_finite_reaches_its_planes_only(main, value):
+    """A point whose energy is not finite spoils the gradients along the three
+    lines through it and the fluxes along the lines that cross those: the three
+    planes through it.  Every other point keeps its bits, also where the point
+    is the first of a tile of lines."""
+    f = A.Flow((A.main_config if main else A.tgv_config)(28, 27, 24))
+    q = periodic_field(f.cfg, 8)
+    f.upload(q)
+    want = f.rhscal()
+    q[4, 8, 0, 0] = value
+    f.upload(q)
+    got = f.rhscal()
+    keep = np.ones(q[0].shape, bool)
+    keep[8], keep[:, 0], keep[:, :, 0] = False, False, False
+    assert np.array_equal(got[:, keep], want[:, keep])
+    assert not np.isfinite(got[4, 8, 0, 0])

@@ -513,14 +513,17 @@ __device__ __forceinline__ double jac_of(const FlowArgs& a, unsigned g) {
 }
 
 // convrsdcal6 (src/solver.F90:2196-2207) with the full metric row:
-// U = dxi(d,1) u + dxi(d,2) v + dxi(d,3) w, F_m = J (q_m U + dxi(d,m) p)
-__device__ __forceinline__ double conv_flux_full(const MetRow& M, int m, double qm, double u,
-                                                 double v, double w, double p) {
+// U = dxi(d,1) u + dxi(d,2) v + dxi(d,3) w, F_m = J (q_m U + dxi(d,m) p); v
+// minus it, rounded once as in flux_diff (jm, rm: J and dxi(d,m))
+__device__ __forceinline__ double contravariant(const MetRow& M, double u, double v, double w) {
 #pragma clang fp contract(off)
-  const double uu = M.r[0] * u + M.r[1] * v + M.r[2] * w;
-  if (m == 0) return M.j * qm * uu;
-  if (m == 4) return M.j * (qm + p) * uu;
-  return M.j * (qm * uu + M.r[m - 1] * p);
+  return M.r[0] * u + M.r[1] * v + M.r[2] * w;
+}
+__device__ __forceinline__ double flux_diff_full(double jm, double rm, int m, double qm, double uu, double p,
+                                                 double v) {
+#pragma clang fp contract(off)
+  if (m == 0 || m == 4) return fma(-(jm * (m == 4 ? qm + p : qm)), uu, v);
+  return fma(-jm, qm * uu + rm * p, v);
 }
 
 // diffrsdcal6 (src/solver.F90:2623-2635) with the full metric row: column
@@ -900,8 +903,9 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
         __syncthreads();
       }
     }
-    // velocity along dir and pressure of the points; hu, hp those of the halo
-    // copies where they differ (main path)
+    const bool metg = GEN && a.met;
+    // velocity along dir (general grids: contravariant) and pressure of the
+    // points; hu, hp those of the halo copies where they differ (main path)
     double ud[NPT], pp[NPT], hu[NPT], hp[NPT];
     if (!uwd) {
 #pragma unroll
@@ -909,8 +913,10 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
         const unsigned o = S.g[t];
         if constexpr (MAIN) {
           // convrsdcal6 takes the stored vel and prs (src/solver.F90:2196-2207)
-          if (!ONE || field == 4 || field == dir + 1) pp[t] = ldg(a.pr + 4 * fs, o);
-          ud[t] = PROG == V_FIRST_G ? pv[0][t] : ldg(a.pr + (1 + dir) * fs, o);
+          if (!ONE || field == 4 || field == dir + 1 || (metg && field > 0)) pp[t] = ldg(a.pr + 4 * fs, o);
+          if (metg)
+            ud[t] = contravariant(met_row(a, dir, o), ldg(a.pr + fs, o), ldg(a.pr + 2 * fs, o), ldg(a.pr + 3 * fs, o));
+          else ud[t] = PROG == V_FIRST_G ? pv[0][t] : ldg(a.pr + (1 + dir) * fs, o);
         } else {
           if (!ONE || field == 4 || field == dir + 1) pp[t] = ldg(a.p, o);
           ud[t] = PROG == V_FIRST_G ? pv[0][t] : ldg(qc + (1 + dir) * fs, o) / ldg(qc, o);
@@ -924,14 +930,15 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
 #pragma unroll
             for (int m = 0; m < 5; m++) qh[m] = halo_q<C>(a, qc, S, t, dir, m);
             hp[t] = pressure_of(a, qh[0], qh[1], qh[2], qh[3], qh[4]);
-            hu[t] = (dir == 0 ? qh[1] : (dir == 1 ? qh[2] : qh[3])) / qh[0];
+            // a periodic halo copy carries the source point's metrics, which are this point's
+            if (metg) hu[t] = contravariant(met_row(a, dir, S.g[t]), qh[1] / qh[0], qh[2] / qh[0], qh[3] / qh[0]);
+            else hu[t] = (dir == 0 ? qh[1] : (dir == 1 ? qh[2] : qh[3])) / qh[0];
           }
         }
       }
     }
     // inputs of the next solve: q_m and the viscous column (general grids
     // form their column when it is staged)
-    const bool metg = GEN && a.met;
     double qn[NPT], vn[NPT];
     auto load_inputs = [&](int m) __attribute__((always_inline)) {
 #pragma unroll
@@ -943,14 +950,15 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
         }
       }
     };
-    // Stage component m's flux difference with its halo copies (part 1: the
-    // convective flux alone, 2: the viscous one).  The momentum flux along dir
+    // Stage component m's flux difference with its halo copies (without the
+    // convective flux where that is upwind-biased).  The momentum flux along dir
     // carries p ~ 1/(gamma Ma^2), large against everything the derivative keeps
     // of it; f0, the pressure of the tile's first point, drops out of the
     // derivative and goes off it first, exactly where p is within a factor of
     // two of it.  (The reference pressure in its place would round a state of
     // another pressure level at its own size.)  Per-point metrics have no such
-    // constant: there the two parts are solved one after the other.
+    // constant; the fused operation alone keeps their difference to one
+    // rounding at the flux's size.
     double f0 = 0.0;
     if (!uwd && !metg && (!ONE || field == dir + 1)) {
 #pragma clang fp contract(off)
@@ -958,13 +966,13 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
       if (MAIN) f0 = a.jac * (a.inv_d[dir] * f0);
       f0 = uniform(__builtin_isfinite(f0) ? f0 : 0.0);
     }
-    auto stage_kind = [&](auto kind, int m, int part) __attribute__((always_inline)) {
+    auto stage_kind = [&](auto kind, int m) __attribute__((always_inline)) {
       constexpr int KIND = decltype(kind)::value;
 #pragma unroll
       for (int t = 0; t < NPT; t++) {
         const unsigned o = S.g[t];
         double v = 0.0;
-        if (m > 0 && part != 1) {
+        if (m > 0) {
           if constexpr (FIRST) v = sx[m - 1][t];
           else v = metg ? visc_col_full(a, dir, m - 1, o) : vn[t];
           if (MAIN && !metg) {
@@ -976,20 +984,16 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
         if constexpr (!MAIN) {
           put<C>(T, S, t, flux_diff<KIND>(qn[t], ud[t], pp[t], f0, v));
         } else {
-          if (uwd || part == 2) {
+          if (uwd) {
             put<C>(T, S, t, v);
             continue;
           }
           if (metg) {
-            // a periodic halo copy carries the source point's metrics, which are this point's
-            const MetRow M = met_row(a, dir, o);
-            T[kLineOff + S.s[t]] = v - conv_flux_full(M, m, qn[t], ldg(a.pr + fs, o), ldg(a.pr + 2 * fs, o),
-                                                      ldg(a.pr + 3 * fs, o), pp[t]);
+            const double jm = ldg(a.met, o), rm = m > 0 && m < 4 ? ldg(a.met + (1 + dir + 3 * (m - 1)) * fs, o) : 0.0;
+            T[kLineOff + S.s[t]] = flux_diff_full(jm, rm, m, qn[t], ud[t], pp[t], v);
             if (S.h[t] != kDummy) {
-              const double r = halo_q<C>(a, qc, S, t, dir, 0);
-              T[kLineOff + S.h[t]] = v - conv_flux_full(M, m, halo_q<C>(a, qc, S, t, dir, m),
-                                                        halo_q<C>(a, qc, S, t, dir, 1) / r, halo_q<C>(a, qc, S, t, dir, 2) / r,
-                                                        halo_q<C>(a, qc, S, t, dir, 3) / r, hp[t]);
+              const double qh = S.ex[t] >= 0 ? halo_q<C>(a, qc, S, t, dir, m) : qn[t];
+              T[kLineOff + S.h[t]] = flux_diff_full(jm, rm, m, qh, hu[t], hp[t], v);
             }
           } else {
             const Met M = met_of(a, dir);
@@ -1002,32 +1006,16 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
         }
       }
     };
-    auto stage_flux = [&](int m, int part) __attribute__((always_inline)) {
-      if (m == 4) stage_kind(std::integral_constant<int, FLUX_ENERGY>{}, m, part);
-      else if (m == dir + 1) stage_kind(std::integral_constant<int, FLUX_ALONG>{}, m, part);
-      else stage_kind(std::integral_constant<int, FLUX_PLAIN>{}, m, part);
+    auto stage_flux = [&](int m) __attribute__((always_inline)) {
+      if (m == 4) stage_kind(std::integral_constant<int, FLUX_ENERGY>{}, m);
+      else if (m == dir + 1) stage_kind(std::integral_constant<int, FLUX_ALONG>{}, m);
+      else stage_kind(std::integral_constant<int, FLUX_PLAIN>{}, m);
     };
-    // derivative of the staged component; cx: the convective part's, where it
-    // is solved on its own
-    double cx[GEN ? NPT : 1];
-    auto derive_flux = [&](int m) __attribute__((always_inline)) {
-      derive();
-      if constexpr (GEN) {
-        const bool two = metg && m > 0 && !uwd;
-#pragma unroll
-        for (int t = 0; t < NPT; t++) cx[t] = two ? X[S.s[t]] : 0.0;
-        if (two) {
-          stage_flux(m, 2);
-          derive();
-        }
-      }
-    };
-    auto first_part = [&](int m) { return metg && m > 0 && !uwd ? 1 : 0; };
-    // its value at slot t (the main path's fluxes carry the metrics: no 1/dx
-    // after the solve)
+    // its derivative at slot t (the main path's fluxes carry the metrics: no
+    // 1/dx after the solve)
     auto dflux = [&](int t) __attribute__((always_inline)) {
       const double x = X[S.s[t]];
-      return (MAIN ? x : x * idn) + (GEN ? cx[GEN ? t : 0] : 0.0);
+      return MAIN ? x : x * idn;
     };
     if constexpr (!RK) {
       const int m0 = uwd ? 1 : 0;
@@ -1037,7 +1025,7 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
       for (int mm = 0; mm < (ONE ? 1 : 5); mm++) {
         const int m = ONE ? field : mm;
         if (m < m0) continue;
-        stage_flux(m, first_part(m));
+        stage_flux(m);
         double* dst = qrhs + m * fs;
         double qr[NPT];
         if (!FIRST || uwd) {
@@ -1045,7 +1033,7 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
           for (int t = 0; t < NPT; t++) qr[t] = ldg(dst, S.g[t]);
         }
         if (!ONE && m < 4) load_inputs(m + 1);
-        derive_flux(m);
+        derive();
 #pragma unroll
         for (int t = 0; t < NPT; t++) stg(dst, S.g[t], FIRST && !uwd ? dflux(t) : qr[t] + dflux(t));
       }
@@ -1064,108 +1052,43 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
           qs[t] = sa.stage == 0 ? 0.0 : ldg(qo + m * fs, S.g[t]);
         }
       };
-      if constexpr (ONE) {
-        const int m = field;
-        const bool solve = m > 0 || !uwd;  // without convection density has no flux
-        load_inputs(m);
-        load_rk(m);
-        if (solve) {
-          stage_flux(m, 0);
-          derive_flux(m);
-        }
-        double qw[NPT];
-#pragma unroll
-        for (int t = 0; t < NPT; t++) {
-          const double v = solve ? qr[t] + dflux(t) : qr[t];
-          const double s0 = sa.stage == 0 ? qn[t] : qs[t];
-          qw[t] = MAIN ? rk_update_main(sa, a.dt, a.jac, s0 * a.jac, qn[t], v)  // qsave = q J (mainloop.F90:423-427)
-                       : rk_update(sa, a.dt, s0, qn[t], v);
-        }
-        if (MAIN && !a.rk_filter) {
-#pragma unroll
-          for (int t = 0; t < NPT; t++) stg(qnew + m * fs, S.g[t], qw[t]);
-          return;
-        }
-        if constexpr (MAIN) {
-          // updatefvar needs all five components of the unfiltered state:
-          // they go to the first fields of the gradients, which the flux
-          // passes no longer read, for k_fvar
-#pragma unroll
-          for (int t = 0; t < NPT; t++) stg(a.dv + m * fs, S.g[t], qw[t]);
-        }
-        // the filter sweep along dir: the miniapp's of this stage, the main
-        // path's of the next (comsolver.F90:514-632)
-        filter_setup(1);
-#pragma unroll
-        for (int t = 0; t < NPT; t++) put<C>(T, S, t, qw[t]);
-        filter();
-#pragma unroll
-        for (int t = 0; t < NPT; t++) stg(qnew + m * fs, S.g[t], X[S.s[t]]);
-      } else {
-        load_inputs(0);
-        load_rk(0);
-        // the new q, whose updatefvar ends the pass
-        double qw[5][NPT];
-#pragma unroll
-        for (int m = 0; m < 5; m++) {
-          const bool solve = m > 0 || !uwd;  // without convection density has no flux
-          if (solve) stage_flux(m, first_part(m));
-          double qm[NPT], ro[NPT], so[NPT];
-#pragma unroll
-          for (int t = 0; t < NPT; t++) {
-            qm[t] = qn[t];
-            ro[t] = qr[t];
-            so[t] = qs[t];
-          }
-          if (m < 4) {
-            load_inputs(m + 1);
-            load_rk(m + 1);
-          }
-          if (solve) derive_flux(m);
-#pragma unroll
-          for (int t = 0; t < NPT; t++) {
-            const double v = solve ? ro[t] + dflux(t) : ro[t];
-            const double jb = jac_of<GEN>(a, S.g[t]);
-            // qsave = q J (src/mainloop.F90:423-427)
-            const double s0 = (sa.stage == 0 ? qm[t] : so[t]) * jb;
-            qw[m][t] = rk_update_main(sa, a.dt, jb, s0, qm[t], v);
-          }
-        }
-        // updatefvar (fludyna.F90:191-242): rho, u, v, w, p, T of the new q
-#pragma unroll
-        for (int t = 0; t < NPT; t++) {
-          const Prim P = prim_of(a, qw[0][t], qw[1][t], qw[2][t], qw[3][t], qw[4][t]);
-          const unsigned o = S.g[t];
-          stg(a.pr, o, P.r);
-          stg(a.pr + fs, o, P.u);
-          stg(a.pr + 2 * fs, o, P.v);
-          stg(a.pr + 3 * fs, o, P.w);
-          stg(a.pr + 4 * fs, o, P.p);
-          stg(a.pr + 5 * fs, o, P.t);
-        }
-        if (a.rk_filter) {
-          // the next stage's filterq sweep along dir (comsolver.F90:514-632),
-          // as the filter pass does it, on the new q held in registers; the
-          // primitives above stay those of the unfiltered q, as after the
-          // reference's filterq.  The barrier before the solve orders the
-          // staging below after every read of the flux part's LDS.
-          filter_setup(1);
-#pragma unroll
-          for (int m = 0; m < 5; m++) {
-#pragma unroll
-            for (int t = 0; t < NPT; t++) put<C>(T, S, t, qw[m][t]);
-            filter();
-#pragma unroll
-            for (int t = 0; t < NPT; t++) stg(qnew + m * fs, S.g[t], X[S.s[t]]);
-          }
-        } else {
-          // q last: the halo copies of general grids are read from it above
-#pragma unroll
-          for (int t = 0; t < NPT; t++)
-#pragma unroll
-            for (int m = 0; m < 5; m++) stg(qnew + m * fs, S.g[t], qw[m][t]);
-        }
+      const int m = field;
+      const bool solve = m > 0 || !uwd;  // without convection density has no flux
+      load_inputs(m);
+      load_rk(m);
+      if (solve) {
+        stage_flux(m);
+        derive();
       }
+      double qw[NPT];
+#pragma unroll
+      for (int t = 0; t < NPT; t++) {
+        const double v = solve ? qr[t] + dflux(t) : qr[t];
+        const double s0 = sa.stage == 0 ? qn[t] : qs[t];
+        const double jb = MAIN ? jac_of<GEN>(a, S.g[t]) : 1.0;
+        qw[t] = MAIN ? rk_update_main(sa, a.dt, jb, s0 * jb, qn[t], v)  // qsave = q J (mainloop.F90:423-427)
+                     : rk_update(sa, a.dt, s0, qn[t], v);
+      }
+      if (MAIN && !a.rk_filter) {
+#pragma unroll
+        for (int t = 0; t < NPT; t++) stg(qnew + m * fs, S.g[t], qw[t]);
+        return;
+      }
+      if constexpr (MAIN) {
+        // updatefvar needs all five components of the unfiltered state:
+        // they go to the first fields of the gradients, which the flux
+        // passes no longer read, for k_fvar
+#pragma unroll
+        for (int t = 0; t < NPT; t++) stg(a.dv + m * fs, S.g[t], qw[t]);
+      }
+      // the filter sweep along dir: the miniapp's of this stage, the main
+      // path's of the next (comsolver.F90:514-632)
+      filter_setup(1);
+#pragma unroll
+      for (int t = 0; t < NPT; t++) put<C>(T, S, t, qw[t]);
+      filter();
+#pragma unroll
+      for (int t = 0; t < NPT; t++) stg(qnew + m * fs, S.g[t], X[S.s[t]]);
     }
   } else {  // F_ONLY: filter of q along dir, in place (filterq, tgvsolver.F90:791-883)
     filter_setup(0);
@@ -1212,7 +1135,10 @@ constexpr int pass_fields(int prog) {
 // 23.8 -> 25.7, and where they form the pressure too 10.3 -> 9.2, 13.8 -> 16.5.
 // The RK pass solves twice per component and gains at every size (miniapp
 // 33^3 23.5 -> 12, 129^3 132 -> 129, 257^3 1080 -> 1034), so it has that
-// form only, but for directions of the general-grid kernels.
+// form only.  The general-grid kernels follow the same limits: with them, and
+// one solve of each flux difference instead of one per part, a step of a
+// wall-bounded stretched grid takes at 32^3 985 -> 485 us, 96x80x64 2002 ->
+// 1403, 128^3 6321 -> 4935.
 constexpr bool pass_one(int prog, bool pres, int nt) {
   if (pass_fields(prog) == 0) return false;
   if (prog == V_LAST_RK) return true;
@@ -1329,33 +1255,33 @@ void launch_pass_m(int prog, const FlowArgs& a, int dir, hipStream_t st) {
   const int nt = tiles_of(a.n, dir, C::TL);
   const size_t lds = (size_t)lds_doubles<C>(prog, MAIN) * sizeof(double);
   dim3 g(nt), b(C::NT);
-  if constexpr (!GEN) {
-    const bool pres = !MAIN && (prog == GC_FIRST || (a.gradx && dir == 1));
-    if (!(prog == V_MID && dir == 0) && pass_one(prog, pres, nt)) {
-      switch (prog) {
-        case GC_FIRST:
-        case GC_MID:
-        case GC_LAST:
-          if (pres || prog == GC_FIRST)
-            hipLaunchKernelGGL((k_pass_one<C, GC_FIRST, MINB, MAIN>), dim3(4 * nt), b, lds, st, a, dir);
-          else
-            hipLaunchKernelGGL((k_pass_one<C, GC_MID, MINB, MAIN>), dim3(4 * nt), b, lds, st, a, dir);
-          return;
-        case V_MID:
-        case V_LAST_RHS:
-          hipLaunchKernelGGL((k_pass_one<C, V_MID, MINB, MAIN>), dim3(5 * nt), b, lds, st, a, dir);
-          return;
-        case V_LAST_RK:
-          hipLaunchKernelGGL((k_pass_one<C, V_LAST_RK, MINB, MAIN>), dim3(5 * nt), b, lds, st, a, dir);
-          if constexpr (MAIN) {
-            const unsigned pts = (unsigned)a.pitch * (a.n[1] + 1) * (a.n[2] + 1);
-            const double* q = a.rk_filter ? a.dv : (a.stage == 1 ? a.qrhs : a.qsave);
-            hipLaunchKernelGGL(k_fvar, dim3((pts + 255) / 256), dim3(256), 0, st, a, q);
-          }
-          return;
-        case F_ONLY: hipLaunchKernelGGL((k_pass_one<C, F_ONLY, MINB, false>), dim3(5 * nt), b, lds, st, a, dir); return;
-        default: break;
-      }
+  const bool pres = !MAIN && (prog == GC_FIRST || (a.gradx && dir == 1));
+  if (!(prog == V_MID && dir == 0) && pass_one(prog, pres, nt)) {
+    switch (prog) {
+      case GC_FIRST:
+      case GC_MID:
+      case GC_LAST:
+        if (pres || prog == GC_FIRST)
+          hipLaunchKernelGGL((k_pass_one<C, GC_FIRST, MINB, MAIN, GEN>), dim3(4 * nt), b, lds, st, a, dir);
+        else
+          hipLaunchKernelGGL((k_pass_one<C, GC_MID, MINB, MAIN, GEN>), dim3(4 * nt), b, lds, st, a, dir);
+        return;
+      case V_MID:
+      case V_LAST_RHS:
+        hipLaunchKernelGGL((k_pass_one<C, V_MID, MINB, MAIN, GEN>), dim3(5 * nt), b, lds, st, a, dir);
+        return;
+      case V_LAST_RK:
+        hipLaunchKernelGGL((k_pass_one<C, V_LAST_RK, MINB, MAIN, GEN>), dim3(5 * nt), b, lds, st, a, dir);
+        if constexpr (MAIN) {
+          const unsigned pts = (unsigned)a.pitch * (a.n[1] + 1) * (a.n[2] + 1);
+          const double* q = a.rk_filter ? a.dv : (a.stage == 1 ? a.qrhs : a.qsave);
+          hipLaunchKernelGGL(k_fvar, dim3((pts + 255) / 256), dim3(256), 0, st, a, q);
+        }
+        return;
+      case F_ONLY:
+        hipLaunchKernelGGL((k_pass_one<C, F_ONLY, MINB, GEN, GEN>), dim3(5 * nt), b, lds, st, a, dir);
+        return;
+      default: break;
     }
   }
   switch (prog) {
@@ -1386,9 +1312,7 @@ void launch_pass_m(int prog, const FlowArgs& a, int dir, hipStream_t st) {
       }
       [[fallthrough]];
     case V_LAST_RHS: hipLaunchKernelGGL((k_pass<C, V_MID, MINB, MAIN, GEN>), g, b, lds, st, a, dir); break;
-    case V_LAST_RK:
-      if constexpr (GEN) hipLaunchKernelGGL((k_pass<C, V_LAST_RK, MINB, MAIN, GEN>), g, b, lds, st, a, dir);
-      break;
+    case V_LAST_RK: break;  // pass_one always
     // the filtering first pass exists for the miniapp's stage only (the main
     // path filters at the start of its stage); launch_pass_c refuses it there
     case FGC_FIRST:

@@ -53,6 +53,7 @@ def _bind():
                                        C.POINTER(C.c_int)]
     L.astr_hip_reactor_release.argtypes = [C.c_void_p, C.c_int]
     L.astr_hip_reactor_rhs.argtypes = [C.c_void_p, C.c_int, _dp, _dp, _dp, _dp]
+    L.astr_hip_reactor_team_eval.argtypes = [C.c_void_p, C.c_int, _dp, _dp, C.c_double, _dp, _dp, _dp]
     L.astr_hip_reactor_method.argtypes = [_dp, C.c_int]
     L.astr_hip_srccomb.argtypes = [C.c_void_p] + [C.c_int] * 5 + [_dp] * 5
     L.astr_hip_srccomb_device.argtypes = [C.c_void_p] + [C.c_int] * 5 + [C.c_void_p] * 6
@@ -94,8 +95,8 @@ class Mechanism:
 
     def reactor_rhs(self, p, y, jacobian=False):
         """The reactor's d(T, Y)/dt at states y (n, ns+1) and pressures p (n,),
-        and with jacobian=True the analytic Jacobian the integrator uses
-        (n, ns+1, ns+1)."""
+        and with jacobian=True the analytic Jacobian (n, ns+1, ns+1), as the
+        integrator with one lane per reactor evaluates them."""
         p = np.ascontiguousarray(np.atleast_1d(p), dtype=np.float64)
         y = np.ascontiguousarray(np.atleast_2d(y), dtype=np.float64)
         n, m = y.shape
@@ -105,6 +106,19 @@ class Mechanism:
         J = np.empty((n, m, m)) if jacobian else None
         _chk(_bind().astr_hip_reactor_rhs(self.h, n, _p(p), _p(y), _p(f), _p(J)))
         return (f, J) if jacobian else f
+
+    def reactor_team_eval(self, p, y, gh):
+        """(f, J, x) at states y (n, ns+1) and pressures p (n,), as the
+        integrator with 16 lanes per reactor evaluates them: the right-hand
+        side, its Jacobian and the solution of (I - gh J) x = f."""
+        p = np.ascontiguousarray(np.atleast_1d(p), dtype=np.float64)
+        y = np.ascontiguousarray(np.atleast_2d(y), dtype=np.float64)
+        n, m = y.shape
+        if m != self.ns + 1 or p.shape != (n,):
+            raise AstrError("shapes: p (n,), y (n, ns+1)")
+        f, J, x = np.empty((n, m)), np.empty((n, m, m)), np.empty((n, m))
+        _chk(_bind().astr_hip_reactor_team_eval(self.h, n, _p(p), _p(y), gh, _p(f), _p(J), _p(x)))
+        return f, J, x
 
     def rates(self, T, rho_or_p, Y, input_is_p=True, species_h=False):
         """T, rho|p: (n,), Y: (ns, n) -> wdot (ns, n) kg/m^3/s, h_mix, cp_mix[, h_k]."""

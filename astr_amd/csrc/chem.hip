@@ -1054,8 +1054,8 @@ __global__ __launch_bounds__(64) void k_reactor_n(const Mech* __restrict__ M, Re
 }
 
 
-// The reactor's right-hand side and its analytic Jacobian (the integrator's,
-// before the -gamma h scaling) at n states, one thread per state: y, f
+// The right-hand side and the analytic Jacobian of the one-thread integrator
+// (before the -gamma h scaling) at n states, one thread per state: y, f
 // row-major N per state, jac N x N per state (row k, column j)
 template <int NS>
 __global__ __launch_bounds__(64) void k_reactor_eval(const Mech* __restrict__ M, int n, const double* p,
@@ -1550,6 +1550,42 @@ __global__ __launch_bounds__(64) void k_reactor_team(const Mech* __restrict__ M,
     P.nstep[i] = nstep;
     P.nrej[i] = nrej;
     P.status[i] = st;
+  }
+}
+
+// What the team integrator is made of, at n states laid out as in
+// k_reactor_eval: the right-hand side, the Jacobian and the solution of
+// (I - gh J) x = f by its factorisation and solve.  The Jacobian comes out of
+// matrix(), which forms I - g J, with a power of two as -g that is large
+// against any 1/J, so that taking I off costs no digits of J's entries.
+template <int NS, bool UNIT>
+__global__ __launch_bounds__(64) void k_reactor_team_eval(const Mech* __restrict__ M, int n, const double* p,
+                                                          const double* y, double gh, double* f, double* jac,
+                                                          double* sol) {
+  using TeamN = Team<NS, UNIT>;
+  constexpr int N = NS + 1;
+  constexpr double kScale = 0x1p60;
+  __shared__ typename TeamN::Lds lds[64 / kTeam];
+  const int team = threadIdx.x / kTeam, lane = threadIdx.x % kTeam;
+  const int i = blockIdx.x * (64 / kTeam) + team;
+  if (i >= n) return;  // the whole team leaves
+  TeamN R(M, lds[team], lane, p[i]);
+  const double fl = R.template rhs<true>(lane < N ? y[(size_t)i * N + lane] : 0.0);
+  if (lane < N) f[(size_t)i * N + lane] = fl;
+  double row[N];
+  if (jac) {
+    R.matrix(fl, -kScale, row);
+    if (lane < N)
+#pragma unroll
+      for (int j = 0; j < N; j++) jac[((size_t)i * N + lane) * N + j] = (row[j] - (lane == j ? 1.0 : 0.0)) / kScale;
+  }
+  if (sol) {
+    double lw[N], up[N], dinv;
+    int src;
+    R.matrix(fl, gh, row);
+    const bool ok = R.factor(row, lw, up, dinv, src);
+    const double x = R.solve(lw, up, dinv, src, fl);
+    if (lane < N) sol[(size_t)i * N + lane] = ok ? x : __longlong_as_double(0x7ff8000000000000ll);
   }
 }
 
@@ -2068,6 +2104,35 @@ int astr_hip_reactor_rhs(astr_chem* chem, int n, const double* p, const double* 
         hipMemcpy(f, df, ny * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess ||
         (jac && hipMemcpy(jac, dj, nj * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess))
       rc = cfail("reactor_rhs: kernel or copy out failed");
+  }
+  (void)hipFree(d);
+  return rc;
+}
+
+int astr_hip_reactor_team_eval(astr_chem* chem, int n, const double* p, const double* y, double gh, double* f,
+                               double* jac, double* sol) {
+  if (!chem || !p || !y || !f || n < 1) return cfail("reactor_team_eval: null argument or no states");
+  if (chem->host.ns != 9) return cfail("reactor_team_eval: 9-species mechanisms only (the team kernel)");
+  CHIP_OK(hipSetDevice(chem->device));
+  constexpr int N = 10;
+  double* d = nullptr;
+  const size_t ny = (size_t)n * N, nj = ny * N;
+  CHIP_OK(hipMalloc(&d, (n + 3 * ny + nj) * sizeof(double)));
+  double *dp = d, *dy = d + n, *df = dy + ny, *ds = df + ny, *dj = ds + ny;
+  int rc = 0;
+  if (hipMemcpy(dp, p, n * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(dy, y, ny * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+    rc = cfail("reactor_team_eval: copy in failed");
+  } else {
+    constexpr int per = 64 / kTeam;
+    hipLaunchKernelGGL((chem->host.unit ? k_reactor_team_eval<9, true> : k_reactor_team_eval<9, false>),
+                       dim3((n + per - 1) / per), dim3(64), 0, nullptr, chem->dev, n, dp, dy, gh, df,
+                       jac ? dj : nullptr, sol ? ds : nullptr);
+    if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess ||
+        hipMemcpy(f, df, ny * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess ||
+        (sol && hipMemcpy(sol, ds, ny * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess) ||
+        (jac && hipMemcpy(jac, dj, nj * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess))
+      rc = cfail("reactor_team_eval: kernel or copy out failed");
   }
   (void)hipFree(d);
   return rc;

@@ -378,7 +378,7 @@ int astr_hip_chem_temperature_device(astr_chem *chem, long long n, const double 
  *
  * The integrator: RODAS4, the stiffly accurate L-stable Rosenbrock method of
  * order 4 with an embedded order-3 solution (Hairer and Wanner 1996,
- * Sect. VI.4), with a finite-difference Jacobian and error control at rtol,
+ * Sect. VI.4), with the analytic Jacobian and error control at rtol,
  * atol (mass fractions; temperature uses atol 1e-6 K).  reactor_method
  * writes its table: gamma, a21, a31, a32, a41..a43, a51..a54, c21, c31,
  * c32, c41..c43, c51..c54, c61..c65 (26 values; n must be at least 26).
@@ -415,10 +415,15 @@ int astr_hip_reactor_get(astr_reactor_pool *pool, int slot, double *t, double *T
 int astr_hip_reactor_release(astr_reactor_pool *pool, int slot);
 int astr_hip_reactor_method(double *coef, int n);
 /* The reactor's right-hand side d(T, Y)/dt at n states (p[n], y and f n x
- * (ns+1) row-major) and, if jac is not null, the analytic Jacobian the
- * integrator uses (n x (ns+1) x (ns+1), row k = component, column j =
- * variable); 9-species mechanisms. */
+ * (ns+1) row-major) and, if jac is not null, the analytic Jacobian
+ * (n x (ns+1) x (ns+1), row k = component, column j = variable), as the
+ * integrator with one lane per reactor evaluates them; 9-species mechanisms. */
 int astr_hip_reactor_rhs(astr_chem *chem, int n, const double *p, const double *y, double *f, double *jac);
+/* The same as the integrator with 16 lanes per reactor evaluates them, and, if
+ * sol is not null, the solution x (n x (ns+1)) of (I - gh J) x = f by its
+ * factorisation and solve (NaN where a pivot is zero); 9-species mechanisms. */
+int astr_hip_reactor_team_eval(astr_chem *chem, int n, const double *p, const double *y, double gh, double *f,
+                               double *jac, double *sol);
 
 /* ------------------------------------------------------------------------
  * HBM streaming probe (no reference counterpart): dst[0:n] = src[0:n] in

@@ -2493,7 +2493,7 @@ int upload_jobs(astr_hip_batch* b) {
 int enqueue_step(astr_hip_batch* b) {
   static const double rk[3][3] = {{1.0, 0.0, 1.0}, {0.75, 0.25, 0.25}, {1.0 / 3.0, 2.0 / 3.0, 2.0 / 3.0}};
   for (int s = 0; s < 3; s++) {
-    StageArgs sa{s, s == 0 ? 1 : 0, rk[s][0], rk[s][1], rk[s][2], s};
+    StageArgs sa{s, s == 0 ? 1 : 0, rk[s][0], rk[s][1], rk[s][2], s, 0};
     StageArgs sv = sa;
     sv.dostats = 0;
     StageArgs sf = sv;  // the filter passes after the update
@@ -2663,7 +2663,7 @@ int astr_hip_batch_autotune(astr_hip_batch* b, int reps) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (!rc && (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess))
     rc = fail("hipEventCreate failed");
-  const StageArgs sa{0, 0, 1.0, 0.0, 1.0, 0};
+  const StageArgs sa{0, 0, 1.0, 0.0, 1.0, 0, 0};
   for (int sl = 0; sl < 8 && !rc; sl++) {
     const int kind = kSlotKind[sl], d = kSlotDir[sl];
     // classes: cases of this slot with the same program and the same set of

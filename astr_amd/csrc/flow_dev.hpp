@@ -70,7 +70,8 @@ struct FlowArgs {
   // its direction to the new q, after updatefvar took the primitives
   int rk_filter;
   // the stress pass computes the x gradients itself (its lines are x-lines),
-  // no x gradient pass before it; store_gx: it also stores them
+  // no x gradient pass before it; store_gx: it also stores them (read through
+  // StageArgs: a batch copies these arguments whatever call set them last)
   int gradx, store_gx;
 };
 
@@ -426,6 +427,7 @@ struct StageArgs {
   int dostats;          // stage-1 KE/enstrophy partial sums (1) or none (0)
   double rk_a, rk_b, rk_c;
   int alt;              // batches: stages whose change of array roles applies (0, 1, 2)
+  int store_gx;         // the stress pass also stores the x gradients it computes (batches: never)
 };
 
 // the arrays in their roles after `alt` stages of a step
@@ -439,7 +441,7 @@ __device__ __forceinline__ Arrays arrays_of(const FlowArgs& a, int alt) {
 }
 
 __device__ __forceinline__ StageArgs stage_of(const FlowArgs& a) {
-  return StageArgs{a.stage, a.dostats, a.rk_a, a.rk_b, a.rk_c, 0};
+  return StageArgs{a.stage, a.dostats, a.rk_a, a.rk_b, a.rk_c, 0, a.store_gx};
 }
 
 // q <- a*qsave + b*q + c*qrhs*dt in the reference's order (tgvsolver.F90:1055-1057)
@@ -836,7 +838,7 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
 #pragma unroll
           for (int t = 0; t < NPT; t++) {
             gx[c][t] = X[S.s[t]] * (MAIN ? met_of(a, dir).d : idn);
-            if (a.store_gx) stg(a.dv + (c < 3 ? c : 9) * fs, S.g[t], gx[c][t]);
+            if (sa.store_gx) stg(a.dv + (c < 3 ? c : 9) * fs, S.g[t], gx[c][t]);
           }
         }
       }

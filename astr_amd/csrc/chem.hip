@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "../../include/astr_hip.h"
+#include "rate_exp.hpp"
 
 namespace {
 
@@ -180,39 +181,18 @@ struct RegArray {
   }
 };
 
-// e^x for the rate constants: x = n ln 2 + r with the nearest n (Cody and
-// Waite's two-part ln 2), e^r = 1 + r + r^2 P(r) with P of degree 9 through
-// the Chebyshev nodes of |r| <= ln 2 / 2 (its error 2e-17), scaled by 2^n.
-// About 20 instructions where exp takes 33: exp's constants sit in vector
-// registers that its multiply-adds overwrite, so each is copied first; here
-// they are scalar operands (ExpK, made once per thread in scalar registers),
-// and the checks for overflow and underflow are one comparison, with exp's
-// own result for the lanes outside +-700.
-struct ExpK {
-  double l2e = 0x1.71547652b82fep+0, rnd = 0x1.8p52, hi = 0x1.62e42fefa39efp-1, lo = 0x1.abc9e3b39803fp-56;
-  double c3 = 0x1.5555555555556p-3, c4 = 0x1.5555555553d4fp-5, c5 = 0x1.11111111109adp-7,
-         c6 = 0x1.6c16c17893833p-10, c7 = 0x1.a01a01a7c8d47p-13, c8 = 0x1.a019b8ef67c6cp-16,
-         c9 = 0x1.71de0d9c145d0p-19, c10 = 0x1.2891a8c1d838dp-22, c11 = 0x1.af38d53857513p-26;
+// e^x for the rate constants (rate_exp.hpp) in about 20 instructions where exp
+// takes 33: exp's constants sit in vector registers that its multiply-adds
+// overwrite, so each is copied first; here they are scalar operands (ExpK, made
+// once per thread in scalar registers), and the checks for overflow and
+// underflow are one comparison, with exp's own result for the lanes outside
+// +-700.
+struct ExpK : astr::RateExpConstants {
   __device__ __forceinline__ ExpK() {
-    asm volatile("" : "+s"(l2e), "+s"(rnd), "+s"(hi), "+s"(lo), "+s"(c3), "+s"(c4), "+s"(c5), "+s"(c6));
-    asm volatile("" : "+s"(c7), "+s"(c8), "+s"(c9), "+s"(c10), "+s"(c11));
+    asm volatile("" : "+s"(l2e), "+s"(rnd), "+s"(hi), "+s"(lo), "+s"(c3), "+s"(c4), "+s"(c5));
+    asm volatile("" : "+s"(c6), "+s"(c7), "+s"(c8), "+s"(c9), "+s"(c10), "+s"(c11), "+s"(c12));
   }
 };
-__device__ __forceinline__ double rate_exp_in(double x, const ExpK& K) {  // |x| < 700
-  const double t = fma(x, K.l2e, K.rnd);  // n in the low bits
-  const double n = t - K.rnd;
-  const double r = fma(-n, K.lo, fma(-n, K.hi, x));
-  double p = fma(K.c11, r, K.c10);
-  p = fma(p, r, K.c9);
-  p = fma(p, r, K.c8);
-  p = fma(p, r, K.c7);
-  p = fma(p, r, K.c6);
-  p = fma(p, r, K.c5);
-  p = fma(p, r, K.c4);
-  p = fma(p, r, K.c3);
-  p = fma(p, r, 0.5);
-  return ldexp(1.0 + fma(r * r, p, r), __double2loint(t));
-}
 // several at once, with one branch after their chains of multiply-adds
 template <int N>
 __device__ __forceinline__ void rate_exps(const double (&x)[N], const ExpK& K, double (&e)[N]) {

@@ -44,7 +44,7 @@ class Layout(C.Structure):
 
 
 EXPORTS = [
-    "astr_hip_last_error", "astr_hip_create", "astr_hip_destroy", "astr_hip_set_stream",
+    "astr_hip_last_error", "astr_hip_case_bytes", "astr_hip_create", "astr_hip_destroy", "astr_hip_set_stream",
     "astr_hip_set_deltat", "astr_hip_field_info", "astr_hip_init_tgv", "astr_hip_upload",
     "astr_hip_download", "astr_hip_filterq", "astr_hip_gradcal", "astr_hip_rhscal",
     "astr_hip_rk3_steps", "astr_hip_rk3_steps_stats", "astr_hip_sync", "astr_hip_line_batch",
@@ -86,6 +86,7 @@ def lib():
         L.astr_hip_last_error.restype = C.c_char_p
         L.astr_hip_create.argtypes = [C.POINTER(Config), C.POINTER(C.c_void_p)]
         L.astr_hip_destroy.argtypes = [C.c_void_p]
+        L.astr_hip_case_bytes.argtypes = [C.POINTER(Config), C.POINTER(C.c_longlong)]
         L.astr_hip_set_stream.argtypes = [C.c_void_p, C.c_void_p]
         L.astr_hip_set_deltat.argtypes = [C.c_void_p, C.c_double]
         L.astr_hip_field_info.argtypes = [C.c_void_p, C.POINTER(Layout)]
@@ -166,6 +167,13 @@ def main_config(im, jm=None, km=None, deltat=1e-3, reynolds=1600.0, mach=0.1, re
                      ref_tem=ref_tem, lx=lx, ly=ly, lz=lz, semantics=SEM_MAIN)
     cfg.beta_bound = 0.98   # filter_coefficient_cal's beter_bouond (src/comsolver.F90:121)
     return cfg
+
+
+def case_field_bytes(cfg: Config) -> int:
+    """Device memory of the fields of a case of this configuration."""
+    v = C.c_longlong()
+    _chk(lib().astr_hip_case_bytes(C.byref(cfg), C.byref(v)))
+    return v.value
 
 
 class Flow:

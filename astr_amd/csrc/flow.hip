@@ -1371,9 +1371,44 @@ int rk3_run(astr_hip_ctx* c, int nsteps, const StatsBufs& sb, double* ke, double
 
 }  // namespace
 
+namespace {
+// sizes, layout of a field and (main path) of the halo sources, from the
+// configuration alone
+void field_layout(const astr_hip_config& cfg, FlowArgs& a) {
+  a.n[0] = cfg.im; a.n[1] = cfg.jm; a.n[2] = cfg.km;
+  a.ndir = cfg.km > 0 ? 3 : 2;
+  a.main_sem = cfg.semantics == ASTR_SEM_MAIN ? 1 : 0;
+  // rows start on a cache line of 128 bytes, or, from 400 000 points on, on half
+  // of one: there the passes are bound by bytes and shorter rows are fewer
+  // (129^3 3.7% and 257^3 1% of a step, 97x81x64 1%), below it by latency and
+  // by requests (33^3 1.4% slower with half lines, 98x62x46 0.7%)
+  const long long points = (long long)(cfg.im + 1) * (cfg.jm + 1) * (cfg.km + 1);
+  const int unit = points < 400000 ? 16 : 8;
+  a.pitch = (cfg.im + unit) / unit * unit;
+  a.plane = (long long)a.pitch * (cfg.jm + 1);
+  a.trash = (int)(a.plane * (cfg.km + 1));
+  a.fs = (a.plane * (cfg.km + 1) + 1 + 63) / 64 * 64;
+  if (a.main_sem) {
+    a.hxs = hx_lines(a.n, a.ndir) * kHaloSrcRows;
+    a.hys = hy_lines(a.n, a.ndir) * kHaloSrcRows;
+  }
+}
+// fields: q 5, qsave 5, qrhs 5, dv 12, sg 9; then the miniapp's pressure or
+// the main path's primitives 6
+long long field_count(const FlowArgs& a) { return a.main_sem ? 42 : 37; }
+}  // namespace
+
 extern "C" {
 
 const char* astr_hip_last_error(void) { return g_err.c_str(); }
+
+int astr_hip_case_bytes(const astr_hip_config* cfg, long long* bytes) {
+  if (!cfg || !bytes) return fail("null argument");
+  FlowArgs a{};
+  field_layout(*cfg, a);
+  *bytes = (field_count(a) * a.fs + 5 * (a.hxs + a.hys)) * (long long)sizeof(double);
+  return 0;
+}
 
 int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   if (!cfg || !out) return fail("null argument");
@@ -1389,18 +1424,7 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   (void)hipGetDevice(&c->device);
   FlowArgs& a = c->a;
   std::memset(&a, 0, sizeof(a));
-  a.n[0] = cfg->im; a.n[1] = cfg->jm; a.n[2] = cfg->km;
-  a.ndir = cfg->km > 0 ? 3 : 2;
-  // rows start on a cache line of 128 bytes, or, from 400 000 points on, on half
-  // of one: there the passes are bound by bytes and shorter rows are fewer
-  // (129^3 3.7% and 257^3 1% of a step, 97x81x64 1%), below it by latency and
-  // by requests (33^3 1.4% slower with half lines, 98x62x46 0.7%)
-  const long long points = (long long)(cfg->im + 1) * (cfg->jm + 1) * (cfg->km + 1);
-  const int unit = points < 400000 ? 16 : 8;
-  a.pitch = (cfg->im + unit) / unit * unit;
-  a.plane = (long long)a.pitch * (cfg->jm + 1);
-  a.trash = (int)(a.plane * (cfg->km + 1));
-  a.fs = (a.plane * (cfg->km + 1) + 1 + 63) / 64 * 64;
+  field_layout(*cfg, a);
   // point offsets inside a field are 32-bit byte offsets (flow_dev.hpp ldg/stg)
   if ((unsigned long long)a.fs * sizeof(double) >= (1ull << 32)) {
     delete c;
@@ -1418,7 +1442,6 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   a.inv_d[1] = (double)cfg->jm / cfg->ly;
   a.inv_d[2] = cfg->km > 0 ? (double)cfg->km / cfg->lz : 0.0;
   a.dt = cfg->deltat;
-  a.main_sem = cfg->semantics == ASTR_SEM_MAIN ? 1 : 0;
   // the Jacobian of the uniform grid until set_metrics gives gridgeom's
   a.jac = (cfg->lx / cfg->im) * (cfg->ly / cfg->jm) * (cfg->km > 0 ? cfg->lz / cfg->km : 1.0);
   a.alfa = cfg->alfa_filter;
@@ -1438,10 +1461,7 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
       c->tuned_ms[pr][d] = 0.f;
     }
   }
-  // fields: q 5, qsave 5, qrhs 5, dv 12, sg 9; then the miniapp's pressure or
-  // the main path's primitives 6
-  const long long nfield = a.main_sem ? 42 : 37;
-  size_t bytes = (size_t)(nfield * a.fs) * sizeof(double);
+  const size_t bytes = (size_t)(field_count(a) * a.fs) * sizeof(double);
   if (hipMalloc(&c->base, bytes) != hipSuccess) { delete c; return fail("hipMalloc of fields failed"); }
   (void)hipMemset(c->base, 0, bytes);
   a.q = c->base;
@@ -1453,8 +1473,6 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   a.p = a.main_sem ? nullptr : a.sg + 9 * a.fs;
   if (a.main_sem) {
     // halo sources kept by qswap: hx then hy, 5 fields each
-    a.hxs = hx_lines(a.n, a.ndir) * kHaloSrcRows;
-    a.hys = hy_lines(a.n, a.ndir) * kHaloSrcRows;
     if (hipMalloc(&c->halo, (size_t)(5 * (a.hxs + a.hys) + 1) * sizeof(double)) != hipSuccess) {
       (void)hipFree(c->base); delete c; return fail("hipMalloc of the halo sources failed");
     }

@@ -68,12 +68,8 @@ class Result:
 
 
 def case_bytes(cfg: A.Config) -> int:
-    """Device memory of one context: 37 padded FP64 fields plus tables."""
-    unit = 16 if (cfg.im + 1) * (cfg.jm + 1) * (cfg.km + 1) < 400000 else 8
-    pitch = (cfg.im + unit) // unit * unit
-    plane = pitch * (cfg.jm + 1)
-    fs = (plane * (cfg.km + 1) + 1 + 63) // 64 * 64
-    return 37 * fs * 8 + 64 * 1024
+    """Device memory of one context: its fields plus tables."""
+    return A.case_field_bytes(cfg) + 64 * 1024
 
 
 def h2_air(names, W, phi):

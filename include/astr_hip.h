@@ -76,6 +76,9 @@ const char *astr_hip_last_error(void);
 /* alloccommarray + solver_init: tgvsolver.F90:13-38, :236-261 */
 int astr_hip_create(const astr_hip_config *cfg, astr_hip_ctx **out);
 int astr_hip_destroy(astr_hip_ctx *ctx);
+/* Device memory of the fields that create would allocate (needs no GPU); a
+ * context's tables add a few 10 KiB. */
+int astr_hip_case_bytes(const astr_hip_config *cfg, long long *bytes);
 int astr_hip_set_stream(astr_hip_ctx *ctx, void *hip_stream);
 int astr_hip_set_deltat(astr_hip_ctx *ctx, double deltat);
 int astr_hip_field_info(astr_hip_ctx *ctx, astr_hip_layout *layout);

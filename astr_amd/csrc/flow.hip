@@ -447,12 +447,17 @@ hipError_t launch_pass(int shape, int prog, int minb, const FlowArgs& a, int dir
 // system needs once a pass is bound by it (256^3 y gradients 380 on 8 lines,
 // 436 on 4, 593 on 2), in the register footprint the pass has room for.  With
 // fewer lines than fill the chip with such tiles, two lines per workgroup
-// (2-D 300 x 181: RK pass 23 against 32).
+// (2-D 300 x 181: RK pass 23 against 32).  The filter sweep, whose five fields
+// are read and written once, gains by wider row segments earlier: 16 lines up
+// to n = 137 with 8192 lines or more (100^3 y 36 -> 30, 128^3 x 53 -> 50), and
+// four lines of 9-row chunks above n = 313 (320^3 x 1214 -> 928, y 1512 -> 998,
+// z 1507 -> 1004; 512 x 200 x 200 x 518 -> 397).
 int default_shape(int prog, int dir, const int n3[3], int ndir) {
   const int n = n3[dir];
   const long long lines = (long long)(n3[0] + 1) * (n3[1] + 1) * (n3[2] + 1) / (n + 1);
   const bool few = lines < 1024;
   if (n <= 73 && !few) return 2;
+  if (n <= 137 && prog == F_ONLY && lines >= 8192) return 10;
   if (n <= 153 && !few) return 4;
   if (n <= 313) {
     if (few) return dir == 0 ? 8 : 7;
@@ -461,6 +466,7 @@ int default_shape(int prog, int dir, const int n3[3], int ndir) {
     if (n <= 281 && (prog == F_ONLY || prog == V_MID || prog == V_LAST_RHS)) return 3;
     return 5;
   }
+  if (prog == F_ONLY && !few) return 1;
   if (dir == 0) return 12;
   return few || ndir == 2 ? 1 : 11;
 }

@@ -1387,9 +1387,13 @@ void field_layout(const astr_hip_config& cfg, FlowArgs& a) {
   // rows start on a cache line of 128 bytes, or, from 400 000 points on, on half
   // of one: there the passes are bound by bytes and shorter rows are fewer
   // (129^3 3.7% and 257^3 1% of a step, 97x81x64 1%), below it by latency and
-  // by requests (33^3 1.4% slower with half lines, 98x62x46 0.7%)
+  // by requests (33^3 1.4% slower with half lines, 98x62x46 0.7%).  Between 161
+  // and 301 points a side the two differ by less than 1% either way; rows past
+  // 314 points, where half a line is 2% of a row at most and the passes take
+  // fewer lines at a time, lose by it (321^3 a step 2.2%, the filter sweeps
+  // 2.1%; 341^3 1.8% and 3.2%)
   const long long points = (long long)(cfg.im + 1) * (cfg.jm + 1) * (cfg.km + 1);
-  const int unit = points < 400000 ? 16 : 8;
+  const int unit = points < 400000 || cfg.im > 313 ? 16 : 8;
   a.pitch = (cfg.im + unit) / unit * unit;
   a.plane = (long long)a.pitch * (cfg.jm + 1);
   a.trash = (int)(a.plane * (cfg.km + 1));

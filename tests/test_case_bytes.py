@@ -1,5 +1,5 @@
 """The memory a case is admitted with is that of the layout it is created with,
-on both sides of the row padding's limit (400 000 points)."""
+on both sides of the row padding's limits (400 000 points, rows of 314)."""
 import ctypes as C
 
 import pytest
@@ -10,6 +10,7 @@ from astr_amd import serve as S
 # (configuration, points, row pitch, fields): 72 x 73 x 75 points are 394 200, 74 x 73 x 75 are 405 150
 CASES = [(A.tgv_config(32), 33 * 33, 48, 37), (A.tgv_config(71, 72, 74), 73 * 75, 80, 37),
          (A.tgv_config(73, 72, 74), 73 * 75, 80, 37), (A.tgv_config(128), 129 * 129, 136, 37),
+         (A.tgv_config(313, 40, 40), 41 * 41, 320, 37), (A.tgv_config(320, 40, 40), 41 * 41, 336, 37),
          (A.vortex_config(64), 65, 80, 37), (A.main_config(128), 129 * 129, 136, 42)]
 
 

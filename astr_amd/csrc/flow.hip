@@ -967,19 +967,9 @@ __global__ __launch_bounds__(256) void k_qswap_box(FlowArgs a) {
 
 // updatefvar (fludyna.F90:191-242): rho, u, v, w, p, T of q at every computed
 // point into the stored primitives
-__global__ void k_updatefvar(FlowArgs a) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y, k = blockIdx.z;
-  if (i > a.n[0]) return;
-  const long long o = (long long)k * a.plane + (long long)j * a.pitch + i;
-  const long long fs = a.fs;
-  const Prim P = prim_of(a, a.q[o], a.q[fs + o], a.q[2 * fs + o], a.q[3 * fs + o], a.q[4 * fs + o]);
-  a.pr[o] = P.r;
-  a.pr[fs + o] = P.u;
-  a.pr[2 * fs + o] = P.v;
-  a.pr[3 * fs + o] = P.w;
-  a.pr[4 * fs + o] = P.p;
-  a.pr[5 * fs + o] = P.t;
+hipError_t fvar_of_q(const FlowArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(k_fvar, fvar_grid(a), dim3(256), 0, st, a, a.q);
+  return hipGetLastError();
 }
 }  // namespace
 
@@ -1202,8 +1192,7 @@ int build_tables(astr_hip_ctx* c) {
 
 // updatefvar into the stored primitives (main path)
 int updatefvar_dev(astr_hip_ctx* c) {
-  hipLaunchKernelGGL(k_updatefvar, pt_grid(c->a), dim3(64), 0, c->stream, c->a);
-  HIP_OK(hipGetLastError());
+  HIP_OK(fvar_of_q(c->a, c->stream));
   c->halo_valid = false;
   return 0;
 }
@@ -1225,8 +1214,7 @@ int qswap_main(astr_hip_ctx* c, bool average) {
     HIP_OK(hipGetLastError());
     // a 2-D case still takes the k step, see below
     if (a.ndir == 2) {
-      hipLaunchKernelGGL(k_updatefvar, pt_grid(a), dim3(64), 0, c->stream, a);
-      HIP_OK(hipGetLastError());
+      HIP_OK(fvar_of_q(a, c->stream));
     }
     c->halo_valid = true;
     return 0;
@@ -1264,8 +1252,7 @@ int qswap_main(astr_hip_ctx* c, bool average) {
     // its slabs -hm..0 and 0..hm hold the plane k = 0, so q2fvar refreshes
     // the primitives of every computed point
     if (a.ndir == 2) {
-      hipLaunchKernelGGL(k_updatefvar, pt_grid(a), dim3(64), 0, c->stream, a);
-      HIP_OK(hipGetLastError());
+      HIP_OK(fvar_of_q(a, c->stream));
     }
   }
   c->halo_valid = true;

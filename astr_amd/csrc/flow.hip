@@ -447,7 +447,10 @@ hipError_t launch_pass(int shape, int prog, int minb, const FlowArgs& a, int dir
 // system needs once a pass is bound by it (256^3 y gradients 380 on 8 lines,
 // 436 on 4, 593 on 2), in the register footprint the pass has room for.  With
 // fewer lines than fill the chip with such tiles, two lines per workgroup
-// (2-D 300 x 181: RK pass 23 against 32).  The filter sweep, whose five fields
+// (2-D 300 x 181: RK pass 23 against 32); three-dimensional cases have 144 lines
+// at least and lose by it up to 73 points (24^3 a step 157 against 234, 30^3
+// 167 against 274, in batches four times that), along y and z up to 153 (20 x
+// 100 x 20 190 against 204; 100 x 20 x 20 along x 190 against 187).  The filter sweep, whose five fields
 // are read and written once, gains by wider row segments earlier: 16 lines up
 // to n = 137 with 8192 lines or more (100^3 y 36 -> 30, 128^3 x 53 -> 50), and
 // four lines of 9-row chunks above n = 313 (320^3 x 1214 -> 928, y 1512 -> 998,
@@ -456,9 +459,9 @@ int default_shape(int prog, int dir, const int n3[3], int ndir) {
   const int n = n3[dir];
   const long long lines = (long long)(n3[0] + 1) * (n3[1] + 1) * (n3[2] + 1) / (n + 1);
   const bool few = lines < 1024;
-  if (n <= 73 && !few) return 2;
+  if (n <= 73 && (!few || ndir == 3)) return 2;
   if (n <= 137 && prog == F_ONLY && lines >= 8192) return 10;
-  if (n <= 153 && !few) return 4;
+  if (n <= 153 && (!few || (ndir == 3 && (dir > 0 || lines >= 640)))) return 4;
   if (n <= 313) {
     if (few) return dir == 0 ? 8 : 7;
     if (dir == 0) return prog == F_ONLY && n <= 281 ? 6 : 8;

@@ -437,7 +437,12 @@ hipError_t launch_pass(int shape, int prog, int minb, const FlowArgs& a, int dir
   }
 }
 
-// The launch shape a pass uses until tuned, from sweeps of every shape over
+long long lines_along(const int n3[3], int dir) {
+  return (long long)(n3[0] + 1) * (n3[1] + 1) * (n3[2] + 1) / (n3[dir] + 1);
+}
+
+// The launch shape a pass of so many lines (a case's own, or those of the cases
+// that share a launch) uses until tuned, from sweeps of every shape over
 // boxes of side 32..256 and 64^2..512^2 (microseconds per launch in brackets).
 // The shortest chunks that hold the line win wherever the kernels wait on
 // their own chains, which is everywhere below about 150 points a side: the 16 x 5
@@ -450,14 +455,14 @@ hipError_t launch_pass(int shape, int prog, int minb, const FlowArgs& a, int dir
 // (2-D 300 x 181: RK pass 23 against 32); three-dimensional cases have 144 lines
 // at least and lose by it up to 73 points (24^3 a step 157 against 234, 30^3
 // 167 against 274, in batches four times that), along y and z up to 153 (20 x
-// 100 x 20 190 against 204; 100 x 20 x 20 along x 190 against 187).  The filter sweep, whose five fields
-// are read and written once, gains by wider row segments earlier: 16 lines up
-// to n = 137 with 8192 lines or more (100^3 y 36 -> 30, 128^3 x 53 -> 50), and
+// 100 x 20 190 against 204), along x from 640 lines on (80 x 28 x 28, 841 lines,
+// 209 against 232; 100 x 20 x 20, 441 lines, 190 against 187).  The filter
+// sweep, whose five fields are read and written once, gains by wider row
+// segments earlier: 16 lines up to n = 137 with 8192 lines or more (100^3 y 36 -> 30, 128^3 x 53 -> 50), and
 // four lines of 9-row chunks above n = 313 (320^3 x 1214 -> 928, y 1512 -> 998,
 // z 1507 -> 1004; 512 x 200 x 200 x 518 -> 397).
-int default_shape(int prog, int dir, const int n3[3], int ndir) {
+int default_shape(int prog, int dir, const int n3[3], int ndir, long long lines) {
   const int n = n3[dir];
-  const long long lines = (long long)(n3[0] + 1) * (n3[1] + 1) * (n3[2] + 1) / (n + 1);
   const bool few = lines < 1024;
   if (n <= 73 && (!few || ndir == 3)) return 2;
   if (n <= 137 && prog == F_ONLY && lines >= 8192) return 10;
@@ -490,6 +495,7 @@ struct astr_hip_ctx {
   int shape[kNumProgs][3];
   int minb[kNumProgs][3];
   float tuned_ms[kNumProgs][3];
+  bool chosen[kNumProgs][3] = {};  // by a caller or an autotuner; otherwise the defaults
   // set and read back by astr_hip_set/get_last_split; the last gradient pass
   // has one form
   int split_last = 0;
@@ -1452,7 +1458,7 @@ int astr_hip_create(const astr_hip_config* cfg, astr_hip_ctx** out) {
   for (int d = 0; d < a.ndir; d++) {
     if (pick_shape(a.n[d]) < 0) { delete c; return fail("no launch shape fits this line length"); }
     for (int pr = 0; pr < kNumProgs; pr++) {
-      int use = default_shape(pr, d, a.n, a.ndir);
+      int use = default_shape(pr, d, a.n, a.ndir, lines_along(a.n, d));
       for (int k = 0; k < kNumShapes && !selection_ok(use, pr, a.n[d], c->device); k++)
         use = k;
       if (!selection_ok(use, pr, a.n[d], c->device)) { delete c; return fail("no launch shape fits the LDS"); }
@@ -1924,6 +1930,7 @@ int astr_hip_autotune(astr_hip_ctx* c, int reps) {
             best = ms;
             c->shape[pr][d] = sh;
             c->minb[pr][d] = mb;
+            c->chosen[pr][d] = true;
             c->tuned_ms[pr][d] = ms;
           }
         }
@@ -1982,6 +1989,7 @@ int astr_hip_set_pass_config(astr_hip_ctx* c, int prog, int dir, int shape, int 
   if (minb < 1 || minb > kMinbVariants) return fail("register budget must be 1 or 2");
   c->shape[prog][dir] = shape;
   c->minb[prog][dir] = minb;
+  c->chosen[prog][dir] = true;
   c->tuned_ms[prog][dir] = 0.f;
   return 0;
 }
@@ -2418,6 +2426,28 @@ void drop_graph(astr_hip_batch* b) {
   b->graph_valid = false;
 }
 
+// The launch shape and register budget a case's pass takes in a batch: the
+// case's own, but for two-dimensional cases with lines of at most 153 points
+// that nobody chose a shape for.  Those share a launch, so the default for the
+// lines of all of them serves: by each case's own count of lines, 32 cases of
+// 64 x 64 took one- and two-line tiles (a step 342 us; 189 with 16-line tiles;
+// 32 of 150 x 150 655 -> 405), which win only alone (64 x 64 105 us against 113).
+// Three-dimensional cases do not have that rule, and longer lines have the same
+// chunks either way.
+struct Selection {
+  int shape, minb;
+};
+Selection batch_selection(const astr_hip_batch* b, const astr_hip_ctx* c, int prog, int d) {
+  if (!c->chosen[prog][d] && c->a.ndir == 2 && c->a.n[d] <= 153) {
+    long long lines = 0;
+    for (const astr_hip_ctx* o : b->cases)
+      if (o->a.ndir == 2) lines += lines_along(o->a.n, d);
+    const int sh = default_shape(prog, d, c->a.n, c->a.ndir, lines);
+    if (selection_ok(sh, prog, c->a.n[d], c->device)) return {sh, default_minb(sh)};
+  }
+  return {c->shape[prog][d], c->minb[prog][d]};
+}
+
 // group the cases of every slot by (program, shape, budget) from each case's
 // launch selection; upload the groups' case arrays and tile offsets
 int build_groups(astr_hip_batch* b) {
@@ -2430,7 +2460,7 @@ int build_groups(astr_hip_batch* b) {
       astr_hip_ctx* c = b->cases[i];
       const int prog = slot_prog(kind, d, c->a.ndir);
       if (prog < 0) continue;
-      const int sh = c->shape[prog][d], mb = c->minb[prog][d];
+      const auto [sh, mb] = batch_selection(b, c, prog, d);
       BatchGroup* g = nullptr;
       for (auto& h : here)
         if (h.prog == prog && h.shape == sh && h.minb == mb) g = &h;
@@ -2499,7 +2529,7 @@ int upload_jobs(astr_hip_batch* b) {
   for (int i = 0; i < nc; i++) {
     astr_hip_ctx* c = b->cases[i];
     jobs[i].part = c->stats_part;
-    jobs[i].ntiles = tiles_of(c->a.n, 0, kShapes[c->shape[V_MID][0]].TL);
+    jobs[i].ntiles = tiles_of(c->a.n, 0, kShapes[batch_selection(b, c, V_MID, 0).shape].TL);
     jobs[i].scale = c->ke_scale;
     jobs[i].out = b->d_stats + kBatchStats * (size_t)i * b->stats_cap;
   }
@@ -2745,6 +2775,7 @@ int astr_hip_batch_autotune(astr_hip_batch* b, int reps) {
         for (int i : cl.second) {
           b->cases[i]->shape[prog][d] = bsh;
           b->cases[i]->minb[prog][d] = bmb;
+          b->cases[i]->chosen[prog][d] = true;
           b->cases[i]->tuned_ms[prog][d] = best / reps;
           // the batch's stress pass computes the x gradients; so does the
           // case's own with both on one shape (own_gradx)

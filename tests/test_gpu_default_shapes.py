@@ -17,7 +17,7 @@ def err(a, b):
 
 # n = 137 | 138 and 313 | 314 with 8192 lines or more (137 x 91 x 90 along x) or 1024 or more
 # and 3-D cases of fewer than 1024 lines along a direction
-@pytest.mark.parametrize("dims", [(12, 12, 12), (30, 31, 30), (153, 12, 14), (154, 12, 14), (12, 73, 74), (137, 91, 90), (138, 91, 90), (137, 90, 88), (40, 137, 200), (36, 200, 137), (313, 40, 36),
+@pytest.mark.parametrize("dims", [(12, 12, 12), (30, 31, 30), (153, 12, 14), (154, 12, 14), (12, 73, 74), (80, 24, 24), (80, 25, 24), (137, 91, 90), (138, 91, 90), (137, 90, 88), (40, 137, 200), (36, 200, 137), (313, 40, 36),
                                   (314, 40, 36), (30, 314, 36), (32, 34, 314), (314, 30, 0), (400, 30, 0)])
 def test_filter_and_step_on_default_shapes(dims):
     s = O.OracleState(O.tgv_cfg(*dims, dt=2e-4))

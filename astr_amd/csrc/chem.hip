@@ -310,7 +310,7 @@ constexpr int kCellBlock = 64;
 // reaction are 760 of them), 64 us of issue for 2^20 cells against 38 us for
 // the cells' 176 bytes.  124 registers leave four wavefronts per SIMD to cover
 // the scalar loads of the reaction records (96 spill: 220 us; three: 93 us).
-// 2^20 cells 178 -> 88 us, 1000 cells 29 -> 13 us against divisions in the
+// 2^20 cells 190 -> 88 us, 1000 cells 29 -> 12 us against divisions in the
 // thermodynamics, indexed sums and the library's exponential; 8 species in
 // the NSMAX instance 253 -> 129 us, with general orders 264 -> 168 us.
 template <int NSA, bool UNIT>
@@ -764,8 +764,8 @@ __device__ __forceinline__ double conc_pow_d(double c, double nu) {
 //   dq_r/dT   = [M] (fwd dln kf/dT - rev dln kr/dT) - s_r / T,
 //   dln kf/dT = b/T + E/(R T^2),  dln kr/dT = dln kf/dT - dH_r/(R T^2) + dnu_r/T;
 // then f_Y = w W / rho and f_T = -sum_k h_k f_Yk / cp give the column.  f0 is
-// f(y).  Every column is computed alone, so a team evaluates them on separate
-// lanes with the arithmetic of the one-thread kernel's sequential loop.
+// f(y).  The one-thread kernel's form, a column at a time; the team forms its
+// columns from the reactions' derivatives (Team::matrix).
 template <int NS>
 __device__ __forceinline__ void reactor_jac_col(const Mech* __restrict__ M, double p, const double (&yv)[NS + 1],
                                                 const double (&f0)[NS + 1], int j, double (&col)[NS + 1]) {
@@ -864,11 +864,11 @@ __device__ __forceinline__ void reactor_jac_col(const Mech* __restrict__ M, doub
   col[0] = -(dH + f0[0] * dcp) / cp;
 }
 
-// solve with LU factors in LDS, element (r,c) at a[(r*N + c)*S]: S = 64 for
-// the one-thread kernel's interleaved matrices, 1 for a team's own matrix
+// solve with LU factors in LDS, element (r,c) of this thread's matrix at
+// a[(r*N + c)*64]: the matrices of a wavefront's reactors are interleaved.
 // The factorization swaps whole rows (its stored multipliers included), so
 // every interchange is applied to b before the unit lower triangular solve.
-template <int N, int S = 64>
+template <int N>
 __device__ __forceinline__ void lu_solve_n(const double* a, const int (&piv)[N], double (&b)[N]) {
 #pragma unroll
   for (int k = 0; k < N; k++) {
@@ -885,20 +885,20 @@ __device__ __forceinline__ void lu_solve_n(const double* a, const int (&piv)[N],
 #pragma unroll
   for (int k = 0; k < N; k++) {
 #pragma unroll
-    for (int r = k + 1; r < N; r++) b[r] -= a[(r * N + k) * S] * b[k];
+    for (int r = k + 1; r < N; r++) b[r] -= a[(r * N + k) * 64] * b[k];
   }
 #pragma unroll
   for (int k = N - 1; k >= 0; k--) {
     double sum = b[k];
 #pragma unroll
-    for (int c = k + 1; c < N; c++) sum -= a[(k * N + c) * S] * b[c];
-    b[k] = sum / a[(k * N + k) * S];
+    for (int c = k + 1; c < N; c++) sum -= a[(k * N + c) * 64] * b[c];
+    b[k] = sum / a[(k * N + k) * 64];
   }
 }
 
-// RODAS4's six stages from the factored A = I - gamma h J (in LDS, stride S)
+// RODAS4's six stages from the factored A = I - gamma h J (in LDS)
 // and f0 = f(y): the new state into ynew, the scaled error as the result
-template <int NS, int S>
+template <int NS>
 __device__ __forceinline__ double ro_stages(const Mech* __restrict__ M, double p, double h, const double* a,
                                             const int (&piv)[NS + 1], const double (&y)[NS + 1],
                                             const double (&f0)[NS + 1], double (&ynew)[NS + 1], double rtol,
@@ -908,7 +908,7 @@ __device__ __forceinline__ double ro_stages(const Mech* __restrict__ M, double p
   const double gh = kRoGamma * h;
 #pragma unroll
   for (int k = 0; k < N; k++) U[0][k] = f0[k];
-  lu_solve_n<N, S>(a, piv, U[0]);
+  lu_solve_n<N>(a, piv, U[0]);
 #pragma unroll
   for (int k = 0; k < N; k++) U[0][k] = gh * U[0][k];
 #pragma unroll
@@ -933,7 +933,7 @@ __device__ __forceinline__ double ro_stages(const Mech* __restrict__ M, double p
       for (int j = 0; j < s; j++) c += (kRoC[s - 1][j] / h) * U[j][k];
       U[s][k] = f1[k] + c;
     }
-    lu_solve_n<N, S>(a, piv, U[s]);
+    lu_solve_n<N>(a, piv, U[s]);
 #pragma unroll
     for (int k = 0; k < N; k++) U[s][k] = gh * U[s][k];
   }
@@ -1010,7 +1010,7 @@ __global__ __launch_bounds__(64) void k_reactor_n(const Mech* __restrict__ M, Re
       }
     }
     double err = 2.0;
-    if (ok) err = ro_stages<NS, 64>(M, p, h, a, piv, y, f0, yt, rtol, atol);
+    if (ok) err = ro_stages<NS>(M, p, h, a, piv, y, f0, yt, rtol, atol);
     if (err <= 1.0) {
       t += h;
 #pragma unroll

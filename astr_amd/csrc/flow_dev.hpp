@@ -64,7 +64,7 @@ struct FlowArgs {
   int bnd[3];
   const double* met;
   // main path: the convective term is the upwind-biased one (upwind.hip),
-  // which the gradient passes then leave out
+  // which the flux passes then leave out
   int uwd;
   // main path: the RK pass also applies the next stage's filterq sweep along
   // its direction to the new q, after updatefvar took the primitives

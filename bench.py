@@ -539,7 +539,6 @@ def main():
         tune_s = time.perf_counter() - t0
     launch = {f"{k[0]}_{k[1]}": {"shape": A.SHAPES[v[0]], "minb": v[1]}
               for k, v in f.pass_configs().items()}
-    launch["last_pass_split"] = f.split_last
     if args.warmup:
         f.rk3(args.warmup, stats=True)
     f.sync()

@@ -2427,25 +2427,31 @@ void drop_graph(astr_hip_batch* b) {
 }
 
 // The launch shape and register budget a case's pass takes in a batch: the
-// case's own, but for two-dimensional cases with lines of at most 153 points
-// that nobody chose a shape for.  Those share a launch, so the default for the
-// lines of all of them serves: by each case's own count of lines, 32 cases of
-// 64 x 64 took one- and two-line tiles (a step 342 us; 189 with 16-line tiles;
-// 32 of 150 x 150 655 -> 405), which win only alone (64 x 64 105 us against 113).
-// Three-dimensional cases do not have that rule, and longer lines have the same
-// chunks either way.
+// case's own, but where every two-dimensional case that nobody chose a shape for
+// has lines of at most 153 points.  Those share a launch, so the default for
+// the longest of their lines and for all of them together serves: by each case's
+// own count of lines, 32 cases of 64 x 64 took one- and two-line tiles (a step
+// 342 us; 189 with 16-line tiles; 32 of 150 x 150 655 -> 405), which win only
+// alone (64 x 64 105 us against 113).  With longer lines among them the cases
+// stay on the small tiles: a shape per length would split the launch (sides 64
+// to 256 mixed, 32 cases 737 us, split 879).  Three-dimensional cases do not
+// have that rule.
 struct Selection {
   int shape, minb;
 };
 Selection batch_selection(const astr_hip_batch* b, const astr_hip_ctx* c, int prog, int d) {
-  if (!c->chosen[prog][d] && c->a.ndir == 2 && c->a.n[d] <= 153) {
-    long long lines = 0;
-    for (const astr_hip_ctx* o : b->cases)
-      if (o->a.ndir == 2) lines += lines_along(o->a.n, d);
-    const int sh = default_shape(prog, d, c->a.n, c->a.ndir, lines);
-    if (selection_ok(sh, prog, c->a.n[d], c->device)) return {sh, default_minb(sh)};
+  const Selection own{c->shape[prog][d], c->minb[prog][d]};
+  if (c->chosen[prog][d] || c->a.ndir != 2) return own;
+  long long lines = 0;
+  const FlowArgs* longest = &c->a;
+  for (const astr_hip_ctx* o : b->cases) {
+    if (o->a.ndir != 2 || o->chosen[prog][d]) continue;
+    lines += lines_along(o->a.n, d);
+    if (o->a.n[d] > longest->n[d]) longest = &o->a;
   }
-  return {c->shape[prog][d], c->minb[prog][d]};
+  if (longest->n[d] > 153) return own;
+  const int sh = default_shape(prog, d, longest->n, 2, lines);
+  return selection_ok(sh, prog, c->a.n[d], c->device) ? Selection{sh, default_minb(sh)} : own;
 }
 
 // group the cases of every slot by (program, shape, budget) from each case's

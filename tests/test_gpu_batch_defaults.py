@@ -54,3 +54,18 @@ def test_batch_of_a_mixed_size_keeps_each_case(n=9):
         g.rk3(2, stats=False)
     check_equal(flows, alone)
     b.close()
+
+
+@pytest.mark.parametrize("sides,groups", [((64, 100, 73, 150), 4), ((64, 100, 73, 154), 4), ((40, 73, 66, 50), 4)])
+def test_cases_of_several_lengths_share_each_launch(sides, groups):
+    """Nobody chose a shape: cases of different lengths stay one group per slot."""
+    flows, alone = [[A.Flow(A.vortex_config(n)) for n in sides for _ in range(4)] for _ in range(2)]
+    for f in flows + alone:
+        f.init_vortex()
+    b = A.Batch(flows)
+    assert b.info()["groups"] == groups
+    b.rk3(2, stats=False)
+    for f in alone:
+        f.rk3(2, stats=False)
+    check_equal(flows, alone)
+    b.close()

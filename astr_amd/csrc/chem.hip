@@ -305,7 +305,7 @@ constexpr int kCellBlock = 64;
 
 // NSA: the per-cell arrays' size.  NSA = NSMAX serves any mechanism (up to
 // M->ns); an instance with NSA = the mechanism's species count has every loop
-// over the species unrolled.  Bound by FP64 arithmetic: about 2400 vector
+// over the species unrolled.  Bound by FP64 arithmetic: about 2500 vector
 // instructions a cell with 9 species and 19 reactions (two exponentials per
 // reaction are 760 of them), 64 us of issue for 2^20 cells against 38 us for
 // the cells' 176 bytes.  124 registers leave four wavefronts per SIMD to cover

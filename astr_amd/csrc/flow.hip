@@ -458,9 +458,9 @@ long long lines_along(const int n3[3], int dir) {
 // 100 x 20 190 against 204), along x from 640 lines on (80 x 28 x 28, 841 lines,
 // 209 against 232; 100 x 20 x 20, 441 lines, 190 against 187).  The filter
 // sweep, whose five fields are read and written once, gains by wider row
-// segments earlier: 16 lines up to n = 137 with 8192 lines or more (100^3 y 36 -> 30, 128^3 x 53 -> 50), and
-// four lines of 9-row chunks above n = 313 (320^3 x 1214 -> 928, y 1512 -> 998,
-// z 1507 -> 1004; 512 x 200 x 200 x 518 -> 397).
+// segments earlier: 16 lines up to n = 137 with 8192 lines or more (100^3 y 36
+// -> 30, 128^3 x 53 -> 50), and four lines of 9-row chunks above n = 313 (320^3 x
+// 1214 -> 928, y 1512 -> 998, z 1507 -> 1004; 512 x 200 x 200 x 518 -> 397).
 int default_shape(int prog, int dir, const int n3[3], int ndir, long long lines) {
   const int n = n3[dir];
   const bool few = lines < 1024;

@@ -1136,7 +1136,7 @@ constexpr int pass_fields(int prog) {
 // 11.7 -> 8.4, 16.1 -> 15.5, 33 -> 39; gradients 10.3 -> 7.6, 13.5 -> 12.2,
 // 23.8 -> 25.7, and where they form the pressure too 10.3 -> 9.2, 13.8 -> 16.5.
 // The RK pass solves twice per component and gains at every size (miniapp
-// 33^3 23.5 -> 12, 129^3 132 -> 129, 257^3 1080 -> 1034), so it has that
+// 33^3 23.5 -> 12, 129^3 132 -> 129; 257^3 1113 in a step), so it has that
 // form only.  The general-grid kernels follow the same limits: with them, and
 // one solve of each flux difference instead of one per part, a step of a
 // wall-bounded stretched grid takes at 32^3 985 -> 485 us, 96x80x64 2002 ->

@@ -67,7 +67,7 @@ typedef struct astr_hip_ctx astr_hip_ctx;
  * batch it belongs to: inside a step the state moves through q, a saved copy
  * and qrhs in turn and is back in q at the step's end.  qrhs holds the
  * right-hand side after astr_hip_rhscal and astr_hip_gradcal; after rk3 or
- * batch steps it holds an intermediate state. */
+ * batch steps and autotuning it holds an intermediate state. */
 typedef struct astr_hip_layout {
   int pitch;               /* doubles between consecutive j rows */
   long long plane;         /* doubles between consecutive k planes */

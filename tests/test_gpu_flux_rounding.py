@@ -125,6 +125,41 @@ def test_viscous_flux_adds_no_rounding_at_the_convective_size(path, dims):
         assert ratio[m] < 1.05, (m, ratio)
 
 
+def rhs_double_apart(cfg, q):
+    """The convective right-hand side's momenta in double as the reference forms
+    them: primitives, products and sums rounded one after the other, each
+    flux differentiated on its own (here in extended precision)."""
+    nd = 3 if cfg.km > 0 else 2
+    u = [q[1 + m] / q[0] for m in range(3)]
+    p = (q[4] - 0.5 * q[0] * (u[0] * u[0] + u[1] * u[1] + u[2] * u[2])) / (1.0 / (cfg.gamma - 1.0))
+    n, l = (cfg.im, cfg.jm, cfg.km), (cfg.lx, cfg.ly, cfg.lz)
+    out = np.zeros((3,) + p.shape, LD)
+    for d in range(nd):
+        for m in range(3):
+            f = q[1 + m] * u[d] + p if m == d else q[1 + m] * u[d]
+            out[m] -= derivative(f.astype(LD), 2 - d) * (LD(n[d]) / LD(l[d]))
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("main", [False, True])
+@pytest.mark.parametrize("mach", [0.5, 1.0])
+@pytest.mark.parametrize("dims", [(28, 27, 24), (150, 131, 0)])
+def test_momentum_is_as_exact_as_the_parts_apart(main, mach, dims):
+    """Where p is of the momentum flux's size, the momenta's error, that of
+    the line solves included, stays below the error that the rounded primitives
+    and fluxes of the reference's order alone leave."""
+    f = A.Flow((A.main_config if main else A.tgv_config)(*dims, mach=mach))
+    q = periodic_field(f.cfg, 8)
+    f.upload(q)
+    got = f.rhscal()[1:4] / (jacobian(f.cfg) if main else 1.0)
+    want = rhs_extended(f.cfg, q, True)[1:4]
+    plain = rhs_double_apart(f.cfg, q) - rhs_extended(f.cfg, q, False)[1:4]
+    rms = lambda e: np.sqrt((e.astype(float) ** 2).mean(axis=(1, 2, 3)))  # noqa: E731
+    for m in range(3 if dims[2] else 2):
+        assert rms(got - want)[m] <= rms(plain)[m], (m, rms(got - want), rms(plain))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("main", [False, True])
 @pytest.mark.parametrize("dims", [(28, 27, 24), (150, 131, 0)])

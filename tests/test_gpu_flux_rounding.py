@@ -85,14 +85,20 @@ def test_extended_derivative_is_sixth_order():
 
 
 def per_point_metrics(f):
-    """The uniform grid's metrics with one entry off the diagonal that is not
-    zero (and adds nothing): the passes read metrics at every point."""
+    """The uniform grid's metrics but for one entry at one point, off the
+    diagonal and large enough for the passes to read metrics at every point; it
+    reaches the three lines through the point."""
     n, l = (f.cfg.im, f.cfg.jm, f.cfg.km), (f.cfg.lx, f.cfg.ly, f.cfg.lz)
     dxi = np.zeros((3, 3) + f.shape)
     for d in range(3 if f.cfg.km else 2):
         dxi[d, d] = n[d] / l[d]
-    dxi[0, 1, 0, 0, 0] = 1e-300
+    dxi[0, 1, 0, 0, 0] = 1e-6
     f.set_metrics(np.full(f.shape, jacobian(f.cfg)), dxi)
+
+
+def off_origin(a):
+    """Without the planes through the first point."""
+    return a[:, 1:, 1:, 1:] if a.shape[1] > 1 else a[:, :, 1:, 1:]
 
 
 def jacobian(cfg):
@@ -115,6 +121,7 @@ def test_viscous_flux_adds_no_rounding_at_the_convective_size(path, dims):
         want = rhs_extended(f.cfg, q, re < 1e20)
         if path != "miniapp":  # the main path's right-hand side carries the Jacobian
             got = got / jacobian(f.cfg)
+        got, want = off_origin(got), off_origin(want)
         assert float(np.abs(got - want).max() / np.abs(want).max()) < 1e-12
         err[re] = np.sqrt(((got - want).astype(float) ** 2).mean(axis=(1, 2, 3)))
         f.close()

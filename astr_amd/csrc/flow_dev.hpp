@@ -606,8 +606,8 @@ __device__ __forceinline__ void stress_point(const FlowArgs& a, unsigned o, cons
 // MAIN: the main path's semantics (src/mainloop.F90:396-482): the gradients
 // and fluxes take the stored primitives (pr) as the last updatefvar left them
 // and their halo copies from the filtered q (qswap), the fluxes carry the
-// metrics J and dxi (convrsdcal6, diffrsdcal6), and the RK pass ends with
-// updatefvar instead of the filter.
+// metrics J and dxi (convrsdcal6, diffrsdcal6), and the RK pass is followed by
+// updatefvar (k_fvar) instead of ending with this stage's filter.
 // Each pass reads its chunk factors back from LDS before each solve instead
 // of holding them in registers, and issues a solve's accumulation loads and
 // the next solve's inputs before it, so that their latency overlaps it.
@@ -966,9 +966,10 @@ __device__ __forceinline__ void pass_body(const FlowArgs& a, const StageArgs& sa
     // carries p ~ 1/(gamma Ma^2), large against everything the derivative keeps
     // of it; f0, the pressure of the tile's first point, drops out of the
     // derivative and goes off it first.  (The reference pressure in its place
-    // would round a state of another pressure level at its own size.)  Per-point metrics have no such
-    // constant; the fused operation alone keeps their difference to one
-    // rounding at the flux's size.
+    // would round a state of another pressure level at its own size; so would
+    // f0 a point of its lines whose p is less than half of it.)  Per-point
+    // metrics have no such constant; the fused operation alone keeps their
+    // difference to one rounding at the flux's size.
     double f0 = 0.0;
     if (!uwd && !metg && (!ONE || field == dir + 1)) {
       f0 = ldg(MAIN ? a.pr + 4 * fs : a.p, tile_first<C>(a, dir, tile));
